@@ -118,6 +118,19 @@ int jf_shadow_write(const uint16_t* key, int64_t k_stride_t, int64_t k_stride_h,
                     uint16_t* k_shadow, uint16_t* v_shadow, int64_t shadow_stride_h, int64_t shadow_stride_slot,
                     int64_t num_slots, void* stream);
 
+/* The append of one layer in one launch: rows of key and value (T, H_kv, 128) bf16 quantised into the packed cache as by
+ * jf_quant_write_sym (k_zp != NULL: the keys as by jf_quant_write_int2_asym), slot_filled[slot] set to 1 where it is given
+ * (the filled-slot bookkeeping of jetfire_vllm/adapter/cache_store.py:686-759), and the rows mirrored as by
+ * jf_shadow_write where k_shadow / v_shadow are given.  slots[t] < 0 and slots[t] >= num_slots are skipped everywhere.
+ * Token rows 16-byte aligned; row strides of tokens and caches below 2^32; other callers use the separate entry points. */
+int jf_append_rows(const uint16_t* key, int64_t k_stride_t, int64_t k_stride_h, const uint16_t* value, int64_t v_stride_t,
+                   int64_t v_stride_h, const int64_t* slots, int64_t T, int H_kv, uint8_t* k_data, int64_t k_data_stride_h,
+                   int64_t k_data_stride_slot, uint16_t* k_scale, int64_t k_scale_stride_h, int64_t k_scale_stride_slot,
+                   uint16_t* k_zp, int64_t zp_stride_h, int64_t zp_stride_slot, uint8_t* v_data, int64_t v_data_stride_h,
+                   int64_t v_data_stride_slot, uint16_t* v_scale, int64_t v_scale_stride_h, int64_t v_scale_stride_slot,
+                   int64_t num_slots, int group_size, int k_nbits, int v_nbits, uint8_t* slot_filled, uint16_t* k_shadow,
+                   uint16_t* v_shadow, int64_t shadow_stride_h, int64_t shadow_stride_slot, void* stream);
+
 /* Address under which the GPU reaches a pinned host buffer (hipHostMalloc, torch's pin_memory=True), or
  * JF_ERR_ARG when host_ptr is pageable or device memory.  The reference allocates its mapped buffers itself
  * (alloc_mapped_pinned_pair, jetfire_vllm/csrc/cpu_topk_attn.cpp:972-1023); here the caller owns them. */

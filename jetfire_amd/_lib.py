@@ -24,6 +24,7 @@ SIGNATURES = {
     "jf_quant_write_sym": (I, [P, L, L, P, L, I, P, L, L, P, L, L, L, I, I, P]),
     "jf_quant_write_int4_sym_kv": (I, [P, L, L, P, L, L, P, L, I, P, L, L, P, L, L, P, L, L, P, L, L, L, I, P]),
     "jf_shadow_write": (I, [P, L, L, P, L, L, P, L, I, P, P, L, L, L, P]),
+    "jf_append_rows": (I, [P, L, L, P, L, L, P, L, I, P, L, L, P, L, L, P, L, L, P, L, L, P, L, L, L, I, I, I, P, P, P, L, L, P]),
     "jf_host_buffer_device_pointer": (I, [P, P]),
     "jf_int3_qk_scores": (I, [P, P, P, P, P, I, I, I, I, I, L, I, I, F, P, P]),
     "jf_intn_qk_scores": (I, [I, P, P, P, P, P, P, I, I, I, I, I, L, I, I, F, P, P]),

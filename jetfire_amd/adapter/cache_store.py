@@ -4,11 +4,11 @@
 Layout (kept byte for byte): `k_data (Hkv, num_slots, Pk) u8`, `k_scales (Hkv, num_slots, D/group) bf16`,
 the same for V, `slot = block * block_size + offset`; shadow `(Hkv, num_slots, D)` bf16 in pinned host memory.
 
-Appends never synchronise with the host.  The quantise-on-write kernels run on the caller's stream.  The
-shadow mirror is ONE kernel that stores the bf16 rows straight into the pinned shadow across PCIe
-(`ops.shadow_write`); it takes the place of the reference's three mirror paths: the serial host copy +
-`index_copy_` (`:686-759`), the prefill pipeline of D2H copies into pinned staging buffers and a worker
-thread's scatter (`:1075-1338`), and the graph-mode decode append with its host callback (`:531-642`).
+Appends never synchronise with the host.  An append is one launch on the caller's stream (`ops.append_rows`): both
+tensors quantised, the slots marked, and the bf16 rows of decode tokens stored straight into the pinned shadow across
+PCIe.  The mirror of a chunk is a launch of its own (`ops.shadow_write`).  The mirror takes the place of the
+reference's three mirror paths: the serial host copy + `index_copy_` (`:686-759`), the prefill pipeline of D2H copies
+into pinned staging buffers and a worker thread's scatter (`:1075-1338`), and the graph-mode decode append with its host callback (`:531-642`).
 Chunks of at least `JETFIRE_PIPELINE_MIN_TOKENS` tokens (prefill) are mirrored on a side stream so that
 the model's stream does not wait for PCIe; `flush_pending_writes` waits for those, as in the reference.
 Smaller appends (decode tokens) stay on the caller's stream, ahead of the hand-off kernel that publishes
@@ -144,9 +144,26 @@ class JetFireInt4CacheStore:
             sym[self.k_nbits](key_tok, slots, self.k_data, self.k_scales, self.group_size)
             sym[self.v_nbits](value_tok, slots, self.v_data, self.v_scales, self.group_size)
 
-    def _mirror(self, key_tok, value_tok, slots) -> None:
+    def _shadow_addresses(self) -> tuple[int, int]:
         if self._shadow_dev is None:
             self._shadow_dev = (ops.host_buffer_device_pointer(self.k_shadow), ops.host_buffer_device_pointer(self.v_shadow))
+        return self._shadow_dev
+
+    def _append(self, key_tok, value_tok, slots, *, mark: bool, mirror: bool) -> None:
+        """Quantise, mark and (optionally) mirror on the current stream: one launch where the token rows allow it."""
+        shadows = dict(k_shadow=self.k_shadow, v_shadow=self.v_shadow, shadow_dev=self._shadow_addresses()) if mirror else {}
+        if self.head_dim == ops.HEAD_DIM and ops.append_rows(
+                key_tok, value_tok, slots, self.k_data, self.k_scales, self.k_zp, self.v_data, self.v_scales, self.group_size,
+                self.k_nbits, self.v_nbits, slot_filled=self.slot_filled if mark else None, **shadows):
+            return
+        self._quantise(key_tok, value_tok, slots)
+        if mark:
+            self._slot_filled_buf.index_fill_(0, torch.where(slots >= 0, slots, self.num_slots), True)
+        if mirror:
+            self._mirror(key_tok, value_tok, slots)
+
+    def _mirror(self, key_tok, value_tok, slots) -> None:
+        self._shadow_addresses()
         ops.shadow_write(key_tok, value_tok, slots, self.k_shadow, self.v_shadow,
                          k_shadow_dev=self._shadow_dev[0], v_shadow_dev=self._shadow_dev[1])
 
@@ -159,26 +176,23 @@ class JetFireInt4CacheStore:
         n, slots, key_tok, value_tok = self._prepare(key, value, slot_mapping)
         if n <= 0:
             return 0
-        self._quantise(key_tok, value_tok, slots)
-        self._slot_filled_buf.index_fill_(0, torch.where(slots >= 0, slots, self.num_slots), True)
-        if self.shadow_enabled and _shadow_needed():
-            side = (_prefill_pipeline_enabled() and n >= _pipeline_min_tokens()
-                    and not torch.cuda.is_current_stream_capturing())
-            if side:
-                # prefill chunk: PCIe-bound, so off the model's stream (cache_store.py:1075-1110)
-                if self._mirror_stream is None:
-                    self._mirror_stream = torch.cuda.Stream(device=self.device)
-                main = torch.cuda.current_stream(self.device)
-                produced = torch.cuda.Event()
-                produced.record(main)
-                with torch.cuda.stream(self._mirror_stream):
-                    self._mirror_stream.wait_event(produced)
-                    self._mirror(key_tok, value_tok, slots)
-                    done = torch.cuda.Event()
-                    done.record(self._mirror_stream)
-                self._pending_mirrors.append((done, key_tok, value_tok, slots))
-            else:
+        mirror = self.shadow_enabled and _shadow_needed()
+        side = (mirror and n >= _pipeline_min_tokens() and _prefill_pipeline_enabled()
+                and not torch.cuda.is_current_stream_capturing())
+        self._append(key_tok, value_tok, slots, mark=True, mirror=mirror and not side)
+        if side:
+            # prefill chunk: PCIe-bound, so off the model's stream (cache_store.py:1075-1110)
+            if self._mirror_stream is None:
+                self._mirror_stream = torch.cuda.Stream(device=self.device)
+            main = torch.cuda.current_stream(self.device)
+            produced = torch.cuda.Event()
+            produced.record(main)
+            with torch.cuda.stream(self._mirror_stream):
+                self._mirror_stream.wait_event(produced)
                 self._mirror(key_tok, value_tok, slots)
+                done = torch.cuda.Event()
+                done.record(self._mirror_stream)
+            self._pending_mirrors.append((done, key_tok, value_tok, slots))
         self.written_count += n
         return n
 
@@ -203,19 +217,18 @@ class JetFireInt4CacheStore:
         if key.dtype != torch.bfloat16 or value.dtype != torch.bfloat16:
             raise RuntimeError("JetFire graph KV append requires BF16 K/V.")
         key_tok, value_tok = key[:n], value[:n]
-        self._quantise(key_tok, value_tok, slots)
-        if self.shadow_enabled and _shadow_needed():
-            if self._shadow_dev is None and torch.cuda.is_current_stream_capturing():
-                raise RuntimeError("JetFire graph KV append context was not pre-created before graph capture "
-                                   "(call warmup_graph_append first).")
-            self._mirror(key_tok, value_tok, slots)
+        mirror = self.shadow_enabled and _shadow_needed()
+        if mirror and self._shadow_dev is None and torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("JetFire graph KV append context was not pre-created before graph capture "
+                               "(call warmup_graph_append first).")
+        self._append(key_tok, value_tok, slots, mark=False, mirror=mirror)
         return n
 
     def warmup_graph_append(self, max_batch_size: int) -> None:
         """Everything `write_slots_graph` may not do while a graph is being captured
         (`cache_store.py:411-419`): here only the look-up of the shadows' device-visible addresses."""
         if max_batch_size > 0 and self.shadow_enabled and self._shadow_dev is None:
-            self._shadow_dev = (ops.host_buffer_device_pointer(self.k_shadow), ops.host_buffer_device_pointer(self.v_shadow))
+            self._shadow_addresses()
 
     def flush_pending_writes(self) -> None:
         """Wait until every mirror launched on the side stream has landed in the shadow, so that the host may

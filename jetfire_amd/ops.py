@@ -234,6 +234,47 @@ def unpack(data, scales, group_size: int = 128, nbits: int = 4, zps=None):
     return out.view(*lead, HEAD_DIM)
 
 
+def append_rows(key_tok, value_tok, slot_idx, k_data, k_scales, k_zp, v_data, v_scales, group_size: int, k_nbits: int,
+                v_nbits: int, slot_filled=None, k_shadow=None, v_shadow=None, shadow_dev=(None, None)) -> bool:
+    """The append of one layer in one launch (jf_append_rows): K and V quantised into the cache (k_zp: asymmetric INT2
+    keys), the slots marked in `slot_filled` (bool, (num_slots,)), the rows mirrored into the pinned shadows when they
+    are given (`shadow_dev`: their device-visible addresses).  Slots outside the cache are skipped.  False, with nothing
+    done, for operands the kernel does not take (rows that are not 16-byte aligned); the separate operators do."""
+    T, H_kv, D = key_tok.shape
+    _check(key_tok.is_cuda and value_tok.is_cuda and key_tok.dtype == torch.bfloat16 and value_tok.dtype == torch.bfloat16,
+           "tokens must be bf16 on the GPU")
+    _check(D == HEAD_DIM and value_tok.shape == key_tok.shape, "key/value tokens must both be (T, H_kv, 128)")
+    _check(slot_idx.is_cuda and slot_idx.dtype == torch.int64 and slot_idx.shape == (T,) and slot_idx.is_contiguous(),
+           "slots must be contiguous (T,) int64")
+    kst, vst = key_tok.stride(), value_tok.stride()
+    kds, kss, vds, vss = k_data.stride(), k_scales.stride(), v_data.stride(), v_scales.stride()
+    kp, vp = key_tok.data_ptr(), value_tok.data_ptr()
+    if (kst[2] != 1 or vst[2] != 1 or (kp | vp) & 15 or (kst[0] | kst[1] | vst[0] | vst[1]) & 7
+            or not all(0 <= n < 1 << 32 for n in (kst[0], vst[0], kds[1], kss[1], vds[1], vss[1]))):
+        return False
+    S, ng = k_data.size(1), D // group_size
+    for d, s, ds, ss, bits in ((k_data, k_scales, kds, kss, k_nbits), (v_data, v_scales, vds, vss, v_nbits)):
+        _check(d.dtype == torch.uint8 and s.dtype == torch.bfloat16, "cache must be uint8 data + bf16 scales")
+        _check(d.shape == (H_kv, S, D * bits // 8) and ds[2] == 1 and s.shape == (H_kv, S, ng) and (ng == 1 or ss[2] == 1),
+               "bad cache shape")
+    zs = (0, 0) if k_zp is None else k_zp.stride()
+    _check(k_zp is None or (k_zp.dtype == torch.bfloat16 and k_zp.shape == k_scales.shape), "bad zero-point shape")
+    _check(slot_filled is None or (slot_filled.dtype == torch.bool and slot_filled.shape == (S,) and slot_filled.is_contiguous()),
+           "slot_filled must be (num_slots,) bool")
+    sh = (0, 0)
+    if k_shadow is not None:
+        _check(k_shadow.shape == (H_kv, S, D) and v_shadow.shape == k_shadow.shape and k_shadow.dtype == torch.bfloat16
+               and v_shadow.dtype == torch.bfloat16 and k_shadow.stride() == v_shadow.stride() and k_shadow.stride(2) == 1,
+               "shadows must be (H_kv, num_slots, 128) bf16 host tensors")
+        sh = k_shadow.stride()
+    _lib.check(_lib.load().jf_append_rows(
+        kp, kst[0], kst[1], vp, vst[0], vst[1], slot_idx.data_ptr(), T, H_kv,
+        k_data.data_ptr(), kds[0], kds[1], k_scales.data_ptr(), kss[0], kss[1], _ptr(k_zp), zs[0], zs[1],
+        v_data.data_ptr(), vds[0], vds[1], v_scales.data_ptr(), vss[0], vss[1], S, group_size, k_nbits, v_nbits,
+        _ptr(slot_filled), *(shadow_dev if k_shadow is not None else (None, None)), sh[0], sh[1], _stream(key_tok)))
+    return True
+
+
 def host_buffer_device_pointer(t: torch.Tensor) -> int:
     """Address under which the GPU reaches the pinned host tensor `t`; raises for pageable memory."""
     import ctypes
