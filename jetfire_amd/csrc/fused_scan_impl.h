@@ -33,6 +33,7 @@
 //   M = max m_i, l = sum l_i e^{m_i-M}, o_hat = sum o_i e^{m_i-M} / l
 // (the split-KV combine of jetfire_vllm/csrc/fused_decode_wmma.cu:1226-1253), and computes the
 // pre-correction terms o_old_unnorm, W over the winners (jetfire_vllm/csrc/int2_softmax_v.cu:738-788).
+// Where one split covers the sequence (short contexts, large batches) launch 1 does both (template argument ONE).
 // Both kernels take a template argument MODE: the whole step, or one stage alone (Stage A: scores written out,
 // top-k, statistics; Stage B: scores and winners given, value stream; selection alone), for callers that keep the
 // reference's separate operators.
@@ -122,6 +123,7 @@ struct FusedParams {
   const int64_t* block_table;
   const int32_t* seq_lens;
   int B, H_q, H_kv, max_S, max_blocks;
+  int one_split;  // (host) the scan merges by itself: n_splits == 1 and ScanTail fits (one_split_fits)
   int g_act;  // query heads per kv-head (H_q / H_kv); the kernel's G is this rounded up to 1, 2, 4, 8 or 16
   int64_t num_slots;
   float attn_scale;
@@ -241,6 +243,17 @@ struct ScanLds {
   }
 };
 
+// LDS behind the staging area of a scan workgroup that holds the whole sequence and merges by itself (ONE): per head
+// the candidate positions, the members of the cut bucket, the winners' slots and weights, o_hat and a few words.
+template <int G, int SEG>
+struct ScanTail {
+  static constexpr int MEM = 64;  // members of the cut bucket that are ranked from a list, one per lane
+  static constexpr int INTS = ((5 + SEG + 3) * G * 4 + 15) & ~15;
+  __host__ __device__ static constexpr size_t bytes(int top_k, int kc) {
+    return INTS + (size_t)G * (D * 4 + 8 * (size_t)top_k + 8 * MEM + 2 * (size_t)kc);
+  }
+};
+
 __device__ inline float key_to_score(uint32_t key) {
   const uint32_t u = (key & 0x80000000u) ? (key & 0x7fffffffu) : ~key;
   return __builtin_bit_cast(float, u);
@@ -288,8 +301,115 @@ __device__ inline float uniform_f(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
 
+// Pre-correction terms over the winners' packed V rows, shared by the merge kernel and the scan's in-kernel merge: DW
+// lanes per row, lane dwi holds dword dwi of it (INT2, INT4) or two bytes of each of the three planes (INT3) = CPD
+// codes; a wavefront instruction covers WPI rows, sixteen wavefronts (or roles) and UNR requests per lane 256 rows.
+template <int VBITS>
+struct PreCorr {
+  static constexpr int VP = D * VBITS / 8;
+  static constexpr int DW = (VBITS == 3) ? 8 : VP / 4;
+  static constexpr int CPD = (VBITS == 3) ? 16 : 32 / VBITS;
+  static constexpr int WPI = 64 / DW;
+  static constexpr int UNR = (256 / (16 * WPI) > 0) ? 256 / (16 * WPI) : 1;
+  static __device__ inline void fetch(const uint8_t* vbase, uint32_t slot, int dwi, uint32_t& word, uint32_t& word_b) {
+    if constexpr (VBITS == 3) {  // bytes 2*dwi, 2*dwi+1 of every plane -> the 24-bit words of two 8-code groups
+      const uint8_t* row = vbase + (size_t)(slot * (uint32_t)VP) + dwi * 2;
+      const uint32_t h0 = *reinterpret_cast<const uint16_t*>(row), h1 = *reinterpret_cast<const uint16_t*>(row + 16),
+                     h2 = *reinterpret_cast<const uint16_t*>(row + 32);
+      word = ((h0 & 0xffu) << 16) | ((h1 & 0xffu) << 8) | (h2 & 0xffu);
+      word_b = ((h0 >> 8) << 16) | ((h1 >> 8) << 8) | (h2 >> 8);
+    } else {
+      word = *reinterpret_cast<const uint32_t*>(vbase + (size_t)(slot * (uint32_t)VP) + dwi * 4);
+      word_b = 0;
+    }
+  }
+  // acc[c] += ws * (code c - offset).  Byte `byte` of the dword holds its codes MSB first; channel of code c in the
+  // dword = dwi*CPD + c.  code - offset is the code with its top bit flipped, read as a two's complement field.  INT4
+  // and INT2: the field goes to the top of a nibble, and one conversion with a byte select turns the nibble into a
+  // sixteenth (INT2: a quarter) of its value; the factor, a power of two, sits in the weight, so every product is the
+  // same number.  Two instructions per code; the bit-field extract, conversion and multiply-add of the INT3 words
+  // take three, and with 256 winners for each of a workgroup's four heads the multiply-adds fill the vector ALU.
+  static __device__ inline void add(uint32_t word, uint32_t word_b, float ws, float (&acc)[CPD]) {
+    if constexpr (VBITS == 3) {
+      const uint32_t xa = word ^ 0x00924924u, xb = word_b ^ 0x00924924u;
+#pragma unroll
+      for (int c = 0; c < CPD; ++c) {
+        const int sh = 21 - 3 * (c & 7);
+        const int code = (int)((c >= 8 ? xb : xa) << (32 - VBITS - sh)) >> (32 - VBITS);
+        acc[c] = __builtin_fmaf(ws, (float)code, acc[c]);
+      }
+    } else if constexpr (VBITS == 4) {  // even codes: high nibbles
+      const float w = ws * 16.f;
+      const uint32_t x = word ^ 0x88888888u, xh = x >> 4;
+      add_bytes<0, 2>(xh, w, acc);
+      add_bytes<1, 2>(x, w, acc);
+    } else {
+      const float w = ws * 4.f;
+      const uint32_t x = word ^ 0xaaaaaaaau;
+      add_bytes<0, 4>((x >> 4) & 0x0c0c0c0cu, w, acc);
+      add_bytes<1, 4>((x >> 2) & 0x0c0c0c0cu, w, acc);
+      add_bytes<2, 4>(x & 0x0c0c0c0cu, w, acc);
+      add_bytes<3, 4>((x << 2) & 0x0c0c0c0cu, w, acc);
+    }
+  }
+  // the low nibbles of the four bytes belong to codes FIRST, FIRST + STEP, ...
+  template <int FIRST, int STEP>
+  static __device__ inline void add_bytes(uint32_t x, float w, float (&acc)[CPD]) {
+    float f0, f1, f2, f3;
+    asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(f0) : "v"(x));
+    asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(f1) : "v"(x));
+    asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(f2) : "v"(x));
+    asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(f3) : "v"(x));
+    acc[FIRST] = __builtin_fmaf(w, f0, acc[FIRST]);
+    acc[FIRST + STEP] = __builtin_fmaf(w, f1, acc[FIRST + STEP]);
+    acc[FIRST + 2 * STEP] = __builtin_fmaf(w, f2, acc[FIRST + 2 * STEP]);
+    acc[FIRST + 3 * STEP] = __builtin_fmaf(w, f3, acc[FIRST + 3 * STEP]);
+  }
+  // Sums over the WPI rows of a wavefront instruction (lanes with equal dwi): every exchange step halves the channels
+  // a lane is responsible for (the lane whose offset bit is clear keeps the lower half), so after log2(WPI) steps
+  // every lane holds the sums of two channels, acc[0] and acc[1]; -> the first of them.
+  static __device__ inline int reduce(float (&acc)[CPD], int lane) {
+    int chan = (lane % DW) * CPD;
+    auto halve = [&](auto off_c, auto n_c) {
+      constexpr int OFF = decltype(off_c)::value, N = decltype(n_c)::value;
+      const bool upper = (lane & OFF) != 0;
+#pragma unroll
+      for (int i = 0; i < N / 2; ++i) {
+        if constexpr (OFF == 32) {  // one half-wave swap serves both directions
+          const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, acc[i]), __builtin_bit_cast(uint32_t, acc[i + N / 2]), false, false);
+          acc[i] = __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
+        } else {
+          const float keep = upper ? acc[i + N / 2] : acc[i];
+          const int send = __builtin_bit_cast(int, upper ? acc[i] : acc[i + N / 2]);
+          // lane ^ 8: rotation by 8 inside the 16-lane row; lane ^ 16: swizzle inside 32 lanes
+          const int recv = (OFF == 8) ? dpp_mov<0x128, 0xf>(0, send) : __builtin_amdgcn_ds_swizzle(send, 0x401F);
+          acc[i] = keep + __builtin_bit_cast(float, recv);
+        }
+      }
+      chan += upper ? N / 2 : 0;
+    };
+    static_assert(DW == 8 || DW == 16, "eight or sixteen lanes per V row");
+    if constexpr (DW == 8) {
+      halve(std::integral_constant<int, 8>{}, std::integral_constant<int, CPD>{});
+      halve(std::integral_constant<int, 16>{}, std::integral_constant<int, CPD / 2>{});
+      halve(std::integral_constant<int, 32>{}, std::integral_constant<int, CPD / 4>{});
+    } else {
+      halve(std::integral_constant<int, 16>{}, std::integral_constant<int, CPD>{});
+      halve(std::integral_constant<int, 32>{}, std::integral_constant<int, CPD / 2>{});
+    }
+    static_assert(CPD / WPI == 2, "two channels per lane after the exchange");
+    return chan;
+  }
+};
+
 // ---------------------------------------------------------------------------------------------------
-template <int MODE, int SCHEME, int G, int NG>
+// ONE: the split is the whole sequence (n_splits == 1), so this workgroup holds everything the merge kernel would
+// fetch: it selects the winners, forms the pre-correction terms and writes the step's outputs itself, and no merge is
+// launched.  A merge launch costs 9 - 10 us whatever it merges (its loads are first touches, its intervals a chain of
+// barriers), 18 us at 1024 rows; the same steps from LDS, four wavefronts per head, cost 4 to 8 us at the end of the
+// scan.  Per layer, MI355X, graph replay: 32 sequences x 2048 positions, K3V2, 8 kv-heads, top-k 256 37.5 -> 26.7 us;
+// 32 x 464, K3V4, 4 kv-heads, top-k 64 30.1 -> 19.4; 7 x 311, K4V4, 8 kv-heads, G = 2 20.7 -> 16.5.
+template <int MODE, int SCHEME, int G, int NG, bool ONE = false>
 __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kernel(FusedParams p) {
   using Lds = ScanLds<SCHEME, G, NG>;
   constexpr bool HAS_K = (MODE == FS_FULL || MODE == FS_STAGE_A);  // key stream and phase A
@@ -368,6 +488,26 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         p.scores[(head0 + i / n_cover) * (size_t)p.max_S + s0 + (i % n_cover)] = -INFINITY;
     if constexpr (MODE == FS_STAGE_A)
       if (p.scores_only) return;
+    if constexpr (ONE) {  // no winners, zero sums
+      for (int i = tid; HAS_TOPK && i < GA * p.top_k; i += NT) {
+        p.topk_idx[head0 * p.top_k + i] = -1;
+        p.topk_slots[head0 * p.top_k + i] = -1;
+      }
+      for (int i = tid; HAS_V && i < GA * D; i += NT) {
+        p.o_hat[head0 * D + i] = 0.f;
+        p.o_old[head0 * D + i] = 0.f;
+        if (MODE == FS_FULL && p.blend_out)
+          p.blend_out[head0 * D + i] = f32_to_bf16(__builtin_fmaf(0.f, bf16_to_f32(p.blend_o_new[head0 * D + i]), 0.f) - 0.f);
+      }
+      if (tid < GA) {
+        if (HAS_V) p.W[head0 + tid] = 0.f;
+        if (p.softmax_m) {
+          p.softmax_m[head0 + tid] = 0.f;
+          p.softmax_inv_z[head0 + tid] = 0.f;
+        }
+      }
+      return;
+    }
     for (int i = tid; i < GA * D; i += NT) p.part_o[(part_base + (size_t)(i / D) * p.n_splits) * D + (i % D)] = 0.f;
     if (tid < GA) {
       p.part_m[part_base + (size_t)tid * p.n_splits] = -INFINITY;
@@ -1517,6 +1657,40 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // the constant row (75 * sum of codes) for l = 3.  Item j = (register i = j >> 2 of set i / AR, component j & 3)
   // lives at xacc[j * 64 + lane].
   int* xacc = reinterpret_cast<int*>(stage);
+  // ONE: what the in-kernel merge keeps behind the staging area (see ScanTail)
+  using Tail = ScanTail<G, SEG>;
+  const int Kcap = p.Kc;
+  [[maybe_unused]] const int K = p.top_k;
+  uint8_t* tail = stage + Lds::stage_bytes() + 64;
+  [[maybe_unused]] int* tl_cnt = reinterpret_cast<int*>(tail);              // [G] candidates of the head
+  [[maybe_unused]] int* tl_cut = tl_cnt + G;                                // [G] the cut bucket
+  [[maybe_unused]] int* tl_need = tl_cut + G;                               // [G] winners among the cut bucket's members; -1: every candidate wins
+  [[maybe_unused]] int* tl_mem = tl_need + G;                               // [G] members of the cut bucket
+  [[maybe_unused]] int* tl_nout = tl_mem + G;                               // [G] winners
+  [[maybe_unused]] int* tl_segc = tl_nout + G;                              // [G][SEG] winners per wavefront
+  [[maybe_unused]] float* tl_m = reinterpret_cast<float*>(tl_segc + G * SEG);  // [G] softmax maximum, 1 / sum, e^{m - M}
+  [[maybe_unused]] float* tl_iz = tl_m + G;
+  [[maybe_unused]] float* tl_coef = tl_iz + G;
+  [[maybe_unused]] float* tl_ohat = reinterpret_cast<float*>(tail + Tail::INTS);          // [G][D]
+  [[maybe_unused]] int* tl_wslot = reinterpret_cast<int*>(tl_ohat + G * D);               // [G][top_k] paged slot of a winner
+  [[maybe_unused]] float* tl_ww = reinterpret_cast<float*>(tl_wslot + (size_t)G * K);     // [G][top_k] its softmax weight
+  // [G][MEM] members of the cut bucket: key over inverted position, so that the larger word is the earlier winner
+  [[maybe_unused]] unsigned long long* tl_mlist = reinterpret_cast<unsigned long long*>(tl_ww + (size_t)G * K);
+  [[maybe_unused]] uint16_t* tl_list = reinterpret_cast<uint16_t*>(tl_mlist + G * Tail::MEM);  // [G][Kcap] candidate positions, ascending
+  if constexpr (ONE) {
+    if (tid < G) {
+      float l = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) l += lsum_sh[w][tid];
+      const float pm = m_sh[tid], M = isfinite(pm) ? pm : 0.f;
+      const float coef = (pm == -INFINITY) ? 0.f : __expf(pm - M);
+      l *= coef;
+      tl_m[tid] = M;
+      tl_coef[tid] = coef;
+      tl_iz[tid] = (l > 0.f) ? 1.0f / l : 0.f;
+      tl_mem[tid] = 0;
+    }
+  }
   constexpr int ACC_TOTAL = NSET * AR, ACC_HALF = (ACC_TOTAL + 1) / 2;
   bool acc_issued = false;  // (uniform) this wavefront's sums are on their way
   auto add_acc_range = [&](const int first, const int last) {  // (constants once the caller's loop is unrolled)
@@ -1556,7 +1730,14 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       const int w0 = wa[0], w1 = wa[64], w2 = wa[128];   // |sum| < 2^24: no overflow
       const long long wsum = (long long)w2 * 65536ll + (long long)w1 * 256ll + (long long)w0 + 32896ll * 64ll * (long long)nch;
       const long long tot = (long long)i2 * 65536ll + (long long)i1 * 256ll + (long long)i0 + 32896ll * (long long)cs - (long long)VOFF * wsum;
-      p.part_o[(part_base + (size_t)h * p.n_splits) * D + d] = (float)ldexp((double)tot, -E[g]);
+      const float o = (float)ldexp((double)tot, -E[g]);
+      if constexpr (ONE) {
+        const float o_hat = __builtin_fmaf(o, tl_coef[h], 0.f) * tl_iz[h];
+        p.o_hat[(head0 + h) * D + d] = o_hat;
+        tl_ohat[h * D + d] = o_hat;
+      } else {
+        p.part_o[(part_base + (size_t)h * p.n_splits) * D + d] = o;
+      }
     }
   };
 
@@ -1566,7 +1747,6 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // `cut` with count(bucket <= cut) >= Kt.  If that count fits, every position whose bucket is <= cut is
   // emitted, one wavefront per (head, segment of the split), each segment starting where the counts of the segments
   // before it end.  Otherwise (heavily tied scores) one wavefront falls back to an exact radix select over the keys.
-  const int Kcap = p.Kc;
   const int Kt = min(p.top_k, n);
   for (int hs = wave; HAS_TOPK && hs < G * SEG; hs += NW) {
     const int h = hs / SEG, seg = hs % SEG;
@@ -1615,7 +1795,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     // lane's four counts
     const unsigned long long who = __ballot((incl & 0xffff) >= Kt);
     bool ok = false;
-    int cut = 255, tot = 0, before_me = 0;
+    int cut = 255, tot = 0, before_me = 0, above_cut = 0;
     if (who != 0ull) {
       const int src = __ffsll((long long)who) - 1;
       const int ex = __builtin_amdgcn_readlane(incl - packed, src);  // exclusive sums at that lane
@@ -1630,6 +1810,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           before_me += mu;
           if (run >= Kt) {
             found = true;
+            above_cut = run - cu;
             cut = 4 * src + u;
             tot = run;
           }
@@ -1641,6 +1822,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     const float* srow = sc + h * L;
     uint32_t* ck = p.cand_key + (part_base + (size_t)h * p.n_splits) * Kcap;
     int32_t* ci = p.cand_idx + (part_base + (size_t)h * p.n_splits) * Kcap;
+    uint16_t* cl = tl_list + h * Kcap;
     if (ok) {
       // bucket(s) <= cut  <=>  not (s * ba + bb >= cut + 1): the bucket is the floor of that value clamped to
       // [0, 255]; with cut = 255 every position qualifies
@@ -1652,7 +1834,15 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       // unused slots hold key 0 (no score maps to it); the planned total is known, so the head's wavefronts
       // share the padding and its stores leave before the emission's
       const int etot = min(Kcap, tot);
-      for (int i = etot + seg * 64 + lane; i < Kcap; i += SEG * 64) ck[i] = 0u;
+      if constexpr (ONE) {
+        if (seg == 0 && lane == 0) {
+          tl_cnt[h] = etot;
+          tl_cut[h] = cut;
+          tl_need[h] = (etot == Kt) ? -1 : Kt - above_cut;
+        }
+      } else {
+        for (int i = etot + seg * 64 + lane; i < Kcap; i += SEG * 64) ck[i] = 0u;
+      }
       // Blocks of 1024 positions, 16 consecutive ones per lane: the lane's candidates are consecutive in the output,
       // so a block costs one comparison per position, one wavefront scan of the lanes' counts, and a loop over the
       // few set bits of every lane.  The lane reads its four 16-byte quads starting at quad (lane >> 2) & 3 (the
@@ -1703,8 +1893,12 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           const int i_next = (mask != 0u) ? __ffs((int)mask) - 1 : 0;
           const float s_next = lp[i_next];
           if (o < (uint32_t)Kcap) {  // the bound only matters for non-finite scores
-            ck[o] = score_key(sco);
-            ci[o] = s0 + lt + i;
+            if constexpr (ONE) {
+              cl[o] = (uint16_t)(lt + i);
+            } else {
+              ck[o] = score_key(sco);
+              ci[o] = s0 + lt + i;
+            }
           }
           ++o;
           i = i_next;
@@ -1725,7 +1919,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         acc_issued = true;
       }
       for (; t0 < te; t0 += 1024) emit_block(t0, plain);
-      if (seg == SEG - 1) {
+      if (!ONE && seg == SEG - 1) {
         if (lane == 0) p.cand_cnt[part_base + (size_t)h * p.n_splits] = min(Kcap, count);
         for (int i = count + lane; i < etot; i += 64) ck[i] = 0u;  // (only if a segment emitted less than planned)
       }
@@ -1796,23 +1990,242 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         if (above || (tie && pt < quota)) {
           const int pos = pa + min(pt, quota);
           if (pos < Kcap) {
-            ck[pos] = k;
-            ci[pos] = s0 + t;
+            if constexpr (ONE) {
+              cl[pos] = (uint16_t)t;
+            } else {
+              ck[pos] = k;
+              ci[pos] = s0 + t;
+            }
           }
         }
         count += __popcll(ma);
         base_tie += __popcll(mt);
       }
       count += min(base_tie, quota);
-      if (lane == 0) p.cand_cnt[part_base + (size_t)h * p.n_splits] = min(Kcap, count);
-      for (int i = count + lane; i < Kcap; i += 64) ck[i] = 0u;
+      if constexpr (ONE) {
+        if (lane == 0) {
+          tl_cnt[h] = min(Kcap, count);
+          tl_need[h] = -1;
+        }
+      } else {
+        if (lane == 0) p.cand_cnt[part_base + (size_t)h * p.n_splits] = min(Kcap, count);
+        for (int i = count + lane; i < Kcap; i += 64) ck[i] = 0u;
+      }
     }
   }
   if (clk && tid == 0) clk[3] = JF_CLK();
 
   if constexpr (HAS_V) {  // whatever the emission did not carry (no batch of this wavefront, a short split, the exact selection)
     if (!acc_issued) add_acc_range(0, ACC_TOTAL * 4);
-    lds_barrier();
+  }
+  if constexpr (HAS_V || ONE) lds_barrier();
+  if constexpr (ONE) {
+    if (p.softmax_m && tid < GA) {
+      p.softmax_m[head0 + tid] = tl_m[tid];
+      p.softmax_inv_z[head0 + tid] = tl_iz[tid];
+    }
+    if constexpr (HAS_V) {
+#pragma unroll
+      for (int set = 0; set < NSET; ++set) combine(set);
+    }
+    constexpr int NHS = (G * SEG + NW - 1) / NW;  // (head, segment) pairs per wavefront
+    if constexpr (HAS_TOPK) {
+      // The candidates whose bucket lies before the cut bucket win; of the cut bucket's members the `need` largest
+      // (ties: the lowest positions).  A wavefront takes a contiguous run of its head's list.
+      auto rank_word = [](uint32_t key, int pos) { return ((unsigned long long)key << 32) | (uint32_t)~pos; };
+      auto pair_of = [&](int it, int& h, int& lo, int& hi) -> int {  // -> segment, -1: nothing for this wavefront
+        const int hs = wave + it * NW;
+        h = hs / SEG;
+        if (hs >= G * SEG || h >= GA) return -1;
+        const int cnt = __builtin_amdgcn_readfirstlane(tl_cnt[h]);
+        const int run = (cnt + SEG * 64 - 1) / (SEG * 64) * 64;
+        lo = (hs % SEG) * run;
+        hi = min(cnt, lo + run);
+        return hs % SEG;
+      };
+#pragma unroll
+      for (int it = 0; it < NHS; ++it) {
+        int h, lo, hi;
+        if (pair_of(it, h, lo, hi) < 0 || tl_need[h] < 0) continue;
+        const int cut = tl_cut[h];
+        const float ba = bin_a_sh[h], bb = bin_b_sh[h], thr = (float)cut;
+        for (int i = lo + lane; i < hi; i += 64) {
+          const int pos = min((int)tl_list[h * Kcap + i], n - 1);
+          const float s = sc[h * L + pos];
+          // (bucket 0: also the degenerate ranges, whose buckets say nothing about the order)
+          if (cut == 0 || __builtin_fmaf(s, ba, bb) >= thr) {
+            const int k = atomicAdd(&tl_mem[h], 1);
+            if (k < Tail::MEM) tl_mlist[h * Tail::MEM + k] = rank_word(score_key(s), pos);
+            tl_list[h * Kcap + i] = (uint16_t)(pos | 0x8000);  // (positions are below 4096)
+          }
+        }
+      }
+      lds_barrier();
+      uint32_t wmask[NHS];  // bit j: this lane's candidate of step j wins (at most 32 steps: one_split_fits)
+#pragma unroll
+      for (int it = 0; it < NHS; ++it) {
+        wmask[it] = 0u;
+        int h, lo, hi;
+        const int seg = pair_of(it, h, lo, hi);
+        if (seg < 0) continue;
+        const int need = __builtin_amdgcn_readfirstlane(tl_need[h]), m = __builtin_amdgcn_readfirstlane(tl_mem[h]);
+        const uint16_t* cl = tl_list + h * Kcap;
+        // the last winner among the members: every wavefront of the head ranks them itself, one member per lane, the
+        // others' words as scalars (no exchange, no LDS latency per member)
+        unsigned long long last = 0ull;
+        const bool from_list = m <= Tail::MEM;
+        if (need >= 0 && from_list) {
+          const unsigned long long own = (lane < m) ? tl_mlist[h * Tail::MEM + lane] : 0ull;
+          int rank = 0;
+          for (int k = 0; k < m; ++k) {
+            const unsigned long long o = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), k) << 32) |
+                                         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, k);
+            rank += (o > own) ? 1 : 0;
+          }
+          const unsigned long long who = __builtin_amdgcn_ballot_w64(lane < m && rank == need - 1);
+          const int src = (who != 0ull) ? __ffsll((long long)who) - 1 : 0;
+          last = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), src) << 32) |
+                 (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, src);
+        }
+        int total = 0;
+        for (int i0 = lo, j = 0; i0 < hi; i0 += 64, ++j) {
+          const int i = i0 + lane;
+          const uint32_t e = (i < hi) ? cl[i] : 0u;
+          bool win = i < hi;
+          if (e & 0x8000u) {
+            const int pos = min((int)(e & 0x7fffu), n - 1);
+            const unsigned long long own = rank_word(score_key(sc[h * L + pos]), pos);
+            if (from_list) {
+              win = own >= last;
+            } else {  // heavily tied: against every member in the list
+              const int cnt = tl_cnt[h];
+              int rank = 0;
+              for (int k = 0; k < cnt; ++k) {
+                const uint32_t f = cl[k];
+                const int fp = min((int)(f & 0x7fffu), n - 1);
+                rank += ((f & 0x8000u) && rank_word(score_key(sc[h * L + fp]), fp) > own) ? 1 : 0;
+              }
+              win = rank < need;
+            }
+          }
+          wmask[it] |= (win ? 1u : 0u) << j;
+          total += __popcll(__builtin_amdgcn_ballot_w64(win));
+        }
+        if (lane == 0) tl_segc[h * SEG + seg] = total;
+      }
+      lds_barrier();
+      // the winners in position order: outputs, and slot and weight for the pre-correction
+#pragma unroll
+      for (int it = 0; it < NHS; ++it) {
+        int h, lo, hi;
+        const int seg = pair_of(it, h, lo, hi);
+        if (seg < 0) continue;
+        int base = 0, all = 0;
+#pragma unroll
+        for (int sg = 0; sg < SEG; ++sg) {
+          const int c = tl_segc[h * SEG + sg];
+          base += (sg < seg) ? c : 0;
+          all += c;
+        }
+        const int n_out = min(K, all);
+        if (seg == 0 && lane == 0) tl_nout[h] = n_out;
+        int64_t* out_idx = p.topk_idx + (head0 + h) * (size_t)K;
+        int64_t* out_slot = p.topk_slots + (head0 + h) * (size_t)K;
+        const float M = tl_m[h], iz = tl_iz[h];
+        for (int i0 = lo, j = 0; i0 < hi; i0 += 64, ++j) {
+          const bool win = ((wmask[it] >> j) & 1u) != 0u;
+          const unsigned long long mw = __builtin_amdgcn_ballot_w64(win);
+          const int r = base + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mw >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mw, 0u));
+          base += __popcll(mw);
+          if (win && r < K) {
+            const int pos = min((int)(tl_list[h * Kcap + i0 + lane] & 0x7fffu), n - 1);
+            const int slot = sbase[pos >> 4] + (pos & 15);
+            out_idx[r] = pos;
+            out_slot[r] = slot;
+            if constexpr (HAS_V) {
+              tl_wslot[h * K + r] = (slot >= 0 && slot < p.num_slots) ? slot : -1;
+              tl_ww[h * K + r] = __expf(sc[h * L + pos] - M) * iz;
+            }
+          }
+        }
+        for (int r = n_out + seg * 64 + lane; r < K; r += SEG * 64) {
+          out_idx[r] = -1;
+          out_slot[r] = -1;
+        }
+      }
+    } else {  // Stage B alone: the winners are given (or none)
+      const int n_out = p.topk_idx ? K : 0;
+      if (tid < G) tl_nout[tid] = n_out;
+      for (int i = tid; i < GA * n_out; i += NT) {
+        const int h = i / K;
+        const int64_t pos = p.topk_idx[head0 * K + i];
+        const bool valid = pos >= 0 && pos < n;
+        const int slot = valid ? sbase[(int)pos >> 4] + ((int)pos & 15) : -1;
+        tl_wslot[i] = (slot >= 0 && slot < p.num_slots) ? slot : -1;
+        tl_ww[i] = valid ? __expf(sc[h * L + (int)pos] - tl_m[h]) * tl_iz[h] : 0.f;
+      }
+    }
+    if constexpr (HAS_V) {
+      lds_barrier();
+      // ---- pre-correction over the winners
+      using Pre = PreCorr<SCHEME % 10>;
+      const int dwi = lane % Pre::DW, w_in = lane / Pre::DW;
+      const int g_of_lane = (NG == 1) ? 0 : ((dwi * Pre::CPD) / (D / NG));
+      // WPH wavefronts per head (more heads than wavefronts: one after the other), each a contiguous-stride share of the
+      // winners, PB requests per lane in flight; one reduction over the lanes per wavefront and head
+      constexpr int WPH = (NW >= G) ? NW / G : 1, PB = (Pre::CPD == 16) ? 8 : 16;
+      static_assert(NW * Lds::WAVE_STAGE >= G * WPH * (D + 1) * 4, "the wavefronts' sums lie in the staging area");
+      float* old_sh = reinterpret_cast<float*>(stage);  // [G][WPH][D] (the accumulator sums are dead)
+      float* w_sh = old_sh + G * WPH * D;               // [G][WPH]
+      for (int hw = wave; hw < GA * WPH; hw += NW) {
+        const int h = hw / WPH, part = hw % WPH, n_out = __builtin_amdgcn_readfirstlane(tl_nout[h]);
+        float acc[Pre::CPD], accw = 0.f;
+#pragma unroll
+        for (int c = 0; c < Pre::CPD; ++c) acc[c] = 0.f;
+        for (int k0 = part * Pre::WPI + w_in; k0 - w_in < n_out; k0 += PB * WPH * Pre::WPI) {
+          uint32_t word[PB], word_b[PB];
+          uint16_t sb[PB];
+          float wv[PB];
+#pragma unroll
+          for (int u = 0; u < PB; ++u) {
+            const int k = k0 + u * WPH * Pre::WPI;
+            const int slot = (k < n_out) ? tl_wslot[h * K + k] : -1;
+            wv[u] = (slot >= 0) ? tl_ww[h * K + k] : 0.f;
+            const uint32_t sl = (uint32_t)max(slot, 0);
+            Pre::fetch(vbase, sl, dwi, word[u], word_b[u]);
+            sb[u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
+          }
+#pragma unroll
+          for (int u = 0; u < PB; ++u) {
+            Pre::add(word[u], word_b[u], wv[u] * bf16_to_f32(sb[u]), acc);
+            if (dwi == 0) accw += wv[u];
+          }
+        }
+        const int chan = Pre::reduce(acc, lane);
+        old_sh[hw * D + chan] = acc[0];
+        old_sh[hw * D + chan + 1] = acc[1];
+        const float wsum = wave_sum(accw);
+        if (lane == 0) w_sh[hw] = wsum;
+      }
+      lds_barrier();
+      for (int i = tid; i < GA * D; i += NT) {
+        const int h = i >> 7, d = i & 127;
+        float o = 0.f, wt = 0.f;
+#pragma unroll
+        for (int w = 0; w < WPH; ++w) {
+          o += old_sh[(h * WPH + w) * D + d];
+          wt += w_sh[h * WPH + w];
+        }
+        p.o_old[(head0 + h) * D + d] = o;
+        if (d == 0) p.W[head0 + h] = wt;
+        if (MODE == FS_FULL && p.blend_out) {
+          const size_t at = (head0 + h) * D + d;
+          p.blend_out[at] = f32_to_bf16(__builtin_fmaf(wt, bf16_to_f32(p.blend_o_new[at]), tl_ohat[h * D + d]) - o);
+        }
+      }
+    }
+    if (clk && tid == 0) clk[4] = JF_CLK();
+    return;
   }
   float lfin = 0.f;
   if (tid < G) {
@@ -1891,12 +2304,9 @@ template <int MODE, int VBITS, int NG, int MG_THREADS, int MG_REGK, bool PARTIAL
 __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) {
   static_assert(!(PARTIAL && MODE == FS_STAGE_B), "Stage B alone selects nothing");
   constexpr int MG_WAVES = MG_THREADS / 64;
-  constexpr int VP = D * VBITS / 8;
-  // lanes per winner row and codes per lane: a dword of the row each (INT2, INT4), or (INT3, planar) two bytes of
-  // each of the three planes = 16 codes
-  constexpr int DW = (VBITS == 3) ? 8 : VP / 4;
-  constexpr int CPD = (VBITS == 3) ? 16 : 32 / VBITS;
-  constexpr int WPI = 64 / DW;          // winners per wavefront instruction
+  using Pre = PreCorr<VBITS>;
+  constexpr int DW = Pre::DW, CPD = Pre::CPD;  // lanes per winner row, codes per lane
+  constexpr int WPI = Pre::WPI;         // winners per wavefront instruction
   // The floating-point sums (o_hat over the splits, the pre-correction terms over the winners) are organised
   // as if eight thread groups of 128 and sixteen wavefronts were at work, whatever MG_THREADS is: a smaller
   // workgroup takes several of those roles one after the other, so every shape of this kernel adds the same
@@ -2384,11 +2794,11 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   // ---- pre-correction over the winners.  One winner row per DW lanes: lane (w_in, dwi) holds dword dwi of
   // the winner's packed V row (CPD codes) and accumulates its CPD channels; winners are visited in a fixed
   // order, so the sums are run-to-run deterministic.  UNR rows per lane are requested before any is used.
-  const uint8_t* vbase = p.v_data + (size_t)hkv * p.num_slots * VP;
+  const uint8_t* vbase = p.v_data + (size_t)hkv * p.num_slots * Pre::VP;
   const uint8_t* vsbase = reinterpret_cast<const uint8_t*>(p.v_scales + (size_t)hkv * p.num_slots * NG);
   const int dwi = lane % DW, w_in = lane / DW;
   const int g_of_lane = (NG == 1) ? 0 : ((dwi * CPD) / (D / NG));
-  constexpr int UNR = (256 / (VWAVES * WPI) > 0) ? 256 / (VWAVES * WPI) : 1;  // 256 winners per pass
+  constexpr int UNR = Pre::UNR;  // 256 winners per pass
   for (int vw = wave; vw < VWAVES; vw += MG_WAVES) {  // (one turn unless the workgroup has fewer than sixteen wavefronts)
   float acc[CPD];
 #pragma unroll
@@ -2404,75 +2814,18 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
       const int slot = (k < n_out) ? win_idx[k] : -1;
       wv[u] = (slot >= 0) ? __builtin_bit_cast(float, win_key[k]) : 0.f;
       const uint32_t sl = (uint32_t)max(slot, 0);
-      if constexpr (VBITS == 3) {  // bytes 2*dwi, 2*dwi+1 of every plane -> the 24-bit words of two 8-code groups
-        const uint8_t* row = vbase + (size_t)(sl * (uint32_t)VP) + dwi * 2;
-        const uint32_t h0 = *reinterpret_cast<const uint16_t*>(row), h1 = *reinterpret_cast<const uint16_t*>(row + 16),
-                       h2 = *reinterpret_cast<const uint16_t*>(row + 32);
-        word[u] = ((h0 & 0xffu) << 16) | ((h1 & 0xffu) << 8) | (h2 & 0xffu);
-        word_b[u] = ((h0 >> 8) << 16) | ((h1 >> 8) << 8) | (h2 >> 8);
-      } else {
-        word[u] = *reinterpret_cast<const uint32_t*>(vbase + (size_t)(sl * (uint32_t)VP) + dwi * 4);
-        word_b[u] = 0;
-      }
+      Pre::fetch(vbase, sl, dwi, word[u], word_b[u]);
       sbits[u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
     }
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
       const float ws = wv[u] * bf16_to_f32(sbits[u]);  // zero for padding rows
-      // byte `byte` of the dword holds its codes MSB first; channel of code c in the dword = dwi*CPD + c.
-      // code - VOFF is the code with its top bit flipped, read as a two's complement field: one signed bit-field
-      // extract per code after one exclusive-or per word.
-      constexpr uint32_t FLIP = (VBITS == 3) ? 0x00924924u : ((VBITS == 2) ? 0xaaaaaaaau : 0x88888888u);
-      const uint32_t xa = word[u] ^ FLIP, xb = word_b[u] ^ FLIP;
-#pragma unroll
-      for (int c = 0; c < CPD; ++c) {
-        int sh;
-        if constexpr (VBITS == 3) {
-          sh = 21 - 3 * (c & 7);
-        } else {
-          const int byte = c / (8 / VBITS), inb = c % (8 / VBITS);
-          sh = 8 * byte + (8 - VBITS * (inb + 1));
-        }
-        const uint32_t x = (VBITS == 3 && c >= 8) ? xb : xa;
-        const int code = (int)(x << (32 - VBITS - sh)) >> (32 - VBITS);
-        acc[c] = __builtin_fmaf(ws, (float)code, acc[c]);
-      }
+      Pre::add(word[u], word_b[u], ws, acc);
       if (dwi == 0) accw += wv[u];
     }
   }
-  // reduce over the WPI winners of a wavefront instruction (lanes with equal dwi): every exchange step halves
-  // the channels a lane is responsible for (the lane whose offset bit is clear keeps the lower half), so after
-  // log2(WPI) steps every lane holds the sums of CPD / WPI = 2 channels; then over wavefronts through LDS
-  {
-    int chan = dwi * CPD;
-    auto halve = [&](auto off_c, auto n_c) {
-      constexpr int OFF = decltype(off_c)::value, N = decltype(n_c)::value;
-      const bool upper = (lane & OFF) != 0;
-#pragma unroll
-      for (int i = 0; i < N / 2; ++i) {
-        if constexpr (OFF == 32) {  // one half-wave swap serves both directions
-          const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, acc[i]), __builtin_bit_cast(uint32_t, acc[i + N / 2]), false, false);
-          acc[i] = __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
-        } else {
-          const float keep = upper ? acc[i + N / 2] : acc[i];
-          const int send = __builtin_bit_cast(int, upper ? acc[i] : acc[i + N / 2]);
-          // lane ^ 8: rotation by 8 inside the 16-lane row; lane ^ 16: swizzle inside 32 lanes
-          const int recv = (OFF == 8) ? dpp_mov<0x128, 0xf>(0, send) : __builtin_amdgcn_ds_swizzle(send, 0x401F);
-          acc[i] = keep + __builtin_bit_cast(float, recv);
-        }
-      }
-      chan += upper ? N / 2 : 0;
-    };
-    static_assert(DW == 8 || DW == 16, "eight or sixteen lanes per V row");
-    if constexpr (DW == 8) {
-      halve(std::integral_constant<int, 8>{}, std::integral_constant<int, CPD>{});
-      halve(std::integral_constant<int, 16>{}, std::integral_constant<int, CPD / 2>{});
-      halve(std::integral_constant<int, 32>{}, std::integral_constant<int, CPD / 4>{});
-    } else {
-      halve(std::integral_constant<int, 16>{}, std::integral_constant<int, CPD>{});
-      halve(std::integral_constant<int, 32>{}, std::integral_constant<int, CPD / 2>{});
-    }
-    static_assert(CPD / WPI == 2, "two channels per lane after the exchange");
+  {  // over the WPI winners of a wavefront instruction; then over wavefronts through LDS
+    const int chan = Pre::reduce(acc, lane);
     old_sh[vw][chan] = acc[0];
     old_sh[vw][chan + 1] = acc[1];
     const float wsum = wave_sum(accw);  // only the dwi == 0 lanes hold weights
@@ -2498,51 +2851,66 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
 constexpr size_t LDS_BUDGET_2WG = 80 * 1024 - 512;    // two workgroups per CU (160 KB LDS)
 constexpr size_t LDS_BUDGET_1WG = 160 * 1024 - 1024;
 
+// LDS a scan workgroup has left for what grows with the split: the scores, the page table (and, with one split, ScanTail)
 template <int SCHEME, int G, int NG>
-int lmax_for() {
+long lds_room_for() {
   using Lds = ScanLds<SCHEME, G, NG>;
   const size_t budget = (G <= 4 && Lds::NW == 8) ? LDS_BUDGET_2WG : LDS_BUDGET_1WG;
   const size_t fixed = Lds::AUX + Lds::stage_bytes() + 64 + 832 + (Lds::KB4 ? 1536 : (Lds::K3 ? 512 : 0));  // + static LDS of the kernel (incl. the rounding tables)
-  long lm = (long)((budget - fixed) / (Lds::per_position() + 1));  // +1: page table (4 bytes per 16 positions)
-  lm = lm / 256 * 256;
-  if (lm > Lds::LMAX) lm = Lds::LMAX;
-  if (lm < 256) lm = 256;
-  return (int)lm;
+  return (long)budget - (long)fixed;
 }
 
-inline int lmax_dispatch(int scheme, int G, int NG) {
-#define JF_LMAX_CASE(SCH, GG, NGG) if (scheme == SCH && G == GG && NG == NGG) return lmax_for<SCH, GG, NGG>()
-  JF_LMAX_CASE(JF_SCHEME_K3V2, 1, 1); JF_LMAX_CASE(JF_SCHEME_K3V2, 2, 1); JF_LMAX_CASE(JF_SCHEME_K3V2, 4, 1);
-  JF_LMAX_CASE(JF_SCHEME_K3V2, 8, 1); JF_LMAX_CASE(JF_SCHEME_K3V2, 16, 1);
-  JF_LMAX_CASE(JF_SCHEME_K3V2, 1, 2); JF_LMAX_CASE(JF_SCHEME_K3V2, 2, 2); JF_LMAX_CASE(JF_SCHEME_K3V2, 4, 2);
-  JF_LMAX_CASE(JF_SCHEME_K3V2, 8, 2); JF_LMAX_CASE(JF_SCHEME_K3V2, 16, 2);
-  JF_LMAX_CASE(JF_SCHEME_K4V4, 1, 1); JF_LMAX_CASE(JF_SCHEME_K4V4, 2, 1); JF_LMAX_CASE(JF_SCHEME_K4V4, 4, 1);
-  JF_LMAX_CASE(JF_SCHEME_K4V4, 8, 1); JF_LMAX_CASE(JF_SCHEME_K4V4, 16, 1);
-  JF_LMAX_CASE(JF_SCHEME_K3V4, 1, 1); JF_LMAX_CASE(JF_SCHEME_K3V4, 2, 1); JF_LMAX_CASE(JF_SCHEME_K3V4, 4, 1);
-  JF_LMAX_CASE(JF_SCHEME_K3V4, 8, 1); JF_LMAX_CASE(JF_SCHEME_K3V4, 16, 1);
-  JF_LMAX_CASE(JF_SCHEME_K4V2, 1, 1); JF_LMAX_CASE(JF_SCHEME_K4V2, 2, 1); JF_LMAX_CASE(JF_SCHEME_K4V2, 4, 1);
-  JF_LMAX_CASE(JF_SCHEME_K4V2, 8, 1); JF_LMAX_CASE(JF_SCHEME_K4V2, 16, 1);
-  JF_LMAX_CASE(JF_SCHEME_K2V2, 1, 1); JF_LMAX_CASE(JF_SCHEME_K2V2, 2, 1); JF_LMAX_CASE(JF_SCHEME_K2V2, 4, 1);
-  JF_LMAX_CASE(JF_SCHEME_K2V2, 8, 1); JF_LMAX_CASE(JF_SCHEME_K2V2, 16, 1);
-  JF_LMAX_CASE(JF_SCHEME_K2V2, 1, 2); JF_LMAX_CASE(JF_SCHEME_K2V2, 2, 2); JF_LMAX_CASE(JF_SCHEME_K2V2, 4, 2);
-  JF_LMAX_CASE(JF_SCHEME_K2V2, 8, 2); JF_LMAX_CASE(JF_SCHEME_K2V2, 16, 2);
-  JF_LMAX_CASE(JF_SCHEME_K2V4, 1, 1); JF_LMAX_CASE(JF_SCHEME_K2V4, 2, 1); JF_LMAX_CASE(JF_SCHEME_K2V4, 4, 1);
-  JF_LMAX_CASE(JF_SCHEME_K2V4, 8, 1); JF_LMAX_CASE(JF_SCHEME_K2V4, 16, 1);
-#define JF_LMAX_ALL_G(SCH, NGG)                                                                      \
-  JF_LMAX_CASE(SCH, 1, NGG); JF_LMAX_CASE(SCH, 2, NGG); JF_LMAX_CASE(SCH, 4, NGG); JF_LMAX_CASE(SCH, 8, NGG); \
-  JF_LMAX_CASE(SCH, 16, NGG)
-  JF_LMAX_ALL_G(JF_SCHEME_K2V3, 1); JF_LMAX_ALL_G(JF_SCHEME_K2V3, 2);
-  JF_LMAX_ALL_G(JF_SCHEME_K3V3, 1); JF_LMAX_ALL_G(JF_SCHEME_K3V3, 2);
-  JF_LMAX_ALL_G(JF_SCHEME_K4V3, 1);
-  JF_LMAX_ALL_G(JF_SCHEME_A2V2, 1); JF_LMAX_ALL_G(JF_SCHEME_A2V2, 2);
-  JF_LMAX_ALL_G(JF_SCHEME_A2V3, 1); JF_LMAX_ALL_G(JF_SCHEME_A2V3, 2);
-  JF_LMAX_ALL_G(JF_SCHEME_A2V4, 1);
-  JF_LMAX_ALL_G(JF_SCHEME_K3V4, 2); JF_LMAX_ALL_G(JF_SCHEME_K2V4, 2); JF_LMAX_ALL_G(JF_SCHEME_A2V4, 2);
-  JF_LMAX_ALL_G(JF_SCHEME_B4V2, 1); JF_LMAX_ALL_G(JF_SCHEME_B4V2, 2); JF_LMAX_ALL_G(JF_SCHEME_B4V3, 1);
-  JF_LMAX_ALL_G(JF_SCHEME_B4V3, 2); JF_LMAX_ALL_G(JF_SCHEME_B4V4, 1); JF_LMAX_ALL_G(JF_SCHEME_B4V4, 2);
-#undef JF_LMAX_ALL_G
-#undef JF_LMAX_CASE
-  return 256;
+inline long lds_room(int scheme, int G, int NG) {
+#define JF_ROOM_CASE(SCH, GG, NGG) if (scheme == SCH && G == GG && NG == NGG) return lds_room_for<SCH, GG, NGG>()
+  JF_ROOM_CASE(JF_SCHEME_K3V2, 1, 1); JF_ROOM_CASE(JF_SCHEME_K3V2, 2, 1); JF_ROOM_CASE(JF_SCHEME_K3V2, 4, 1);
+  JF_ROOM_CASE(JF_SCHEME_K3V2, 8, 1); JF_ROOM_CASE(JF_SCHEME_K3V2, 16, 1);
+  JF_ROOM_CASE(JF_SCHEME_K3V2, 1, 2); JF_ROOM_CASE(JF_SCHEME_K3V2, 2, 2); JF_ROOM_CASE(JF_SCHEME_K3V2, 4, 2);
+  JF_ROOM_CASE(JF_SCHEME_K3V2, 8, 2); JF_ROOM_CASE(JF_SCHEME_K3V2, 16, 2);
+  JF_ROOM_CASE(JF_SCHEME_K4V4, 1, 1); JF_ROOM_CASE(JF_SCHEME_K4V4, 2, 1); JF_ROOM_CASE(JF_SCHEME_K4V4, 4, 1);
+  JF_ROOM_CASE(JF_SCHEME_K4V4, 8, 1); JF_ROOM_CASE(JF_SCHEME_K4V4, 16, 1);
+  JF_ROOM_CASE(JF_SCHEME_K3V4, 1, 1); JF_ROOM_CASE(JF_SCHEME_K3V4, 2, 1); JF_ROOM_CASE(JF_SCHEME_K3V4, 4, 1);
+  JF_ROOM_CASE(JF_SCHEME_K3V4, 8, 1); JF_ROOM_CASE(JF_SCHEME_K3V4, 16, 1);
+  JF_ROOM_CASE(JF_SCHEME_K4V2, 1, 1); JF_ROOM_CASE(JF_SCHEME_K4V2, 2, 1); JF_ROOM_CASE(JF_SCHEME_K4V2, 4, 1);
+  JF_ROOM_CASE(JF_SCHEME_K4V2, 8, 1); JF_ROOM_CASE(JF_SCHEME_K4V2, 16, 1);
+  JF_ROOM_CASE(JF_SCHEME_K2V2, 1, 1); JF_ROOM_CASE(JF_SCHEME_K2V2, 2, 1); JF_ROOM_CASE(JF_SCHEME_K2V2, 4, 1);
+  JF_ROOM_CASE(JF_SCHEME_K2V2, 8, 1); JF_ROOM_CASE(JF_SCHEME_K2V2, 16, 1);
+  JF_ROOM_CASE(JF_SCHEME_K2V2, 1, 2); JF_ROOM_CASE(JF_SCHEME_K2V2, 2, 2); JF_ROOM_CASE(JF_SCHEME_K2V2, 4, 2);
+  JF_ROOM_CASE(JF_SCHEME_K2V2, 8, 2); JF_ROOM_CASE(JF_SCHEME_K2V2, 16, 2);
+  JF_ROOM_CASE(JF_SCHEME_K2V4, 1, 1); JF_ROOM_CASE(JF_SCHEME_K2V4, 2, 1); JF_ROOM_CASE(JF_SCHEME_K2V4, 4, 1);
+  JF_ROOM_CASE(JF_SCHEME_K2V4, 8, 1); JF_ROOM_CASE(JF_SCHEME_K2V4, 16, 1);
+#define JF_ROOM_ALL_G(SCH, NGG)                                                                      \
+  JF_ROOM_CASE(SCH, 1, NGG); JF_ROOM_CASE(SCH, 2, NGG); JF_ROOM_CASE(SCH, 4, NGG); JF_ROOM_CASE(SCH, 8, NGG); \
+  JF_ROOM_CASE(SCH, 16, NGG)
+  JF_ROOM_ALL_G(JF_SCHEME_K2V3, 1); JF_ROOM_ALL_G(JF_SCHEME_K2V3, 2);
+  JF_ROOM_ALL_G(JF_SCHEME_K3V3, 1); JF_ROOM_ALL_G(JF_SCHEME_K3V3, 2);
+  JF_ROOM_ALL_G(JF_SCHEME_K4V3, 1);
+  JF_ROOM_ALL_G(JF_SCHEME_A2V2, 1); JF_ROOM_ALL_G(JF_SCHEME_A2V2, 2);
+  JF_ROOM_ALL_G(JF_SCHEME_A2V3, 1); JF_ROOM_ALL_G(JF_SCHEME_A2V3, 2);
+  JF_ROOM_ALL_G(JF_SCHEME_A2V4, 1);
+  JF_ROOM_ALL_G(JF_SCHEME_K3V4, 2); JF_ROOM_ALL_G(JF_SCHEME_K2V4, 2); JF_ROOM_ALL_G(JF_SCHEME_A2V4, 2);
+  JF_ROOM_ALL_G(JF_SCHEME_B4V2, 1); JF_ROOM_ALL_G(JF_SCHEME_B4V2, 2); JF_ROOM_ALL_G(JF_SCHEME_B4V3, 1);
+  JF_ROOM_ALL_G(JF_SCHEME_B4V3, 2); JF_ROOM_ALL_G(JF_SCHEME_B4V4, 1); JF_ROOM_ALL_G(JF_SCHEME_B4V4, 2);
+#undef JF_ROOM_ALL_G
+#undef JF_ROOM_CASE
+  return 0;
+}
+
+// Longest split: what fits LDS (scores and one page-table entry per 16 positions), at most four chunks per wavefront.
+inline int split_len_max(int scheme, int G, int NG) {
+  long lm = lds_room(scheme, G, NG) / (4 * G + 1) / 256 * 256;
+  const long cap = (G <= 4 ? 16 : 8) * 256;
+  if (lm > cap) lm = cap;
+  return lm < 256 ? 256 : (int)lm;
+}
+
+// Whether a scan whose single split of L positions covers the sequence can merge by itself: its tables fit the LDS
+// that is left, and a wavefront's share of a candidate list fits the 32 bits of its win mask.
+inline bool one_split_fits(int scheme, int G, int NG, int L, int top_k, int kc) {
+  const int seg = G <= 4 ? 4 : 1;
+  const size_t tail = G == 1 ? ScanTail<1, 4>::bytes(top_k, kc) : G == 2 ? ScanTail<2, 4>::bytes(top_k, kc) :
+                      G == 4 ? ScanTail<4, 4>::bytes(top_k, kc) : G == 8 ? ScanTail<8, 1>::bytes(top_k, kc) :
+                               ScanTail<16, 1>::bytes(top_k, kc);
+  return kc <= seg * 64 * 32 && (long)((4 * G + 1) * (long)L + (long)tail) <= lds_room(scheme, G, NG);
 }
 
 // Estimated microseconds of the merge (fitted on MI355X): a fixed part per launch plus a part proportional to
@@ -2593,10 +2961,10 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
   // MI355X: a scan workgroup costs a fixed part plus a part proportional to the 64-position chunks each of
   // its wavefronts works through; a last, partly filled round of workgroups runs faster than a full one; the
   // merge costs a fixed part per launch plus a part proportional to the candidates one workgroup visits.
-  const int lmax = lmax_dispatch(scheme, G, NG);
+  const int lmax = split_len_max(scheme, G, NG);
   const int nw = (G <= 4) ? 16 : 8;
   const int kCUs = device_cus();
-  constexpr double kScanFixed = 8.5;
+  constexpr double kScanFixed = 8.5, kOneTail = 3.5, kOneTailPerWinner = 0.0025, kManyRows = 5.0, kPerRowBeyond = 0.005;
   // one chunk per wavefront, all wavefronts; the mixed schemes are priced like the wider one
   const double per_chunk = (scheme == JF_SCHEME_K3V2 || scheme == JF_SCHEME_K2V2) ? 5.9 : 6.6;  // (INT3 values, asymmetric keys: as INT4)
   int L = 256;
@@ -2610,8 +2978,15 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
     double cost = (double)full * (kScanFixed + stream);
     if (rem > 0) cost += kScanFixed + stream * (0.5 + 0.5 * (double)rem / kCUs);
     const int kc = (top_k + FS_CAND_SLACK) < cand ? (top_k + FS_CAND_SLACK) : cand;
-    int parts, spp;
-    cost += merge_plan(rows, (int)nsp, kc, top_k, &parts, &spp);
+    // One split that merges by itself (measured: 4 - 5 us for 64 winners per head of four, 6 for 256 of four; the sums
+    // over the winners fill the vector ALU); a merge launch of more rows than CUs takes 16 us at 512 rows, 18 at 1024.
+    if (nsp == 1 && one_split_fits(scheme, G, NG, cand, top_k, kc)) {
+      cost += kOneTail + kOneTailPerWinner * (double)(G * top_k);
+    } else {
+      int parts, spp;
+      cost += merge_plan(rows, (int)nsp, kc, top_k, &parts, &spp);
+      if (rows > kCUs) cost += kManyRows + kPerRowBeyond * (double)(rows - kCUs);
+    }
     if (best < 0.0 || cost <= best) {
       best = cost;
       L = cand;
@@ -2659,16 +3034,18 @@ inline WsLayout ws_layout(int B, int H_q, int ns, int kc, int parts, int top_k) 
 
 template <int MODE, int SCHEME, int G, int NG>
 int launch_scan(const FusedParams& p, hipStream_t st) {
-  const size_t smem = ScanLds<SCHEME, G, NG>::total(p.L);
-  auto kern = fused_scan_kernel<MODE, SCHEME, G, NG>;
+  using Lds = ScanLds<SCHEME, G, NG>;
+  const bool one = p.one_split != 0;
+  const size_t smem = Lds::total(p.L) + (one ? ScanTail<G, Lds::SEG>::bytes(p.top_k, p.Kc) : 0);
+  auto kern = one ? fused_scan_kernel<MODE, SCHEME, G, NG, true> : fused_scan_kernel<MODE, SCHEME, G, NG, false>;
   // per instantiation: raise the dynamic-LDS limit only when it grows (launches may come from several threads)
   static std::mutex attr_mu;
-  static size_t attr_smem = 0;
+  static size_t attr_smem[2] = {0, 0};
   {
     std::lock_guard<std::mutex> lock(attr_mu);
-    if (smem > attr_smem) {
+    if (smem > attr_smem[one]) {
       JF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-      attr_smem = smem;
+      attr_smem[one] = smem;
     }
   }
 #ifdef JF_DEBUG_HOOKS
@@ -2806,6 +3183,7 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   JF_CHECK_ARG(p.n_splits <= MG_MAX_SPLITS, "fused_scan: too many splits (%d > %d)", p.n_splits, MG_MAX_SPLITS);
   merge_plan(B * H_q, p.n_splits, p.Kc, top_k, &p.mg_parts, &p.mg_spp);
   if (MODE == FS_STAGE_B) { p.mg_parts = 1; p.mg_spp = p.n_splits; }
+  p.one_split = !scores_only && p.n_splits == 1 && one_split_fits(scheme, G, NGv, p.L, top_k, p.Kc);
   const WsLayout wl = ws_layout(B, H_q, p.n_splits, p.Kc, p.mg_parts, top_k);
   if (!scores_only) {
     JF_CHECK_ARG(workspace && workspace_bytes >= wl.total, "fused_scan: workspace too small (%zu < %zu)", workspace_bytes, wl.total);
@@ -2869,7 +3247,7 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   }
 #undef JF_FUSED_BY_G
 #undef JF_FUSED_CASE
-  if (rc != JF_OK || scores_only) return rc;
+  if (rc != JF_OK || scores_only || p.one_split) return rc;
   dim3 mgrid(B, H_q);
   const bool wide = top_k > FS_LDS_TOPK;  // the winners' arrays do not fit the kernels' static LDS
   if (p.mg_parts > 1) {  // first stage: every part's top_k, as new candidate lists (the same kernel for every form)

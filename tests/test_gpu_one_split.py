@@ -1,0 +1,92 @@
+"""The scan that merges by itself (one split covers the sequence, no merge launch): the sizes where it can go wrong --
+single rows, page and chunk edges, fewer positions than winners, empty sequences, ties at the cut that fill more than one
+wavefront's rank list, corrections at the edge of its LDS -- against the oracle, and against the same call cut into splits
+of 256 positions, which takes the merge kernel."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import make_case, to_device
+from tests.test_gpu_fused import check_against_oracle, run_fused
+
+pytestmark = pytest.mark.gpu
+
+SCALE = 128 ** -0.5
+
+
+def _plan(scheme_id, gs, B, Hq, Hkv, S, K):
+    from jetfire_amd import _lib
+    out = [C.c_int() for _ in range(4)]
+    _lib.check(_lib.load().jf_fused_plan(scheme_id, gs, B, Hq, Hkv, S, K, *[C.byref(o) for o in out]))
+    return [o.value for o in out]
+
+
+def _both(scheme, c, d, S, K):
+    """The call with one split, and with splits of 256 positions."""
+    from jetfire_amd import _lib
+    res = []
+    for split in (4096, 256):
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(split))
+        try:
+            res.append([t.clone() for t in run_fused(scheme, c, d, S, K)])
+        finally:
+            _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    return res
+
+
+@pytest.mark.parametrize("scheme,kb,vb,gs,G,S,lens,K", [
+    ("k4v4", 4, 4, 128, 4, 1, [1], 32),
+    ("k4v4", 4, 4, 128, 4, 257, [257, 0, 256, 17], 64),
+    ("k3v2", 3, 2, 64, 4, 1024, [1024, 1023, 63, 65], 256),
+    ("k3v2", 3, 2, 64, 4, 2040, [2040, 1, 0], 512),
+    ("k3v2", 3, 2, 64, 8, 1111, [1111, 700], 128),
+    ("k3v2", 3, 2, 64, 8, 512, [512, 300], 512),
+    ("k2v2", 2, 2, 64, 1, 3900, [3900, 16], 2048),
+    ("k3v3", 3, 3, 64, 2, 1500, [1500, 64], 256),
+    ("k3v3", 3, 3, 128, 7, 800, [800, 799], 64),
+    ("b4v4", 4, 4, 64, 4, 900, [900, 450], 128),
+    ("a2v4", 2, 4, 128, 16, 400, [400, 33], 64),
+])
+def test_one_split_matches_oracle_and_merge(scheme, kb, vb, gs, G, S, lens, K):
+    Hkv = 2 if G < 16 else 1
+    c = make_case(91, len(lens), G * Hkv, Hkv, S, kb, vb, gs, lens=lens, k_asym=scheme.startswith("a"))
+    d = to_device(c)
+    one, cut = _both(scheme, c, d, S, K)
+    check_against_oracle(scheme, c, S, K, one)
+    # same winners; the sums differ by the order of fp32 additions over the splits (and, over the winners, of at most
+    # 2048 terms of one sign pattern): 3e-6, the bound both hold against the oracle
+    assert torch.equal(one[4], cut[4]) and torch.equal(one[1], cut[1])
+    for a, b in ((one[0], cut[0]), (one[2], cut[2]), (one[3], cut[3])):
+        assert float((a - b).abs().max()) <= 6e-6
+
+
+@pytest.mark.parametrize("levels", [1, 3, 40])
+@pytest.mark.parametrize("S,K", [(300, 64), (300, 512), (1500, 256)])
+def test_one_split_ties(levels, S, K):
+    """Key rows copied from a few distinct ones: the cut bucket holds more members than a rank list (levels 3: hundreds
+    of equal scores; 1: all of them), or more than the candidate list (the exact selection).  Lowest positions win."""
+    c = make_case(92, 2, 8, 2, S, 4, 4, 128, lens=[S, S - 37])
+    d = to_device(c)
+    kd, ks, bt = d["kd"].clone(), d["ks"].clone(), d["bt"]
+    pos = torch.arange(S, device="cuda")
+    for b in range(2):
+        slot = bt[b, pos // 16] * 16 + pos % 16
+        src = slot[pos % levels]
+        kd[:, slot], ks[:, slot] = d["kd"][:, src], d["ks"][:, src]
+    d["kd"], d["ks"] = kd, ks
+    one, cut = _both("k4v4", c, d, S, K)
+    assert torch.equal(one[4], cut[4]) and torch.equal(one[1], cut[1])
+    scores = one[7].cpu().numpy()
+    for b, n in enumerate((S, S - 37)):
+        for h in range(8):
+            want = np.sort(np.lexsort((np.arange(n), -scores[b, h, :n]))[:K])
+            got = one[4][b, h].cpu().numpy()
+            assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -1).all()
+
+
+def test_plan_takes_one_split_for_short_and_many_sequences():
+    assert _plan(44, 128, 1, 32, 8, 777, 64)[1] == 1
+    assert _plan(32, 64, 32, 32, 8, 2048, 256)[1] == 1
+    assert _plan(44, 128, 1, 32, 8, 4096, 64)[1] > 1
