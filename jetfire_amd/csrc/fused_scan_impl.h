@@ -132,7 +132,7 @@ struct FusedParams {
   float* scores;  // optional (B, H_q, max_S)
   const float* scores_in;  // FS_STAGE_B: the scores (B, H_q, max_S)
   const float* stats_m;    // FS_STAGE_B merge, optional: softmax statistics (B, H_q) that replace the ones derived
-  const float* stats_iz;   //   from the split partials (pre-correction terms alone: n_splits == 0, o_hat == NULL)
+  const float* stats_iz;   //   from the split partials (which are then already normalised; part_m, part_l NULL)
   int scores_only;         // FS_STAGE_A: stop after writing `scores`
   float* part_m;  // (B, H_q, NS)
   float* part_l;  // (B, H_q, NS)
@@ -2372,9 +2372,9 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   constexpr bool HAS_LISTS = (MODE != FS_STAGE_B);
   float pm = -INFINITY, pl = 0.f;
   int my_cnt = 0;
-  // (given statistics, jf_stage_b_softmax_v: no partial results at all, NS = 0 and the pointers are null; those
-  // loads then read the page table, which every caller of this kernel passes, and every one of them is masked)
-  const bool has_parts = NS > 0;
+  // (given statistics, jf_softmax_v_int8_tiles: the partial rows are already normalised and come without maxima and
+  // sums; those loads then read the page table, which every caller of this kernel passes, and are masked)
+  const bool has_parts = MODE != FS_STAGE_B || p.part_m != nullptr;
   const float* dummy_f = reinterpret_cast<const float*>(bt);
   // The first MG_REGK * MG_THREADS candidates live in registers: group g = r / 4 of a thread holds the four
   // consecutive candidates (g * MG_THREADS + tid) * 4 + (r % 4), fetched with one 16-byte load.  Candidate
@@ -2416,7 +2416,7 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
     for (int i = 0; i < PO_PRE; ++i) {
       po[i] = 0.f;
       if constexpr (MODE != FS_STAGE_A && !PARTIAL)
-        po[i] = *(has_parts ? p.part_o + (bh * NS + min(q4 + VGRP * i, NS - 1)) * D + d : dummy_f);
+        po[i] = p.part_o[(bh * NS + min(q4 + VGRP * i, NS - 1)) * D + d];
     }
   }
   // page-table entries for the table in LDS: stored after the first barrier, so that the wait for them (the
@@ -2433,7 +2433,7 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   for (int i = tid; i < MG_BINS; i += MG_THREADS) hist[i] = 0;
   if (tid == 0) lcount_sh = 0;
   // the masks of the loads the first interval uses (the others follow its barrier)
-  if (tid >= NS) pm = -INFINITY;
+  if (tid >= NS || !has_parts) pm = -INFINITY;
   if (tid >= NL) my_cnt = 0;
 #pragma unroll
   for (int g = 0; g < NGRP; ++g) {
@@ -2483,7 +2483,7 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   if (lane == 0) { wred_u[wave] = kmin; wred_k[wave] = kmax; }
   lds_barrier();
   if (mclk && tid == 0) mclk[6] = JF_CLK();
-  if (tid >= NS) pl = 0.f;
+  if (tid >= NS || !has_parts) pl = 0.f;
   if (MODE == FS_FULL && !PARTIAL && p.blend_out && tid < D) blend_new = bf16_to_f32(blend_raw);
 #pragma unroll
   for (int g = 0; g < NGRP; ++g) {
@@ -2501,7 +2501,8 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   if (!PARTIAL) {
     M = waves_max_f<MG_WAVES>(wred_f, lane);
     if (!isfinite(M)) M = 0.f;
-    const float coef = (pm == -INFINITY) ? 0.f : __expf(pm - M);
+    float coef = (pm == -INFINITY) ? 0.f : __expf(pm - M);
+    if (!has_parts) coef = 1.f;
     if (tid < NS) coef_sh[tid] = coef;
     const float v = wave_sum(pl * coef);  // fixed reduction tree: deterministic
     if (lane == 0) wred_g[wave] = v;
@@ -2592,8 +2593,8 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
       float o2 = red_sh[0][tid];
 #pragma unroll
       for (int q = 1; q < VGRP; ++q) o2 += red_sh[q][tid];  // fixed order
-      blend_hat = o2 * inv_z;
-      if (MODE != FS_STAGE_B || p.o_hat) p.o_hat[bh * D + tid] = blend_hat;
+      blend_hat = !has_parts ? o2 : o2 * inv_z;
+      p.o_hat[bh * D + tid] = blend_hat;
     }
   }
   if (mclk && tid == 0) mclk[1] = JF_CLK();
@@ -3297,19 +3298,19 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   return JF_OK;
 }
 
-// The pre-correction terms alone (Stage B merge kernel with the caller's softmax statistics):
+// Stage B merge kernel with the caller's softmax statistics: o_hat is the plain sum of normalised partial rows, and
 //   W = sum_j p_j, o_old_unnorm = sum_j p_j * Vhat_j over the given winners, p_j = exp(score_j - m) * inv_z.
 template <int VBITS, int NG>
 static int launch_precorr_given_stats(const float* scores, const float* softmax_m, const float* softmax_inv_z,
                                       const uint8_t* v_data, const uint16_t* v_scales, const int64_t* block_table,
                                       const int32_t* seq_lens, const int64_t* topk_idx, int B, int H_q, int H_kv,
-                                      int max_S, int max_blocks, int64_t num_slots, int top_k, float* o_old_unnorm,
-                                      float* W, hipStream_t st) {
+                                      int max_S, int max_blocks, int64_t num_slots, int top_k, const float* partial,
+                                      int n_partial, float* o_hat, float* o_old_unnorm, float* W, hipStream_t st) {
   FusedParams p = {};
   p.v_data = v_data; p.v_scales = v_scales; p.block_table = block_table; p.seq_lens = seq_lens;
   p.B = B; p.H_q = H_q; p.H_kv = H_kv; p.max_S = max_S; p.max_blocks = max_blocks; p.num_slots = num_slots;
   p.top_k = top_k;
-  p.n_splits = 0; p.mg_parts = 1; p.mg_spp = 0; p.Kc = 0;
+  p.n_splits = n_partial; p.part_o = const_cast<float*>(partial); p.o_hat = o_hat; p.mg_parts = 1; p.mg_spp = 0; p.Kc = 0;
   p.scores_in = scores; p.stats_m = softmax_m; p.stats_iz = softmax_inv_z;
   p.topk_idx = const_cast<int64_t*>(topk_idx);
   p.o_old = o_old_unnorm; p.W = W;

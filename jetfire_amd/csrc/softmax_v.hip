@@ -129,95 +129,190 @@ __global__ __launch_bounds__(SV_THREADS) void weighted_v_split_kernel(
 //     rs   = max_t |pv_t| / 127,  pq_t = clamp(rint(pv_t * (1 / rs)), -127, 127)   (rs == 0: pq = 0)
 //     o_hat[d] += f32(sum_t pq_t * (nibble_t,d - 8)) * rs
 // with an exact int32 sum per tile and an fp32 running sum over the tiles in ascending order.
-// grid (TQ_SPLITS * sub_count, H_kv, B); thread = output channel d; the 32-lane quarters of the workgroup take the heads
-// in turn.  A range's tiles are dealt out in runs to `sub_count` workgroups (the tiles themselves, and with them every
-// quantisation step, stay those of the reference's eight ranges; only the association of the fp32 sum over tiles
-// changes, at the 1e-7 level), so that a long context fills the chip.
+// grid (TQ_SPLITS * sub_count, H_kv, B).  A range's tiles are dealt out in runs to `sub_count` workgroups and inside a
+// run to four wavefronts (the tiles themselves, and with them every quantisation step, stay those of the reference's
+// eight ranges; only the association of the fp32 sum over tiles changes, at the 1e-7 level).
+// A wavefront takes two tiles (64 positions) at a time on v_mfma_i32_16x16x64_i8, contracting over the positions: lane =
+// token quantises the heads' weights and stores one 16-byte row whose byte 4h + t is head h's weight if the token lies
+// in tile t and 0 otherwise, so accumulator register t of lane 16h + c is tile t's exact sum for head h and column c;
+// the -8 of the codes enters as the C operand (the weights against a tile of eights, negated).  V rows are fetched with
+// 16-byte loads consecutive inside a page, one step ahead, staged in wavefront-private LDS with swapped quarters and
+// transposed by ds_read_b64_tr_b4.  B 4, 32 / 8 heads, 8192 to 16384 positions: 12 - 14 us = 2.9 TB/s of rows, scales
+// and scores (a thread per channel with scalar products took 30.7 us); a wavefront's chain of load, exponential, two
+// divisions per head, LDS turn-around and MFMA bounds it, not the memory.
+__device__ inline void wave_lds_order() {  // a wavefront's earlier LDS accesses before its later ones
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 constexpr int TQ_SPLITS = 8;
 constexpr int TQ_TILE = 2 * BS;
-template <int G>
-__global__ __launch_bounds__(SV_THREADS) void tile_quantised_v_split_kernel(
+constexpr int TQ_WAVES = 4;
+typedef int tq_v2i __attribute__((ext_vector_type(2)));
+typedef int tq_v4i __attribute__((ext_vector_type(4)));
+typedef tq_v4i tq_row __attribute__((aligned(4)));  // 16 bytes of a packed row (the tensor may start at any dword)
+template <int NSET>
+__global__ __launch_bounds__(TQ_WAVES * 64) void tile_quantised_v_split_kernel(
     const float* __restrict__ scores, const float* __restrict__ softmax_m, const float* __restrict__ softmax_inv_z,
     const uint8_t* __restrict__ v_data, const uint16_t* __restrict__ v_scales, const int64_t* __restrict__ block_table,
     const int32_t* __restrict__ seq_lens, float* __restrict__ partial, int H_q, int H_kv, int max_S, int max_blocks,
     int64_t num_slots, int sub_count, int ga) {
-  constexpr int P = D / 2;
-  __shared__ __align__(16) uint8_t vbuf[TQ_TILE * P];
-  __shared__ int pq[G][TQ_TILE];
-  __shared__ float rs_sh[G];
-  const int split = blockIdx.x / sub_count, sub = blockIdx.x % sub_count;
-  const int hkv = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
+  constexpr int P = D / 2, G = NSET * 4;
+  constexpr int VST = 64 * P, WST = NSET * 64 * 16;
+  __shared__ __align__(16) uint8_t stage[TQ_WAVES][VST + WST];
+  const int range = blockIdx.x / sub_count, sub = blockIdx.x % sub_count;
+  const int hkv = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int S = max(0, min(max_S, seq_lens[b]));
-  const int chunk = (max_S + TQ_SPLITS - 1) / TQ_SPLITS;
-  const int s_start = split * chunk, s_end = min(s_start + chunk, S);
-  float acc[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) acc[g] = 0.0f;
+  const int len = (max_S + TQ_SPLITS - 1) / TQ_SPLITS;
+  const int s_start = range * len, s_end = min(s_start + len, S);
   const uint8_t* vbase = v_data + (size_t)hkv * num_slots * P;
   const uint16_t* sbase = v_scales + (size_t)hkv * num_slots;
   const int64_t* bt = block_table + (size_t)b * max_blocks;
-  const int q32 = tid >> 5, l32 = tid & 31;
+  const size_t head0 = (size_t)b * H_q + (size_t)hkv * ga;
   const int t_first = (s_start / BS) * BS;
-  const int n_tiles = (s_end > t_first) ? (s_end - t_first + TQ_TILE - 1) / TQ_TILE : 0;
-  const int per_sub = (n_tiles + sub_count - 1) / sub_count;
-  const int tile_end = min(n_tiles, (sub + 1) * per_sub);
-  for (int tile = sub * per_sub; tile < tile_end; ++tile) {
-    const int t0 = t_first + tile * TQ_TILE;
-    __syncthreads();
-    // the two pages of the tile (a page past the table or the sequence contributes zero weights; its codes are not read)
-    int64_t base_slot[2];
+  const int n_pairs = (s_end > t_first) ? (s_end - t_first + 2 * TQ_TILE - 1) / (2 * TQ_TILE) : 0;  // pairs of tiles
+  const int per_sub = (n_pairs + sub_count - 1) / sub_count;
+  const int p_end = min(n_pairs, (sub + 1) * per_sub);
+  uint8_t* vst = stage[wave];
+  uint8_t* wl = vst + VST;
+  float m[G], iz[G];
 #pragma unroll
-    for (int pg = 0; pg < 2; ++pg) {
+  for (int h = 0; h < G; ++h) {
+    m[h] = softmax_m[head0 + min(h, ga - 1)];
+    iz[h] = softmax_inv_z[head0 + min(h, ga - 1)];
+  }
+  // everything a pair of tiles needs from memory; a page past the table or the sequence contributes zero weights and
+  // its rows are not read
+  struct Fetch {
+    tq_v4i row[4];
+    float sc[G];
+    uint32_t vs;
+    bool live;
+  };
+  auto fetch = [&](int pair) -> Fetch {
+    Fetch f;
+    const int t0 = t_first + pair * 2 * TQ_TILE;
+    int64_t slot0[4];
+#pragma unroll
+    for (int pg = 0; pg < 4; ++pg) {
       const int blk = t0 / BS + pg;
       const int64_t e = (blk < max_blocks && blk * BS < s_end) ? bt[blk] : -1;
-      base_slot[pg] = (e >= 0 && (e + 1) * BS <= num_slots) ? e * BS : -1;
+      slot0[pg] = (e >= 0 && (e + 1) * BS <= num_slots) ? e * BS : -1;
     }
-    {
-      constexpr int NDW = BS * P / 4;  // 256 dwords per page
 #pragma unroll
-      for (int pg = 0; pg < 2; ++pg) {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(vbase + (base_slot[pg] < 0 ? 0 : base_slot[pg]) * P);
+    for (int pg = 0; pg < 4; ++pg) {
+      f.row[pg] = (tq_v4i){0, 0, 0, 0};
+      if (slot0[pg] >= 0) f.row[pg] = *reinterpret_cast<const tq_row*>(vbase + slot0[pg] * P + 16 * lane);  // (uniform)
+    }
+    const int pg = lane >> 4, pos = t0 + lane;
+    const int64_t s0 = pg == 0 ? slot0[0] : pg == 1 ? slot0[1] : pg == 2 ? slot0[2] : slot0[3];
+    f.live = pos >= s_start && pos < s_end && s0 >= 0;
+    f.vs = f.live ? sbase[s0 + (lane & 15)] : 0;
 #pragma unroll
-        for (int i = 0; i < NDW / SV_THREADS; ++i)
-          reinterpret_cast<uint32_t*>(vbuf)[pg * NDW + tid + i * SV_THREADS] = base_slot[pg] < 0 ? 0x88888888u : src[tid + i * SV_THREADS];
+    for (int h = 0; h < G; ++h) f.sc[h] = f.live ? scores[(head0 + min(h, ga - 1)) * (size_t)max_S + pos] : 0.f;
+    return f;
+  };
+  const int r16 = lane & 15, kb4 = lane >> 4;
+  const int tr_tok = (((r16 >> 1) & 3) << 1) | ((r16 >> 3) & 1);
+  const uint8_t* wrow = wl + (kb4 * 16 + tr_tok) * 16 + (r16 & 1) * 8;
+  const uint8_t* vrow = vst + lane * P;
+  const int vx = 16 * ((lane >> 2) & 3);
+  const tq_v4i minus8 = {(int)0xf8f8f8f8, (int)0xf8f8f8f8, (int)0xf8f8f8f8, (int)0xf8f8f8f8};
+  float acc[NSET][8];
+#pragma unroll
+  for (int s = 0; s < NSET; ++s)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[s][t] = 0.f;
+  int pair = sub * per_sub + wave;
+  Fetch nxt = {};
+  if (pair < p_end) nxt = fetch(pair);
+  for (; pair < p_end; pair += TQ_WAVES) {
+    const Fetch cur = nxt;
+    if (pair + TQ_WAVES < p_end) nxt = fetch(pair + TQ_WAVES);
+#pragma unroll
+    for (int pg = 0; pg < 4; ++pg) {  // row 16 pg + lane / 4, quarter lane % 4
+      const int row = 16 * pg + (lane >> 2);
+      *reinterpret_cast<tq_v4i*>(vst + row * P + (((lane & 3) ^ ((row >> 2) & 3)) * 16)) = cur.row[pg];
+    }
+    const float vs = bf16_to_f32((uint16_t)cur.vs);
+    const int shift = (lane >> 5) * 8;  // byte of the token's tile
+    float rs[NSET][2];
+#pragma unroll
+    for (int s = 0; s < NSET; ++s) {
+      tq_v4i row;
+      float r0 = 0.f, r1 = 0.f;
+#pragma unroll
+      for (int hh = 0; hh < 4; ++hh) {
+        const int h = s * 4 + hh;
+        float pv = 0.0f;
+        if (cur.live && h < ga) {
+          const float pr = __expf(cur.sc[h] - m[h]) * iz[h];
+          pv = pr * vs;
+        }
+        float a = fabsf(pv);  // maximum over the 32 tokens of the tile
+        a = fmaxf(a, __builtin_bit_cast(float, dpp_mov<0xb1, 0xf>(0, __builtin_bit_cast(int, a))));   // lane ^ 1
+        a = fmaxf(a, __builtin_bit_cast(float, dpp_mov<0x4e, 0xf>(0, __builtin_bit_cast(int, a))));   // lane ^ 2
+        a = fmaxf(a, __builtin_bit_cast(float, dpp_mov<0x141, 0xf>(0, __builtin_bit_cast(int, a))));  // mirrored in 8 lanes
+        a = fmaxf(a, __builtin_bit_cast(float, dpp_mov<0x140, 0xf>(0, __builtin_bit_cast(int, a))));  // mirrored in 16 lanes
+        a = fmaxf(a, __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, a), 0x401F)));  // lane ^ 16
+        const float row_scale = a / 127.0f;
+        const float inv_scale = (row_scale > 0.0f) ? (1.0f / row_scale) : 0.0f;
+        int qv = (int)rintf(pv * inv_scale);
+        qv = max(-127, min(127, qv));
+        row[hh] = (qv & 0xff) << shift;
+        const float lo = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, row_scale), 0));
+        const float hi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, row_scale), 32));
+        r0 = (kb4 == hh) ? lo : r0;
+        r1 = (kb4 == hh) ? hi : r1;
+      }
+      rs[s][0] = r0;
+      rs[s][1] = r1;
+      *reinterpret_cast<tq_v4i*>(wl + (s * 64 + lane) * 16) = row;
+    }
+    wave_lds_order();
+    tq_v4i A[NSET], C[NSET];
+#pragma unroll
+    for (int s = 0; s < NSET; ++s) {
+      const uint8_t* src = wrow + s * 1024;
+      const tq_v2i x0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) tq_v2i*)(src));
+      const tq_v2i x1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) tq_v2i*)(src + 128));
+      A[s] = (tq_v4i){x0[0], x0[1], x1[0], x1[1]};
+      C[s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[s], minus8, (tq_v4i){0, 0, 0, 0}, 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const tq_v2i x = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) tq_v2i*)(vrow + ((8 * t) ^ vx)));
+      const uint32_t x0 = (uint32_t)x[0], x1 = (uint32_t)x[1];
+      const tq_v4i Bv = {(int)(x0 & 0x0f0f0f0fu), (int)((x0 >> 4) & 0x0f0f0f0fu),
+                         (int)(x1 & 0x0f0f0f0fu), (int)((x1 >> 4) & 0x0f0f0f0fu)};
+#pragma unroll
+      for (int s = 0; s < NSET; ++s) {
+        const tq_v4i dot = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[s], Bv, C[s], 0, 0, 0);
+        acc[s][t] = __builtin_fmaf((float)dot[0], rs[s][0], acc[s][t]);
+        acc[s][t] = __builtin_fmaf((float)dot[1], rs[s][1], acc[s][t]);
       }
     }
-    for (int g = q32; g < G; g += SV_THREADS / 32) {
-      const size_t bh = (size_t)b * H_q + (size_t)hkv * ga + g;
-      const int pos = t0 + l32;
-      const int64_t bs = base_slot[l32 / BS];
-      float pv = 0.0f;
-      if (pos >= s_start && pos < s_end && bs >= 0 && g < ga) {
-        const float pr = __expf(scores[bh * (size_t)max_S + pos] - softmax_m[bh]) * softmax_inv_z[bh];
-        pv = pr * bf16_to_f32(sbase[bs + (l32 % BS)]);
-      }
-      float a = fabsf(pv);
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1) a = fmaxf(a, __shfl_xor(a, o, 32));
-      const float row_scale = a / 127.0f;
-      const float inv_scale = (row_scale > 0.0f) ? (1.0f / row_scale) : 0.0f;
-      int qv = (int)rintf(pv * inv_scale);
-      qv = max(-127, min(127, qv));
-      pq[g][l32] = qv;
-      if (l32 == 0) rs_sh[g] = row_scale;
-    }
-    __syncthreads();
-    int dot[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) dot[g] = 0;
-#pragma unroll 8
-    for (int j = 0; j < TQ_TILE; ++j) {
-      const int c = v_code<4>(vbuf + j * P, tid);
-#pragma unroll
-      for (int g = 0; g < G; ++g) dot[g] += pq[g][j] * c;
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) acc[g] += (float)dot[g] * rs_sh[g];
+    wave_lds_order();
   }
+  // the wavefronts' sums, in wavefront order: one head set at a time through LDS
+  float* red = reinterpret_cast<float*>(&stage[0][0]);  // [TQ_WAVES][8][64]
+  static_assert(sizeof(stage) >= TQ_WAVES * 8 * 64 * 4, "the final sums fit the staging areas");
 #pragma unroll
-  for (int g = 0; g < G; ++g)
-    if (g < ga)
-      partial[(((size_t)b * H_q + (size_t)hkv * ga + g) * (TQ_SPLITS * sub_count) + blockIdx.x) * D + tid] = acc[g];
+  for (int s = 0; s < NSET; ++s) {
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 8; ++t) red[(wave * 8 + t) * 64 + lane] = acc[s][t];
+    __syncthreads();
+    for (int i = tid; i < 8 * 64; i += TQ_WAVES * 64) {
+      float o = 0.f;
+#pragma unroll
+      for (int w = 0; w < TQ_WAVES; ++w) o += red[w * 512 + i];
+      const int t = i >> 6, h = s * 4 + ((i >> 4) & 3), c = i & 15;
+      const int d = t * 16 + 2 * (c >> 1) + (1 - (c & 1));
+      if (h < ga) partial[((head0 + h) * (size_t)(TQ_SPLITS * sub_count) + blockIdx.x) * D + d] = o;
+    }
+  }
 }
 
 // grid (B, H_q); adds split partials in order, then the top-k pre-correction.
@@ -394,27 +489,34 @@ extern "C" int jf_softmax_v_int8_tiles(const float* scores, const float* softmax
                "int8tc_softmax_v: workspace too small");
   hipStream_t st = (hipStream_t)stream;
   float* partial = reinterpret_cast<float*>(workspace);
-  // runs of at least four tiles per workgroup, at most sixteen workgroups per range (8 * sub_count <= max_S / 128
-  // partial rows: inside the workspace, which holds max(8, max_S / 64))
-  const int tiles_per_range = ((max_S + TQ_SPLITS - 1) / TQ_SPLITS + TQ_TILE - 1) / TQ_TILE + 1;
-  int sub_count = tiles_per_range / 4;
+  // A range is cut into `sub_count` runs (at most sixteen): enough workgroups of four wavefronts for four per CU, and
+  // at least two pairs of tiles per wavefront (8 * sub_count <= max_S / 64 partial rows: inside the workspace, which
+  // holds max(8, max_S / 64))
+  const int pairs_per_range = ((max_S + TQ_SPLITS - 1) / TQ_SPLITS + 2 * TQ_TILE - 1) / (2 * TQ_TILE) + 1;
+  const int want = (4 * 256 + TQ_SPLITS * H_kv * B - 1) / (TQ_SPLITS * H_kv * B);
+  int sub_count = pairs_per_range / (2 * TQ_WAVES);
+  sub_count = sub_count < want ? sub_count : want;
   sub_count = sub_count < 1 ? 1 : (sub_count > 16 ? 16 : sub_count);
   while (sub_count > 1 && (size_t)TQ_SPLITS * sub_count > (size_t)(max_S + 63) / 64) --sub_count;
-  dim3 grid(TQ_SPLITS * sub_count, H_kv, B), block(SV_THREADS);
-  JF_DISPATCH_G2(G, {
-    hipLaunchKernelGGL((tile_quantised_v_split_kernel<GG>), grid, block, 0, st, scores, softmax_m, softmax_inv_z, v_data,
-                       v_scales, block_table, seq_lens, partial, H_q, H_kv, max_S, max_blocks, num_slots, sub_count, G);
-  });
+  const dim3 grid(TQ_SPLITS * sub_count, H_kv, B);
+#define JF_TQ_LAUNCH(NSET)                                                                                              \
+  hipLaunchKernelGGL((tile_quantised_v_split_kernel<NSET>), grid, dim3(TQ_WAVES * 64), 0, st, scores, softmax_m,        \
+                     softmax_inv_z, v_data, v_scales, block_table, seq_lens, partial, H_q, H_kv, max_S, max_blocks,     \
+                     num_slots, sub_count, G)
+  if (G <= 4) JF_TQ_LAUNCH(1);
+  else if (G <= 8) JF_TQ_LAUNCH(2);
+  else JF_TQ_LAUNCH(4);
+#undef JF_TQ_LAUNCH
   JF_CHECK_LAUNCH();
-  // the pre-correction terms run on the merge kernel of the fused step where its limits allow (the same
-  // formula, p_j = exp(score_j - m) * inv_z with the caller's statistics), else in the combine kernel
-  const bool fast_precorr = topk_idx != nullptr && top_k <= 2048 && num_slots <= (1ll << 26) && ((uintptr_t)v_data & 3) == 0;
-  hipLaunchKernelGGL((combine_precorr_kernel<4, 1>), dim3(B, H_q), block, 0, st, partial, scores, softmax_m, softmax_inv_z,
-                     v_data, v_scales, block_table, seq_lens, fast_precorr ? nullptr : topk_idx, o_hat, o_old_unnorm, W, H_q,
-                     H_kv, max_S, max_blocks, num_slots, TQ_SPLITS * sub_count, top_k);
-  JF_CHECK_LAUNCH();
-  if (fast_precorr)
+  // the sum of the partials and the pre-correction terms run on the merge kernel of the fused step where its limits
+  // allow (the same formula, p_j = exp(score_j - m) * inv_z with the caller's statistics), else in the combine kernel
+  if (topk_idx != nullptr && top_k <= 2048 && num_slots <= (1ll << 26) && ((uintptr_t)v_data & 3) == 0)
     return precorr_int4_given_stats(scores, softmax_m, softmax_inv_z, v_data, v_scales, block_table, seq_lens, topk_idx, B,
-                                    H_q, H_kv, max_S, max_blocks, num_slots, top_k, o_old_unnorm, W, stream);
+                                    H_q, H_kv, max_S, max_blocks, num_slots, top_k, partial, TQ_SPLITS * sub_count, o_hat,
+                                    o_old_unnorm, W, stream);
+  hipLaunchKernelGGL((combine_precorr_kernel<4, 1>), dim3(B, H_q), dim3(SV_THREADS), 0, st, partial, scores, softmax_m,
+                     softmax_inv_z, v_data, v_scales, block_table, seq_lens, topk_idx, o_hat, o_old_unnorm, W, H_q, H_kv,
+                     max_S, max_blocks, num_slots, TQ_SPLITS * sub_count, top_k);
+  JF_CHECK_LAUNCH();
   return JF_OK;
 }

@@ -591,8 +591,10 @@ def _softmax_v(scores, m, iz, v_data, v_scales, block_table, seq_lens, topk_idx,
     dev = sc.device
     if outs is None:
         o_hat = torch.empty((B, H_q, HEAD_DIM), dtype=torch.float32, device=dev)
-        o_old = torch.zeros((B, H_q, HEAD_DIM), dtype=torch.float32, device=dev)
-        W = torch.zeros((B, H_q), dtype=torch.float32, device=dev)
+        # (with winners every kernel writes all of these; without, o_old and W may stay untouched)
+        fresh = torch.empty if topk_idx is not None else torch.zeros
+        o_old = fresh((B, H_q, HEAD_DIM), dtype=torch.float32, device=dev)
+        W = fresh((B, H_q), dtype=torch.float32, device=dev)
     else:
         o_hat, o_old, W = outs
         for t in outs:
