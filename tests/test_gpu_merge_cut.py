@@ -1,0 +1,43 @@
+"""The merge kernel's threshold search at the sizes of its three paths: a cut bucket of at most 64 members (ranked in
+registers), of up to 1024 (a list in LDS), of more (bisection), with ties across the cut, in both shapes of the kernel
+(1024 threads; 256 threads for more rows than compute units)."""
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import make_case, to_device
+from tests.test_gpu_fused import run_fused
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B", [1, 40])
+@pytest.mark.parametrize("copies", [40, 64, 65, 500, 1100])
+def test_equal_scores_around_the_cut(B, copies):
+    from jetfire_amd import _lib
+    S, K, Hq, Hkv = 2048, 64, 8, 1
+    c = make_case(93, 1, Hq, Hkv, S, 4, 4, 128, lens=[S])
+    if B > 1:      # the same sequence B times: the same pages, the same queries
+        for key in ("q", "bt", "lens"):
+            c[key] = np.repeat(c[key], B, axis=0)
+        c["B"] = B
+    d = to_device(c)
+    base = run_fused("k4v4", c, d, S, 32)
+    # `copies` positions get the key row of the 20th best position of head 0: one bucket of equal scores at the cut
+    order = torch.argsort(base[7][0, 0], descending=True, stable=True)
+    src, dst = int(order[20]), torch.sort(order[200:200 + copies]).values
+    bt = d["bt"][0]
+    slot = lambda t: bt[t // 16] * 16 + t % 16
+    d["kd"], d["ks"] = d["kd"].clone(), d["ks"].clone()
+    d["kd"][:, slot(dst)] = d["kd"][:, slot(torch.tensor([src], device="cuda"))]
+    d["ks"][:, slot(dst)] = d["ks"][:, slot(torch.tensor([src], device="cuda"))]
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(256))
+    try:
+        out = run_fused("k4v4", c, d, S, K)
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    scores, idx = out[7].cpu().numpy(), out[4].cpu().numpy()
+    for b in (0, B - 1):
+        for h in range(Hq):
+            want = np.sort(np.lexsort((np.arange(S), -scores[b, h]))[:K])
+            assert np.array_equal(idx[b, h], want), (b, h)
