@@ -1,7 +1,7 @@
 // Fused decode scan + top-k for gfx950: one pass over the packed K and V of every (sequence, kv-head),
 // no (B, H_q, S) score tensor in HBM.
 //
-// Launch 1, fused_scan_kernel, grid (n_splits, H_kv, B), 16 wavefronts per workgroup (8 where the register
+// Launch 1, fused_scan_kernel, grid (H_kv, n_splits, B), 16 wavefronts per workgroup (8 where the register
 // budget does not allow 1024 threads).  A workgroup owns L consecutive positions of one (sequence, kv-head)
 // and all G query heads of that kv-head.  The page table of the split is read once into LDS.  Key and value
 // rows are fetched in 64-position chunks with 16-byte loads whose lane addresses are consecutive inside a
@@ -447,7 +447,12 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   __shared__ unsigned long long tmax_sh;
   if (threadIdx.x == 0) tmax_sh = 0ull;
 
-  const int split = blockIdx.x, hkv = blockIdx.y, b = blockIdx.z;
+  // kv-head fastest: workgroups go to the eight XCDs in turn, and the heads of one (sequence, split) have equal work.
+  // With the split fastest an XCD got the same split (mod 8) of every sequence: in a batch of different lengths the
+  // early splits, which all sequences have, on some XCDs and the late, mostly empty ones on others.  Per layer, graph
+  // replay: 16 sequences of 983 .. 16384 positions, K4V4 63.7 -> 62.2 us (with splits of 1024: 125 -> 96); equal
+  // lengths gain too, 4 x 32768 K3V2 37.0 -> 36.3, 131072 K4V4 49.7 -> 48.6.
+  const int hkv = blockIdx.x, split = blockIdx.y, b = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: keeps wave-derived addresses in SGPRs
   const int S = max(0, min(p.max_S, p.seq_lens[b]));
@@ -3084,7 +3089,7 @@ int launch_scan(const FusedParams& p, hipStream_t st) {
   }
   if (prof) JF_CHECK_HIP(hipEventRecord(g_prof.ev[g_prof.used], st));
 #endif
-  hipLaunchKernelGGL(kern, dim3(p.n_splits, p.H_kv, p.B), dim3(ScanLds<SCHEME, G, NG>::NT), smem, st, p);
+  hipLaunchKernelGGL(kern, dim3(p.H_kv, p.n_splits, p.B), dim3(ScanLds<SCHEME, G, NG>::NT), smem, st, p);
   JF_CHECK_LAUNCH();
 #ifdef JF_DEBUG_HOOKS
   if (prof) {
