@@ -30,18 +30,20 @@ def _check(cond: bool, msg: str) -> None:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream of the tensor's device.  (The raw handle: building the Stream object that
+    torch.cuda.current_stream returns takes 2 us, at each of an operator's look-ups.)"""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-def _workspace(device: torch.device, nbytes: int, tag: str) -> torch.Tensor:
+def _workspace(device: torch.device, nbytes: int, tag: str, stream: Optional[int] = None) -> torch.Tensor:
     """Per-(device, stream, tag) scratch buffer that only grows; safe under stream ordering.  A buffer that is
     replaced by a larger one is kept alive: a HIP graph captured earlier on the stream has its address baked into
     its kernels, and the allocator must not hand that memory to anyone else while the graph can be replayed."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream, tag)
+    key = (device, torch.cuda.current_stream(device).cuda_stream if stream is None else stream, tag)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         if buf is not None:
@@ -347,16 +349,17 @@ def _stage_a_fast(fmt: int, q, kd, ks, bt, sl, max_S, H_q, H_kv, attn_scale, top
     B, dev = q.size(0), q.device
     scores = torch.empty((B, H_q, max_S), dtype=torch.float32, device=dev)
     idx = slots = m = iz = ws = None
+    stream = _stream(q)
     if top_k is not None:
         idx = torch.empty((B, H_q, top_k), dtype=torch.int64, device=dev)
         slots = torch.empty((B, H_q, top_k), dtype=torch.int64, device=dev)
         if stats:
             m = torch.empty((B, H_q), dtype=torch.float32, device=dev)
             iz = torch.empty((B, H_q), dtype=torch.float32, device=dev)
-        ws = _workspace(dev, lib.jf_fused_workspace_bytes(fmt, B, H_q, H_kv, int(max_S), int(top_k)), "fused")
+        ws = _workspace(dev, lib.jf_fused_workspace_bytes(fmt, B, H_q, H_kv, int(max_S), int(top_k)), "fused", stream)
     tail = (bt.data_ptr(), sl.data_ptr(), B, H_q, H_kv, int(max_S), bt.size(1), kd.size(1), 16, float(attn_scale),
             0 if top_k is None else int(top_k), scores.data_ptr(), _ptr(idx), _ptr(slots), _ptr(m), _ptr(iz), _ptr(ws),
-            0 if ws is None else ws.numel(), _stream(q))
+            0 if ws is None else ws.numel(), stream)
     if k_zp is None:
         _lib.check(lib.jf_stage_a_topk(fmt, HEAD_DIM // ks.size(2), q.data_ptr(), kd.data_ptr(), ks.data_ptr(), *tail))
     else:       # asymmetric INT2 keys (fmt 12)
@@ -366,9 +369,9 @@ def _stage_a_fast(fmt: int, q, kd, ks, bt, sl, max_S, H_q, H_kv, attn_scale, top
 
 
 def _check_top_k(top_k, name: str, minimum: int = 32) -> None:
-    _check(int(top_k) in SUPPORTED_TOP_K and int(top_k) >= minimum,
-           f"{name}: unsupported radix-select top_k={top_k} (supported: "
-           f"{','.join(str(k) for k in SUPPORTED_TOP_K if k >= minimum)})")
+    if not (int(top_k) in SUPPORTED_TOP_K and int(top_k) >= minimum):
+        raise RuntimeError(f"{name}: unsupported radix-select top_k={top_k} (supported: "
+                           f"{','.join(str(k) for k in SUPPORTED_TOP_K if k >= minimum)})")
 
 
 def _stage_a_args(q, k_data, k_scales, block_table, seq_lens, H_q, H_kv, packed):
@@ -588,7 +591,7 @@ def _softmax_v(scores, m, iz, v_data, v_scales, block_table, seq_lens, topk_idx,
     sc, vd, vs = scores.contiguous(), v_data.contiguous(), vs.contiguous()
     bt, sl = block_table.contiguous(), seq_lens.contiguous()
     B = sc.size(0)
-    dev = sc.device
+    dev, stream = sc.device, _stream(sc)
     if outs is None:
         o_hat = torch.empty((B, H_q, HEAD_DIM), dtype=torch.float32, device=dev)
         # (with winners every kernel writes all of these; without, o_old and W may stay untouched)
@@ -603,26 +606,26 @@ def _softmax_v(scores, m, iz, v_data, v_scales, block_table, seq_lens, topk_idx,
             and _fast_shape(H_q, H_kv, block_size, max_S, vd.size(1), top_k if topk_idx is not None else None)):
         fmt = {2: 32, 3: 33, 4: 44 if ng == 1 else 34}[nbits]      # (value side of the tag; 34: INT4 values, two groups)
         k_eff = int(top_k) if topk_idx is not None else 32
-        ws = _workspace(dev, lib.jf_fused_workspace_bytes(fmt, B, H_q, H_kv, int(max_S), k_eff), "fused")
+        ws = _workspace(dev, lib.jf_fused_workspace_bytes(fmt, B, H_q, H_kv, int(max_S), k_eff), "fused", stream)
         _lib.check(lib.jf_stage_b_softmax_v(
             fmt, HEAD_DIM // ng, sc.data_ptr(), vd.data_ptr(), vs.data_ptr(), bt.data_ptr(), sl.data_ptr(), _ptr(topk_idx),
             B, H_q, H_kv, int(max_S), bt.size(1), vd.size(1), 16, k_eff, o_hat.data_ptr(), o_old.data_ptr(), W.data_ptr(),
-            ws.data_ptr(), ws.numel(), _stream(sc)))
+            ws.data_ptr(), ws.numel(), stream))
         return [o_hat, o_old, W]
     need = lib.jf_softmax_v_workspace_bytes(B, H_q, int(max_S))
-    ws = _workspace(dev, need, "softmax_v")
+    ws = _workspace(dev, need, "softmax_v", stream)
     if m is not None:
         m, iz = m.contiguous(), iz.contiguous()
     if int8_tiles:
         _lib.check(lib.jf_softmax_v_int8_tiles(
             sc.data_ptr(), _ptr(m), _ptr(iz), vd.data_ptr(), vs.data_ptr(), bt.data_ptr(), sl.data_ptr(), _ptr(topk_idx),
             B, H_q, H_kv, int(max_S), bt.size(1), vd.size(1), int(block_size), int(top_k),
-            o_hat.data_ptr(), o_old.data_ptr(), W.data_ptr(), ws.data_ptr(), ws.numel(), _stream(sc)))
+            o_hat.data_ptr(), o_old.data_ptr(), W.data_ptr(), ws.data_ptr(), ws.numel(), stream))
         return [o_hat, o_old, W]
     _lib.check(lib.jf_softmax_v_pre_corr(
         sc.data_ptr(), _ptr(m), _ptr(iz), vd.data_ptr(), vs.data_ptr(), bt.data_ptr(), sl.data_ptr(), _ptr(topk_idx),
         B, H_q, H_kv, int(max_S), bt.size(1), vd.size(1), int(block_size), int(top_k), nbits, ng,
-        o_hat.data_ptr(), o_old.data_ptr(), W.data_ptr(), ws.data_ptr(), ws.numel(), _stream(sc)))
+        o_hat.data_ptr(), o_old.data_ptr(), W.data_ptr(), ws.data_ptr(), ws.numel(), stream))
     return [o_hat, o_old, W]
 
 
@@ -732,7 +735,8 @@ def fused_attn_topk(scheme: str, q, k_data, k_scales, v_data, v_scales, block_ta
     of int4_qk_scores (group 64 or 128), what the reference runs for INT4 keys with 64-channel groups."""
     lib = _lib.load()
     scheme_id = FUSED_SCHEMES.get(scheme)
-    _check(scheme_id is not None, f"unknown scheme {scheme!r} ({', '.join(sorted(FUSED_SCHEMES))})")
+    if scheme_id is None:  # (here and below: a message is put together only when it is raised)
+        raise RuntimeError(f"unknown scheme {scheme!r} ({', '.join(sorted(FUSED_SCHEMES))})")
     asym = scheme_id // 10 == 1
     kp, vp = {1: 32, 5: 64}.get(scheme_id // 10, 16 * (scheme_id // 10)), 16 * (scheme_id % 10)
     q, kd, ks, bt, sl = _stage_a_args(q, k_data, k_scales, block_table, seq_lens, H_q, H_kv, kp)
@@ -742,7 +746,8 @@ def fused_attn_topk(scheme: str, q, k_data, k_scales, v_data, v_scales, block_ta
         _check(k_zp.is_cuda and k_zp.dtype == torch.bfloat16 and k_zp.shape == ks.shape,
                "k_zp must be bf16 with the shape of k_scales")
     _gpu(v_data, v_scales)
-    _check(v_data.dtype == torch.uint8 and v_data.dim() == 3 and v_data.size(2) == vp, f"v_data last dim must be {vp}")
+    if not (v_data.dtype == torch.uint8 and v_data.dim() == 3 and v_data.size(2) == vp):
+        raise RuntimeError(f"v_data last dim must be {vp}")
     _check(v_scales.dtype == torch.bfloat16, "v_scales must be bf16")
     vs = (v_scales.unsqueeze(-1) if v_scales.dim() == 2 else v_scales).contiguous()
     vd = v_data.contiguous()
@@ -750,7 +755,8 @@ def fused_attn_topk(scheme: str, q, k_data, k_scales, v_data, v_scales, block_ta
     gs = HEAD_DIM // ks.size(2)
     if group_size is not None:
         _check(int(group_size) == gs, f"group_size={group_size} does not match the scale tensors ({gs})")
-    _check(int(top_k) in SUPPORTED_TOP_K, f"unsupported top_k={top_k}")
+    if int(top_k) not in SUPPORTED_TOP_K:
+        raise RuntimeError(f"unsupported top_k={top_k}")
     _check(kd.size(1) == vd.size(1), "K and V caches must have the same number of slots")
     B = q.size(0)
     dev = q.device
@@ -763,16 +769,17 @@ def fused_attn_topk(scheme: str, q, k_data, k_scales, v_data, v_scales, block_ta
     iz = torch.empty((B, H_q), dtype=torch.float32, device=dev) if return_stats else None
     scores = torch.empty((B, H_q, max_S), dtype=torch.float32, device=dev) if return_scores else None
     need = lib.jf_fused_workspace_bytes(scheme_id, B, H_q, H_kv, int(max_S), int(top_k))
-    ws = _workspace(dev, need, "fused")
+    stream = _stream(q)
+    ws = _workspace(dev, need, "fused", stream)
     head = (scheme_id, gs, q.data_ptr(), kd.data_ptr(), ks.data_ptr(), *((k_zp.data_ptr(),) if asym else ()),
             vd.data_ptr(), vs.data_ptr(), bt.data_ptr(),
             sl.data_ptr(), B, H_q, H_kv, int(max_S), bt.size(1), kd.size(1), int(block_size), float(attn_scale), int(top_k),
             idx.data_ptr(), slots.data_ptr(), o_hat.data_ptr(), o_old.data_ptr(), W.data_ptr(), _ptr(m), _ptr(iz),
             _ptr(scores))
     if blend is None and not asym:
-        _lib.check(lib.jf_fused_scan_topk(*head, ws.data_ptr(), ws.numel(), _stream(q)))
+        _lib.check(lib.jf_fused_scan_topk(*head, ws.data_ptr(), ws.numel(), stream))
     elif blend is None:
-        _lib.check(lib.jf_fused_scan_topk_asym(*head, None, None, ws.data_ptr(), ws.numel(), _stream(q)))
+        _lib.check(lib.jf_fused_scan_topk_asym(*head, None, None, ws.data_ptr(), ws.numel(), stream))
     else:
         o_new, out = blend
         _gpu(o_new, out)
@@ -781,7 +788,7 @@ def fused_attn_topk(scheme: str, q, k_data, k_scales, v_data, v_scales, block_ta
                "o_new / out must be (B, H_q, 128)")
         _check(o_new.is_contiguous() and out.is_contiguous(), "o_new / out must be contiguous")
         entry = lib.jf_fused_scan_topk_asym if asym else lib.jf_fused_scan_topk_blend
-        _lib.check(entry(*head, o_new.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(q)))
+        _lib.check(entry(*head, o_new.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), stream))
     out = [o_hat, slots, o_old, W, idx]
     if return_stats:
         out += [m, iz]
