@@ -58,7 +58,8 @@ const char* jf_version(void);
  * Replaces fused_quant_write_int{2,3,4}_sym (jetfire_vllm/kernels/fused_quant_write.py:242-270,
  * 337-369, 746-781): per (token, kv-head) and per group: scale = bf16(max(amax/qmax, 1e-8)),
  * code = clamp(rint(x / f32(scale)), +-qmax) + 2^(nbits-1), packed in the reference wire format and
- * scattered to out_data[h, slots[t], :], out_scale[h, slots[t], g].  slots[t] < 0 skips the token.
+ * scattered to out_data[h, slots[t], :], out_scale[h, slots[t], g].  Tokens with slots[t] < 0 (padding) or
+ * slots[t] >= num_slots are skipped, in this and in the other writers; num_slots <= 0 states no bound.
  * x is (T, H_kv, 128) bf16 with element strides x_stride_t / x_stride_h (last dim contiguous).
  * Data strides are in bytes, scale strides in bf16 elements.  nbits in {2,3,4};
  * group_size in {32, 64, 128}. */

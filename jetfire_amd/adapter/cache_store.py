@@ -85,7 +85,7 @@ class JetFireInt4CacheStore:
         self.v_scales = torch.zeros(self.num_kv_heads, self.num_slots, ng, dtype=torch.bfloat16, device=dev)
         self.v_zp = None
         self.k_zp = torch.zeros(self.num_kv_heads, self.num_slots, ng, dtype=torch.bfloat16, device=dev) if self.k_asymmetric else None
-        # one spare entry at the end takes the marks of padding tokens (slot < 0), so that marking needs no mask
+        # one spare entry at the end takes the marks of tokens outside the cache, so that marking needs no mask
         self._slot_filled_buf = torch.zeros(self.num_slots + 1, dtype=torch.bool, device=dev)
         self.slot_filled = self._slot_filled_buf[:self.num_slots]
         self.written_count = 0
@@ -158,7 +158,8 @@ class JetFireInt4CacheStore:
             return
         self._quantise(key_tok, value_tok, slots)
         if mark:
-            self._slot_filled_buf.index_fill_(0, torch.where(slots >= 0, slots, self.num_slots), True)
+            inside = (slots >= 0) & (slots < self.num_slots)
+            self._slot_filled_buf.index_fill_(0, torch.where(inside, slots, self.num_slots), True)
         if mirror:
             self._mirror(key_tok, value_tok, slots)
 
@@ -169,7 +170,7 @@ class JetFireInt4CacheStore:
 
     def write_slots(self, *, key: torch.Tensor, value: torch.Tensor, slot_mapping: torch.Tensor | None) -> int:
         """Quantise `key` / `value` (T, Hkv, D) into the rows named by `slot_mapping` (T,) and mirror them into
-        the shadow; negative slots are padding and are skipped.  Asynchronous: nothing here waits for the GPU.
+        the shadow; slots outside the cache (negative: padding) are skipped.  Asynchronous: nothing here waits for the GPU.
         Returns the number of rows offered (as the reference does)."""
         if slot_mapping is None or slot_mapping.numel() == 0:
             return 0

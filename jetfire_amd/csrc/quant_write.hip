@@ -78,15 +78,15 @@ __device__ inline void quant_row(const uint16_t* __restrict__ xrow, uint8_t* __r
 template <int NBITS>
 __global__ __launch_bounds__(256) void quant_write16_kernel(RowSrc s0, RowDst d0, RowSrc s1, RowDst d1,
                                                             const int64_t* __restrict__ slots, int64_t T,
-                                                            int H_kv, int n_tensors, int group_size) {
+                                                            int64_t num_slots, int H_kv, int n_tensors, int group_size) {
   const int l16 = threadIdx.x & 15;
   const uint32_t r = threadIdx.x >> 4;
   const int64_t t0 = (int64_t)blockIdx.x * 16;  // first token of the block (uniform: its products stay on the scalar unit)
   const int h = blockIdx.y;
   const int which = blockIdx.z;
   // rows past the end still take part in the cross-lane steps (they re-read the block's first row); the row is
-  // requested without waiting for its slot, so the two loads are in flight together; masked rows (slot < 0) only
-  // skip the stores
+  // requested without waiting for its slot, so the two loads are in flight together; masked rows (a slot outside the
+  // cache) only skip the stores
   const bool inside = t0 + r < T;
   const uint32_t re = inside ? r : 0u;
   const int64_t slot = slots[t0 + re];
@@ -96,9 +96,8 @@ __global__ __launch_bounds__(256) void quant_write16_kernel(RowSrc s0, RowDst d0
   // multiply-add instead of a 64 x 64 multiplication)
   const uint16_t* xrow = s.x + t0 * s.stride_t + (int64_t)h * s.stride_h + (uint64_t)re * (uint32_t)s.stride_t;
   const uint4 raw = reinterpret_cast<const uint4*>(xrow)[l16];
-  // (a slot index takes 32 bits: negative = masked row; anything beyond 2^32 cannot be a row of a cache and is
-  // skipped like a masked row)
-  const bool live = inside && (uint64_t)slot < ((uint64_t)1 << 32);
+  // (num_slots <= 2^32: quant16_row takes slots of 32 bits)
+  const bool live = inside && slot >= 0 && slot < num_slots;
   quant16_row<NBITS>(raw, d, h, (uint32_t)slot, live, l16, group_size);
 }
 
@@ -106,7 +105,7 @@ __global__ __launch_bounds__(256) void quant_write16_kernel(RowSrc s0, RowDst d0
 __global__ __launch_bounds__(256) void quant_write16_int2_asym_kernel(RowSrc s, RowDst d, uint16_t* __restrict__ zp_out,
                                                                       int64_t zp_stride_h, int64_t zp_stride_slot,
                                                                       const int64_t* __restrict__ slots, int64_t T,
-                                                                      int group_size) {
+                                                                      int64_t num_slots, int group_size) {
   const int l16 = threadIdx.x & 15;
   const int64_t tq = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
   const int h = blockIdx.y;
@@ -115,7 +114,7 @@ __global__ __launch_bounds__(256) void quant_write16_int2_asym_kernel(RowSrc s, 
   const int64_t slot = slots[t];
   const uint16_t* xrow = s.x + t * s.stride_t + (int64_t)h * s.stride_h;
   const uint4 raw = reinterpret_cast<const uint4*>(xrow)[l16];
-  const bool live = inside && slot >= 0;
+  const bool live = inside && slot >= 0 && slot < num_slots;
   quant16_row_int2_asym(raw, d, zp_out, zp_stride_h, zp_stride_slot, h, slot, live, l16, group_size);
 }
 
@@ -123,7 +122,7 @@ __global__ __launch_bounds__(256) void quant_write16_int2_asym_kernel(RowSrc s, 
 template <int NBITS>
 __global__ __launch_bounds__(256) void quant_write_kernel(RowSrc s0, RowDst d0, RowSrc s1, RowDst d1,
                                                           const int64_t* __restrict__ slots, int64_t T,
-                                                          int H_kv, int n_tensors, int group_size) {
+                                                          int64_t num_slots, int H_kv, int n_tensors, int group_size) {
   const int lane = threadIdx.x & 63;
   const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t total = T * H_kv * n_tensors;
@@ -133,13 +132,21 @@ __global__ __launch_bounds__(256) void quant_write_kernel(RowSrc s0, RowDst d0, 
   const int64_t t = rem / H_kv;
   const int h = (int)(rem - t * H_kv);
   const int64_t slot = slots[t];
-  if (slot < 0) return;
+  if (slot < 0 || slot >= num_slots) return;
   const RowSrc& s = which ? s1 : s0;
   const RowDst& d = which ? d1 : d0;
   const uint16_t* xrow = s.x + t * s.stride_t + (int64_t)h * s.stride_h;
   uint8_t* drow = d.data + (int64_t)h * d.data_stride_h + slot * d.data_stride_slot;
   uint16_t* srow = d.scale + (int64_t)h * d.scale_stride_h + slot * d.scale_stride_slot;
   quant_row<NBITS>(xrow, drow, srow, group_size, lane);
+}
+
+// Rows whose slot is not below the bound are skipped like padding.  num_slots <= 0: a caller that does not state the size
+// of its cache; quant16_row takes slots of 32 bits.
+inline int64_t slot_bound(int64_t num_slots) { return num_slots > 0 ? num_slots : INT64_MAX; }
+inline int64_t slot_bound32(int64_t num_slots) {
+  const int64_t lim = (int64_t)1 << 32;
+  return slot_bound(num_slots) < lim ? slot_bound(num_slots) : lim;
 }
 
 int check_common(const void* x, const int64_t* slots, int64_t T, int H_kv, int group_size,
@@ -167,7 +174,6 @@ extern "C" int jf_quant_write_sym(const uint16_t* x, int64_t x_stride_t, int64_t
                                   uint8_t* out_data, int64_t data_stride_h, int64_t data_stride_slot,
                                   uint16_t* out_scale, int64_t scale_stride_h, int64_t scale_stride_slot,
                                   int64_t num_slots, int group_size, int nbits, void* stream) {
-  (void)num_slots;
   int rc = check_common(x, slots, T, H_kv, group_size, data_stride_slot, nbits, out_data, out_scale);
   if (rc != JF_OK || T == 0) return rc;
   JF_CHECK_ARG(x_stride_t % 2 == 0 && x_stride_h % 2 == 0, "quant_write: x strides must be even");
@@ -177,16 +183,16 @@ extern "C" int jf_quant_write_sym(const uint16_t* x, int64_t x_stride_t, int64_t
   hipStream_t st = (hipStream_t)stream;
   if (rows_16b_aligned(x, x_stride_t, x_stride_h) && strides_fit_32(x_stride_t, data_stride_slot, scale_stride_slot)) {
     dim3 grid16((unsigned)((T + 15) / 16), (unsigned)H_kv, 1), block16(256);
-    if (nbits == 2) hipLaunchKernelGGL(quant_write16_kernel<2>, grid16, block16, 0, st, s, d, s, d, slots, T, H_kv, 1, group_size);
-    else if (nbits == 3) hipLaunchKernelGGL(quant_write16_kernel<3>, grid16, block16, 0, st, s, d, s, d, slots, T, H_kv, 1, group_size);
-    else hipLaunchKernelGGL(quant_write16_kernel<4>, grid16, block16, 0, st, s, d, s, d, slots, T, H_kv, 1, group_size);
+    if (nbits == 2) hipLaunchKernelGGL(quant_write16_kernel<2>, grid16, block16, 0, st, s, d, s, d, slots, T, slot_bound32(num_slots), H_kv, 1, group_size);
+    else if (nbits == 3) hipLaunchKernelGGL(quant_write16_kernel<3>, grid16, block16, 0, st, s, d, s, d, slots, T, slot_bound32(num_slots), H_kv, 1, group_size);
+    else hipLaunchKernelGGL(quant_write16_kernel<4>, grid16, block16, 0, st, s, d, s, d, slots, T, slot_bound32(num_slots), H_kv, 1, group_size);
     JF_CHECK_LAUNCH();
     return JF_OK;
   }
   dim3 grid((unsigned)((units + 3) / 4)), block(256);
-  if (nbits == 2) hipLaunchKernelGGL(quant_write_kernel<2>, grid, block, 0, st, s, d, s, d, slots, T, H_kv, 1, group_size);
-  else if (nbits == 3) hipLaunchKernelGGL(quant_write_kernel<3>, grid, block, 0, st, s, d, s, d, slots, T, H_kv, 1, group_size);
-  else hipLaunchKernelGGL(quant_write_kernel<4>, grid, block, 0, st, s, d, s, d, slots, T, H_kv, 1, group_size);
+  if (nbits == 2) hipLaunchKernelGGL(quant_write_kernel<2>, grid, block, 0, st, s, d, s, d, slots, T, slot_bound(num_slots), H_kv, 1, group_size);
+  else if (nbits == 3) hipLaunchKernelGGL(quant_write_kernel<3>, grid, block, 0, st, s, d, s, d, slots, T, slot_bound(num_slots), H_kv, 1, group_size);
+  else hipLaunchKernelGGL(quant_write_kernel<4>, grid, block, 0, st, s, d, s, d, slots, T, slot_bound(num_slots), H_kv, 1, group_size);
   JF_CHECK_LAUNCH();
   return JF_OK;
 }
@@ -199,7 +205,6 @@ extern "C" int jf_quant_write_int4_sym_kv(const uint16_t* key, int64_t k_stride_
                                           uint8_t* v_data, int64_t v_data_stride_h, int64_t v_data_stride_slot,
                                           uint16_t* v_scale, int64_t v_scale_stride_h, int64_t v_scale_stride_slot,
                                           int64_t num_slots, int group_size, void* stream) {
-  (void)num_slots;
   int rc = check_common(key, slots, T, H_kv, group_size, k_data_stride_slot, 4, k_data, k_scale);
   if (rc != JF_OK) return rc;
   rc = check_common(value, slots, T, H_kv, group_size, v_data_stride_slot, 4, v_data, v_scale);
@@ -213,12 +218,13 @@ extern "C" int jf_quant_write_int4_sym_kv(const uint16_t* key, int64_t k_stride_
       strides_fit_32(k_stride_t, k_data_stride_slot, k_scale_stride_slot) &&
       strides_fit_32(v_stride_t, v_data_stride_slot, v_scale_stride_slot)) {
     dim3 grid16((unsigned)((T + 15) / 16), (unsigned)H_kv, 2), block16(256);
-    hipLaunchKernelGGL(quant_write16_kernel<4>, grid16, block16, 0, (hipStream_t)stream, s0, d0, s1, d1, slots, T, H_kv, 2, group_size);
+    hipLaunchKernelGGL(quant_write16_kernel<4>, grid16, block16, 0, (hipStream_t)stream, s0, d0, s1, d1, slots, T,
+                       slot_bound32(num_slots), H_kv, 2, group_size);
     JF_CHECK_LAUNCH();
     return JF_OK;
   }
   dim3 grid((unsigned)((units + 3) / 4)), block(256);
-  hipLaunchKernelGGL(quant_write_kernel<4>, grid, block, 0, (hipStream_t)stream, s0, d0, s1, d1, slots, T, H_kv, 2, group_size);
+  hipLaunchKernelGGL(quant_write_kernel<4>, grid, block, 0, (hipStream_t)stream, s0, d0, s1, d1, slots, T, slot_bound(num_slots), H_kv, 2, group_size);
   JF_CHECK_LAUNCH();
   return JF_OK;
 }
@@ -228,7 +234,6 @@ extern "C" int jf_quant_write_int2_asym(const uint16_t* x, int64_t x_stride_t, i
                                         int64_t data_stride_slot, uint16_t* out_scale, int64_t scale_stride_h,
                                         int64_t scale_stride_slot, uint16_t* out_zp, int64_t zp_stride_h,
                                         int64_t zp_stride_slot, int64_t num_slots, int group_size, void* stream) {
-  (void)num_slots;
   int rc = check_common(x, slots, T, H_kv, group_size, data_stride_slot, 2, out_data, out_scale);
   if (rc != JF_OK || T == 0) return rc;
   JF_CHECK_ARG(out_zp, "quant_write_int2_asym: null zero-point tensor");
@@ -237,7 +242,7 @@ extern "C" int jf_quant_write_int2_asym(const uint16_t* x, int64_t x_stride_t, i
   RowDst d{out_data, data_stride_h, data_stride_slot, out_scale, scale_stride_h, scale_stride_slot};
   dim3 grid((unsigned)((T + 15) / 16), (unsigned)H_kv, 1), block(256);
   hipLaunchKernelGGL(quant_write16_int2_asym_kernel, grid, block, 0, (hipStream_t)stream, s, d, out_zp, zp_stride_h,
-                     zp_stride_slot, slots, T, group_size);
+                     zp_stride_slot, slots, T, slot_bound(num_slots), group_size);
   JF_CHECK_LAUNCH();
   return JF_OK;
 }

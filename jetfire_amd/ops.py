@@ -98,7 +98,7 @@ def _quant_write(x, slots, out_data, out_scale, group_size: int, nbits: int) -> 
         x.data_ptr(), x.stride(0), x.stride(1), slots.data_ptr(), T, H_kv,
         out_data.data_ptr(), out_data.stride(0), out_data.stride(1),
         out_scale.data_ptr(), out_scale.stride(0), out_scale.stride(1),
-        out_data.shape[1], int(group_size), nbits, _stream(x)))
+        min(out_data.shape[1], out_scale.shape[1]), int(group_size), nbits, _stream(x)))
 
 
 def fused_quant_write_int2_sym(val_tok, slots, out_data, out_scale, group_size: int) -> None:
@@ -138,7 +138,8 @@ def fused_quant_write_int2_asym(key_tok, slots, out_data, out_scale, out_zp, gro
     _lib.check(lib.jf_quant_write_int2_asym(
         key_tok.data_ptr(), key_tok.stride(0), key_tok.stride(1), slots.data_ptr(), T, H_kv,
         out_data.data_ptr(), out_data.stride(0), out_data.stride(1), out_scale.data_ptr(), out_scale.stride(0),
-        out_scale.stride(1), out_zp.data_ptr(), out_zp.stride(0), out_zp.stride(1), out_data.shape[1], int(group_size),
+        out_scale.stride(1), out_zp.data_ptr(), out_zp.stride(0), out_zp.stride(1),
+        min(out_data.shape[1], out_scale.shape[1], out_zp.shape[1]), int(group_size),
         _stream(key_tok)))
 
 
@@ -169,7 +170,7 @@ def fused_quant_write_int4_sym_kv(key_tok, value_tok, slot_idx, k_data, k_scales
         slot_idx.data_ptr(), T, H_kv,
         k_data.data_ptr(), k_data.stride(0), k_data.stride(1), k_scales.data_ptr(), k_scales.stride(0), k_scales.stride(1),
         v_data.data_ptr(), v_data.stride(0), v_data.stride(1), v_scales.data_ptr(), v_scales.stride(0), v_scales.stride(1),
-        k_data.shape[1], int(group_size), _stream(key_tok)))
+        min(t.shape[1] for t in (k_data, k_scales, v_data, v_scales)), int(group_size), _stream(key_tok)))
 
 
 def packed_dim(head_dim: int, nbits: int) -> int:

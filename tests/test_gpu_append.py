@@ -66,3 +66,39 @@ def test_store_append_of_unaligned_rows_takes_the_separate_operators():
     for x, y in ((a.k_data, b.k_data), (a.k_scales, b.k_scales), (a.v_data, b.v_data), (a.v_scales, b.v_scales),
                  (a.slot_filled, b.slot_filled), (a.k_shadow, b.k_shadow), (a.v_shadow, b.v_shadow)):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("kb,vb,asym,gs", [(3, 2, False, 64), (4, 4, False, 128), (2, 3, True, 64), (2, 4, False, 32)])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_slots_beyond_the_cache_are_skipped_by_every_writer(aligned, kb, vb, asym, gs):
+    """The same call does the same whatever the alignment of its token rows: slots past the end of the cache (and of its
+    filled marks and shadow) are dropped like padding.  `store` appends them among valid ones, `want` without them."""
+    from jetfire_amd import ops
+    from jetfire_amd.adapter.cache_store import JetFireInt4CacheStore
+    H, nblk, T = 2, 4, 40
+    rng = np.random.default_rng(kb * 10 + vb)
+    store, want = (JetFireInt4CacheStore(num_kv_heads=H, head_dim=128, group_size=gs, num_blocks=nblk, block_size=16,
+                                         device="cuda", k_nbits=kb, v_nbits=vb, k_asymmetric=asym) for _ in range(2))
+    x = [bf16_tensor(O.bf16_round(rng.standard_normal((T, H, 128)).astype(np.float32))).cuda() for _ in range(2)]
+    slots = rng.permutation(nblk * 16)[:T].astype(np.int64)
+    slots[[0, 7, 16, 31]] = [nblk * 16, nblk * 16 + 3, 2**32 + 5, -1]
+    keep = torch.from_numpy(np.flatnonzero((slots >= 0) & (slots < nblk * 16))).cuda()
+    slots = torch.from_numpy(slots).cuda()
+    rows = list(x)
+    if not aligned:      # rows that start at dwords (asymmetric keys have no writer for those: the values only)
+        for i in range(1 if asym else 0, 2):
+            rows[i] = torch.empty(T * H * 128 + 2, dtype=torch.bfloat16, device="cuda")[2:].view(T, H, 128).copy_(x[i])
+    store.write_slots(key=rows[0], value=rows[1], slot_mapping=slots)
+    want.write_slots(key=x[0][keep], value=x[1][keep], slot_mapping=slots[keep])
+    torch.cuda.synchronize()
+    names = ["k_data", "k_scales", "v_data", "v_scales", "slot_filled", "k_shadow", "v_shadow"] + (["k_zp"] if asym else [])
+    for name in names:
+        assert torch.equal(getattr(store, name), getattr(want, name)), name
+    # the writers called one by one, on caches that are the front part of larger ones
+    for name, tok, bits in (("fused_quant_write_int2_sym", rows[1], 2), ("fused_quant_write_int3_sym", rows[1], 3),
+                            ("fused_quant_write_int4_sym", rows[1], 4)):
+        data = torch.zeros(H, nblk * 32, 16 * bits, dtype=torch.uint8, device="cuda")
+        scales = torch.zeros(H, nblk * 32, 128 // gs, dtype=torch.bfloat16, device="cuda")
+        getattr(ops, name)(tok, slots, data[:, :nblk * 16], scales[:, :nblk * 16], gs)
+        assert not data[:, nblk * 16:].any() and not scales[:, nblk * 16:].any()
+        assert torch.equal(scales[0, :nblk * 16, 0] != 0, want.slot_filled)
