@@ -32,6 +32,9 @@ int jf_debug_phase_clock(void* device_buffer);
  * multiple of 256 and clamped to what fits the kernel's LDS) replaces the planner's choice of the split
  * length in jf_fused_scan_topk and jf_fused_workspace_bytes; 0 restores the planner.  Process-wide. */
 int jf_debug_split_len(int split_len);
+/* Test aid: *one_split = 1 if a call of these sizes (jf_fused_scan_topk, Stage A with top-k, Stage B, selection) runs
+ * as one launch whose scan workgroups merge by themselves, 0 if a merge launch follows; jf_debug_split_len applies. */
+int jf_debug_one_split(int scheme, int group_size, int B, int H_q, int H_kv, int max_S, int top_k, int* one_split);
 /* Test aids for the CPU pool, no counterpart in the reference.  jf_debug_pool_stall: the worker that claims `row` of
  * the next correction job sleeps `microseconds` before it computes the row (one shot), as if it had lost its core.
  * jf_debug_pool_wait_stragglers(0): jf_cpu_topk_attn returns as soon as every row is committed, like the hand-off

@@ -186,6 +186,16 @@ extern "C" int jf_debug_phase_clock(void* device_buffer) {
   return JF_OK;
 }
 
+extern "C" int jf_debug_one_split(int scheme, int group_size, int B, int H_q, int H_kv, int max_S, int top_k, int* one_split) {
+  JF_CHECK_ARG(known_scheme(scheme) && (group_size == 64 || group_size == 128) && B > 0 && H_q > 0 && H_kv > 0 &&
+                   H_q % H_kv == 0 && max_S >= 0 && top_k > 0 && one_split, "debug_one_split: bad arguments");
+  int L, ns, kc;
+  const int ng = scheme_ng(scheme, group_size);
+  fused_plan(scheme, ng, B, H_q, H_kv, max_S, top_k, &L, &ns, &kc);
+  *one_split = ns == 1 && one_split_fits(scheme, padded_group(H_q / H_kv), ng, L, top_k, kc);
+  return JF_OK;
+}
+
 extern "C" int jf_debug_split_len(int split_len) {
   JF_CHECK_ARG(split_len >= 0, "debug_split_len: negative length");
   g_force_split_len.store(split_len);

@@ -1679,7 +1679,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   [[maybe_unused]] float* tl_ohat = reinterpret_cast<float*>(tail + Tail::INTS);          // [G][D]
   [[maybe_unused]] int* tl_wslot = reinterpret_cast<int*>(tl_ohat + G * D);               // [G][top_k] paged slot of a winner
   [[maybe_unused]] float* tl_ww = reinterpret_cast<float*>(tl_wslot + (size_t)G * K);     // [G][top_k] its softmax weight
-  // [G][MEM] members of the cut bucket: key over inverted position, so that the larger word is the earlier winner
+  // [G][MEM] members of the cut bucket, as rank words
   [[maybe_unused]] unsigned long long* tl_mlist = reinterpret_cast<unsigned long long*>(tl_ww + (size_t)G * K);
   [[maybe_unused]] uint16_t* tl_list = reinterpret_cast<uint16_t*>(tl_mlist + G * Tail::MEM);  // [G][Kcap] candidate positions, ascending
   if constexpr (ONE) {
@@ -2037,7 +2037,9 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     if constexpr (HAS_TOPK) {
       // The candidates whose bucket lies before the cut bucket win; of the cut bucket's members the `need` largest
       // (ties: the lowest positions).  A wavefront takes a contiguous run of its head's list.
-      auto rank_word = [](uint32_t key, int pos) { return ((unsigned long long)key << 32) | (uint32_t)~pos; };
+      // (rank word: key over inverted position, 32 + 12 bits, so that the larger word is the earlier winner)
+      static_assert(Lds::LMAX <= 4096, "a position takes twelve bits");
+      auto rank_word = [](uint32_t key, int pos) { return ((unsigned long long)key << 12) | (uint32_t)(4095 - pos); };
       auto pair_of = [&](int it, int& h, int& lo, int& hi) -> int {  // -> segment, -1: nothing for this wavefront
         const int hs = wave + it * NW;
         h = hs / SEG;
@@ -2066,6 +2068,115 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         }
       }
       lds_barrier();
+      // More members than a rank list holds: the buckets are linear between the smallest and the largest score, so one
+      // outlying score (an attention sink) makes them wide, a correction of thousands puts hundreds of positions in
+      // one, and equal scores share one.  Radix select over the rank words, eight bits a pass from the highest bit in
+      // which a head's members differ: the head's wavefronts count the digits of their runs, each finds the digit of
+      // the last winner, and the head is done when the members left are as many as the winners left.  At most six
+      // passes (the words are distinct), two or three where scores differ.  Ranking each such member against the whole
+      // list, as this did at first, took 67 us per layer for 32 sequences x 2048 positions, K3V2, 8 kv-heads, top-k 256
+      // and one score at 40 sigma (this: 29.5, no outlier: 24.9, splits of 256 with a merge launch: 103), and 1055 us
+      // for 16 x 3900, K2V2, one head per kv-head, top-k 2048 and no outlier at all (31.6; 81).
+      unsigned long long last[NHS] = {};  // the last winner among the head's members
+      const unsigned long long crowded = __builtin_amdgcn_ballot_w64(
+          lane < GA && tl_need[min(lane, G - 1)] >= 0 && tl_mem[min(lane, G - 1)] > Tail::MEM);
+      if (crowded != 0ull) {  // (the same in every wavefront)
+        // (the staging area is dead since `combine`) per head the digit counts, the smallest and the largest member's key
+        int* rh = reinterpret_cast<int*>(stage);
+        uint32_t* ends = reinterpret_cast<uint32_t*>(rh + G * 256);
+        static_assert(NW * Lds::WAVE_STAGE >= G * (256 * 4 + 8), "the digit counts lie in the staging area");
+        auto for_members = [&](int h, int lo, int hi, auto&& f) {  // four list entries per lane in flight
+          for (int i0 = lo + lane; i0 - lane < hi; i0 += 256) {
+            uint32_t e[4];
+            float sv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) e[u] = (i0 + 64 * u < hi) ? tl_list[h * Kcap + i0 + 64 * u] : 0u;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) sv[u] = sc[h * L + min((int)(e[u] & 0x7fffu), n - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              if (e[u] & 0x8000u) f(rank_word(score_key(sv[u]), min((int)(e[u] & 0x7fffu), n - 1)));
+          }
+        };
+        for (int i = tid; i < G * 256; i += NT) rh[i] = 0;
+        if (tid < 2 * G) ends[tid] = (tid & 1) ? 0u : 0xffffffffu;
+        lds_barrier();
+#pragma unroll
+        for (int it = 0; it < NHS; ++it) {
+          int h, lo, hi;
+          if (pair_of(it, h, lo, hi) < 0 || !((crowded >> h) & 1ull)) continue;
+          uint32_t kmin = 0xffffffffu, kmax = 0u;
+          for_members(h, lo, hi, [&](unsigned long long w) { kmin = min(kmin, (uint32_t)(w >> 12)); kmax = max(kmax, (uint32_t)(w >> 12)); });
+          kmin = wave_min_u(kmin);
+          kmax = wave_max_u(kmax);
+          if (lane == 0) {
+            atomicMin(&ends[2 * h], kmin);
+            atomicMax(&ends[2 * h + 1], kmax);
+          }
+        }
+        lds_barrier();
+        int bits[NHS], need[NHS], left[NHS];
+        unsigned long long top[NHS];  // members in the running have these bits above the lowest `bits` ones
+#pragma unroll
+        for (int it = 0; it < NHS; ++it) {
+          int h, lo, hi;
+          bits[it] = need[it] = left[it] = 0;
+          top[it] = 0ull;
+          if (pair_of(it, h, lo, hi) < 0 || !((crowded >> h) & 1ull)) continue;
+          const uint32_t kmin = __builtin_amdgcn_readfirstlane(ends[2 * h]), kmax = __builtin_amdgcn_readfirstlane(ends[2 * h + 1]);
+          bits[it] = 12 + ((kmin == kmax) ? 0 : 32 - __clz((int)(kmin ^ kmax)));
+          top[it] = rank_word(kmax, 0) >> bits[it];
+          need[it] = __builtin_amdgcn_readfirstlane(tl_need[h]);
+          left[it] = __builtin_amdgcn_readfirstlane(tl_mem[h]);
+        }
+        for (int pass = 0; pass < 6; ++pass) {
+#pragma unroll
+          for (int it = 0; it < NHS; ++it) {
+            int h, lo, hi;
+            if (pair_of(it, h, lo, hi) < 0 || left[it] == need[it]) continue;
+            const int shift = max(0, bits[it] - 8);
+            for_members(h, lo, hi, [&](unsigned long long w) {
+              if ((w >> bits[it]) == top[it]) atomicAdd(&rh[h * 256 + (int)((w >> shift) & ((1u << (bits[it] - shift)) - 1u))], 1);
+            });
+          }
+          lds_barrier();
+#pragma unroll
+          for (int it = 0; it < NHS; ++it) {
+            int h, lo, hi;
+            const int seg = pair_of(it, h, lo, hi);
+            if (seg < 0) continue;
+            if (left[it] != need[it]) {
+              // lane l owns the digits 255 - 4l .. 252 - 4l: a scan over the lanes counts from the largest digit down
+              const v4i c = *reinterpret_cast<const v4i*>(rh + h * 256 + 252 - 4 * lane);
+              const int mine = (c[0] + c[1]) + (c[2] + c[3]);
+              int above = wave_incl_scan_i(mine) - mine, digit = -1, count = 0, before = 0;
+#pragma unroll
+              for (int u = 3; u >= 0; --u) {
+                if (above < need[it] && need[it] <= above + c[u]) {
+                  digit = 252 - 4 * lane + u;
+                  count = c[u];
+                  before = above;
+                }
+                above += c[u];
+              }
+              const unsigned long long who = __builtin_amdgcn_ballot_w64(digit >= 0);
+              const int src = (who != 0ull) ? __ffsll((long long)who) - 1 : 0;
+              const int shift = max(0, bits[it] - 8);
+              top[it] = (top[it] << (bits[it] - shift)) | (uint32_t)__builtin_amdgcn_readlane(digit, src);
+              need[it] -= __builtin_amdgcn_readlane(before, src);
+              left[it] = __builtin_amdgcn_readlane(count, src);
+              bits[it] = shift;
+            }
+            if (seg == 0 && lane == 0) tl_nout[h] = left[it] - need[it];  // (free until the winners are counted)
+          }
+          lds_barrier();
+          if (__builtin_amdgcn_ballot_w64(lane < GA && tl_nout[min(lane, G - 1)] != 0) == 0ull) break;
+          for (int i = tid; i < G * 256; i += NT) rh[i] = 0;
+          lds_barrier();
+        }
+#pragma unroll
+        for (int it = 0; it < NHS; ++it) last[it] = top[it] << bits[it];
+      }
       uint32_t wmask[NHS];  // bit j: this lane's candidate of step j wins (at most 32 steps: one_split_fits)
 #pragma unroll
       for (int it = 0; it < NHS; ++it) {
@@ -2075,11 +2186,9 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         if (seg < 0) continue;
         const int need = __builtin_amdgcn_readfirstlane(tl_need[h]), m = __builtin_amdgcn_readfirstlane(tl_mem[h]);
         const uint16_t* cl = tl_list + h * Kcap;
-        // the last winner among the members: every wavefront of the head ranks them itself, one member per lane, the
-        // others' words as scalars (no exchange, no LDS latency per member)
-        unsigned long long last = 0ull;
-        const bool from_list = m <= Tail::MEM;
-        if (need >= 0 && from_list) {
+        // a short list: every wavefront of the head ranks the members itself, one per lane, the others' words as
+        // scalars (no exchange, no LDS latency per member)
+        if (need >= 0 && m <= Tail::MEM) {
           const unsigned long long own = (lane < m) ? tl_mlist[h * Tail::MEM + lane] : 0ull;
           int rank = 0;
           for (int k = 0; k < m; ++k) {
@@ -2089,8 +2198,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           }
           const unsigned long long who = __builtin_amdgcn_ballot_w64(lane < m && rank == need - 1);
           const int src = (who != 0ull) ? __ffsll((long long)who) - 1 : 0;
-          last = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), src) << 32) |
-                 (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, src);
+          last[it] = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), src) << 32) |
+                     (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, src);
         }
         int total = 0;
         for (int i0 = lo, j = 0; i0 < hi; i0 += 64, ++j) {
@@ -2099,19 +2208,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           bool win = i < hi;
           if (e & 0x8000u) {
             const int pos = min((int)(e & 0x7fffu), n - 1);
-            const unsigned long long own = rank_word(score_key(sc[h * L + pos]), pos);
-            if (from_list) {
-              win = own >= last;
-            } else {  // heavily tied: against every member in the list
-              const int cnt = tl_cnt[h];
-              int rank = 0;
-              for (int k = 0; k < cnt; ++k) {
-                const uint32_t f = cl[k];
-                const int fp = min((int)(f & 0x7fffu), n - 1);
-                rank += ((f & 0x8000u) && rank_word(score_key(sc[h * L + fp]), fp) > own) ? 1 : 0;
-              }
-              win = rank < need;
-            }
+            win = rank_word(score_key(sc[h * L + pos]), pos) >= last[it];
           }
           wmask[it] |= (win ? 1u : 0u) << j;
           total += __popcll(__builtin_amdgcn_ballot_w64(win));

@@ -23,11 +23,23 @@ def _plan(scheme_id, gs, B, Hq, Hkv, S, K):
     return [o.value for o in out]
 
 
+def _one_split(scheme_id, gs, B, Hq, Hkv, S, K, split_len):
+    """Whether the call merges by itself when its splits are `split_len` positions long."""
+    from jetfire_amd import _lib
+    out = C.c_int(-1)
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
+    try:
+        _lib.check(_lib.debug_hook("jf_debug_one_split")(scheme_id, gs, B, Hq, Hkv, S, K, C.byref(out)))
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    return out.value
+
+
 def _both(scheme, c, d, S, K):
     """The call with one split, and with splits of 256 positions."""
     from jetfire_amd import _lib
     res = []
-    for split in (4096, 256):
+    for split in (-(-S // 256) * 256, 256):
         _lib.check(_lib.debug_hook("jf_debug_split_len")(split))
         try:
             res.append([t.clone() for t in run_fused(scheme, c, d, S, K)])
@@ -90,3 +102,78 @@ def test_plan_takes_one_split_for_short_and_many_sequences():
     assert _plan(44, 128, 1, 32, 8, 777, 64)[1] == 1
     assert _plan(32, 64, 32, 32, 8, 2048, 256)[1] == 1
     assert _plan(44, 128, 1, 32, 8, 4096, 64)[1] > 1
+
+
+def _crowded(d, c, S, kind):
+    """Scores that put far more positions in the bucket of the cut than a rank list holds."""
+    kd, ks, bt = d["kd"].clone(), d["ks"].clone(), d["bt"]
+    pos = torch.arange(S, device="cuda")
+    for b in range(bt.size(0)):
+        slot = bt[b, pos // 16] * 16 + pos % 16
+        if kind == "outlier":      # one key row three hundred times the others: the buckets of every head are that much wider
+            ks[:, slot[S // 3]] *= 300
+        elif kind == "levels":     # eight distinct rows: eight scores, each shared by an eighth of the positions
+            src = slot[pos % 8]
+            kd[:, slot], ks[:, slot] = d["kd"][:, src], d["ks"][:, src]
+    d["kd"], d["ks"] = kd, ks
+
+
+@pytest.mark.parametrize("kind", ["outlier", "levels", "plain"])
+@pytest.mark.parametrize("scheme,kb,vb,gs,G,S,K", [
+    ("k2v2", 2, 2, 64, 1, 3900, 2048),
+    ("k4v4", 4, 4, 128, 2, 2048, 512),
+    ("k4v4", 4, 4, 128, 4, 777, 64),
+    ("k3v2", 3, 2, 64, 4, 2048, 256),
+    ("k3v2", 3, 2, 64, 7, 1000, 256),
+    ("k3v2", 3, 2, 64, 8, 512, 256),
+    ("k3v3", 3, 3, 64, 16, 256, 32),
+])
+def test_one_split_selects_from_a_crowded_bucket(scheme, kb, vb, gs, G, S, K, kind):
+    from jetfire_amd import ops
+    Hkv, lens = 2, [S, S - S // 5]
+    c = make_case(94, 2, G * Hkv, Hkv, S, kb, vb, gs, lens=lens)
+    d = to_device(c)
+    _crowded(d, c, S, kind)
+    assert _one_split(ops.FUSED_SCHEMES[scheme], gs, 2, G * Hkv, Hkv, S, K, -(-S // 256) * 256)
+    one, cut = _both(scheme, c, d, S, K)
+    assert torch.equal(one[4], cut[4]) and torch.equal(one[1], cut[1])
+    scores = one[7].cpu().numpy()
+    for b, n in enumerate(lens):
+        for h in range(G * Hkv):
+            want = np.sort(np.lexsort((np.arange(n), -scores[b, h, :n]))[:K])
+            got = one[4][b, h].cpu().numpy()
+            assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -1).all()
+
+
+@pytest.mark.parametrize("kind", ["outlier", "levels", "plain"])
+@pytest.mark.parametrize("scheme,kb,vb,gs,B,Hkv,G,S,K", [
+    ("k2v2", 2, 2, 64, 16, 8, 1, 3900, 2048),
+    ("k4v4", 4, 4, 128, 32, 8, 4, 1024, 512),
+    ("k3v2", 3, 2, 64, 16, 4, 8, 1000, 256),
+])
+def test_one_split_is_no_slower_than_the_merge_launch(scheme, kb, vb, gs, B, Hkv, G, S, K, kind):
+    """Bounded work per member of the cut bucket: ranking each against the whole list took two to seventeen times the
+    merge launch's time here."""
+    from jetfire_amd import _lib, ops
+    c = make_case(95, B, G * Hkv, Hkv, S, kb, vb, gs)
+    d = to_device(c)
+    _crowded(d, c, S, kind)
+    times = []
+    for split in (-(-S // 256) * 256, 256):
+        assert _one_split(ops.FUSED_SCHEMES[scheme], gs, B, G * Hkv, Hkv, S, K, split) == (split > 256)
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(split))
+        try:
+            best = float("inf")
+            for _ in range(6):
+                e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                torch.cuda.synchronize()
+                e0.record()
+                for _ in range(10):
+                    run_fused(scheme, c, d, S, K)
+                e1.record()
+                e1.synchronize()
+                best = min(best, e0.elapsed_time(e1))
+            times.append(best)
+        finally:
+            _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    assert times[0] <= 1.5 * times[1], times
