@@ -1823,6 +1823,13 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       }
       ok = tot <= Kcap;
     }
+    // A NaN falls into bucket 0, which says nothing about its place in the order of the keys, the order a merge launch
+    // goes by.  Nobody looks at the keys of the buckets before the cut here, so such a head takes the exact selection;
+    // its sum of weights is a NaN too (and where a score is +infinity or all are -infinity).
+    if constexpr (ONE) {
+      const float lw = lsum_sh[min(lane, NW - 1)][h];
+      ok = ok && __builtin_amdgcn_ballot_w64(lw != lw) == 0ull;
+    }
     if (clk && tid == 0) clk[6] = JF_CLK();
     const float* srow = sc + h * L;
     uint32_t* ck = p.cand_key + (part_base + (size_t)h * p.n_splits) * Kcap;

@@ -115,10 +115,14 @@ def _crowded(d, c, S, kind):
         elif kind == "levels":     # eight distinct rows: eight scores, each shared by an eighth of the positions
             src = slot[pos % 8]
             kd[:, slot], ks[:, slot] = d["kd"][:, src], d["ks"][:, src]
+        elif kind == "infinite":   # scores of both signs' infinity: no finite range, everything in one bucket
+            ks[:, slot[5]] = float("inf")
+        elif kind == "nan":        # a finite range, and scores without a place in it
+            ks[:, slot[[5, S // 2]]] = float("nan")
     d["kd"], d["ks"] = kd, ks
 
 
-@pytest.mark.parametrize("kind", ["outlier", "levels", "plain"])
+@pytest.mark.parametrize("kind", ["outlier", "levels", "plain", "infinite", "nan"])
 @pytest.mark.parametrize("scheme,kb,vb,gs,G,S,K", [
     ("k2v2", 2, 2, 64, 1, 3900, 2048),
     ("k4v4", 4, 4, 128, 2, 2048, 512),
@@ -140,7 +144,10 @@ def test_one_split_selects_from_a_crowded_bucket(scheme, kb, vb, gs, G, S, K, ki
     scores = one[7].cpu().numpy()
     for b, n in enumerate(lens):
         for h in range(G * Hkv):
-            want = np.sort(np.lexsort((np.arange(n), -scores[b, h, :n]))[:K])
+            # the order of the kernels' keys: NaNs with the sign bit below everything, the others above
+            u = scores[b, h, :n].view(np.uint32)
+            key = np.where(u >> 31, ~u, u | np.uint32(1 << 31)).astype(np.int64)
+            want = np.sort(np.lexsort((np.arange(n), -key))[:K])
             got = one[4][b, h].cpu().numpy()
             assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -1).all()
 
