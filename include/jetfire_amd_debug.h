@@ -35,6 +35,9 @@ int jf_debug_split_len(int split_len);
 /* Test aid: *one_split = 1 if a call of these sizes (jf_fused_scan_topk, Stage A with top-k, Stage B, selection) runs
  * as one launch whose scan workgroups merge by themselves, 0 if a merge launch follows; jf_debug_split_len applies. */
 int jf_debug_one_split(int scheme, int group_size, int B, int H_q, int H_kv, int max_S, int top_k, int* one_split);
+/* Test aid: how many workgroups of the merge kernel's light shape (many rows, few candidates each) one compute unit
+ * holds, the smallest figure over the value formats. */
+int jf_debug_light_merge_per_cu(int* workgroups);
 /* Test aids for the CPU pool, no counterpart in the reference.  jf_debug_pool_stall: the worker that claims `row` of
  * the next correction job sleeps `microseconds` before it computes the row (one shot), as if it had lost its core.
  * jf_debug_pool_wait_stragglers(0): jf_cpu_topk_attn returns as soon as every row is committed, like the hand-off

@@ -92,6 +92,7 @@ DEBUG_SIGNATURES = {
     "jf_profile_scan_end": (I, [P, P]),
     "jf_debug_phase_clock": (I, [P]),
     "jf_debug_one_split": (I, [I, I, I, I, I, I, I, P]),
+    "jf_debug_light_merge_per_cu": (I, [P]),
     "jf_debug_split_len": (I, [I]),
     "jf_debug_pool_stall": (I, [L, I]),
     "jf_debug_pool_wait_stragglers": (I, [I]),

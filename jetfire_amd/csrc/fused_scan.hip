@@ -196,6 +196,24 @@ extern "C" int jf_debug_one_split(int scheme, int group_size, int B, int H_q, in
   return JF_OK;
 }
 
+extern "C" int jf_debug_light_merge_per_cu(int* workgroups) {
+  JF_CHECK_ARG(workgroups, "debug_light_merge_per_cu: null pointer");
+  const void* kernels[] = {
+      reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 2, 1, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>),
+      reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 2, 2, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>),
+      reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 3, 1, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>),
+      reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 3, 2, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>),
+      reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 4, 1, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>),
+      reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 4, 2, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>)};
+  *workgroups = 0;
+  for (const void* k : kernels) {
+    int n = 0;
+    JF_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, MG_LIGHT_THREADS, 0));
+    if (*workgroups == 0 || n < *workgroups) *workgroups = n;
+  }
+  return JF_OK;
+}
+
 extern "C" int jf_debug_split_len(int split_len) {
   JF_CHECK_ARG(split_len >= 0, "debug_split_len: negative length");
   g_force_split_len.store(split_len);

@@ -2924,48 +2924,55 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   const int dwi = lane % DW, w_in = lane / DW;
   const int g_of_lane = (NG == 1) ? 0 : ((dwi * CPD) / (D / NG));
   constexpr int UNR = Pre::UNR;  // 256 winners per pass
-  // (a workgroup of fewer than sixteen wavefronts takes several roles per wavefront; their rows are requested together,
-  // one gather latency instead of one per role: 9.4 k -> 7.8 k cycles at 512 rows of 256 INT4 winners)
-  constexpr int RPW = VWAVES / MG_WAVES;
-  float acc[RPW][CPD], accw[RPW];
+  // A workgroup of fewer than sixteen wavefronts takes several roles per wavefront, two at a time: their rows are
+  // requested together (one gather latency for both), roles past the last winner are left out, and the kernel stays
+  // below the 96 registers that five workgroups of the light shape per CU allow:
+  // 73 - 87 instead of the 105 - 126 that all four roles at once take (four workgroups per CU).  Per layer: 20
+  // sequences x 64 heads of up to 2806 positions, K4V4, top-k 256 52.9 -> 47.6 us; 10 x 128 heads of up to 636, INT4
+  // with 64-channel groups, top-k 512 55.2 -> 48.2; 29 x 128 heads of up to 77, INT2 values 72.9 -> 66.0; 512 rows as before.
+  constexpr int RPW = VWAVES / MG_WAVES, RP = (RPW >= 2) ? 2 : 1;
 #pragma unroll
-  for (int r = 0; r < RPW; ++r) {
-    accw[r] = 0.f;
+  for (int r0 = 0; r0 < RPW; r0 += RP) {
+    float acc[RP][CPD], accw[RP];
 #pragma unroll
-    for (int c = 0; c < CPD; ++c) acc[r][c] = 0.f;
-  }
-  for (int kb = 0; kb + wave * WPI < n_out; kb += UNR * VWAVES * WPI) {
-    uint32_t word[RPW][UNR], word_b[RPW][UNR];  // (word_b: INT3 only)
-    uint16_t sbits[RPW][UNR];
-    float wv[RPW][UNR];
+    for (int r = 0; r < RP; ++r) {
+      accw[r] = 0.f;
 #pragma unroll
-    for (int r = 0; r < RPW; ++r)
+      for (int c = 0; c < CPD; ++c) acc[r][c] = 0.f;
+    }
+    for (int kb = (wave + r0 * MG_WAVES) * WPI; kb < n_out; kb += UNR * VWAVES * WPI) {
+      uint32_t word[RP][UNR], word_b[RP][UNR];  // (word_b: INT3 only)
+      uint16_t sbits[RP][UNR];
+      float wv[RP][UNR];
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        const int k = kb + (wave + r * MG_WAVES) * WPI + u * VWAVES * WPI + w_in;
-        const int slot = (k < n_out) ? win_idx[k] : -1;
-        wv[r][u] = (slot >= 0) ? __builtin_bit_cast(float, win_key[k]) : 0.f;
-        const uint32_t sl = (uint32_t)max(slot, 0);
-        Pre::fetch(vbase, sl, dwi, word[r][u], word_b[r][u]);
-        sbits[r][u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
-      }
+      for (int r = 0; r < RP; ++r)
 #pragma unroll
-    for (int r = 0; r < RPW; ++r)
+        for (int u = 0; u < UNR; ++u) {
+          const int k = kb + (r * MG_WAVES + u * VWAVES) * WPI + w_in;
+          const int slot = (k < n_out) ? win_idx[k] : -1;
+          wv[r][u] = (slot >= 0) ? __builtin_bit_cast(float, win_key[k]) : 0.f;
+          const uint32_t sl = (uint32_t)max(slot, 0);
+          Pre::fetch(vbase, sl, dwi, word[r][u], word_b[r][u]);
+          sbits[r][u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
+        }
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        const float ws = wv[r][u] * bf16_to_f32(sbits[r][u]);  // zero for padding rows
-        Pre::add(word[r][u], word_b[r][u], ws, acc[r]);
-        if (dwi == 0) accw[r] += wv[r][u];
-      }
-  }
+      for (int r = 0; r < RP; ++r)
 #pragma unroll
-  for (int r = 0; r < RPW; ++r) {  // over the WPI winners of a wavefront instruction; then over the roles through LDS
-    const int vw = wave + r * MG_WAVES;
-    const int chan = Pre::reduce(acc[r], lane);
-    old_sh[vw][chan] = acc[r][0];
-    old_sh[vw][chan + 1] = acc[r][1];
-    const float wsum = wave_sum(accw[r]);  // only the dwi == 0 lanes hold weights
-    if (lane == 0) w_sh[vw] = wsum;
+        for (int u = 0; u < UNR; ++u) {
+          const float ws = wv[r][u] * bf16_to_f32(sbits[r][u]);  // zero for padding rows
+          Pre::add(word[r][u], word_b[r][u], ws, acc[r]);
+          if (dwi == 0) accw[r] += wv[r][u];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < RP; ++r) {  // over the WPI winners of a wavefront instruction; then over the roles through LDS
+      const int vw = wave + (r0 + r) * MG_WAVES;
+      const int chan = Pre::reduce(acc[r], lane);
+      old_sh[vw][chan] = acc[r][0];
+      old_sh[vw][chan + 1] = acc[r][1];
+      const float wsum = wave_sum(accw[r]);  // only the dwi == 0 lanes hold weights
+      if (lane == 0) w_sh[vw] = wsum;
+    }
   }
   lds_barrier();
   if (tid < D) {

@@ -41,3 +41,14 @@ def test_equal_scores_around_the_cut(B, copies):
         for h in range(Hq):
             want = np.sort(np.lexsort((np.arange(S), -scores[b, h]))[:K])
             assert np.array_equal(idx[b, h], want), (b, h)
+
+
+def test_five_rows_of_the_light_shape_share_a_compute_unit():
+    """What the light shape is for (many rows, few candidates each): its registers and LDS leave room for five
+    workgroups per compute unit."""
+    import ctypes as C
+
+    from jetfire_amd import _lib
+    n = C.c_int(0)
+    _lib.check(_lib.debug_hook("jf_debug_light_merge_per_cu")(C.byref(n)))
+    assert n.value >= 5
