@@ -192,7 +192,7 @@ extern "C" int jf_debug_one_split(int scheme, int group_size, int B, int H_q, in
   int L, ns, kc;
   const int ng = scheme_ng(scheme, group_size);
   fused_plan(scheme, ng, B, H_q, H_kv, max_S, top_k, &L, &ns, &kc);
-  *one_split = ns == 1 && one_split_fits(scheme, padded_group(H_q / H_kv), ng, L, top_k, kc);
+  *one_split = ns == 1 && one_split_merges(scheme, padded_group(H_q / H_kv), ng, B, H_q, H_kv, max_S, L, top_k, kc);
   return JF_OK;
 }
 

@@ -123,7 +123,7 @@ struct FusedParams {
   const int64_t* block_table;
   const int32_t* seq_lens;
   int B, H_q, H_kv, max_S, max_blocks;
-  int one_split;  // (host) the scan merges by itself: n_splits == 1 and ScanTail fits (one_split_fits)
+  int one_split;  // (host) the scan merges by itself: n_splits == 1 and one_split_merges
   int g_act;  // query heads per kv-head (H_q / H_kv); the kernel's G is this rounded up to 1, 2, 4, 8 or 16
   int64_t num_slots;
   float attn_scale;
@@ -3065,12 +3065,11 @@ inline double merge_pass_us(double fixed, long cands) {
 
 // Two-stage merge when one workgroup per row would face more than MG_REG_CANDS candidates: the number of
 // parts (at most MG_REG_CANDS / top_k, so that the final merge keeps its candidates in registers, and at least
-// two lists per part) with the smallest estimated time.  parts == 1: single stage.
+// two lists per part) with the smallest estimated time, which is returned.  parts == 1: single stage.
 inline double merge_plan(int rows, int ns, int kc, int top_k, int* parts_out, int* spp_out) {
   *parts_out = 1;
   *spp_out = ns;
-  const double wide = 1.5 * (top_k > 256 ? (double)top_k / 256.0 - 1.0 : 0.0);  // slots and pre-correction of the winners
-  double best = merge_pass_us(kMergeFixed, (long)ns * kc) + wide;
+  double best = merge_pass_us(kMergeFixed, (long)ns * kc);
   if ((long long)ns * kc <= MG_REG_CANDS || ns < 4) return best;
   // (wide corrections run the 32-register shape throughout: its 32768 candidates bound the final merge)
   int cap = (top_k > FS_LDS_TOPK ? 4 * MG_REG_CANDS : MG_REG_CANDS) / top_k;
@@ -3081,7 +3080,7 @@ inline double merge_plan(int rows, int ns, int kc, int top_k, int* parts_out, in
     const long wgs = (long)(rows > 0 ? rows : 1) * parts;
     const double rounds = (double)((wgs + 511) / 512);  // two workgroups per CU
     const double us = kPartialFixed + rounds * (merge_pass_us(kPartialFixed, (long)spp * kc) - kPartialFixed) +
-                      merge_pass_us(kMergeFixed, (long)parts * top_k) + wide;
+                      merge_pass_us(kMergeFixed, (long)parts * top_k);
     if (us < best) {
       best = us;
       *parts_out = parts;
@@ -3089,6 +3088,37 @@ inline double merge_plan(int rows, int ns, int kc, int top_k, int* parts_out, in
     }
   }
   return best;
+}
+
+// Estimated microseconds of the merge launches: the above, the slots and pre-correction of the winners, and what a launch
+// of more rows than CUs takes (16 us at 512 rows, 18 at 1024).
+inline double merge_us(int rows, int max_S, int ns, int kc, int top_k) {
+  constexpr double kManyRows = 5.0, kPerRowBeyond = 0.005;
+  const int winners = top_k < max_S ? top_k : max_S, cus = device_cus();
+  int parts, spp;
+  double us = merge_plan(rows, ns, kc, top_k, &parts, &spp);
+  if (winners > 256) us += 1.5 * ((double)winners / 256.0 - 1.0);
+  if (rows > cus) us += kManyRows + kPerRowBeyond * (double)(rows - cus);
+  return us;
+}
+
+// Estimated microseconds by which a scan workgroup gets longer when it merges by itself.  The sums over the winners'
+// value rows bound it: a wavefront takes 64 rows of one head at a time, the heads of the kv-head share the workgroup's
+// wavefronts (more heads than wavefronts: one after the other), and all wavefronts of a SIMD share its vector ALU.
+// Measured against the merge launch at the same split length, up to 256 rows: 64-row batches per wavefront 1 / 2 / 4 with
+// sixteen wavefronts 3 us faster / equal / 4 us slower, 1 / 2 / 4 / 8 with eight wavefronts 4 and 2 us faster, 2 and up to 10
+// slower; with more rows the launch takes longer and the workgroups here do not.
+inline double one_split_us(int G, int units, int max_S, int top_k) {
+  constexpr double kFixed = 1.4, kPerBatch = 0.25;
+  const int nw = G <= 4 ? 16 : 8, per_head = nw >= G ? nw / G : 1, winners = top_k < max_S ? top_k : max_S;
+  const int batches = (winners + 64 * per_head - 1) / (64 * per_head) * ((G + nw - 1) / nw), cus = device_cus();
+  return (kFixed + kPerBatch * nw * batches) * (double)((units + cus - 1) / cus);
+}
+
+// Whether a scan of one split merges by itself: it can (one_split_fits), and that is estimated to be the shorter way.
+inline bool one_split_merges(int scheme, int G, int NG, int B, int H_q, int H_kv, int max_S, int L, int top_k, int kc) {
+  return one_split_fits(scheme, G, NG, L, top_k, kc) &&
+         one_split_us(G, B * H_kv, max_S, top_k) <= merge_us(B * H_q, max_S, 1, kc, top_k);
 }
 
 inline int padded_group(int g) { return g <= 2 ? g : (g <= 4 ? 4 : (g <= 8 ? 8 : 16)); }
@@ -3106,9 +3136,14 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
   const int lmax = split_len_max(scheme, G, NG);
   const int nw = (G <= 4) ? 16 : 8;
   const int kCUs = device_cus();
-  constexpr double kScanFixed = 8.5, kOneTail = 3.5, kOneTailPerWinner = 0.0025, kManyRows = 5.0, kPerRowBeyond = 0.005;
+  constexpr double kScanFixed = 8.5;
   // one chunk per wavefront, all wavefronts; the mixed schemes are priced like the wider one
   const double per_chunk = (scheme == JF_SCHEME_K3V2 || scheme == JF_SCHEME_K2V2) ? 5.9 : 6.6;  // (INT3 values, asymmetric keys: as INT4)
+  // What one chunk per wavefront costs in an almost empty round, against a full one.  One split for the whole sequence
+  // means few workgroups with several chunks each, and the INT4 keys of the bf16 model then take 4.7 - 5.5 us a chunk
+  // where the others take 1.5 - 3: 3 sequences x 8 kv-heads, 1679 positions, G = 4, top-k 32 in one split 26.6 us, in
+  // splits of 256 22.3.  (Between several split lengths the higher figure changed no choice for the better.)
+  const double lone_split = scheme / 10 == 5 ? 0.8 : 0.5;
   int L = 256;
   double best = -1.0;
   for (int cand = 256; cand <= lmax; cand += 256) {
@@ -3118,17 +3153,13 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
     const long full = nwg / kCUs, rem = nwg % kCUs;
     const double stream = per_chunk * (double)cand / (64.0 * nw);
     double cost = (double)full * (kScanFixed + stream);
-    if (rem > 0) cost += kScanFixed + stream * (0.5 + 0.5 * (double)rem / kCUs);
+    const double lone = nsp == 1 ? lone_split : 0.5;
+    if (rem > 0) cost += kScanFixed + stream * (lone + (1.0 - lone) * (double)rem / kCUs);
     const int kc = (top_k + FS_CAND_SLACK) < cand ? (top_k + FS_CAND_SLACK) : cand;
-    // One split that merges by itself (measured: 4 - 5 us for 64 winners per head of four, 6 for 256 of four; the sums
-    // over the winners fill the vector ALU); a merge launch of more rows than CUs takes 16 us at 512 rows, 18 at 1024.
-    if (nsp == 1 && one_split_fits(scheme, G, NG, cand, top_k, kc)) {
-      cost += kOneTail + kOneTailPerWinner * (double)(G * top_k);
-    } else {
-      int parts, spp;
-      cost += merge_plan(rows, (int)nsp, kc, top_k, &parts, &spp);
-      if (rows > kCUs) cost += kManyRows + kPerRowBeyond * (double)(rows - kCUs);
-    }
+    if (nsp == 1 && one_split_merges(scheme, G, NG, B, H_q, H_kv, max_S, cand, top_k, kc))
+      cost += one_split_us(G, units, max_S, top_k);
+    else
+      cost += merge_us(rows, max_S, (int)nsp, kc, top_k);
     if (best < 0.0 || cost <= best) {
       best = cost;
       L = cand;
@@ -3325,7 +3356,7 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   JF_CHECK_ARG(p.n_splits <= MG_MAX_SPLITS, "fused_scan: too many splits (%d > %d)", p.n_splits, MG_MAX_SPLITS);
   merge_plan(B * H_q, p.n_splits, p.Kc, top_k, &p.mg_parts, &p.mg_spp);
   if (MODE == FS_STAGE_B) { p.mg_parts = 1; p.mg_spp = p.n_splits; }
-  p.one_split = !scores_only && p.n_splits == 1 && one_split_fits(scheme, G, NGv, p.L, top_k, p.Kc);
+  p.one_split = !scores_only && p.n_splits == 1 && one_split_merges(scheme, G, NGv, B, H_q, H_kv, max_S, p.L, top_k, p.Kc);
   const WsLayout wl = ws_layout(B, H_q, p.n_splits, p.Kc, p.mg_parts, top_k);
   if (!scores_only) {
     JF_CHECK_ARG(workspace && workspace_bytes >= wl.total, "fused_scan: workspace too small (%zu < %zu)", workspace_bytes, wl.total);

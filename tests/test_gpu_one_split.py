@@ -128,8 +128,8 @@ def _crowded(d, c, S, kind):
     ("k4v4", 4, 4, 128, 2, 2048, 512),
     ("k4v4", 4, 4, 128, 4, 777, 64),
     ("k3v2", 3, 2, 64, 4, 2048, 256),
-    ("k3v2", 3, 2, 64, 7, 1000, 256),
-    ("k3v2", 3, 2, 64, 8, 512, 256),
+    ("k3v2", 3, 2, 64, 7, 1000, 128),
+    ("k3v2", 3, 2, 64, 8, 512, 128),
     ("k3v3", 3, 3, 64, 16, 256, 32),
 ])
 def test_one_split_selects_from_a_crowded_bucket(scheme, kb, vb, gs, G, S, K, kind):
