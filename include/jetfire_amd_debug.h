@@ -32,9 +32,10 @@ int jf_debug_phase_clock(void* device_buffer);
  * multiple of 256 and clamped to what fits the kernel's LDS) replaces the planner's choice of the split
  * length in jf_fused_scan_topk and jf_fused_workspace_bytes; 0 restores the planner.  Process-wide. */
 int jf_debug_split_len(int split_len);
-/* Test aid: *one_split = 1 if a call of these sizes (jf_fused_scan_topk, Stage A with top-k, Stage B, selection) runs
- * as one launch whose scan workgroups merge by themselves, 0 if a merge launch follows; jf_debug_split_len applies. */
-int jf_debug_one_split(int scheme, int group_size, int B, int H_q, int H_kv, int max_S, int top_k, int* one_split);
+/* Test aid: *one_split = 1 if a call of these sizes runs as one launch whose scan workgroups merge by themselves, 0 if a
+ * merge launch follows.  stage: 0 jf_fused_scan_topk, 1 Stage A with top-k, 2 Stage B, 3 selection from given scores.
+ * jf_debug_split_len applies. */
+int jf_debug_one_split(int stage, int scheme, int group_size, int B, int H_q, int H_kv, int max_S, int top_k, int* one_split);
 /* Test aid: how many workgroups of the merge kernel's light shape (many rows, few candidates each) one compute unit
  * holds, the smallest figure over the value formats. */
 int jf_debug_light_merge_per_cu(int* workgroups);

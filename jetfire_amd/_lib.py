@@ -91,7 +91,7 @@ DEBUG_SIGNATURES = {
     "jf_profile_scan_begin": (I, [I]),
     "jf_profile_scan_end": (I, [P, P]),
     "jf_debug_phase_clock": (I, [P]),
-    "jf_debug_one_split": (I, [I, I, I, I, I, I, I, P]),
+    "jf_debug_one_split": (I, [I, I, I, I, I, I, I, I, P]),
     "jf_debug_light_merge_per_cu": (I, [P]),
     "jf_debug_split_len": (I, [I]),
     "jf_debug_pool_stall": (I, [L, I]),

@@ -186,13 +186,15 @@ extern "C" int jf_debug_phase_clock(void* device_buffer) {
   return JF_OK;
 }
 
-extern "C" int jf_debug_one_split(int scheme, int group_size, int B, int H_q, int H_kv, int max_S, int top_k, int* one_split) {
-  JF_CHECK_ARG(known_scheme(scheme) && (group_size == 64 || group_size == 128) && B > 0 && H_q > 0 && H_kv > 0 &&
-                   H_q % H_kv == 0 && max_S >= 0 && top_k > 0 && one_split, "debug_one_split: bad arguments");
+extern "C" int jf_debug_one_split(int stage, int scheme, int group_size, int B, int H_q, int H_kv, int max_S, int top_k,
+                                  int* one_split) {
+  JF_CHECK_ARG(stage >= FS_FULL && stage <= FS_TOPK && known_scheme(scheme) && (group_size == 64 || group_size == 128) &&
+                   B > 0 && H_q > 0 && H_kv > 0 && H_q % H_kv == 0 && max_S >= 0 && top_k > 0 && one_split,
+               "debug_one_split: bad arguments");
   int L, ns, kc;
   const int ng = scheme_ng(scheme, group_size);
   fused_plan(scheme, ng, B, H_q, H_kv, max_S, top_k, &L, &ns, &kc);
-  *one_split = ns == 1 && one_split_merges(scheme, padded_group(H_q / H_kv), ng, B, H_q, H_kv, max_S, L, top_k, kc);
+  *one_split = ns == 1 && one_split_merges(stage, scheme, padded_group(H_q / H_kv), ng, B, H_q, H_kv, max_S, L, top_k, kc);
   return JF_OK;
 }
 

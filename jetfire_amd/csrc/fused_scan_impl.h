@@ -2264,7 +2264,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       }
     } else {  // Stage B alone: the winners are given (or none)
       const int n_out = p.topk_idx ? K : 0;
-      if (tid < G) tl_nout[tid] = n_out;
+      if (tid < G) tl_nout[tid] = 0;
+      lds_barrier();
       for (int i = tid; i < GA * n_out; i += NT) {
         const int h = i / K;
         const int64_t pos = p.topk_idx[head0 * K + i];
@@ -2272,6 +2273,10 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         const int slot = valid ? sbase[(int)pos >> 4] + ((int)pos & 15) : -1;
         tl_wslot[i] = (slot >= 0 && slot < p.num_slots) ? slot : -1;
         tl_ww[i] = valid ? __expf(sc[h * L + (int)pos] - tl_m[h]) * tl_iz[h] : 0.f;
+        // A head's list ends with its last entry that names a position (the padding of a short sequence is not gone
+        // over: 1024 entries for eight heads over 16 positions took 50 us).  K >= 32: 32 lanes hold entries of one head.
+        const uint32_t named = (uint32_t)(__builtin_amdgcn_ballot_w64(valid) >> (lane & 32));
+        if (valid && (named >> (lane & 31)) == 1u) atomicMax(&tl_nout[h], i - h * K + 1);
       }
     }
     if constexpr (HAS_V) {
@@ -3115,14 +3120,19 @@ inline double one_split_us(int G, int units, int max_S, int top_k) {
   return (kFixed + kPerBatch * nw * batches) * (double)((units + cus - 1) / cus);
 }
 
-// Whether a scan of one split merges by itself: it can (one_split_fits), and that is estimated to be the shorter way.
-inline bool one_split_merges(int scheme, int G, int NG, int B, int H_q, int H_kv, int max_S, int L, int top_k, int kc) {
+// Whether a scan of one split merges by itself: it can (one_split_fits), and that is estimated to be the shorter way
+// (selection alone always is: 64 heads over 4 kv-heads, 190 positions, top-k 128 17.4 us, with the launch 20.8).  The same
+// for the whole step and Stage B alone, whose sums over the winners are then the same numbers.
+inline bool one_split_merges(int mode, int scheme, int G, int NG, int B, int H_q, int H_kv, int max_S, int L, int top_k,
+                             int kc) {
   return one_split_fits(scheme, G, NG, L, top_k, kc) &&
-         one_split_us(G, B * H_kv, max_S, top_k) <= merge_us(B * H_q, max_S, 1, kc, top_k);
+         (mode == FS_STAGE_A || mode == FS_TOPK ||
+          one_split_us(G, B * H_kv, max_S, top_k) <= merge_us(B * H_q, max_S, 1, kc, top_k));
 }
 
 inline int padded_group(int g) { return g <= 2 ? g : (g <= 4 ? 4 : (g <= 8 ? 8 : 16)); }
 
+// (One plan for the whole step and for either stage alone, so that their sums over the splits are the same numbers.)
 inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, int top_k, int* L_out, int* ns_out,
                        int* kc_out) {
   const int G = padded_group(H_q / H_kv);
@@ -3156,7 +3166,7 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
     const double lone = nsp == 1 ? lone_split : 0.5;
     if (rem > 0) cost += kScanFixed + stream * (lone + (1.0 - lone) * (double)rem / kCUs);
     const int kc = (top_k + FS_CAND_SLACK) < cand ? (top_k + FS_CAND_SLACK) : cand;
-    if (nsp == 1 && one_split_merges(scheme, G, NG, B, H_q, H_kv, max_S, cand, top_k, kc))
+    if (nsp == 1 && one_split_merges(FS_FULL, scheme, G, NG, B, H_q, H_kv, max_S, cand, top_k, kc))
       cost += one_split_us(G, units, max_S, top_k);
     else
       cost += merge_us(rows, max_S, (int)nsp, kc, top_k);
@@ -3356,7 +3366,8 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   JF_CHECK_ARG(p.n_splits <= MG_MAX_SPLITS, "fused_scan: too many splits (%d > %d)", p.n_splits, MG_MAX_SPLITS);
   merge_plan(B * H_q, p.n_splits, p.Kc, top_k, &p.mg_parts, &p.mg_spp);
   if (MODE == FS_STAGE_B) { p.mg_parts = 1; p.mg_spp = p.n_splits; }
-  p.one_split = !scores_only && p.n_splits == 1 && one_split_merges(scheme, G, NGv, B, H_q, H_kv, max_S, p.L, top_k, p.Kc);
+  p.one_split = !scores_only && p.n_splits == 1 &&
+                one_split_merges(MODE, scheme, G, NGv, B, H_q, H_kv, max_S, p.L, top_k, p.Kc);
   const WsLayout wl = ws_layout(B, H_q, p.n_splits, p.Kc, p.mg_parts, top_k);
   if (!scores_only) {
     JF_CHECK_ARG(workspace && workspace_bytes >= wl.total, "fused_scan: workspace too small (%zu < %zu)", workspace_bytes, wl.total);

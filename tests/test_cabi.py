@@ -405,21 +405,25 @@ def test_fused_plan_geometry_is_consistent(scheme, gs, B, Hq, Hkv, S, K):
     assert out[0].value == L
 
 
-@pytest.mark.parametrize("scheme,gs,B,Hq,Hkv,S,K,merges", [
-    (44, 128, 1, 32, 8, 777, 64, True),          # a chat turn
-    (32, 64, 32, 32, 8, 2048, 256, True),        # a full batch: a merge launch of 1024 rows
-    (32, 64, 16, 32, 4, 1000, 256, True),        # one wavefront per head, but 512 rows
-    (33, 64, 1, 16, 2, 1092, 512, False),        # one wavefront per head and 512 winners: 42 us, 30 with the merge launch
-    (24, 128, 1, 16, 1, 237, 256, False),        # sixteen heads in one workgroup: 39 us, 27
-    (33, 64, 2, 32, 8, 1045, 1024, False),       # 34.5 us, 29
-    (54, 64, 3, 32, 8, 1679, 32, False),         # INT4 keys of the bf16 model, long for one split: 26.6 us, 22
+@pytest.mark.parametrize("stage,scheme,gs,B,Hq,Hkv,S,K,merges", [
+    (0, 44, 128, 1, 32, 8, 777, 64, True),       # a chat turn
+    (0, 32, 64, 32, 32, 8, 2048, 256, True),     # a full batch: a merge launch of 1024 rows
+    (0, 32, 64, 16, 32, 4, 1000, 256, True),     # one wavefront per head, but 512 rows
+    (0, 33, 64, 1, 16, 2, 1092, 512, False),     # one wavefront per head and 512 winners: 42 us, 30 with the merge launch
+    (0, 24, 128, 1, 16, 1, 237, 256, False),     # sixteen heads in one workgroup: 39 us, 27
+    (0, 33, 64, 2, 32, 8, 1045, 1024, False),    # 34.5 us, 29
+    (0, 54, 64, 3, 32, 8, 1679, 32, False),      # INT4 keys of the bf16 model, long for one split: 26.6 us, 22
+    (2, 33, 64, 1, 16, 2, 1092, 512, False),     # Stage B: as the whole step
+    (2, 33, 64, 13, 16, 2, 16, 1024, True),      # (sixteen winners, whatever the list's length)
+    (1, 32, 64, 1, 64, 4, 190, 128, True),       # Stage A: selection alone, 17.4 us, 20.8
+    (3, 44, 128, 1, 64, 4, 190, 64, True),
 ])
-def test_plan_merges_in_the_scan_only_where_that_is_shorter(scheme, gs, B, Hq, Hkv, S, K, merges):
+def test_plan_merges_in_the_scan_only_where_that_is_shorter(stage, scheme, gs, B, Hq, Hkv, S, K, merges):
     """Measured shapes on both sides of the line between the scan that merges by itself and the merge launch."""
     import ctypes as C
     from jetfire_amd import _lib
     one = C.c_int(-1)
-    _lib.check(_lib.debug_hook("jf_debug_one_split")(scheme, gs, B, Hq, Hkv, S, K, C.byref(one)))
+    _lib.check(_lib.debug_hook("jf_debug_one_split")(stage, scheme, gs, B, Hq, Hkv, S, K, C.byref(one)))
     assert one.value == merges
 
 

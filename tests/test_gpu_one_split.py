@@ -29,7 +29,7 @@ def _one_split(scheme_id, gs, B, Hq, Hkv, S, K, split_len):
     out = C.c_int(-1)
     _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
     try:
-        _lib.check(_lib.debug_hook("jf_debug_one_split")(scheme_id, gs, B, Hq, Hkv, S, K, C.byref(out)))
+        _lib.check(_lib.debug_hook("jf_debug_one_split")(0, scheme_id, gs, B, Hq, Hkv, S, K, C.byref(out)))
     finally:
         _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
     return out.value
@@ -184,3 +184,34 @@ def test_one_split_is_no_slower_than_the_merge_launch(scheme, kb, vb, gs, B, Hkv
         finally:
             _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
     assert times[0] <= 1.5 * times[1], times
+
+
+@pytest.mark.parametrize("G,S,K,filled", [(2, 300, 512, "first"), (8, 600, 128, "holes"), (4, 700, 256, "last"),
+                                          (7, 290, 32, "holes"), (2, 400, 64, "none"), (1, 300, 1024, "ascending")])
+def test_stage_b_goes_over_the_entries_that_name_positions(G, S, K, filled):
+    """Stage B alone, merging in the scan: given lists that end early, have holes, or name positions past the end."""
+    from jetfire_amd import _lib, ops
+    Hkv = 2
+    c = make_case(96, 2, G * Hkv, Hkv, S, 3, 3, 64, lens=[S, S - 40])
+    d = to_device(c)
+    sc = ops.int3_qk_scores(d["q"], d["kd"], d["ks"], d["bt"], d["lens"], S, G * Hkv, Hkv, 16, SCALE)
+    idx = torch.full((2, G * Hkv, K), -1, dtype=torch.int64, device="cuda")
+    n = min(K, S)
+    if filled in ("first", "ascending"):
+        idx[..., :n] = torch.arange(n, device="cuda") if filled == "ascending" else torch.randperm(S, device="cuda")[:n]
+    elif filled == "holes":
+        idx[..., ::3] = torch.arange(0, K, 3, device="cuda")
+        idx[..., 1::3] = S + 5
+    elif filled == "last":
+        idx[..., -1] = S // 2
+    res = []
+    for split in (-(-S // 256) * 256, 256):
+        assert _one_split(33, 64, 2, G * Hkv, Hkv, S, K, split) == (split > 256)
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(split))
+        try:
+            res.append([t.clone() for t in ops.int3_softmax_v_with_pre_corr_wvs2(sc, d["vd"], d["vs"], d["bt"], d["lens"], idx,
+                                                                                  S, G * Hkv, Hkv, 16, K)])
+        finally:
+            _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    for a, b in zip(*res):      # (the bound of the comparison above)
+        assert float((a - b).abs().max()) <= 6e-6
