@@ -207,6 +207,7 @@ extern "C" int jf_debug_light_merge_per_cu(int* workgroups) {
       reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 3, 2, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>),
       reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 4, 1, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>),
       reinterpret_cast<const void*>(fused_merge_kernel<FS_FULL, 4, 2, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>)};
+  // (the form for more rows than four per compute unit)
   *workgroups = 0;
   for (const void* k : kernels) {
     int n = 0;

@@ -2414,7 +2414,7 @@ constexpr int MG_LIGHT_THREADS = 256, MG_LIGHT_REGK = 16, MG_LIGHT_TOPK = 512;  
 // new candidate list; the final merge (PARTIAL = false, mg_parts > 1) reads these lists instead of the
 // scan's.  The top K of a union is the top K of the parts' top K's, ties included: a candidate that a part
 // drops is beaten by K candidates of that part.
-template <int MODE, int VBITS, int NG, int MG_THREADS, int MG_REGK, bool PARTIAL, bool WIDE = false>
+template <int MODE, int VBITS, int NG, int MG_THREADS, int MG_REGK, bool PARTIAL, bool WIDE = false, int ROLES = 1>
 __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) {
   static_assert(!(PARTIAL && MODE == FS_STAGE_B), "Stage B alone selects nothing");
   constexpr int MG_WAVES = MG_THREADS / 64;
@@ -2929,13 +2929,13 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   const int dwi = lane % DW, w_in = lane / DW;
   const int g_of_lane = (NG == 1) ? 0 : ((dwi * CPD) / (D / NG));
   constexpr int UNR = Pre::UNR;  // 256 winners per pass
-  // A workgroup of fewer than sixteen wavefronts takes several roles per wavefront, two at a time: their rows are
-  // requested together (one gather latency for both), roles past the last winner are left out, and the kernel stays
-  // below the 96 registers that five workgroups of the light shape per CU allow:
-  // 73 - 87 instead of the 105 - 126 that all four roles at once take (four workgroups per CU).  Per layer: 20
-  // sequences x 64 heads of up to 2806 positions, K4V4, top-k 256 52.9 -> 47.6 us; 10 x 128 heads of up to 636, INT4
-  // with 64-channel groups, top-k 512 55.2 -> 48.2; 29 x 128 heads of up to 77, INT2 values 72.9 -> 66.0; 512 rows as before.
-  constexpr int RPW = VWAVES / MG_WAVES, RP = (RPW >= 2) ? 2 : 1;
+  // A workgroup of fewer than sixteen wavefronts takes several roles per wavefront, ROLES at a time: the rows of those are
+  // requested together.  All four at once: one gather latency instead of four, 105 - 126 registers and so four workgroups
+  // of the light shape per CU; one at a time: 73, five workgroups, and no rows fetched for roles without winners.  Per
+  // layer, one / four at a time: 16 sequences x 32 heads, 700 positions, K4V4, top-k 256 37.1 / 36.3 us; 32 x 64 heads of
+  // 512, top-k 128 53.6 / 55.6; 22 x 128 heads of 39, INT4 with 64-channel groups, top-k 128 54.8 / 60.8.
+  constexpr int RPW = VWAVES / MG_WAVES, RP = ROLES;
+  static_assert(RPW % RP == 0, "whole turns");
 #pragma unroll
   for (int r0 = 0; r0 < RPW; r0 += RP) {
     float acc[RP][CPD], accw[RP];
@@ -3450,6 +3450,9 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   // the kernel).
   const bool light = (MODE == FS_FULL) && !big && p.mg_parts == 1 && top_k <= MG_LIGHT_TOPK &&
                      (long long)B * H_q > (long long)device_cus() && (long long)p.n_splits * p.Kc <= MG_LIGHT_THREADS * MG_LIGHT_REGK;
+  // its gathers all at once where four workgroups per CU hold every row and most roles have winners (see ROLES)
+  const bool gather = light && (long long)B * H_q <= 4ll * device_cus() && top_k >= 256 && max_S >= 256;
+  (void)gather;
 #define JF_MERGE(VB, NGG)                                                                                            \
   do {                                                                                                               \
     if (wide) {                                                                                                      \
@@ -3457,8 +3460,10 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
       else rc = launch_wide_merge<fused_merge_kernel<MODE, VB, NGG, 1024, 32, false, true>>(mgrid, p, st);            \
     } else if (big) hipLaunchKernelGGL((fused_merge_kernel<MODE, VB, NGG, 1024, 32, false>), mgrid, dim3(1024), 0, st, p); \
     else if (light) {                                                                                                \
-      if constexpr (MODE == FS_FULL)                                                                                 \
-        hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, p); \
+      if constexpr (MODE == FS_FULL) {                                                                               \
+        if (gather) hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false, false, 4>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, p); \
+        else hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, p); \
+      }                                                                                                              \
     } else hipLaunchKernelGGL((fused_merge_kernel<MODE, VB, NGG, 1024, 8, false>), mgrid, dim3(1024), 0, st, p);       \
   } while (0)
   if constexpr (MODE == FS_STAGE_A || MODE == FS_TOPK) {  // no value rows are read: one instantiation serves every format
