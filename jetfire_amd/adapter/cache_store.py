@@ -158,8 +158,8 @@ class JetFireInt4CacheStore:
             return
         self._quantise(key_tok, value_tok, slots)
         if mark:
-            inside = (slots >= 0) & (slots < self.num_slots)
-            self._slot_filled_buf.index_fill_(0, torch.where(inside, slots, self.num_slots), True)
+            # (slots on either side of the cache mark the spare entry, which is number num_slots and number -1)
+            self._slot_filled_buf.index_fill_(0, slots.clamp(-1, self.num_slots), True)
         if mirror:
             self._mirror(key_tok, value_tok, slots)
 
