@@ -29,10 +29,16 @@ def _check(cond: bool, msg: str) -> None:
         raise RuntimeError(msg)
 
 
+# (the raw handle: building the Stream object that torch.cuda.current_stream returns takes 2 us, at each of an operator's
+# look-ups; the function is torch's own, not part of its documented interface, hence the way round)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
-    """The current stream of the tensor's device.  (The raw handle: building the Stream object that
-    torch.cuda.current_stream returns takes 2 us, at each of an operator's look-ups.)"""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    """The current stream of the tensor's device."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -526,3 +526,15 @@ def test_committed_counter_summaries_belong_to_the_sources_in_the_tree():
     assert files
     for f in files:
         assert f"build {want}" in json.load(open(f)).get("lib_version", ""), f
+
+
+def test_stream_look_up_without_the_raw_handle(monkeypatch):
+    """A torch without the undocumented look-up: the documented one, with the tensor's own device."""
+    import types
+    from jetfire_amd import ops
+    asked = []
+    monkeypatch.setattr(ops, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: asked.append(d) or types.SimpleNamespace(cuda_stream=77))
+    assert ops._stream(types.SimpleNamespace(device="cuda:3")) == 77 and asked == ["cuda:3"]
+    monkeypatch.setattr(ops, "_raw_stream", lambda index: 100 + index)
+    assert ops._stream(types.SimpleNamespace(get_device=lambda: 3)) == 103
