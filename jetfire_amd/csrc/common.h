@@ -117,6 +117,10 @@ __device__ inline int wave_incl_scan_i(int v) {
   return v;
 }
 
+// Compute units of the current device (launchers balance workgroups over them); 256, the MI355X count, when no device
+// can be asked (planning on a host without a GPU).
+int device_cus();
+
 inline bool is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 
 // Pre-correction terms of INT4 values (one scale per row) over given winners with given softmax statistics, on the

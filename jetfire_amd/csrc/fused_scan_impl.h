@@ -77,10 +77,7 @@ constexpr bool kDebugHooks = true;
 #define JF_CLK() 0ll
 constexpr bool kDebugHooks = false;
 #endif
-// Compute units of the current device (the planner balances workgroups over them); 256, the MI355X count, when
-// no device can be asked (planning on a host without a GPU).
-int device_cus();
-// The one-pass scan kernels are instantiated in four translation units (fused_full_*.hip), one per family of
+// The one-pass scan kernels are instantiated in five translation units (fused_full_*.hip), one per family of
 // schemes, so that they compile side by side; `params` points to the launcher's FusedParams.
 int launch_full_scan_a(int scheme, int G, int NG, const void* params, void* stream);  // K3V2, K4V4, K3V4, K4V2
 int launch_full_scan_b(int scheme, int G, int NG, const void* params, void* stream);  // K2V2, K2V3, K2V4

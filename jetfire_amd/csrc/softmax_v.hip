@@ -493,7 +493,7 @@ extern "C" int jf_softmax_v_int8_tiles(const float* scores, const float* softmax
   // at least two pairs of tiles per wavefront (8 * sub_count <= max_S / 64 partial rows: inside the workspace, which
   // holds max(8, max_S / 64))
   const int pairs_per_range = ((max_S + TQ_SPLITS - 1) / TQ_SPLITS + 2 * TQ_TILE - 1) / (2 * TQ_TILE) + 1;
-  const int want = (4 * 256 + TQ_SPLITS * H_kv * B - 1) / (TQ_SPLITS * H_kv * B);
+  const int want = (4 * device_cus() + TQ_SPLITS * H_kv * B - 1) / (TQ_SPLITS * H_kv * B);
   int sub_count = pairs_per_range / (2 * TQ_WAVES);
   sub_count = sub_count < want ? sub_count : want;
   sub_count = sub_count < 1 ? 1 : (sub_count > 16 ? 16 : sub_count);
