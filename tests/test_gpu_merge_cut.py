@@ -1,6 +1,6 @@
 """The merge kernel's threshold search at the sizes of its three paths: a cut bucket of at most 64 members (ranked in
-registers), of up to 1024 (a list in LDS), of more (bisection), with ties across the cut, in both shapes of the kernel
-(1024 threads; 256 threads for more rows than compute units)."""
+registers), of up to 1024 (a list in LDS), of more (bisection), with ties across the cut (and once without), in both
+shapes of the kernel (1024 threads; 256 threads for more rows than compute units)."""
 import numpy as np
 import pytest
 import torch
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B", [1, 40])
-@pytest.mark.parametrize("copies", [40, 64, 65, 500, 1100])
+@pytest.mark.parametrize("copies", [40, 45, 58, 64, 65, 500, 1100])
 def test_equal_scores_around_the_cut(B, copies):
     from jetfire_amd import _lib
     S, K, Hq, Hkv = 2048, 64, 8, 1
@@ -37,6 +37,9 @@ def test_equal_scores_around_the_cut(B, copies):
     finally:
         _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
     scores, idx = out[7].cpu().numpy(), out[4].cpu().numpy()
+    # (head 0: twenty better positions, the copied one and its copies; the tie lies across the cut from 44 copies on)
+    ranked = np.sort(scores[0, 0])[::-1]
+    assert (ranked[K - 1] == ranked[K]) == (copies >= 44)
     for b in (0, B - 1):
         for h in range(Hq):
             want = np.sort(np.lexsort((np.arange(S), -scores[b, h]))[:K])

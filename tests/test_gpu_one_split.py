@@ -36,10 +36,11 @@ def _one_split(scheme_id, gs, B, Hq, Hkv, S, K, split_len):
 
 
 def _both(scheme, c, d, S, K):
-    """The call with one split, and with splits of 256 positions."""
-    from jetfire_amd import _lib
+    """The call with one split, which merges by itself, and with splits of 256 positions and the merge launch."""
+    from jetfire_amd import _lib, ops
     res = []
     for split in (-(-S // 256) * 256, 256):
+        assert _one_split(ops.FUSED_SCHEMES[scheme], c["gs"], c["B"], c["Hq"], c["Hkv"], S, K, split) == (split >= S)
         _lib.check(_lib.debug_hook("jf_debug_split_len")(split))
         try:
             res.append([t.clone() for t in run_fused(scheme, c, d, S, K)])
@@ -54,7 +55,7 @@ def _both(scheme, c, d, S, K):
     ("k3v2", 3, 2, 64, 4, 1024, [1024, 1023, 63, 65], 256),
     ("k3v2", 3, 2, 64, 4, 2040, [2040, 1, 0], 512),
     ("k3v2", 3, 2, 64, 8, 1111, [1111, 700], 128),
-    ("k3v2", 3, 2, 64, 8, 512, [512, 300], 512),
+    ("k3v2", 3, 2, 64, 8, 512, [512, 100], 128),
     ("k2v2", 2, 2, 64, 1, 3900, [3900, 16], 2048),
     ("k3v3", 3, 3, 64, 2, 1500, [1500, 64], 256),
     ("k3v3", 3, 3, 128, 7, 800, [800, 799], 64),
@@ -75,10 +76,11 @@ def test_one_split_matches_oracle_and_merge(scheme, kb, vb, gs, G, S, lens, K):
 
 
 @pytest.mark.parametrize("levels", [1, 3, 40])
-@pytest.mark.parametrize("S,K", [(300, 64), (300, 512), (1500, 256)])
+@pytest.mark.parametrize("S,K", [(300, 64), (300, 256), (1500, 256)])
 def test_one_split_ties(levels, S, K):
-    """Key rows copied from a few distinct ones: the cut bucket holds more members than a rank list (levels 3: hundreds
-    of equal scores; 1: all of them), or more than the candidate list (the exact selection).  Lowest positions win."""
+    """Key rows copied from a few distinct ones: the cut bucket holds fewer members than a rank list (levels 40), more
+    (levels 3: hundreds of equal scores; 1: all of them), or more than the candidate list (1500 positions of level
+    1: the exact selection).  Lowest positions win."""
     c = make_case(92, 2, 8, 2, S, 4, 4, 128, lens=[S, S - 37])
     d = to_device(c)
     kd, ks, bt = d["kd"].clone(), d["ks"].clone(), d["bt"]
@@ -99,8 +101,8 @@ def test_one_split_ties(levels, S, K):
 
 
 def test_plan_takes_one_split_for_short_and_many_sequences():
-    assert _plan(44, 128, 1, 32, 8, 777, 64)[1] == 1
-    assert _plan(32, 64, 32, 32, 8, 2048, 256)[1] == 1
+    assert _plan(44, 128, 1, 32, 8, 777, 64)[1] == 1 and _one_split(44, 128, 1, 32, 8, 777, 64, 0)
+    assert _plan(32, 64, 32, 32, 8, 2048, 256)[1] == 1 and _one_split(32, 64, 32, 32, 8, 2048, 256, 0)
     assert _plan(44, 128, 1, 32, 8, 4096, 64)[1] > 1
 
 
@@ -133,12 +135,10 @@ def _crowded(d, c, S, kind):
     ("k3v3", 3, 3, 64, 16, 256, 32),
 ])
 def test_one_split_selects_from_a_crowded_bucket(scheme, kb, vb, gs, G, S, K, kind):
-    from jetfire_amd import ops
     Hkv, lens = 2, [S, S - S // 5]
     c = make_case(94, 2, G * Hkv, Hkv, S, kb, vb, gs, lens=lens)
     d = to_device(c)
     _crowded(d, c, S, kind)
-    assert _one_split(ops.FUSED_SCHEMES[scheme], gs, 2, G * Hkv, Hkv, S, K, -(-S // 256) * 256)
     one, cut = _both(scheme, c, d, S, K)
     assert torch.equal(one[4], cut[4]) and torch.equal(one[1], cut[1])
     scores = one[7].cpu().numpy()
