@@ -2082,9 +2082,17 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       // and one score at 40 sigma (this: 29.5, no outlier: 24.9, splits of 256 with a merge launch: 103), and 1055 us
       // for 16 x 3900, K2V2, one head per kv-head, top-k 2048 and no outlier at all (31.6; 81).
       unsigned long long last[NHS] = {};  // the last winner among the head's members
-      const unsigned long long crowded = __builtin_amdgcn_ballot_w64(
-          lane < GA && tl_need[min(lane, G - 1)] >= 0 && tl_mem[min(lane, G - 1)] > Tail::MEM);
-      if (crowded != 0ull) {  // (the same in every wavefront)
+      // (the same in every wavefront; this wavefront's heads are read along)
+      const int any_need = tl_need[min(lane, G - 1)], any_mem = tl_mem[min(lane, G - 1)];
+      int need_of[NHS], mem_of[NHS];
+#pragma unroll
+      for (int it = 0; it < NHS; ++it) {
+        const int h = min((wave + it * NW) / SEG, G - 1);
+        need_of[it] = tl_need[h];
+        mem_of[it] = tl_mem[h];
+      }
+      const unsigned long long crowded = __builtin_amdgcn_ballot_w64(lane < GA && any_need >= 0 && any_mem > Tail::MEM);
+      if (__builtin_expect(crowded != 0ull, 0)) {
         // (the staging area is dead since `combine`) per head the digit counts, the smallest and the largest member's key
         int* rh = reinterpret_cast<int*>(stage);
         uint32_t* ends = reinterpret_cast<uint32_t*>(rh + G * 256);
@@ -2130,8 +2138,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           const uint32_t kmin = __builtin_amdgcn_readfirstlane(ends[2 * h]), kmax = __builtin_amdgcn_readfirstlane(ends[2 * h + 1]);
           bits[it] = 12 + ((kmin == kmax) ? 0 : 32 - __clz((int)(kmin ^ kmax)));
           top[it] = rank_word(kmax, 0) >> bits[it];
-          need[it] = __builtin_amdgcn_readfirstlane(tl_need[h]);
-          left[it] = __builtin_amdgcn_readfirstlane(tl_mem[h]);
+          need[it] = __builtin_amdgcn_readfirstlane(need_of[it]);
+          left[it] = __builtin_amdgcn_readfirstlane(mem_of[it]);
         }
         for (int pass = 0; pass < 6; ++pass) {
 #pragma unroll
@@ -2188,7 +2196,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         int h, lo, hi;
         const int seg = pair_of(it, h, lo, hi);
         if (seg < 0) continue;
-        const int need = __builtin_amdgcn_readfirstlane(tl_need[h]), m = __builtin_amdgcn_readfirstlane(tl_mem[h]);
+        const int need = __builtin_amdgcn_readfirstlane(need_of[it]), m = __builtin_amdgcn_readfirstlane(mem_of[it]);
         const uint16_t* cl = tl_list + h * Kcap;
         // a short list: every wavefront of the head ranks the members itself, one per lane, the others' words as
         // scalars (no exchange, no LDS latency per member)
