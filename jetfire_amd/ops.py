@@ -266,8 +266,9 @@ def append_rows(key_tok, value_tok, slot_idx, k_data, k_scales, k_zp, v_data, v_
         _check(d.dtype == torch.uint8 and s.dtype == torch.bfloat16, "cache must be uint8 data + bf16 scales")
         _check(d.shape == (H_kv, S, D * bits // 8) and ds[2] == 1 and s.shape == (H_kv, S, ng) and (ng == 1 or ss[2] == 1),
                "bad cache shape")
-    zs = (0, 0) if k_zp is None else k_zp.stride()
-    _check(k_zp is None or (k_zp.dtype == torch.bfloat16 and k_zp.shape == k_scales.shape), "bad zero-point shape")
+    zs = (0, 0, 1) if k_zp is None else k_zp.stride()
+    _check(k_zp is None or (k_zp.dtype == torch.bfloat16 and k_zp.shape == k_scales.shape and (ng == 1 or zs[2] == 1)),
+           "bad zero-point shape")
     _check(slot_filled is None or (slot_filled.dtype == torch.bool and slot_filled.shape == (S,) and slot_filled.is_contiguous()),
            "slot_filled must be (num_slots,) bool")
     sh = (0, 0)

@@ -102,3 +102,18 @@ def test_slots_beyond_the_cache_are_skipped_by_every_writer(aligned, kb, vb, asy
         getattr(ops, name)(tok, slots, data[:, :nblk * 16], scales[:, :nblk * 16], gs)
         assert not data[:, nblk * 16:].any() and not scales[:, nblk * 16:].any()
         assert torch.equal(scales[0, :nblk * 16, 0] != 0, want.slot_filled)
+
+
+def test_append_refuses_zero_points_whose_groups_do_not_lie_side_by_side():
+    """The kernel stores a row's zero-points next to each other, as the separate writer checks they are."""
+    from jetfire_amd import ops
+    T, H, S = 4, 2, 32
+    tok = torch.zeros(T, H, 128, dtype=torch.bfloat16, device="cuda")
+    data = [torch.zeros(H, S, 32, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    scales = [torch.zeros(H, S, 2, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    zp = torch.zeros(H, S, 4, dtype=torch.bfloat16, device="cuda")[:, :, ::2]
+    slots = torch.arange(T, device="cuda")
+    for call in (lambda: ops.append_rows(tok, tok, slots, data[0], scales[0], zp, data[1], scales[1], 64, 2, 2),
+                 lambda: ops.fused_quant_write_int2_asym(tok, slots, data[0], scales[0], zp, 64)):
+        with pytest.raises(RuntimeError):
+            call()
