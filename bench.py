@@ -101,8 +101,8 @@ def _median_ms(fn, sync, n=10, warm=2):
 
 
 def component_append(args):
-    """A prefill chunk of --tokens tokens appended to one layer's store at the workload's geometry: the
-    quantise-on-write kernels, the mirror kernel that stores the bf16 rows into the pinned host shadow, the
+    """A prefill chunk of --tokens tokens appended to one layer's store at the workload's geometry: the one
+    launch that quantises K and V and marks the slots, the mirror kernel that stores the bf16 rows into the pinned host shadow, the
     store's whole `write_slots` + `flush_pending_writes`, and beside it the serial host mirror the reference
     falls back to (device-to-host copy of the permuted chunk + `index_copy_`, cache_store.py:744-759)."""
     import torch
@@ -120,7 +120,7 @@ def component_append(args):
     blocks = torch.randperm(nblk, generator=g)[:(T + 15) // 16]
     slots = (blocks[:, None] * 16 + torch.arange(16)[None, :]).reshape(-1)[:T].cuda()     # paged: runs of 16 slots
     sync = torch.cuda.synchronize
-    quant_ms = _median_ms(lambda: store._quantise(key, value, slots), sync)
+    quant_ms = _median_ms(lambda: store._append(key, value, slots, mark=True, mirror=False), sync)
     mirror_ms = _median_ms(lambda: store._mirror(key, value, slots), sync)
 
     def whole():
