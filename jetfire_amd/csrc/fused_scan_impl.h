@@ -3055,14 +3055,33 @@ inline int split_len_max(int scheme, int G, int NG) {
   return lm < 256 ? 256 : (int)lm;
 }
 
+inline size_t scan_tail_bytes(int G, int top_k, int kc) {
+  return G == 1 ? ScanTail<1, 4>::bytes(top_k, kc) : G == 2 ? ScanTail<2, 4>::bytes(top_k, kc) :
+         G == 4 ? ScanTail<4, 4>::bytes(top_k, kc) : G == 8 ? ScanTail<8, 1>::bytes(top_k, kc) :
+                  ScanTail<16, 1>::bytes(top_k, kc);
+}
+
+// Entries a head's candidate list can have where the scan merges by itself: a wavefront's share fits the 32 bits of its
+// win mask.
+inline int one_split_list_max(int G) { return (G <= 4 ? 4 : 1) * 64 * 32; }
+
 // Whether a scan whose single split of L positions covers the sequence can merge by itself: its tables fit the LDS
-// that is left, and a wavefront's share of a candidate list fits the 32 bits of its win mask.
+// that is left, and so does a list of kc candidates.
 inline bool one_split_fits(int scheme, int G, int NG, int L, int top_k, int kc) {
-  const int seg = G <= 4 ? 4 : 1;
-  const size_t tail = G == 1 ? ScanTail<1, 4>::bytes(top_k, kc) : G == 2 ? ScanTail<2, 4>::bytes(top_k, kc) :
-                      G == 4 ? ScanTail<4, 4>::bytes(top_k, kc) : G == 8 ? ScanTail<8, 1>::bytes(top_k, kc) :
-                               ScanTail<16, 1>::bytes(top_k, kc);
-  return kc <= seg * 64 * 32 && (long)((4 * G + 1) * (long)L + (long)tail) <= lds_room(scheme, G, NG);
+  return kc <= one_split_list_max(G) &&
+         (long)((4 * G + 1) * (long)L + (long)scan_tail_bytes(G, top_k, kc)) <= lds_room(scheme, G, NG);
+}
+
+// The candidate list such a scan gets: as much of the LDS that is left (one workgroup per CU either way) as the split can
+// fill.  A bucket at the cut with more positions than the list has room for (one outlying score makes the buckets wide)
+// takes the exact selection, one wavefront per head; a list that holds them goes on with all of the head's wavefronts:
+// 16 sequences x 8 kv-heads, 3900 positions, K2V2, one head each, top-k 1024, per layer with no outlier / one score at 20
+// / at 40 sigma: top_k + 256 entries 26.8 / 52.8 / 61.1 us, this 26.7 / 28.8 / 29.5 (splits of 2048 and a merge launch:
+// 28.5 / 29.2 / 35.3).
+inline int one_split_list(int scheme, int G, int NG, int L, int top_k, int kc) {
+  const long room = lds_room(scheme, G, NG) - (4 * G + 1) * (long)L - (long)scan_tail_bytes(G, top_k, kc);
+  const long most = L < one_split_list_max(G) ? L : one_split_list_max(G), more = kc + room / (2 * G);
+  return (int)(more < most ? more : most);
 }
 
 // Estimated microseconds of the merge (fitted on MI355X): a fixed part per launch plus a part proportional to
@@ -3378,6 +3397,7 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
     JF_CHECK_ARG(workspace && workspace_bytes >= wl.total, "fused_scan: workspace too small (%zu < %zu)", workspace_bytes, wl.total);
     JF_CHECK_ARG(((uintptr_t)workspace & 255) == 0, "fused_scan: workspace must be 256-byte aligned");
   }
+  if (p.one_split) p.Kc = one_split_list(scheme, G, NGv, p.L, top_k, p.Kc);  // (in LDS, not in the workspace)
   uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
   p.scores = HAS_K ? scores : nullptr;
   p.scores_in = scores_in;

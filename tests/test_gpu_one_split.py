@@ -153,21 +153,23 @@ def test_one_split_selects_from_a_crowded_bucket(scheme, kb, vb, gs, G, S, K, ki
 
 
 @pytest.mark.parametrize("kind", ["outlier", "levels", "plain"])
-@pytest.mark.parametrize("scheme,kb,vb,gs,B,Hkv,G,S,K", [
-    ("k2v2", 2, 2, 64, 16, 8, 1, 3900, 2048),
-    ("k4v4", 4, 4, 128, 32, 8, 4, 1024, 512),
-    ("k3v2", 3, 2, 64, 16, 4, 8, 1000, 256),
+@pytest.mark.parametrize("scheme,kb,vb,gs,B,Hkv,G,S,K,other", [
+    ("k2v2", 2, 2, 64, 16, 8, 1, 3900, 2048, 256),
+    ("k2v2", 2, 2, 64, 16, 8, 1, 3900, 1024, 2048),
+    ("k4v4", 4, 4, 128, 32, 8, 4, 1024, 512, 256),
+    ("k3v2", 3, 2, 64, 16, 4, 8, 1000, 256, 256),
 ])
-def test_one_split_is_no_slower_than_the_merge_launch(scheme, kb, vb, gs, B, Hkv, G, S, K, kind):
+def test_one_split_is_no_slower_than_the_merge_launch(scheme, kb, vb, gs, B, Hkv, G, S, K, other, kind):
     """Bounded work per member of the cut bucket: ranking each against the whole list took two to seventeen times the
-    merge launch's time here."""
+    merge launch's time here, and the exact selection by one wavefront per head, where the list was too short for the
+    bucket, twice that of the longest splits with a launch (`other`: their length)."""
     from jetfire_amd import _lib, ops
     c = make_case(95, B, G * Hkv, Hkv, S, kb, vb, gs)
     d = to_device(c)
     _crowded(d, c, S, kind)
     times = []
-    for split in (-(-S // 256) * 256, 256):
-        assert _one_split(ops.FUSED_SCHEMES[scheme], gs, B, G * Hkv, Hkv, S, K, split) == (split > 256)
+    for split in (-(-S // 256) * 256, other):
+        assert _one_split(ops.FUSED_SCHEMES[scheme], gs, B, G * Hkv, Hkv, S, K, split) == (split > other)
         _lib.check(_lib.debug_hook("jf_debug_split_len")(split))
         try:
             best = float("inf")
