@@ -244,7 +244,8 @@ struct ScanLds {
 // the candidate positions, the members of the cut bucket, the winners' slots and weights, o_hat and a few words.
 template <int G, int SEG>
 struct ScanTail {
-  static constexpr int MEM = 64;  // members of the cut bucket that are ranked from a list, one per lane
+  static constexpr int MEM = 64;  // members of the cut bucket that are selected from a list, one per lane
+  static constexpr int RANK = 24;  // up to here against each other, beyond by bits
   static constexpr int INTS = ((5 + SEG + 3) * G * 4 + 15) & ~15;
   __host__ __device__ static constexpr size_t bytes(int top_k, int kc) {
     return INTS + (size_t)G * (D * 4 + 8 * (size_t)top_k + 8 * MEM + 2 * (size_t)kc);
@@ -254,6 +255,28 @@ struct ScanTail {
 __device__ inline float key_to_score(uint32_t key) {
   const uint32_t u = (key & 0x80000000u) ? (key & 0x7fffffffu) : ~key;
   return __builtin_bit_cast(float, u);
+}
+
+// Narrows `active` to the lanes that hold the `need`-th largest of the active lanes' words (need: 1 .. their number, uniform;
+// afterwards its place among those equal lanes).  One ballot per bit from the highest in which the words differ, the rest on
+// the scalar unit, until one lane is left: about 1 us whatever the number of words.  (Comparing every word with every other
+// one, as a loop over scalars, costs five vector instructions per word in each of the workgroup's wavefronts: 2 us at 60.)
+__device__ inline void nth_largest(uint32_t word, unsigned long long& active, int& need) {
+  if (active == 0ull) return;
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)word, __ffsll((long long)active) - 1);
+  const bool in = (active >> (threadIdx.x & 63)) & 1ull;
+  const uint32_t differ = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_u(in ? word ^ first : 0u));
+  if (differ == 0u) return;
+  for (int b = 31 - __clz((int)differ); b >= 0 && (active & (active - 1)) != 0ull; --b) {
+    const unsigned long long ones = __builtin_amdgcn_ballot_w64(((word >> b) & 1u) != 0u) & active;
+    const int c = __popcll(ones);
+    if (need <= c || ones == active) {
+      active = ones;
+    } else {
+      need -= c;
+      active &= ~ones;
+    }
+  }
 }
 
 // Orders this wavefront's earlier LDS writes before its later LDS reads (the LDS pipe executes one
@@ -2198,18 +2221,26 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         if (seg < 0) continue;
         const int need = __builtin_amdgcn_readfirstlane(need_of[it]), m = __builtin_amdgcn_readfirstlane(mem_of[it]);
         const uint16_t* cl = tl_list + h * Kcap;
-        // a short list: every wavefront of the head ranks the members itself, one per lane, the others' words as
-        // scalars (no exchange, no LDS latency per member)
+        // a short list: every wavefront of the head finds the last winner itself, one member per lane (no exchange): few
+        // members are ranked against each other as scalars (40 ns per member), more by bits (1 us)
         if (need >= 0 && m <= Tail::MEM) {
           const unsigned long long own = (lane < m) ? tl_mlist[h * Tail::MEM + lane] : 0ull;
-          int rank = 0;
-          for (int k = 0; k < m; ++k) {
-            const unsigned long long o = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), k) << 32) |
-                                         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, k);
-            rank += (o > own) ? 1 : 0;
+          unsigned long long held;
+          if (m <= Tail::RANK) {
+            int rank = 0;
+            for (int k = 0; k < m; ++k) {
+              const unsigned long long o = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), k) << 32) |
+                                           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, k);
+              rank += (o > own) ? 1 : 0;
+            }
+            held = __builtin_amdgcn_ballot_w64(lane < m && rank == need - 1);
+          } else {
+            held = (m < 64) ? (1ull << m) - 1ull : ~0ull;
+            int place = need;
+            nth_largest((uint32_t)(own >> 12), held, place);   // the key,
+            nth_largest((uint32_t)own & 4095u, held, place);   // and among equal ones the position
           }
-          const unsigned long long who = __builtin_amdgcn_ballot_w64(lane < m && rank == need - 1);
-          const int src = (who != 0ull) ? __ffsll((long long)who) - 1 : 0;
+          const int src = (held != 0ull) ? __ffsll((long long)held) - 1 : 0;
           last[it] = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), src) << 32) |
                      (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, src);
         }
@@ -2397,6 +2428,9 @@ __device__ inline void waves_prefix_i(const int* arr, int lane, int wave, int* b
 constexpr int MG_MAX_SPLITS = 256;
 constexpr int MG_BINS = 1024;      // linear score buckets of the threshold search
 constexpr int MG_LIST = 1024;      // members of the cut bucket resolved by rank counting
+// Up to here in the registers of every wavefront, beyond over the list in LDS, one member per thread: the sixteen
+// wavefronts share four SIMDs, so a member costs all of them 40 ns, and the list one barrier and half a microsecond.
+constexpr int MG_RANK = 16;
 constexpr int MG_BT_LDS = 4096;    // block-table entries cached in LDS (65536 positions)
 constexpr int MG_LIGHT_THREADS = 256, MG_LIGHT_REGK = 16, MG_LIGHT_TOPK = 512;  // the light shape of the merge
 
@@ -2749,7 +2783,7 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
     }
     lds_barrier();
     const int m = __builtin_amdgcn_readfirstlane(lcount_sh);
-    if (m <= 64) {
+    if (m <= MG_RANK) {
       // (the usual case: one member per lane, the others as scalars, in every wavefront: no LDS latency per member and
       // no barrier to hand the result around)
       const uint32_t own = (lane < m) ? lkey[lane] : 0u;
