@@ -79,8 +79,7 @@ def test_one_split_matches_oracle_and_merge(scheme, kb, vb, gs, G, S, lens, K):
 @pytest.mark.parametrize("S,K", [(300, 64), (300, 256), (1500, 256)])
 def test_one_split_ties(levels, S, K):
     """Key rows copied from a few distinct ones: the cut bucket holds fewer members than a rank list (levels 40), more
-    (levels 3: hundreds of equal scores; 1: all of them), or more than the candidate list (1500 positions of level
-    1: the exact selection).  Lowest positions win."""
+    (levels 3: hundreds of equal scores; 1: all of them, more than top_k and its slack).  Lowest positions win."""
     c = make_case(92, 2, 8, 2, S, 4, 4, 128, lens=[S, S - 37])
     d = to_device(c)
     kd, ks, bt = d["kd"].clone(), d["ks"].clone(), d["bt"]
