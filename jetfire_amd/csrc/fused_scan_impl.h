@@ -3211,7 +3211,10 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
   // means few workgroups with several chunks each, and the INT4 keys of the bf16 model then take 4.7 - 5.5 us a chunk
   // where the others take 1.5 - 3: 3 sequences x 8 kv-heads, 1679 positions, G = 4, top-k 32 in one split 26.6 us, in
   // splits of 256 22.3.  (Between several split lengths the higher figure changed no choice for the better.)
-  const double lone_split = scheme / 10 == 5 ? 0.8 : 0.5;
+  // Asymmetric keys with two scale groups (three contractions per group) lie between: 4 sequences x 4 kv-heads, 1181
+  // positions, A2V2, G = 2, top-k 1024 in one split 28.9 us, in splits of 256 25.5; 4 x 1, 1262 positions, A2V4 24.4 / 22.6.
+  // (With one group, or at 0.8, as many shapes lost as gained.)
+  const double lone_split = scheme / 10 == 5 ? 0.8 : (scheme / 10 == 1 && NG == 2) ? 0.65 : 0.5;
   int L = 256;
   double best = -1.0;
   for (int cand = 256; cand <= lmax; cand += 256) {

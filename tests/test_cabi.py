@@ -413,6 +413,8 @@ def test_fused_plan_geometry_is_consistent(scheme, gs, B, Hq, Hkv, S, K):
     (0, 24, 128, 1, 16, 1, 237, 256, False),     # sixteen heads in one workgroup: 39 us, 27
     (0, 33, 64, 2, 32, 8, 1045, 1024, False),    # 34.5 us, 29
     (0, 54, 64, 3, 32, 8, 1679, 32, False),      # INT4 keys of the bf16 model, long for one split: 26.6 us, 22
+    (0, 12, 64, 4, 8, 4, 1181, 1024, False),     # asymmetric keys in two groups, likewise: 28.9 us, 25.5
+    (0, 12, 128, 10, 16, 2, 823, 64, True),      # (in one group not)
     (2, 33, 64, 1, 16, 2, 1092, 512, False),     # Stage B: as the whole step
     (2, 33, 64, 13, 16, 2, 16, 1024, True),      # (sixteen winners, whatever the list's length)
     (1, 32, 64, 1, 64, 4, 190, 128, True),       # Stage A: selection alone, 17.4 us, 20.8
