@@ -136,13 +136,13 @@ struct FusedParams {
   float* part_o;  // (B, H_q, NS, D)
   uint32_t* cand_key;  // (B, H_q, NS, Kc)
   int32_t* cand_idx;   // (B, H_q, NS, Kc)
-  int32_t* cand_cnt;   // (B, H_q, NS)
+  float* cand_edge;    // (B, H_q, NS) about the smallest score of the list: where it holds top_k, that many lie no lower
   // two-stage merge (long contexts): `mg_parts` workgroups per row first reduce `mg_spp` consecutive
   // candidate lists each to the row's top_k among them; the final merge then reads those lists
   int mg_parts, mg_spp;
   uint32_t* key2;      // (B, H_q, mg_parts, top_k)
   int32_t* idx2;       // (B, H_q, mg_parts, top_k)
-  int32_t* cnt2;       // (B, H_q, mg_parts)
+  float* edge2;        // (B, H_q, mg_parts)
   // merge outputs
   int64_t* topk_idx;
   int64_t* topk_slots;
@@ -156,6 +156,60 @@ struct FusedParams {
   uint16_t* blend_out;
   long long* phase_clock;  // optional: 10 s_memtime stamps per scan workgroup, 8 per merge workgroup (measurement aid)
 };
+
+// What the merge kernel takes (its first loads depend on the first block: one round trip for the arguments).
+struct MergeParams {
+  const uint32_t* list_key;  // (B, H_q, lists, list_cap) candidate lists: the scan's or, in the final of two stages, the first stage's
+  const int32_t* list_idx;   // (B, H_q, lists, list_cap)
+  const float* list_edge;    // (B, H_q, lists)
+  const float* part_m;       // (B, H_q, n_splits); NULL (Stage B, given statistics): part_o is already normalised
+  const float* part_l;
+  const float* part_o;
+  const int64_t* block_table;
+  const int32_t* seq_lens;
+  const uint16_t* blend_o_new;
+  int H_q, g_act, n_splits, lists, list_cap, list_len, top_k, max_blocks, max_S, mg_spp, mg_parts;
+  int64_t num_slots;
+  const uint8_t* v_data;
+  const uint16_t* v_scales;
+  const float* scores_in;  // FS_STAGE_B
+  const float* stats_m;
+  const float* stats_iz;
+  int64_t* topk_idx;
+  int64_t* topk_slots;
+  float* o_hat;
+  float* o_old;
+  float* W;
+  float* softmax_m;
+  float* softmax_inv_z;
+  uint16_t* blend_out;
+  uint32_t* out_key;  // first stage: (B, H_q, mg_parts, top_k), and (B, H_q, mg_parts)
+  int32_t* out_idx;
+  float* out_edge;
+  long long* phase_clock;
+};
+
+// The merge of one scan (`first`: its first stage) as the kernel takes it.
+inline MergeParams merge_params(const FusedParams& p, bool first) {
+  MergeParams m = {};
+  const bool staged = !first && p.mg_parts > 1;
+  m.list_key = staged ? p.key2 : p.cand_key;
+  m.list_idx = staged ? p.idx2 : p.cand_idx;
+  m.list_edge = staged ? p.edge2 : p.cand_edge;
+  m.lists = staged ? p.mg_parts : p.n_splits;
+  m.list_cap = staged ? p.top_k : p.Kc;
+  m.list_len = staged ? p.mg_spp * p.L : p.L;
+  m.part_m = p.part_m; m.part_l = p.part_l; m.part_o = p.part_o;
+  m.block_table = p.block_table; m.seq_lens = p.seq_lens; m.blend_o_new = p.blend_o_new;
+  m.H_q = p.H_q; m.g_act = p.g_act; m.n_splits = p.n_splits; m.top_k = p.top_k; m.max_blocks = p.max_blocks;
+  m.max_S = p.max_S; m.mg_spp = p.mg_spp; m.mg_parts = p.mg_parts; m.num_slots = p.num_slots;
+  m.v_data = p.v_data; m.v_scales = p.v_scales; m.scores_in = p.scores_in; m.stats_m = p.stats_m; m.stats_iz = p.stats_iz;
+  m.topk_idx = p.topk_idx; m.topk_slots = p.topk_slots; m.o_hat = p.o_hat; m.o_old = p.o_old; m.W = p.W;
+  m.softmax_m = p.softmax_m; m.softmax_inv_z = p.softmax_inv_z; m.blend_out = p.blend_out;
+  m.out_key = p.key2; m.out_idx = p.idx2; m.out_edge = p.edge2;
+  m.phase_clock = p.phase_clock ? p.phase_clock + (size_t)p.B * p.H_kv * p.n_splits * 10 : nullptr;
+  return m;
+}
 
 // Phase-A constants of the INT3 path, built once per workgroup in LDS.
 template <int NSET>
@@ -319,6 +373,21 @@ __device__ inline void set_wave_prio(int p) {
 
 __device__ inline float uniform_f(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+// Range-checked loads through a buffer descriptor (raw, the offsets in bytes): past its end a load returns zero, and the
+// scalar base and offset take the place of 64-bit vector address arithmetic.
+__device__ inline __amdgpu_buffer_rsrc_t buffer_of(const void* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
+__device__ inline int buffer_i32(__amdgpu_buffer_rsrc_t r, int voffset, int soffset) {
+  return (int)__builtin_amdgcn_raw_buffer_load_b32(r, voffset, soffset, 0);
+}
+__device__ inline v4i buffer_i32x4(__amdgpu_buffer_rsrc_t r, int voffset, int soffset) {
+  return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, voffset, soffset, 0));
+}
+__device__ inline float buffer_f32(__amdgpu_buffer_rsrc_t r, int voffset, int soffset) {
+  return __builtin_bit_cast(float, buffer_i32(r, voffset, soffset));
 }
 
 // Pre-correction terms over the winners' packed V rows, shared by the merge kernel and the scan's in-kernel merge: DW
@@ -537,7 +606,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     if (tid < GA) {
       p.part_m[part_base + (size_t)tid * p.n_splits] = -INFINITY;
       p.part_l[part_base + (size_t)tid * p.n_splits] = 0.f;
-      p.cand_cnt[part_base + (size_t)tid * p.n_splits] = 0;
+      p.cand_edge[part_base + (size_t)tid * p.n_splits] = -INFINITY;
     }
     for (int i = tid; i < GA * p.Kc; i += NT)  // unused candidate slots hold key 0 (no score maps to it)
       p.cand_key[(part_base + (size_t)(i / p.Kc) * p.n_splits) * p.Kc + (i % p.Kc)] = 0u;
@@ -1717,7 +1786,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     }
   }
   constexpr int ACC_TOTAL = NSET * AR, ACC_HALF = (ACC_TOTAL + 1) / 2;
-  bool acc_issued = false;  // (uniform) this wavefront's sums are on their way
+  // (uniform) this wavefront's sums are on their way (or it had no chunk: a short split occupies a few wavefronts only)
+  bool acc_issued = wave >= nch;
   auto add_acc_range = [&](const int first, const int last) {  // (constants once the caller's loop is unrolled)
 #pragma unroll
     for (int j = 0; j < ACC_TOTAL * 4; ++j) {
@@ -1952,7 +2022,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       }
       for (; t0 < te; t0 += 1024) emit_block(t0, plain);
       if (!ONE && seg == SEG - 1) {
-        if (lane == 0) p.cand_cnt[part_base + (size_t)h * p.n_splits] = min(Kcap, count);
+        // the lower edge of the cut bucket (a degenerate range: one bucket, the largest score)
+        if (lane == 0) p.cand_edge[part_base + (size_t)h * p.n_splits] = (ba < 0.f) ? (bb - (float)(cut + 1)) * __builtin_amdgcn_rcpf(-ba) : m_sh[h];
         for (int i = count + lane; i < etot; i += 64) ck[i] = 0u;  // (only if a segment emitted less than planned)
       }
     } else if (seg == 0) {
@@ -2040,7 +2111,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           tl_need[h] = -1;
         }
       } else {
-        if (lane == 0) p.cand_cnt[part_base + (size_t)h * p.n_splits] = min(Kcap, count);
+        if (lane == 0) p.cand_edge[part_base + (size_t)h * p.n_splits] = key_to_score(T);
         for (int i = count + lane; i < Kcap; i += 64) ck[i] = 0u;
       }
     }
@@ -2397,12 +2468,6 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
 // instructions instead of a loop over the sixteen entries in every thread.  Integer and min/max only: the result
 // does not depend on the order.
 template <int NWV>
-__device__ inline float waves_max_f(const float* arr, int lane) {
-  float v = (lane < NWV) ? arr[lane] : -INFINITY;
-  JF_DPP_ROW_REDUCE(v, op_fmax, float, -INFINITY);
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 15));
-}
-template <int NWV>
 __device__ inline uint32_t waves_max_u(const uint32_t* arr, int lane) {
   uint32_t v = (lane < NWV) ? arr[lane] : 0u;
   JF_DPP_ROW_REDUCE(v, op_umax, uint32_t, 0u);
@@ -2426,35 +2491,41 @@ __device__ inline void waves_prefix_i(const int* arr, int lane, int wave, int* b
 
 // ---------------------------------------------------------------------------------------------------
 constexpr int MG_MAX_SPLITS = 256;
-constexpr int MG_BINS = 1024;      // linear score buckets of the threshold search
+constexpr int MG_BINS = 512;       // linear score buckets of the threshold search; the last one holds all that lies below
 constexpr int MG_LIST = 1024;      // members of the cut bucket resolved by rank counting
-// Up to here in the registers of every wavefront, beyond over the list in LDS, one member per thread: the sixteen
-// wavefronts share four SIMDs, so a member costs all of them 40 ns, and the list one barrier and half a microsecond.
-constexpr int MG_RANK = 16;
+constexpr int MG_RANK = 16;        // up to here all pairs at once in every wavefront, beyond over the list in LDS
 constexpr int MG_BT_LDS = 4096;    // block-table entries cached in LDS (65536 positions)
 constexpr int MG_LIGHT_THREADS = 256, MG_LIGHT_REGK = 16, MG_LIGHT_TOPK = 512;  // the light shape of the merge
 
 // Launch 2: one workgroup per (sequence, query head).
-//   1. split statistics -> M, l, o_hat
-//   2. the K-th largest candidate key tau (and how many keys equal to tau still belong to the top K): the
-//      candidates are dropped into MG_BINS linear score buckets between the smallest and the largest, a scan
-//      finds the bucket that holds the K-th largest, and the few members of that bucket are ranked against
-//      each other (a bisection over the key range covers the case of more than MG_LIST members)
-//   3. ordered compaction of the winners (key > tau, or key == tau while the quota lasts; candidates are stored
-//      in position order, so ties resolve to the lower position and the output is ascending)
+//   1. split statistics -> M, l, o_hat; a lower bound of the K-th largest score from the splits' own cuts
+//   2. the K-th largest candidate: the candidates are dropped into MG_BINS linear score buckets between that bound and
+//      the largest score, a scan finds the bucket that holds the K-th largest, and the few members of that bucket are
+//      ranked against each other (a bisection over the key range covers the case of more than MG_LIST members)
+//   3. ordered compaction of the winners (candidates are stored in position order, so ties resolve to the lower
+//      position and the output is ascending)
 //   4. slots, softmax weights, and the pre-correction terms over the winners' V rows.
 // The first MG_REGK * MG_THREADS candidates stay in registers from a single load; anything beyond that is
 // re-read from global memory in every pass.
-// Two shapes: 1024 threads x 8 register-resident candidates each (up to 8192 candidates, the common case;
-// the phases are chains of LDS round trips and barriers, so more, lighter threads beat fewer, heavier ones)
+// Two shapes: 1024 threads x 8 register-resident candidates each (up to 8192 candidates, the common case)
 // and 1024 x 32 for first-stage parts that exceed it.
+//
+// What bounds it is neither memory nor launch: run a second time over warm caches the same workgroup takes as long.  It
+// is the length of the chain every wavefront goes through, some 900 instructions and a dozen round trips to LDS, which
+// four wavefronts per SIMD share.  So: the arguments come in one block, first the ones the first loads need (scattered
+// over the scan's they were four dependent scalar loads); the loads are range-checked buffer loads, 16 bytes of candidates
+// each, instead of clamped and masked ones; every wavefront reduces the splits' statistics for itself (lane = split); the
+// range of the buckets comes with the lists instead of from a pass over the candidates; few members of the cut bucket are
+// ranked all pairs at once, in every wavefront.  Six barriers instead of twelve.  Per layer, graph replay, before / now:
+// 1 x 4096 positions, K4V4, top-k 64 20.5 / 18.3 us; 4 x 8100, B4V4 30.3 / 28.9; 4 x 32768, K3V2 36.1 / 35.0;
+// the same with G = 8 33.4 / 32.3; 1 x 131072, K4V4, top-k 512 (two stages) 49.3 / 48.0.
 // PARTIAL = true is the first stage of the two-stage merge: blockIdx.z selects a run of mg_spp candidate
 // lists, steps 2 and 3 run on those alone and the winners (still in position order) are written out as one
 // new candidate list; the final merge (PARTIAL = false, mg_parts > 1) reads these lists instead of the
 // scan's.  The top K of a union is the top K of the parts' top K's, ties included: a candidate that a part
 // drops is beaten by K candidates of that part.
 template <int MODE, int VBITS, int NG, int MG_THREADS, int MG_REGK, bool PARTIAL, bool WIDE = false, int ROLES = 1>
-__global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) {
+__global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) {
   static_assert(!(PARTIAL && MODE == FS_STAGE_B), "Stage B alone selects nothing");
   constexpr int MG_WAVES = MG_THREADS / 64;
   using Pre = PreCorr<VBITS>;
@@ -2469,10 +2540,9 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   // the light shape (many rows per launch, few candidates per row) trades table sizes for workgroups per CU
   constexpr int MG_BT = (MG_THREADS >= 1024) ? MG_BT_LDS : 1024;  // block-table entries cached in LDS
   constexpr int MG_WIN = (MG_THREADS >= 1024) ? FS_LDS_TOPK : 512;  // widest correction of this shape (WIDE: any)
-  __shared__ int hist[MG_BINS];
+  __shared__ __align__(16) int hist[MG_BINS];
   __shared__ uint32_t lkey[MG_LIST];
-  __shared__ float coef_sh[MG_MAX_SPLITS];
-  __shared__ int cnt_sh[MG_MAX_SPLITS];
+  __shared__ int lpos[MG_RANK];  // candidate number of the first members
   __shared__ int bt_sh[MG_BT];
   // winners: key and position while they are selected; the thread that turns winner r into its softmax weight and
   // paged slot overwrites the two entries in place (weight bits over the key, slot over the position)
@@ -2482,219 +2552,536 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   extern __shared__ __align__(16) uint32_t win_dyn[];
   uint32_t* const win_key = WIDE ? win_dyn : win_key_s;
   int* const win_idx = WIDE ? reinterpret_cast<int*>(win_dyn + p.top_k) : win_idx_s;
-  __shared__ uint32_t cnt_a[MG_REGK / 4 * MG_WAVES];  // packed (winners, ties) per (group, wavefront)
   __shared__ float red_sh[VGRP][D];
   __shared__ float old_sh[VWAVES][D];
+  __shared__ float ohat_sh[D];
   __shared__ float w_sh[VWAVES];
-  __shared__ float wred_f[MG_WAVES];
   __shared__ uint32_t wred_u[MG_WAVES], wred_k[MG_WAVES];
-  __shared__ float wred_g[MG_WAVES];
   __shared__ int wred_i[MG_WAVES], wred_j[MG_WAVES];
-  __shared__ int lcount_sh, cut_sh, above_sh, quota_sh;
+  __shared__ int lcount_sh, quota_sh;
   __shared__ uint32_t tau_sh;
 
-  const int b = blockIdx.x, hq = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  // (first stage: x = sequence, y = query head, z = part; else x = head of the group, y = kv-head, z = sequence)
+  const int b = PARTIAL ? blockIdx.x : blockIdx.z, hkv = PARTIAL ? 0 : blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int hq = PARTIAL ? blockIdx.y : hkv * p.g_act + blockIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const size_t bh = (size_t)b * p.H_q + hq;
-  const int NS = p.n_splits, K = p.top_k;
-  const int hkv = hq / (p.H_q / p.H_kv);
-  // candidate lists of this workgroup: NL lists of capacity Kc
-  const bool staged = !PARTIAL && p.mg_parts > 1;
+  const int NS = p.n_splits, K = p.top_k, Kc = p.list_cap, LL = p.list_len;
+  // candidate lists of this workgroup: NL lists of capacity Kc, each over LL positions
   const int part = PARTIAL ? (int)blockIdx.z : 0;
   const int l0 = PARTIAL ? part * p.mg_spp : 0;
   // (Stage B alone: the winners are an input, there are no candidate lists)
-  const int NL = (MODE == FS_STAGE_B) ? 0 : (PARTIAL ? min(p.mg_spp, NS - l0) : (staged ? p.mg_parts : NS));
-  const int Kc = staged ? K : p.Kc;
-  const uint32_t* ck = staged ? p.key2 + bh * p.mg_parts * K : p.cand_key + (bh * NS + l0) * Kc;
-  const int32_t* ci = staged ? p.idx2 + bh * p.mg_parts * K : p.cand_idx + (bh * NS + l0) * Kc;
-  const int32_t* cc = staged ? p.cnt2 + bh * p.mg_parts : p.cand_cnt + bh * NS + l0;
+  constexpr bool HAS_LISTS = (MODE != FS_STAGE_B);
+  const int NL = !HAS_LISTS ? 0 : (PARTIAL ? min(p.mg_spp, p.lists - l0) : p.lists);
+  const size_t list0 = bh * p.lists + l0, split0 = bh * NS + l0;
+  const uint32_t* ck = p.list_key + list0 * Kc;
+  const int32_t* ci = p.list_idx + list0 * Kc;
+  const float* ce = p.list_edge + list0;
   const int64_t* bt = p.block_table + (size_t)b * p.max_blocks;
-  int64_t* out_idx = p.topk_idx + bh * (size_t)K;
-  int64_t* out_slot = p.topk_slots + bh * (size_t)K;
   const int flat = NL * Kc;
-  const int rounds = (flat + MG_THREADS - 1) / MG_THREADS;
   const int nblk_lds = min(p.max_blocks, MG_BT);
 
-  long long* mclk = (kDebugHooks && p.phase_clock && !PARTIAL) ? p.phase_clock + (size_t)p.B * p.H_kv * p.n_splits * 10 + bh * 8 : nullptr;
+  long long* mclk = (kDebugHooks && p.phase_clock && !PARTIAL) ? p.phase_clock + bh * 8 : nullptr;
   if (mclk && tid == 0) mclk[0] = JF_CLK();
 
-  // ---- everything that does not depend on anything else is requested first, in the order of its use.  Every load
-  // is unconditional, on a clamped index, and its mask is applied further down: under a condition the compiler waits
-  // for a load inside its branch, and these loads (first touches of what other XCDs wrote) would cost one round trip
-  // after the other instead of one for all.
-  constexpr bool HAS_LISTS = (MODE != FS_STAGE_B);
-  float pm = -INFINITY, pl = 0.f;
-  int my_cnt = 0;
+  // ---- everything that does not depend on anything else is requested first, in the order of its use: one round trip
+  // of first touches (what other XCDs wrote) instead of one after the other.  Buffer loads: past the end of what the
+  // descriptor covers they return zero, so neither clamps nor masks are needed.
   // (given statistics, jf_softmax_v_int8_tiles: the partial rows are already normalised and come without maxima and
-  // sums; those loads then read the page table, which every caller of this kernel passes, and are masked)
+  // sums)
   const bool has_parts = MODE != FS_STAGE_B || p.part_m != nullptr;
-  const float* dummy_f = reinterpret_cast<const float*>(bt);
-  // The first MG_REGK * MG_THREADS candidates live in registers: group g = r / 4 of a thread holds the four
-  // consecutive candidates (g * MG_THREADS + tid) * 4 + (r % 4), fetched with one 16-byte load.  Candidate
-  // order = (group, thread, element).  Slots past a list's count hold key 0 (written by the producer).
+  constexpr int SPL = MG_MAX_SPLITS / 64;  // splits per lane
+  const int NV = PARTIAL ? NL : NS;        // splits whose statistics are read
+  float pm[SPL], pl[SPL], pe[SPL];
+  // (a vector load: a wait for the kernel's arguments would wait for any scalar load that is under way)
+  const int len_mine = buffer_i32(buffer_of(p.seq_lens + b, 4), 0, 0);
+  const auto rm = buffer_of(p.part_m + split0, has_parts ? NV * 4 : 0), rl = buffer_of(p.part_l + split0, has_parts ? NV * 4 : 0);
+  const auto re = buffer_of(ce, NL * 4);
+  const bool many = NV > 64;  // (uniform) more splits than lanes
+#pragma unroll
+  for (int i = 0; i < SPL; ++i) pm[i] = pl[i] = pe[i] = 0.f;
+  auto request_split = [&](int i) {
+    pm[i] = buffer_f32(rm, lane * 4, i * 256);
+    if constexpr (HAS_LISTS) pe[i] = buffer_f32(re, lane * 4, i * 256);
+    pl[i] = buffer_f32(rl, lane * 4, i * 256);
+  };
+  request_split(0);
+  if (many) {
+#pragma unroll
+    for (int i = 1; i < SPL; ++i) request_split(i);
+  }
+  // The first MG_REGK * MG_THREADS candidates live in registers: wavefront w holds `per` x 64 consecutive ones, 256 per group
+  // of four registers, of which lane l has the four at 4 l (one 16-byte load).  Slots past a list's end hold key 0 (written
+  // by the producer).
   static_assert(MG_REGK % 4 == 0, "register candidates come in groups of four");
   constexpr int NGRP = MG_REGK / 4;
-  const int rreg = min((flat + 4 * MG_THREADS - 1) / (4 * MG_THREADS), NGRP) * 4;  // register slots in use (uniform)
+  constexpr bool LAZY = MG_REGK > 16;  // the positions of the winners are fetched when they are known
+  const int per = min((flat + 4 * MG_THREADS - 1) / (4 * MG_THREADS), NGRP) * 4;  // registers in use (uniform)
+  const int f0 = wave * per * 64;  // number of this wavefront's first candidate
+  auto f_of = [&](int r) -> int { return f0 + (r >> 2) * 256 + lane * 4 + (r & 3); };
+  const auto rk = buffer_of(ck, flat * 4), ri = buffer_of(ci, flat * 4);
   uint32_t kreg[MG_REGK];
-  int ireg[MG_REGK];
-  v4u k4[NGRP];
-  v4i i4[NGRP];
-  // what the first barrier interval needs goes first (loads return in order): the split maxima, the list counts,
-  // the candidate keys
-  if constexpr (!PARTIAL) pm = *(has_parts ? p.part_m + bh * NS + min(tid, NS - 1) : dummy_f);
-  if constexpr (HAS_LISTS) my_cnt = cc[min(tid, NL - 1)];
+  int ireg[LAZY ? 1 : MG_REGK];
 #pragma unroll
   for (int g = 0; g < NGRP; ++g) {
-    k4[g] = (v4u){0u, 0u, 0u, 0u};
-    if constexpr (HAS_LISTS)  // (flat is a multiple of 4; groups past the end are not requested)
-      if (g == 0 || 4 * g < rreg) k4[g] = *reinterpret_cast<const v4u*>(ck + min((g * MG_THREADS + tid) * 4, flat - 4));
-  }
-  if constexpr (!PARTIAL) pl = *(has_parts ? p.part_l + bh * NS + min(tid, NS - 1) : dummy_f);
+    v4i x = {0, 0, 0, 0};
+    if (HAS_LISTS && (g == 0 || 4 * g < per)) x = buffer_i32x4(rk, lane * 16, (f0 + g * 256) * 4);
 #pragma unroll
-  for (int g = 0; g < NGRP; ++g) {
-    i4[g] = (v4i){0, 0, 0, 0};
-    if constexpr (HAS_LISTS)
-      if (g == 0 || 4 * g < rreg) i4[g] = *reinterpret_cast<const v4i*>(ci + min((g * MG_THREADS + tid) * 4, flat - 4));
+    for (int j = 0; j < 4; ++j) kreg[4 * g + j] = (uint32_t)x[j];
   }
-  uint16_t blend_raw = 0;
-  float blend_new = 0.f, blend_hat = 0.f;
-  if constexpr (MODE == FS_FULL && !PARTIAL)  // (no blend: any readable address)
-    blend_raw = *(p.blend_out ? p.blend_o_new + bh * D + (tid & (D - 1)) : reinterpret_cast<const uint16_t*>(ck));
-  // o_hat: the thread groups of 128 take the splits round-robin (first terms requested now)
-  constexpr int PO_PRE = 2, PO_GRP = MG_THREADS / D;
-  float po[PO_PRE];
-  {
-    const int d = tid & (D - 1), q4 = tid >> 7;
+  if constexpr (!LAZY) {
 #pragma unroll
-    for (int i = 0; i < PO_PRE; ++i) {
-      po[i] = 0.f;
-      if constexpr (MODE != FS_STAGE_A && !PARTIAL)
-        po[i] = p.part_o[(bh * NS + min(q4 + VGRP * i, NS - 1)) * D + d];
+    for (int g = 0; g < NGRP; ++g) {
+      v4i x = {0, 0, 0, 0};
+      if (HAS_LISTS && (g == 0 || 4 * g < per)) x = buffer_i32x4(ri, lane * 16, (f0 + g * 256) * 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ireg[4 * g + j] = x[j];
     }
   }
-  // page-table entries for the table in LDS: stored after the first barrier, so that the wait for them (the
-  // youngest loads) is not part of the first interval
+  // o_hat: the thread groups of 128 take the splits round-robin (first terms requested now)
+  constexpr int PO_PRE = 2, PO_GRP = MG_THREADS / D;
+  const int q4 = wave / (D / 64);
+  const auto ro = buffer_of(p.part_o + bh * NS * D, NS * D * 4);
+  float po[PO_PRE];
+#pragma unroll
+  for (int i = 0; i < PO_PRE; ++i) {
+    po[i] = 0.f;
+    if constexpr (MODE != FS_STAGE_A && !PARTIAL) po[i] = buffer_f32(ro, (tid & (D - 1)) * 4, (q4 + VGRP * i) * (D * 4));
+  }
+  // page-table entries for the table in LDS (the low half of the 64-bit entry only)
   constexpr int BTPT = (MG_BT + MG_THREADS - 1) / MG_THREADS;
   int bt_mine[BTPT];
+  const auto rb = buffer_of(bt, nblk_lds * 8);
 #pragma unroll
-  for (int i = 0; i < BTPT; ++i) {
-    bt_mine[i] = 0;
-    // (the low half of the 64-bit entry only: the unused half of a wider load is a register the compiler hands out
-    // again at once, and writing it has to wait for the load)
-    if constexpr (!PARTIAL) bt_mine[i] = reinterpret_cast<const int*>(bt)[2 * min(tid + i * MG_THREADS, p.max_blocks - 1)];
+  for (int i = 0; i < BTPT; ++i) bt_mine[i] = 0;
+  if constexpr (!PARTIAL) {
+    bt_mine[0] = buffer_i32(rb, tid * 8, 0);
+    if (nblk_lds > MG_THREADS) {  // (uniform)
+#pragma unroll
+      for (int i = 1; i < BTPT; ++i) bt_mine[i] = buffer_i32(rb, tid * 8, i * MG_THREADS * 8);
+    }
   }
+  uint16_t blend_raw = 0;
+  if constexpr (MODE == FS_FULL && !PARTIAL)  // (no blend: any readable address)
+    blend_raw = *(p.blend_o_new ? p.blend_o_new + bh * D + (tid & (D - 1)) : reinterpret_cast<const uint16_t*>(ck));
   for (int i = tid; i < MG_BINS; i += MG_THREADS) hist[i] = 0;
   if (tid == 0) lcount_sh = 0;
-  // the masks of the loads the first interval uses (the others follow its barrier)
-  if (tid >= NS || !has_parts) pm = -INFINITY;
-  if (tid >= NL) my_cnt = 0;
-#pragma unroll
-  for (int g = 0; g < NGRP; ++g) {
-    const bool in = (g * MG_THREADS + tid) * 4 < flat;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) kreg[4 * g + j] = in ? k4[g][j] : 0u;
-  }
-  if (tid < NL) cnt_sh[tid] = my_cnt;
+  lds_barrier();
 
+  // positions the lists stand for; not more than K of them: every candidate wins
+  const int S = max(0, min(p.max_S, __builtin_amdgcn_readfirstlane(len_mine))) - l0 * LL;
+  const bool take_all = (PARTIAL ? min(S, NL * LL) : S) <= K;  // (uniform)
+  // ---- interval 1: the statistics, in every wavefront; the candidates drop into the buckets
+  // The K-th largest score is no smaller than the cut of any list that stands for at least K positions (K of its own
+  // lie above), nor than the smallest of all cuts.
+  // (reduced as order-preserving integers, 0 below every score: one instruction a step)
+  const bool whole = LL >= K;  // (uniform) lists of K positions: their largest cut; else the smallest cut
+  const uint32_t flip = whole ? 0u : 0xffffffffu;
+  uint32_t m_key = 0u, e_key = 0u;
+  auto take_split = [&](int i) {
+    const int s = lane + 64 * i;
+    pm[i] = (s < NV && has_parts) ? pm[i] : -INFINITY;
+    m_key = max(m_key, score_key(pm[i]));
+    const int n_list = S - s * LL;  // (a list past the end of the sequence: not above zero)
+    const uint32_t e = score_key(pe[i]) ^ flip;
+    e_key = max(e_key, (s < NL && n_list >= (whole ? K : 1)) ? e : 0u);
+  };
+  take_split(0);
+  if (many) {
+#pragma unroll
+    for (int i = 1; i < SPL; ++i) take_split(i);
+  }
+  m_key = wave_max_u(m_key);
+  e_key = wave_max_u(e_key) ^ flip;
+  float M = key_to_score(m_key);
+  const float hi = M, lo = key_to_score(e_key);
+  if (!isfinite(M)) M = 0.f;
+  float coef[SPL], lsum = 0.f;
+#pragma unroll
+  for (int i = 0; i < SPL; ++i) coef[i] = 0.f;
+  auto weigh_split = [&](int i) {
+    coef[i] = (pm[i] == -INFINITY) ? 0.f : __expf(pm[i] - M);
+    lsum += wave_sum(pl[i] * coef[i]);  // fixed reduction tree: deterministic
+    if (!has_parts) coef[i] = 1.f;
+  };
+  weigh_split(0);
+  if (many) {
+#pragma unroll
+    for (int i = 1; i < SPL; ++i) weigh_split(i);
+  }
+  // (bucket 0 = largest scores; the last one, for what lies below `lo`, is not counted)
+  const float range = hi - lo;
+  const float iw = ((float)MG_BINS - 1.5f) * __builtin_amdgcn_rcpf(range);
+  const float bb = hi * iw;
+  // No usable range (all cuts at the largest score, infinite scores), or a NaN among the scores, whose place in the order
+  // of the keys the buckets do not know (its split's sum of weights is a NaN too): bisection over the keys.
+  const bool exact = !take_all && !(range > 0.f && isfinite(range) && isfinite(iw) && isfinite(bb) && lsum == lsum);  // (uniform)
+  // (an unused slot's key 0 stands for a NaN, which the minimum turns into the last bucket)
+  auto bin_of = [&](uint32_t k) -> int {
+    return (int)__builtin_fmaxf(__builtin_fminf(__builtin_fmaf(key_to_score(k), -iw, bb), (float)(MG_BINS - 1)), 0.f);
+  };
   // key of candidate f in pass-over-all-candidates loops: registers first, global memory beyond
+  const int rounds = (flat + MG_THREADS - 1) / MG_THREADS;
   auto key_of = [&](int r) -> uint32_t {
     const int f = r * MG_THREADS + tid;
     return (f < flat) ? ck[f] : 0u;
   };
-  // number of candidates with key >= x (x > 0), identical in every thread
-  auto count_ge = [&](uint32_t x) -> int {
-    int c = 0;
+  int bin[MG_REGK];
 #pragma unroll
-    for (int r = 0; r < MG_REGK; ++r)
-      if (r < rreg) c += __popcll(__builtin_amdgcn_ballot_w64(kreg[r] >= x));
-    for (int r = MG_REGK; r < rounds; ++r) c += __popcll(__builtin_amdgcn_ballot_w64(key_of(r) >= x));
-    lds_barrier();
-    if (lane == 0) wred_i[wave] = c;
-    lds_barrier();
-    int before, t;
-    waves_prefix_i<MG_WAVES>(wred_i, lane, 0, &before, &t);
-    return t;
-  };
-
-  // The split statistics (M, coefficients e^{m_i - M}, l, o_hat) and the threshold search (range of the candidate
-  // keys, bucket histogram, bucket scan) do not depend on each other: their steps share the barrier intervals.
-  // ---- interval 1: per-wavefront maximum of the split maxima and range of the candidate keys
-  if (!PARTIAL) {
-    const float v = wave_max(pm);
-    if (lane == 0) wred_f[wave] = v;
-  }
-  uint32_t kmin = 0xffffffffu, kmax = 0u;
+  for (int r = 0; r < MG_REGK; ++r) bin[r] = MG_BINS - 1;
+  if constexpr (HAS_LISTS) {
+    if (take_all) {
 #pragma unroll
-  for (int r = 0; r < MG_REGK; ++r)
-    if (r < rreg && kreg[r] != 0u) { kmin = min(kmin, kreg[r]); kmax = max(kmax, kreg[r]); }
-  for (int r = MG_REGK; r < rounds; ++r) {
-    const uint32_t k = key_of(r);
-    if (k != 0u) { kmin = min(kmin, k); kmax = max(kmax, k); }
-  }
-  kmin = wave_min_u(kmin);
-  kmax = wave_max_u(kmax);
-  if (lane == 0) { wred_u[wave] = kmin; wred_k[wave] = kmax; }
-  lds_barrier();
-  if (mclk && tid == 0) mclk[6] = JF_CLK();
-  if (tid >= NS || !has_parts) pl = 0.f;
-  if (MODE == FS_FULL && !PARTIAL && p.blend_out && tid < D) blend_new = bf16_to_f32(blend_raw);
+      for (int r = 0; r < MG_REGK; ++r) bin[r] = (kreg[r] != 0u) ? 0 : MG_BINS - 1;
+    } else if (!exact) {
 #pragma unroll
-  for (int g = 0; g < NGRP; ++g) {
-    const bool in = (g * MG_THREADS + tid) * 4 < flat;
+      for (int g = 0; g < NGRP; ++g)
+        if (g == 0 || 4 * g < per) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) ireg[4 * g + j] = in ? i4[g][j] : 0;
-  }
-  if constexpr (!PARTIAL) {  // (first read long after the next barrier)
-#pragma unroll
-    for (int i = 0; i < BTPT; ++i)
-      if (tid + i * MG_THREADS < nblk_lds) bt_sh[tid + i * MG_THREADS] = bt_mine[i];
-  }
-  // ---- interval 2: M, the coefficients, per-wavefront sums of l; the candidates drop into MG_BINS linear buckets
-  float M = -INFINITY;
-  if (!PARTIAL) {
-    M = waves_max_f<MG_WAVES>(wred_f, lane);
-    if (!isfinite(M)) M = 0.f;
-    float coef = (pm == -INFINITY) ? 0.f : __expf(pm - M);
-    if (!has_parts) coef = 1.f;
-    if (tid < NS) coef_sh[tid] = coef;
-    const float v = wave_sum(pl * coef);  // fixed reduction tree: deterministic
-    if (lane == 0) wred_g[wave] = v;
-  }
-  int total = 0;
-  for (int s2 = lane; s2 < NL; s2 += 64) total += cnt_sh[s2];
-  total = wave_sum_i(total);
-  kmin = waves_min_u<MG_WAVES>(wred_u, lane);
-  kmax = waves_max_u<MG_WAVES>(wred_k, lane);
-  const float hi = key_to_score(kmax), lo = key_to_score(kmin);
-  const float range = hi - lo;
-  const float iw = (range > 0.f && isfinite(range)) ? ((float)MG_BINS - 0.01f) / range : 0.f;
-  const float ba = -iw, bb = isfinite(hi) ? hi * iw : 0.f;
-  auto bin_of = [&](uint32_t k) -> int {
-    return (int)__builtin_amdgcn_fmed3f(__builtin_fmaf(key_to_score(k), ba, bb), 0.f, (float)(MG_BINS - 1));
-  };
-  const bool take_all = (total <= K);  // (uniform) every candidate wins: no threshold
-  if (!take_all) {
-#pragma unroll
-    for (int r = 0; r < MG_REGK; ++r)
-      if (r < rreg && kreg[r] != 0u) atomicAdd(&hist[bin_of(kreg[r])], 1);
-    for (int r = MG_REGK; r < rounds; ++r) {
-      const uint32_t k = key_of(r);
-      if (k != 0u) atomicAdd(&hist[bin_of(k)], 1);
+          for (int r = 4 * g; r < 4 * g + 4; ++r) {
+            bin[r] = bin_of(kreg[r]);
+            if (bin[r] < MG_BINS - 1) atomicAdd(&hist[bin[r]], 1);
+          }
+        }
+      for (int r = MG_REGK; r < rounds; ++r) {
+        const uint32_t k = key_of(r);
+        if (k != 0u) {
+          const int c = bin_of(k);
+          if (c < MG_BINS - 1) atomicAdd(&hist[c], 1);
+        }
+      }
     }
   }
+  if constexpr (!PARTIAL) {
+    bt_sh[tid] = bt_mine[0];
+    if (nblk_lds > MG_THREADS) {
+#pragma unroll
+      for (int i = 1; i < BTPT; ++i) bt_sh[tid + i * MG_THREADS] = bt_mine[i];
+    }
+  }
+  if constexpr (!PARTIAL && MODE != FS_STAGE_A) {
+    // o_hat: group vg of the eight takes every eighth split, then a fixed-order sum (after the next barrier)
+    auto coef_of = [&](int sp) -> float {  // (sp is uniform)
+      float c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, coef[0]), sp & 63));
+      if (!many) return c;
+#pragma unroll
+      for (int i = 1; i < SPL; ++i)
+        if (sp / 64 == i) c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, coef[i]), sp & 63));
+      return c;
+    };
+    const int d4 = (tid & (D - 1)) * 4;
+#pragma unroll
+    for (int v = 0; v < VGRP / PO_GRP; ++v) {
+      const int vg = q4 + v * PO_GRP;
+      float o = 0.f;
+#pragma unroll
+      for (int i = 0; i < PO_PRE; ++i) {
+        const int sp = vg + VGRP * i;
+        if (sp < NS) o = __builtin_fmaf((v == 0) ? po[i] : buffer_f32(ro, d4, sp * (D * 4)), coef_of(sp), o);
+      }
+      // the remaining splits eight at a time: the loads of a batch are in flight together, the sum keeps its order
+      constexpr int PO_B = 8;
+      for (int sp0 = vg + VGRP * PO_PRE; sp0 < NS; sp0 += VGRP * PO_B) {
+        float w[PO_B];
+#pragma unroll
+        for (int u = 0; u < PO_B; ++u) w[u] = buffer_f32(ro, d4, (sp0 + VGRP * u) * (D * 4));
+#pragma unroll
+        for (int u = 0; u < PO_B; ++u)
+          if (sp0 + VGRP * u < NS) o = __builtin_fmaf(w[u], coef_of(sp0 + VGRP * u), o);
+      }
+      red_sh[vg][tid & (D - 1)] = o;
+    }
+  }
+  if (mclk && tid == 0) mclk[6] = JF_CLK();
   lds_barrier();
   if (mclk && tid == 0) mclk[7] = JF_CLK();
-  // ---- interval 3: 1/l, the partial sums of o_hat; first half of the bucket scan
-  float inv_z = 0.f;
-  if (!PARTIAL) {
-    float lsum = 0.f;
+  int n_out = 0;
+  float edge = whole ? -INFINITY : lo;  // PARTIAL: no winner scores less
+  if constexpr (HAS_LISTS) {
+    // ---- interval 2, in every wavefront: the bucket of the K-th largest; the wavefront's candidates before it, and the
+    // list of that bucket's members
+    int cut = 1, need = 0;  // (every candidate wins: they are in bucket 0)
+    if (!take_all && !exact) {
+      constexpr int BPL = MG_BINS / 64;  // lane l owns buckets BPL * l .. (ascending bucket = descending score)
+      static_assert(BPL % 4 == 0, "16-byte reads");
+      int mine = 0;
 #pragma unroll
-    for (int w = 0; w < MG_WAVES; ++w) lsum += wred_g[w];
-    inv_z = (lsum > 0.f) ? 1.0f / lsum : 0.f;
-    if (tid == 0 && p.softmax_m) {
-      p.softmax_m[bh] = M;
-      p.softmax_inv_z[bh] = inv_z;
+      for (int u = 0; u < BPL; u += 4) {
+        const v4i x = *reinterpret_cast<const v4i*>(hist + BPL * lane + u);
+        mine += (x[0] + x[1]) + (x[2] + x[3]);
+      }
+      const int incl = wave_incl_scan_i(mine);
+      const unsigned long long who = __builtin_amdgcn_ballot_w64(incl >= K);
+      cut = MG_BINS - 1;
+      int above = __builtin_amdgcn_readlane(incl, 63);
+      if (who != 0ull) {
+        const int src = __ffsll((long long)who) - 1;
+        // the buckets of that lane, one per lane
+        const int own = (lane < BPL) ? hist[BPL * src + lane] : 0;
+        int run = own;
+        JF_DPP_ROW_REDUCE(run, op_iadd, int, 0);  // inclusive scan inside the row
+        run += __builtin_amdgcn_readlane(incl - mine, src);
+        const int u = __ffsll((long long)__builtin_amdgcn_ballot_w64(run >= K)) - 1;  // (the lane's total reaches K)
+        static_assert(BPL <= 16, "one row");
+        cut = BPL * src + u;
+        above = __builtin_amdgcn_readlane(run - own, u);
+      }
+      need = K - above;  // so many of the cut bucket's members belong to the top K
     }
+    int n_above = 0;
+    bool has_members = false;  // (uniform)
+    auto list_member = [&](uint32_t key, int f) {
+      const int i = atomicAdd(&lcount_sh, 1);
+      if (i < MG_LIST) lkey[i] = key;
+      if (i < MG_RANK) lpos[i] = f;
+    };
+    if (!exact) {
+#pragma unroll
+      for (int g = 0; g < NGRP; ++g)
+        if (g == 0 || 4 * g < per) {
+#pragma unroll
+          for (int r = 4 * g; r < 4 * g + 4; ++r) {
+            n_above += __popcll(__builtin_amdgcn_ballot_w64(bin[r] < cut));
+            const bool member = bin[r] == cut && kreg[r] != 0u;
+            if (__builtin_amdgcn_ballot_w64(member) != 0ull) {
+              has_members = true;
+              if (member) list_member(kreg[r], f_of(r));
+            }
+          }
+        }
+      if (!take_all) {
+        for (int r = MG_REGK; r < rounds; ++r) {
+          const uint32_t k = key_of(r);
+          if (k != 0u && bin_of(k) == cut) list_member(k, r * MG_THREADS + tid);
+        }
+      }
+    }
+    if (lane == 0) wred_i[wave] = n_above;
+    lds_barrier();
+    if (mclk && tid == 0) mclk[1] = JF_CLK();
+    const int m = __builtin_amdgcn_readfirstlane(lcount_sh);
+    if (!exact && m <= MG_RANK && rounds <= MG_REGK) {
+      // ---- interval 3: the last winner among the members (larger key first, then lower position), then every winner
+      // stores its key and position at its place
+      uint32_t tk = 0u;
+      int tf = -1, own_f = 0;
+      unsigned long long won = 0ull;  // members that win (bit = place in the list)
+      if (m > 0) {  // (uniform) all pairs: lane (i, j) compares member 4 * step + i with member j
+        const int j = lane & 15, i = lane >> 4;
+        const bool vj = j < m;
+        const uint32_t kj = vj ? lkey[j] : 0u;
+        const int fj = vj ? lpos[j] : 0x7fffffff;
+        uint32_t ki[MG_RANK / 4];
+        int fi[MG_RANK / 4], sel = 0;
+#pragma unroll
+        for (int st = 0; st < MG_RANK / 4; ++st) {
+          ki[st] = lkey[4 * st + i];
+          fi[st] = lpos[4 * st + i];
+        }
+        own_f = fj;
+#pragma unroll
+        for (int st = 0; st < MG_RANK / 4; ++st) {
+          if (4 * st < m) {
+            const unsigned long long gt = __builtin_amdgcn_ballot_w64(vj && (kj > ki[st] || (kj == ki[st] && fj < fi[st])));
+            const int rank = __popc((uint32_t)(gt >> (16 * i)) & 0xffffu);
+            const unsigned long long hit = __builtin_amdgcn_ballot_w64(4 * st + i < m && rank == need - 1);
+            if (hit != 0ull) sel = 4 * st + (__ffsll((long long)hit) - 1) / 16;
+          }
+        }
+        tk = (uint32_t)__builtin_amdgcn_readlane((int)kj, sel);
+        tf = __builtin_amdgcn_readlane(fj, sel);
+        won = __builtin_amdgcn_ballot_w64(lane < 16 && vj && (kj > tk || (kj == tk && fj <= tf)));
+      }
+      int before, all;
+      waves_prefix_i<MG_WAVES>(wred_i, lane, wave, &before, &all);
+      int place = before + __popcll(won & __builtin_amdgcn_ballot_w64(own_f < f0));
+      n_out = min(K, all + __popcll(won));
+#pragma unroll
+      for (int g = 0; g < NGRP; ++g)
+        if (g == 0 || 4 * g < per) {
+          bool win[4];
+          int mine = 0;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int r = 4 * g + j;
+            win[j] = bin[r] < cut;
+            if (has_members)  // (uniform)
+              win[j] = win[j] || (bin[r] == cut && kreg[r] != 0u && (kreg[r] > tk || (kreg[r] == tk && f_of(r) <= tf)));
+            mine += win[j] ? 1 : 0;
+          }
+          const int incl = wave_incl_scan_i(mine);
+          int at = place + incl - mine;
+          place += __builtin_amdgcn_readlane(incl, 63);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int r = 4 * g + j;
+            if (win[j]) {
+              if (at < K) {
+                win_key[at] = kreg[r];
+                win_idx[at] = LAZY ? f_of(r) : ireg[LAZY ? 0 : r];
+              }
+              ++at;
+            }
+          }
+        }
+      if (PARTIAL && !take_all) edge = key_to_score(tk);
+    } else {
+      // ---- the general case: tau = the K-th largest key, `quota` of the keys equal to it win
+      uint32_t tau = 0u;
+      int quota = 0;
+      if (take_all) {
+        quota = 0;
+      } else if (!exact && m <= MG_LIST) {
+        // rank counting: the member with fewer than `need` larger members and at least `need` members >= it
+        for (int i = tid; i < m; i += MG_THREADS) {
+          const uint32_t k = lkey[i];
+          int gt = 0, ge = 0;
+          for (int j = 0; j < m; ++j) {
+            const uint32_t o = lkey[j];
+            gt += (o > k) ? 1 : 0;
+            ge += (o >= k) ? 1 : 0;
+          }
+          if (gt < need && need <= ge) {  // every thread that gets here writes the same pair
+            tau_sh = k;
+            quota_sh = need - gt;
+          }
+        }
+        lds_barrier();
+        tau = tau_sh;
+        quota = quota_sh;
+      } else {
+        // bisection over the key range: largest x with count(key >= x) >= K
+        uint32_t kmin = 0xffffffffu, kmax = 0u;
+#pragma unroll
+        for (int r = 0; r < MG_REGK; ++r)
+          if (kreg[r] != 0u) { kmin = min(kmin, kreg[r]); kmax = max(kmax, kreg[r]); }
+        for (int r = MG_REGK; r < rounds; ++r) {
+          const uint32_t k = key_of(r);
+          if (k != 0u) { kmin = min(kmin, k); kmax = max(kmax, k); }
+        }
+        kmin = wave_min_u(kmin);
+        kmax = wave_max_u(kmax);
+        if (lane == 0) { wred_u[wave] = kmin; wred_k[wave] = kmax; }
+        lds_barrier();
+        kmin = waves_min_u<MG_WAVES>(wred_u, lane);
+        kmax = waves_max_u<MG_WAVES>(wred_k, lane);
+        // number of candidates with key >= x (x > 0), identical in every thread
+        auto count_ge = [&](uint32_t x) -> int {
+          int c = 0;
+#pragma unroll
+          for (int r = 0; r < MG_REGK; ++r)
+            if (r < per) c += __popcll(__builtin_amdgcn_ballot_w64(kreg[r] >= x));
+          for (int r = MG_REGK; r < rounds; ++r) c += __popcll(__builtin_amdgcn_ballot_w64(key_of(r) >= x));
+          lds_barrier();
+          if (lane == 0) wred_i[wave] = c;
+          lds_barrier();
+          int before, t;
+          waves_prefix_i<MG_WAVES>(wred_i, lane, 0, &before, &t);
+          return t;
+        };
+        uint32_t lo_k = kmin, hi_k = kmax;  // invariant: count_ge(lo_k) >= K
+        while (lo_k < hi_k) {
+          const uint32_t mid = lo_k + (hi_k - lo_k + 1u) / 2u;
+          if (count_ge(mid) >= K) lo_k = mid;
+          else hi_k = mid - 1u;
+        }
+        tau = lo_k;
+        quota = K - ((tau == 0xffffffffu) ? 0 : count_ge(tau + 1u));
+      }
+      // ordered compaction: winners (key above tau) and ties of every wavefront, then its own, register by register
+      auto is_above = [&](uint32_t key) { return key != 0u && (take_all || key > tau); };
+      auto is_tie = [&](uint32_t key) { return key != 0u && !take_all && key == tau; };
+      int na = 0, nt = 0;
+#pragma unroll
+      for (int r = 0; r < MG_REGK; ++r) {
+        na += __popcll(__builtin_amdgcn_ballot_w64(is_above(kreg[r])));
+        nt += __popcll(__builtin_amdgcn_ballot_w64(is_tie(kreg[r])));
+      }
+      lds_barrier();  // (wred_i has been read)
+      if (lane == 0) {
+        wred_i[wave] = na;
+        wred_j[wave] = nt;
+      }
+      lds_barrier();
+      int base_above, base_tie, all_above, all_tie;
+      waves_prefix_i<MG_WAVES>(wred_i, lane, wave, &base_above, &all_above);
+      waves_prefix_i<MG_WAVES>(wred_j, lane, wave, &base_tie, &all_tie);
+      auto store = [&](uint32_t key, int pa, int pt, auto position) {  // pa, pt: winners above and ties before this one
+        if (is_above(key) || (is_tie(key) && pt < quota)) {
+          const int at = pa + min(pt, quota);
+          if (at < K) {
+            win_key[at] = key;
+            win_idx[at] = position();
+          }
+        }
+      };
+#pragma unroll
+      for (int g = 0; g < NGRP; ++g)
+        if (4 * g < per) {
+          int c = 0;  // low half: winners above, high half: ties (at most 256 of a wavefront's group)
+#pragma unroll
+          for (int r = 4 * g; r < 4 * g + 4; ++r) c += (is_above(kreg[r]) ? 1 : 0) + (is_tie(kreg[r]) ? 0x10000 : 0);
+          const int incl = wave_incl_scan_i(c), last = __builtin_amdgcn_readlane(incl, 63);
+          int pa = base_above + ((incl - c) & 0xffff), pt = base_tie + ((incl - c) >> 16);
+#pragma unroll
+          for (int r = 4 * g; r < 4 * g + 4; ++r) {
+            store(kreg[r], pa, pt, [&]() { return LAZY ? f_of(r) : ireg[LAZY ? 0 : r]; });
+            pa += is_above(kreg[r]) ? 1 : 0;
+            pt += is_tie(kreg[r]) ? 1 : 0;
+          }
+          base_above += last & 0xffff;
+          base_tie += last >> 16;
+        }
+      for (int r = MG_REGK; r < rounds; ++r) {  // candidates beyond the register-resident ones, one round at a time
+        const int f = r * MG_THREADS + tid;
+        const uint32_t key = key_of(r);
+        const unsigned long long ma = __builtin_amdgcn_ballot_w64(is_above(key)), mt = __builtin_amdgcn_ballot_w64(is_tie(key));
+        lds_barrier();
+        if (lane == 0) {
+          wred_i[wave] = __popcll(ma);
+          wred_j[wave] = __popcll(mt);
+        }
+        lds_barrier();
+        int ba, bt_, ra, rt;
+        waves_prefix_i<MG_WAVES>(wred_i, lane, wave, &ba, &ra);
+        waves_prefix_i<MG_WAVES>(wred_j, lane, wave, &bt_, &rt);
+        const int pa = all_above + ba + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(ma >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ma, 0u));
+        const int pt = all_tie + bt_ + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mt >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mt, 0u));
+        store(key, pa, pt, [&]() { return LAZY ? f : ci[f]; });
+        all_above += ra;
+        all_tie += rt;
+      }
+      n_out = min(K, all_above + min(all_tie, quota));
+      if (PARTIAL && !take_all) edge = key_to_score(tau);
+    }
+  } else {
+    // the winners are given (ascending positions, -1 padded, possibly none at all): their keys come from the
+    // caller's score tensor
+    n_out = p.topk_idx ? K : 0;
+    for (int r = tid; r < n_out; r += MG_THREADS) {
+      const int64_t pos = p.topk_idx[bh * (size_t)K + r];
+      const bool ok = pos >= 0 && pos < S;
+      win_idx[r] = ok ? (int)pos : -1;
+      win_key[r] = ok ? score_key(p.scores_in[bh * (size_t)p.max_S + pos]) : 0u;
+    }
+  }
+  if (mclk && tid == 0) mclk[2] = JF_CLK();
+  lds_barrier();
+  if (mclk && tid == 0) mclk[3] = JF_CLK();
+  if (PARTIAL) {  // the winners become one candidate list of the final merge
+    const size_t at = (bh * p.mg_parts + part) * (size_t)K;
+    for (int r = tid; r < K; r += MG_THREADS) {
+      p.out_key[at + r] = (r < n_out) ? win_key[r] : 0u;  // unused slots: key 0
+      if (r < n_out) p.out_idx[at + r] = LAZY ? ci[win_idx[r]] : win_idx[r];
+    }
+    if (tid == 0) p.out_edge[bh * p.mg_parts + part] = edge;
+    return;
+  }
+
+  float inv_z = (lsum > 0.f) ? 1.0f / lsum : 0.f;
+  if (!PARTIAL && tid == 0 && p.softmax_m) {
+    p.softmax_m[bh] = M;
+    p.softmax_inv_z[bh] = inv_z;
   }
   if constexpr (MODE == FS_STAGE_B) {
     if (p.stats_m) {  // (uniform) the caller's statistics
@@ -2702,248 +3089,15 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
       inv_z = p.stats_iz[bh];
     }
   }
-  // thread t owns buckets BPT*t .. BPT*t + BPT-1 (bucket 0 = largest scores): which bucket holds the K-th largest
-  constexpr int BPT = MG_BINS / MG_THREADS;
-  int cb[BPT], mine = 0;
-#pragma unroll
-  for (int u = 0; u < BPT; ++u) {
-    cb[u] = hist[BPT * tid + u];
-    mine += cb[u];
-  }
-  const int incl = wave_incl_scan_i(mine);
-  if (lane == 63) wred_j[wave] = incl;
-  if constexpr (!PARTIAL && MODE != FS_STAGE_A) {
-    // o_hat: group vg of the eight takes every eighth split, then a fixed-order sum
-    const int d = tid & (D - 1), q4 = tid >> 7;
-    for (int vg = q4; vg < VGRP; vg += PO_GRP) {
-      float o = 0.f;
-#pragma unroll
-      for (int i = 0; i < PO_PRE; ++i) {
-        const int sp = vg + VGRP * i;
-        if (sp < NS) o = __builtin_fmaf((vg == q4) ? po[i] : p.part_o[(bh * NS + sp) * D + d], coef_sh[sp], o);
-      }
-      // the remaining splits eight at a time: the loads of a batch are in flight together, the sum keeps its order
-      constexpr int PO_B = 8;
-      for (int sp0 = vg + VGRP * PO_PRE; sp0 < NS; sp0 += VGRP * PO_B) {
-        float v[PO_B];
-#pragma unroll
-        for (int u = 0; u < PO_B; ++u) {
-          const int sp = sp0 + VGRP * u;
-          v[u] = (sp < NS) ? p.part_o[(bh * NS + sp) * D + d] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < PO_B; ++u) {
-          const int sp = sp0 + VGRP * u;
-          if (sp < NS) o = __builtin_fmaf(v[u], coef_sh[sp], o);
-        }
-      }
-      red_sh[vg][d] = o;
-    }
-  }
-  lds_barrier();
-  // ---- interval 4: o_hat; the bucket of the K-th largest candidate
-  if constexpr (!PARTIAL && MODE != FS_STAGE_A) {
-    if (tid < D) {
-      float o2 = red_sh[0][tid];
-#pragma unroll
-      for (int q = 1; q < VGRP; ++q) o2 += red_sh[q][tid];  // fixed order
-      blend_hat = !has_parts ? o2 : o2 * inv_z;
-      p.o_hat[bh * D + tid] = blend_hat;
-    }
-  }
-  if (mclk && tid == 0) mclk[1] = JF_CLK();
-
-  uint32_t tau = 0;
-  int quota = 0;
-  if (!take_all) {
-    {
-      int run, all_waves;
-      waves_prefix_i<MG_WAVES>(wred_j, lane, wave, &run, &all_waves);
-      run += incl - mine;
-#pragma unroll
-      for (int u = 0; u < BPT; ++u) {
-        if (run < K && K <= run + cb[u]) { cut_sh = BPT * tid + u; above_sh = run; }
-        run += cb[u];
-      }
-    }
-    lds_barrier();
-    const int cut = cut_sh, need = K - above_sh;  // `need` of the cut bucket's members belong to the top K
-#pragma unroll
-    for (int r = 0; r < MG_REGK; ++r)
-      if (r < rreg && kreg[r] != 0u && bin_of(kreg[r]) == cut) {
-        const int i = atomicAdd(&lcount_sh, 1);
-        if (i < MG_LIST) lkey[i] = kreg[r];
-      }
-    for (int r = MG_REGK; r < rounds; ++r) {
-      const uint32_t k = key_of(r);
-      if (k != 0u && bin_of(k) == cut) {
-        const int i = atomicAdd(&lcount_sh, 1);
-        if (i < MG_LIST) lkey[i] = k;
-      }
-    }
-    lds_barrier();
-    const int m = __builtin_amdgcn_readfirstlane(lcount_sh);
-    if (m <= MG_RANK) {
-      // (the usual case: one member per lane, the others as scalars, in every wavefront: no LDS latency per member and
-      // no barrier to hand the result around)
-      const uint32_t own = (lane < m) ? lkey[lane] : 0u;
-      int gt = 0, ge = 0;
-      for (int j = 0; j < m; ++j) {
-        const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)own, j);
-        gt += (o > own) ? 1 : 0;
-        ge += (o >= own) ? 1 : 0;
-      }
-      const unsigned long long who = __builtin_amdgcn_ballot_w64(lane < m && gt < need && need <= ge);
-      const int src = (who != 0ull) ? __ffsll((long long)who) - 1 : 0;
-      tau = (uint32_t)__builtin_amdgcn_readlane((int)own, src);
-      quota = need - __builtin_amdgcn_readlane(gt, src);
-    } else if (m <= MG_LIST) {
-      // rank counting: the member with fewer than `need` larger members and at least `need` members >= it
-      for (int i = tid; i < m; i += MG_THREADS) {
-        const uint32_t k = lkey[i];
-        int gt = 0, ge = 0;
-        for (int j = 0; j < m; ++j) {
-          const uint32_t o = lkey[j];
-          gt += (o > k) ? 1 : 0;
-          ge += (o >= k) ? 1 : 0;
-        }
-        if (gt < need && need <= ge) {  // every thread that gets here writes the same pair
-          tau_sh = k;
-          quota_sh = need - gt;
-        }
-      }
-      lds_barrier();
-      tau = tau_sh;
-      quota = quota_sh;
-    } else {
-      // bisection over the key range: largest x with count(key >= x) >= K
-      uint32_t lo_k = kmin, hi_k = kmax;  // invariant: count_ge(lo_k) >= K
-      while (lo_k < hi_k) {
-        const uint32_t mid = lo_k + (hi_k - lo_k + 1u) / 2u;
-        if (count_ge(mid) >= K) lo_k = mid;
-        else hi_k = mid - 1u;
-      }
-      tau = lo_k;
-      quota = K - ((tau == 0xffffffffu) ? 0 : count_ge(tau + 1u));
-    }
-  }
-  if (mclk && tid == 0) mclk[2] = JF_CLK();
-
-  // ---- ordered compaction.  Register candidates: every thread counts its winners and ties per group, a
-  // wavefront scan plus the wavefront totals in LDS give the thread's first place, and the thread places its
-  // (consecutive) candidates one after the other.  The owner of a winner stores its key and position.
-  int base_above = 0, base_tie = 0;
-  {
-    int cnt_g[NGRP];  // low half: winners, high half: ties of this thread in group g
-    int scan_g[NGRP];
-#pragma unroll
-    for (int g = 0; g < NGRP; ++g) {
-      int c = 0;
-      if (4 * g < rreg) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t key = kreg[4 * g + j];
-          const bool above = (key != 0u) && (take_all || key > tau), tie = (key != 0u) && !take_all && key == tau;
-          c += (above ? 1 : 0) + (tie ? 0x10000 : 0);
-        }
-      }
-      cnt_g[g] = c;
-      scan_g[g] = wave_incl_scan_i(c);  // at most 4 * 64 per half: no carry between the halves
-      if (lane == 63) cnt_a[g * MG_WAVES + wave] = (uint32_t)scan_g[g];
-    }
-    lds_barrier();
-    uint32_t run = 0u;  // packed totals of the groups before g (each half stays below 2^16: at most 32768 candidates)
-#pragma unroll
-    for (int g = 0; g < NGRP; ++g) {
-      int before_i, all_i;  // (packed pairs: each half stays below 2^16, so the halves never carry into each other)
-      waves_prefix_i<MG_WAVES>(reinterpret_cast<const int*>(cnt_a) + g * MG_WAVES, lane, wave, &before_i, &all_i);
-      const uint32_t before = (uint32_t)before_i, all = (uint32_t)all_i;
-      if (4 * g < rreg) {
-        const uint32_t start = run + before + (uint32_t)(scan_g[g] - cnt_g[g]);
-        int pa = (int)(start & 0xffffu), pt = (int)(start >> 16);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t key = kreg[4 * g + j];
-          const bool above = (key != 0u) && (take_all || key > tau), tie = (key != 0u) && !take_all && key == tau;
-          if (above || (tie && pt < quota)) {
-            const int pos = pa + min(pt, quota);
-            if (pos < K) {
-              win_key[pos] = key;
-              win_idx[pos] = ireg[4 * g + j];
-            }
-          }
-          pa += above ? 1 : 0;
-          pt += tie ? 1 : 0;
-        }
-      }
-      run += all;
-    }
-    base_above = (int)(run & 0xffffu);
-    base_tie = (int)(run >> 16);
-    lds_barrier();
-  }
-  for (int r = MG_REGK; r < rounds; ++r) {  // candidates beyond the register-resident ones, one round at a time
-    const int f = r * MG_THREADS + tid;
-    const uint32_t key = key_of(r);
-    const bool above = (key != 0u) && (take_all || key > tau), tie = (key != 0u) && !take_all && key == tau;
-    const unsigned long long ma = __builtin_amdgcn_ballot_w64(above), mt = __builtin_amdgcn_ballot_w64(tie);
-    if (lane == 0) {
-      wred_i[wave] = __popcll(ma);
-      wred_j[wave] = __popcll(mt);
-    }
-    lds_barrier();
-    int pa = base_above + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(ma >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ma, 0u));
-    int pt = base_tie + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mt >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mt, 0u));
-    int tot_a = 0, tot_t = 0;
-#pragma unroll
-    for (int w = 0; w < MG_WAVES; ++w) {
-      if (w < wave) { pa += wred_i[w]; pt += wred_j[w]; }
-      tot_a += wred_i[w];
-      tot_t += wred_j[w];
-    }
-    if (above || (tie && pt < quota)) {
-      const int pos = pa + min(pt, quota);
-      if (pos < K) {
-        win_key[pos] = key;
-        win_idx[pos] = ci[f];
-      }
-    }
-    base_above += tot_a;
-    base_tie += tot_t;
-    lds_barrier();
-  }
-  int n_out = min(K, base_above + min(base_tie, quota));
-  if constexpr (MODE == FS_STAGE_B) {
-    // the winners are given (ascending positions, -1 padded, possibly none at all): their keys come from the
-    // caller's score tensor
-    n_out = p.topk_idx ? K : 0;
-    const int64_t s_len = max(0, min(p.max_S, p.seq_lens[b]));
-    for (int r = tid; r < n_out; r += MG_THREADS) {
-      const int64_t pos = p.topk_idx[bh * (size_t)K + r];
-      const bool ok = pos >= 0 && pos < s_len;
-      win_idx[r] = ok ? (int)pos : -1;
-      win_key[r] = ok ? score_key(p.scores_in[bh * (size_t)p.max_S + pos]) : 0u;
-    }
-    lds_barrier();
-  }
-  if (mclk && tid == 0) mclk[3] = JF_CLK();
-  if (PARTIAL) {  // the winners become one candidate list of the final merge
-    const size_t lo = (bh * p.mg_parts + part) * (size_t)K;
-    for (int r = tid; r < K; r += MG_THREADS) {
-      p.key2[lo + r] = (r < n_out) ? win_key[r] : 0u;  // unused slots: key 0
-      if (r < n_out) p.idx2[lo + r] = win_idx[r];
-    }
-    if (tid == 0) p.cnt2[bh * p.mg_parts + part] = n_out;
-    return;
-  }
-
   // one thread per winner: position, paged slot, softmax weight
+  int64_t* out_idx = p.topk_idx + bh * (size_t)K;
+  int64_t* out_slot = p.topk_slots + bh * (size_t)K;
   for (int r = tid; r < K; r += MG_THREADS) {
     int64_t position = -1, slot = -1;
     int wslot = -1;
     float ww = 0.f;
     if (r < n_out && win_idx[r] >= 0) {
-      position = win_idx[r];
+      position = (LAZY && HAS_LISTS) ? ci[win_idx[r]] : win_idx[r];
       const int blk = (int)(position / BS);
       if (blk < p.max_blocks) slot = (int64_t)((blk < nblk_lds) ? (int64_t)bt_sh[blk] : bt[blk]) * BS + (position % BS);
       wslot = (slot >= 0 && slot < p.num_slots) ? (int)slot : -1;
@@ -2957,6 +3111,22 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
     win_key[r] = __builtin_bit_cast(uint32_t, ww);
   }
   if constexpr (MODE == FS_STAGE_A) return;  // Stage A alone ends with the winners and the statistics
+  if constexpr (!PARTIAL && MODE != FS_STAGE_A) {  // o_hat, by the last two wavefronts while the first ones look after the winners
+    const int d = tid - (MG_THREADS - D);
+    if (d >= 0) {
+      float o8[VGRP];
+#pragma unroll
+      for (int q = 0; q < VGRP; ++q) o8[q] = red_sh[q][d];
+#pragma unroll
+      for (int n = VGRP / 2; n >= 1; n /= 2) {  // fixed order
+#pragma unroll
+        for (int q = 0; q < n; ++q) o8[q] += o8[q + n];
+      }
+      const float o2 = has_parts ? o8[0] * inv_z : o8[0];
+      p.o_hat[bh * D + d] = o2;
+      ohat_sh[d] = o2;
+    }
+  }
   lds_barrier();
   if (mclk && tid == 0) mclk[4] = JF_CLK();
 
@@ -2984,14 +3154,15 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
 #pragma unroll
       for (int c = 0; c < CPD; ++c) acc[r][c] = 0.f;
     }
-    for (int kb = (wave + r0 * MG_WAVES) * WPI; kb < n_out; kb += UNR * VWAVES * WPI) {
-      uint32_t word[RP][UNR], word_b[RP][UNR];  // (word_b: INT3 only)
-      uint16_t sbits[RP][UNR];
-      float wv[RP][UNR];
+    auto gather = [&](int kb, auto count) {  // `count` rows per lane and role from winner kb on
+      constexpr int NU = decltype(count)::value;
+      uint32_t word[RP][NU], word_b[RP][NU];  // (word_b: INT3 only)
+      uint16_t sbits[RP][NU];
+      float wv[RP][NU];
 #pragma unroll
       for (int r = 0; r < RP; ++r)
 #pragma unroll
-        for (int u = 0; u < UNR; ++u) {
+        for (int u = 0; u < NU; ++u) {
           const int k = kb + (r * MG_WAVES + u * VWAVES) * WPI + w_in;
           const int slot = (k < n_out) ? win_idx[k] : -1;
           wv[r][u] = (slot >= 0) ? __builtin_bit_cast(float, win_key[k]) : 0.f;
@@ -3002,11 +3173,16 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
 #pragma unroll
       for (int r = 0; r < RP; ++r)
 #pragma unroll
-        for (int u = 0; u < UNR; ++u) {
+        for (int u = 0; u < NU; ++u) {
           const float ws = wv[r][u] * bf16_to_f32(sbits[r][u]);  // zero for padding rows
           Pre::add(word[r][u], word_b[r][u], ws, acc[r]);
           if (dwi == 0) accw[r] += wv[r][u];
         }
+    };
+    for (int kb = (wave + r0 * MG_WAVES) * WPI; kb < n_out; kb += UNR * VWAVES * WPI) {
+      // (narrow corrections: no rows are fetched for winners there are none of)
+      if (UNR > 1 && n_out - (kb - (wave + r0 * MG_WAVES) * WPI) <= VWAVES * WPI) gather(kb, std::integral_constant<int, 1>{});
+      else gather(kb, std::integral_constant<int, UNR>{});
     }
 #pragma unroll
     for (int r = 0; r < RP; ++r) {  // over the WPI winners of a wavefront instruction; then over the roles through LDS
@@ -3020,16 +3196,25 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(FusedParams p) 
   }
   lds_barrier();
   if (tid < D) {
-    float o = 0.f;
+    float o16[VWAVES], w16[VWAVES];
 #pragma unroll
-    for (int w = 0; w < VWAVES; ++w) o += old_sh[w][tid];  // fixed order
+    for (int w = 0; w < VWAVES; ++w) {
+      o16[w] = old_sh[w][tid];
+      w16[w] = w_sh[w];
+    }
+#pragma unroll
+    for (int n = VWAVES / 2; n >= 1; n /= 2) {  // fixed order
+#pragma unroll
+      for (int w = 0; w < n; ++w) {
+        o16[w] += o16[w + n];
+        w16[w] += w16[w + n];
+      }
+    }
+    const float o = o16[0], wt = w16[0];  // (the same wt in every thread)
     p.o_old[bh * D + tid] = o;
-    float wt = 0.f;
-#pragma unroll
-    for (int w = 0; w < VWAVES; ++w) wt += w_sh[w];  // fixed order: the same value in every thread
     if (tid == 0) p.W[bh] = wt;
     // the blend of jetfire_vllm/csrc/blend.cu:202-226 for callers that hold o_new already
-    if (MODE == FS_FULL && p.blend_out) p.blend_out[bh * D + tid] = f32_to_bf16(__builtin_fmaf(wt, blend_new, blend_hat) - o);
+    if (MODE == FS_FULL && p.blend_out) p.blend_out[bh * D + tid] = f32_to_bf16(__builtin_fmaf(wt, bf16_to_f32(blend_raw), ohat_sh[tid]) - o);
   }
   if (mclk && tid == 0) mclk[5] = JF_CLK();
 }
@@ -3253,7 +3438,7 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
 }
 
 struct WsLayout {
-  size_t off_m, off_l, off_o, off_key, off_idx, off_cnt, off_key2, off_idx2, off_cnt2, total;
+  size_t off_m, off_l, off_o, off_key, off_idx, off_edge, off_key2, off_idx2, off_edge2, total;
 };
 inline WsLayout ws_layout(int B, int H_q, int ns, int kc, int parts, int top_k) {
   WsLayout w;
@@ -3265,12 +3450,12 @@ inline WsLayout ws_layout(int B, int H_q, int ns, int kc, int parts, int top_k) 
   w.off_o = take(rows * ns * D * 4);
   w.off_key = take(rows * ns * kc * 4);
   w.off_idx = take(rows * ns * kc * 4);
-  w.off_cnt = take(rows * ns * 4);
-  w.off_key2 = w.off_idx2 = w.off_cnt2 = 0;
+  w.off_edge = take(rows * ns * 4);
+  w.off_key2 = w.off_idx2 = w.off_edge2 = 0;
   if (parts > 1) {
     w.off_key2 = take(rows * parts * top_k * 4);
     w.off_idx2 = take(rows * parts * top_k * 4);
-    w.off_cnt2 = take(rows * parts * 4);
+    w.off_edge2 = take(rows * parts * 4);
   }
   w.total = o + 256;
   return w;
@@ -3344,8 +3529,8 @@ inline int scheme_ng(int scheme, int group_size) { return scheme_any_group(schem
 
 // A merge kernel whose winners live in dynamic LDS (corrections wider than FS_LDS_TOPK): 8 bytes per winner; the
 // dynamic-LDS limit of the instantiation is raised once.
-template <void (*KERN)(FusedParams)>
-int launch_wide_merge(dim3 grid, const FusedParams& p, hipStream_t st) {
+template <void (*KERN)(MergeParams)>
+int launch_wide_merge(dim3 grid, const MergeParams& p, hipStream_t st) {
   static std::mutex mu;
   static bool raised = false;
   {
@@ -3445,10 +3630,10 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   p.part_o = reinterpret_cast<float*>(ws + wl.off_o);
   p.cand_key = reinterpret_cast<uint32_t*>(ws + wl.off_key);
   p.cand_idx = reinterpret_cast<int32_t*>(ws + wl.off_idx);
-  p.cand_cnt = reinterpret_cast<int32_t*>(ws + wl.off_cnt);
+  p.cand_edge = reinterpret_cast<float*>(ws + wl.off_edge);
   p.key2 = reinterpret_cast<uint32_t*>(ws + wl.off_key2);
   p.idx2 = reinterpret_cast<int32_t*>(ws + wl.off_idx2);
-  p.cnt2 = reinterpret_cast<int32_t*>(ws + wl.off_cnt2);
+  p.edge2 = reinterpret_cast<float*>(ws + wl.off_edge2);
   p.topk_idx = topk_idx; p.topk_slots = topk_slots; p.o_hat = o_hat; p.o_old = o_old_unnorm; p.W = W;
   p.softmax_m = softmax_m; p.softmax_inv_z = softmax_inv_z;
   p.blend_o_new = blend_o_new; p.blend_out = blend_out;
@@ -3494,16 +3679,18 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
 #undef JF_FUSED_BY_G
 #undef JF_FUSED_CASE
   if (rc != JF_OK || scores_only || p.one_split) return rc;
-  dim3 mgrid(B, H_q);
+  const dim3 mgrid(g_act, H_kv, B);
   const bool wide = top_k > FS_LDS_TOPK;  // the winners' arrays do not fit the kernels' static LDS
   if (p.mg_parts > 1) {  // first stage: every part's top_k, as new candidate lists (the same kernel for every form)
     const dim3 pgrid(B, H_q, p.mg_parts);
-    if (wide) rc = launch_wide_merge<fused_merge_kernel<FS_FULL, 4, 1, 1024, 32, true, true>>(pgrid, p, st);
-    else if ((long long)p.mg_spp * p.Kc > MG_REG_CANDS) hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, 4, 1, 1024, 32, true>), pgrid, dim3(1024), 0, st, p);
-    else hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, 4, 1, 1024, 8, true>), pgrid, dim3(1024), 0, st, p);
+    const MergeParams mp = merge_params(p, true);
+    if (wide) rc = launch_wide_merge<fused_merge_kernel<FS_FULL, 4, 1, 1024, 32, true, true>>(pgrid, mp, st);
+    else if ((long long)p.mg_spp * p.Kc > MG_REG_CANDS) hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, 4, 1, 1024, 32, true>), pgrid, dim3(1024), 0, st, mp);
+    else hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, 4, 1, 1024, 8, true>), pgrid, dim3(1024), 0, st, mp);
     if (rc != JF_OK) return rc;
     JF_CHECK_LAUNCH();
   }
+  const MergeParams mp = merge_params(p, false);
   const bool big = (MODE != FS_STAGE_B) &&
                    (p.mg_parts > 1 ? (long long)p.mg_parts * top_k : (long long)p.n_splits * p.Kc) > MG_REG_CANDS;
   // Many rows with few candidates each (large batches of short or medium sequences): four wavefronts per row and
@@ -3518,20 +3705,20 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
 #define JF_MERGE(VB, NGG)                                                                                            \
   do {                                                                                                               \
     if (wide) {                                                                                                      \
-      if constexpr (MODE == FS_STAGE_B) rc = launch_wide_merge<fused_merge_kernel<MODE, VB, NGG, 1024, 8, false, true>>(mgrid, p, st); \
-      else rc = launch_wide_merge<fused_merge_kernel<MODE, VB, NGG, 1024, 32, false, true>>(mgrid, p, st);            \
-    } else if (big) hipLaunchKernelGGL((fused_merge_kernel<MODE, VB, NGG, 1024, 32, false>), mgrid, dim3(1024), 0, st, p); \
+      if constexpr (MODE == FS_STAGE_B) rc = launch_wide_merge<fused_merge_kernel<MODE, VB, NGG, 1024, 8, false, true>>(mgrid, mp, st); \
+      else rc = launch_wide_merge<fused_merge_kernel<MODE, VB, NGG, 1024, 32, false, true>>(mgrid, mp, st);            \
+    } else if (big) hipLaunchKernelGGL((fused_merge_kernel<MODE, VB, NGG, 1024, 32, false>), mgrid, dim3(1024), 0, st, mp); \
     else if (light) {                                                                                                \
       if constexpr (MODE == FS_FULL) {                                                                               \
-        if (gather) hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false, false, 4>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, p); \
-        else hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, p); \
+        if (gather) hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false, false, 4>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, mp); \
+        else hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, mp); \
       }                                                                                                              \
-    } else hipLaunchKernelGGL((fused_merge_kernel<MODE, VB, NGG, 1024, 8, false>), mgrid, dim3(1024), 0, st, p);       \
+    } else hipLaunchKernelGGL((fused_merge_kernel<MODE, VB, NGG, 1024, 8, false>), mgrid, dim3(1024), 0, st, mp);       \
   } while (0)
   if constexpr (MODE == FS_STAGE_A || MODE == FS_TOPK) {  // no value rows are read: one instantiation serves every format
-    if (wide) rc = launch_wide_merge<fused_merge_kernel<FS_STAGE_A, 4, 1, 1024, 32, false, true>>(mgrid, p, st);
-    else if (big) hipLaunchKernelGGL((fused_merge_kernel<FS_STAGE_A, 4, 1, 1024, 32, false>), mgrid, dim3(1024), 0, st, p);
-    else hipLaunchKernelGGL((fused_merge_kernel<FS_STAGE_A, 4, 1, 1024, 8, false>), mgrid, dim3(1024), 0, st, p);
+    if (wide) rc = launch_wide_merge<fused_merge_kernel<FS_STAGE_A, 4, 1, 1024, 32, false, true>>(mgrid, mp, st);
+    else if (big) hipLaunchKernelGGL((fused_merge_kernel<FS_STAGE_A, 4, 1, 1024, 32, false>), mgrid, dim3(1024), 0, st, mp);
+    else hipLaunchKernelGGL((fused_merge_kernel<FS_STAGE_A, 4, 1, 1024, 8, false>), mgrid, dim3(1024), 0, st, mp);
   } else if (scheme % 10 == 2) {  // INT2 values
     if (NGv == 2) JF_MERGE(2, 2);
     else JF_MERGE(2, 1);
@@ -3558,13 +3745,13 @@ static int launch_precorr_given_stats(const float* scores, const float* softmax_
                                       int n_partial, float* o_hat, float* o_old_unnorm, float* W, hipStream_t st) {
   FusedParams p = {};
   p.v_data = v_data; p.v_scales = v_scales; p.block_table = block_table; p.seq_lens = seq_lens;
-  p.B = B; p.H_q = H_q; p.H_kv = H_kv; p.max_S = max_S; p.max_blocks = max_blocks; p.num_slots = num_slots;
+  p.B = B; p.H_q = H_q; p.H_kv = H_kv; p.g_act = H_q / H_kv; p.max_S = max_S; p.max_blocks = max_blocks; p.num_slots = num_slots;
   p.top_k = top_k;
-  p.n_splits = n_partial; p.part_o = const_cast<float*>(partial); p.o_hat = o_hat; p.mg_parts = 1; p.mg_spp = 0; p.Kc = 0;
+  p.n_splits = n_partial; p.part_o = const_cast<float*>(partial); p.o_hat = o_hat; p.mg_parts = 1; p.mg_spp = 0; p.Kc = p.L = 0;
   p.scores_in = scores; p.stats_m = softmax_m; p.stats_iz = softmax_inv_z;
   p.topk_idx = const_cast<int64_t*>(topk_idx);
   p.o_old = o_old_unnorm; p.W = W;
-  hipLaunchKernelGGL((fused_merge_kernel<FS_STAGE_B, VBITS, NG, 1024, 8, false>), dim3(B, H_q), dim3(1024), 0, st, p);
+  hipLaunchKernelGGL((fused_merge_kernel<FS_STAGE_B, VBITS, NG, 1024, 8, false>), dim3(p.g_act, H_kv, B), dim3(1024), 0, st, merge_params(p, false));
   JF_CHECK_LAUNCH();
   return JF_OK;
 }
