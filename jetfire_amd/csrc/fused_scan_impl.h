@@ -637,28 +637,31 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   const uint8_t* ksb = reinterpret_cast<const uint8_t*>(p.k_scales + (size_t)hkv * p.num_slots * (KLIMB ? NG : 1));
   const uint8_t* kzb = KA ? reinterpret_cast<const uint8_t*>(p.k_zp + (size_t)hkv * p.num_slots * NG) : nullptr;
   constexpr bool SPREP = HAS_K && Lds::SPREP;
+  // one scale word per lane (lane = token of the chunk), handed to the lanes that work on the token through the table
+  // (SPREP) or a lane permutation; the asymmetric keys load scales and zero-points per page
+  constexpr bool SL = HAS_K && !KA;
   struct KBuf {
     v4u r[KLD];
-    uint32_t s[SPREP ? 1 : 4];   // scale words: of the lane's token (SPREP), or of token t16 of each of the four pages
+    uint32_t s[SL ? 1 : 4];   // scale words: of the lane's token (SL), or of token t16 of each of the four pages
     uint32_t z[KA ? 4 : 1];  // zero-points of the asymmetric keys, packed like the scales
   };
   const int t16 = lane & 15, lg = lane >> 4;
+  constexpr int KNG = KLIMB ? NG : 1;  // key scales per row
   auto issue_k = [&](int chunk) -> KBuf {
     KBuf kbuf;
-    constexpr int KNG = KLIMB ? NG : 1;  // key scales per row
     // (the scales first: they are copied out of the buffer one chunk earlier than the rows are, and loads return in order)
-    if constexpr (SPREP) {
+    if constexpr (SL) {
       const int tl = chunk * 64 + lane;
       const uint32_t slot = (uint32_t)(sbase[tl >> 4] + (tl & 15));
       if (KNG == 2) kbuf.s[0] = *reinterpret_cast<const uint32_t*>(ksb + (size_t)(slot * 4u));
       else kbuf.s[0] = (uint32_t) * reinterpret_cast<const uint16_t*>(ksb + (size_t)(slot * 2u));
     }
 #pragma unroll
-    for (int j = 0; j < (SPREP ? 0 : 4); ++j) {
+    for (int j = 0; j < (SL ? 0 : 4); ++j) {
       const int sb = __builtin_amdgcn_readfirstlane(sbase[chunk * 4 + j]);  // first slot of the page (uniform)
       const uint8_t* srow = ksb + (size_t)sb * (KNG * 2) + t16 * (KNG * 2);
-      if (KNG == 2) kbuf.s[SPREP ? 0 : j] = *reinterpret_cast<const uint32_t*>(srow);
-      else kbuf.s[SPREP ? 0 : j] = *reinterpret_cast<const uint16_t*>(srow);
+      if (KNG == 2) kbuf.s[SL ? 0 : j] = *reinterpret_cast<const uint32_t*>(srow);
+      else kbuf.s[SL ? 0 : j] = *reinterpret_cast<const uint16_t*>(srow);
       if constexpr (KA) {
         const uint8_t* zrow = kzb + (size_t)sb * (KNG * 2) + t16 * (KNG * 2);
         if (KNG == 2) kbuf.z[j] = *reinterpret_cast<const uint32_t*>(zrow);
@@ -673,6 +676,11 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       kbuf.r[i] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(kbase + (size_t)(sb * (uint32_t)KP + kl_off[i])));
     }
     return kbuf;
+  };
+  // the scale word of token t16 of page j
+  auto scale_word = [&](const uint32_t (&Sx)[4], int j) -> uint32_t {
+    if constexpr (SL) return (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (16 * j + t16), (int)Sx[0]);
+    else return Sx[j];
   };
   auto stash_k = [&](const KBuf& kbuf) {
 #pragma unroll
@@ -884,7 +892,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // positions produced.  A chunk past the end (n_local <= 0) is not worked through at all.
   auto clone_last_row = [&](int n_local, uint32_t (&Sx)[4], uint32_t (&Zx)[4]) {
     const int last = n_local - 1, jl = last >> 4;
-    if constexpr (SPREP) {  // one scale word per lane (= token): Sx[0]
+    if constexpr (SL) {  // one scale word per lane (= token): Sx[0]
       const uint32_t sl = (uint32_t)__builtin_amdgcn_readlane((int)Sx[0], last);
       Sx[0] = (lane >= n_local) ? sl : Sx[0];
     } else {
@@ -998,7 +1006,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     auto body = [&](int chunk, const uint32_t (&Sx)[4], const uint32_t (&Zx)[4]) {
       (void)Zx;
       // all LDS reads of the chunk first (plane dwords of the four pages, rounding coefficients), then arithmetic
-      uint32_t Pj[4][KB4 ? 4 : 3];
+      uint32_t Pj[4][3];
       float sgj[4][NG], egj[4][NG];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -1007,10 +1015,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           Pj[j][0] = *reinterpret_cast<const uint32_t*>(rp);
           Pj[j][1] = *reinterpret_cast<const uint32_t*>(rp + 16);
           Pj[j][2] = *reinterpret_cast<const uint32_t*>(rp + 32);
-        } else if constexpr (KB4) {
-          const v4u x = *reinterpret_cast<const v4u*>(rp);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) Pj[j][KB4 ? i : 0] = x[i];
+        } else if constexpr (KB4) {  // (read where they are used: the registers are the tighter resource)
         } else {
           const v2u x = *reinterpret_cast<const v2u*>(rp);
           Pj[j][0] = x[0];
@@ -1030,8 +1035,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
             sgj[j][0] = x[0];
             egj[j][0] = x[1];
           }
-        } else {
-          const uint32_t sw = Sx[j];
+        } else if constexpr (!KB4) {
+          const uint32_t sw = scale_word(Sx, j);
           sgj[j][0] = bf16_to_f32((uint16_t)(sw & 0xffffu));
           egj[j][0] = K3 ? eps_sh[0][sw & 0x7fu] : 0.f;  // (INT4: three coefficients, read where they are used)
           if (NG == 2) {
@@ -1043,10 +1048,19 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const uint32_t P0 = Pj[j][0], P1 = Pj[j][1], P2 = Pj[j][2];
         v4i Bc[2], Br[2];
+        v4u X = {0u, 0u, 0u, 0u};
+        if constexpr (KB4) {
+          // (one page at a time, the scheduler would otherwise hold the operands of all four and spill)
+          __builtin_amdgcn_sched_barrier(0);
+          X = *reinterpret_cast<const v4u*>(krd + j * 16 * KROW);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 3; ++i) X[i] = Pj[j][i];
+        }
+        const uint32_t P0 = X[0], P1 = X[1], P2 = X[2];
         if constexpr (KB4) {  // two codes per byte, the even channel in the high nibble
-          const uint32_t P3 = Pj[j][KB4 ? 3 : 0];
+          const uint32_t P3 = X[3];
           Bc[0] = (v4i){(int)((P0 >> 4) & 0x0f0f0f0fu), (int)(P0 & 0x0f0f0f0fu), (int)((P1 >> 4) & 0x0f0f0f0fu), (int)(P1 & 0x0f0f0f0fu)};
           Bc[1] = (v4i){(int)((P2 >> 4) & 0x0f0f0f0fu), (int)(P2 & 0x0f0f0f0fu), (int)((P3 >> 4) & 0x0f0f0f0fu), (int)(P3 & 0x0f0f0f0fu)};
         } else if constexpr (K3) {
@@ -1077,8 +1091,13 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           // khat = bf16((u - 8) s) for the unsigned nibble u: exact for |u - 8| in {0, 1, 2, 4, 8}; for 3, 5, 7 (and 6 =
           // 2 * 3) the rounding is eps_c(s) * s with the sign of the code, eps_c a function of the scale's mantissa
           // alone.  So next to the code contraction there are three with the signed indicators r3 = [c = +-3] +
-          // 2 [c = +-6], r5 = [c = +-5], r7 = [c = +-7], made by byte look-ups: one table for the codes >= 0 (u >= 8,
-          // selector u - 8 = c) and one for the codes < 0 (selector u = c + 8), chosen per byte by bit 3 of u.
+          // 2 [c = +-6], r5 = [c = +-5], r7 = [c = +-7], each the sum of two byte look-ups: one that is right for the codes
+          // >= 0 (selector u ^ 8 = c) and one for the codes < 0 (selector u = c + 8).  Selectors 8..15 of v_perm_b32 are
+          // not table entries but constants (8..11 the signs of bytes 1, 3, 5, 7, 12 zero, 13..15 minus one); the tables
+          // hold what makes the two sums come out, and the matrix cores, which are idle mostly, do the adding: seven
+          // vector instructions per dword.  (Masking the selectors and choosing between the two results per byte took
+          // fourteen.)  4 x 8100 positions, B4V4 in 64-channel groups, per layer: 29.0 -> 28.0 us, and no scratch any more.
+          const uint32_t sw = scale_word(Sx, j);
           const int tok = chunk * 64 + 16 * j + t16;
           float acc_s[NSET][NG];
 #pragma unroll
@@ -1096,21 +1115,25 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
               (void)zero;
               acc_s[set][g] = (float)join_limbs(Dc[2], Dc[1], Dc[0]);
             }
+          v4i Bw[2];  // u ^ 8
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Bw[u][e] = Bc[u][e] ^ 0x08080808;
 #pragma unroll
           for (int c = 0; c < 3; ++c) {  // c = 0, 1, 2: the indicators of +-3 (and +-6), +-5, +-7
-            const uint32_t pos_hi = (c == 0) ? 0x00020000u : ((c == 1) ? 0x00000100u : 0x01000000u);  // selectors 4..7
-            const uint32_t pos_lo = (c == 0) ? 0x01000000u : 0u;                                       // selectors 0..3
-            const uint32_t neg_hi = (c == 0) ? 0x0000ff00u : 0u;
+            const uint32_t pos_hi = (c == 0) ? 0x01030100u : ((c == 1) ? 0x01010200u : 0x02010100u);
+            const uint32_t pos_lo = (c == 0) ? 0x01000000u : ((c == 1) ? 0x00000100u : 0x00000001u);
+            const uint32_t neg_hi = (c == 0) ? 0x01010000u : ((c == 1) ? 0x01010100u : 0x01010100u);
             const uint32_t neg_lo = (c == 0) ? 0x00fe0000u : ((c == 1) ? 0xff000000u : 0x0000ff00u);
-            v4i Bi[2];
+            __builtin_amdgcn_sched_barrier(0);
+            v4i Bp[2], Bn[2];
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                const uint32_t x = (uint32_t)Bc[u][e], sel = x & 0x07070707u;
-                const uint32_t t = (x >> 3) & 0x01010101u, hm = (t << 8) - t;  // 0xff in the bytes whose code is >= 0
-                const uint32_t rp_ = __builtin_amdgcn_perm(pos_hi, pos_lo, sel), rn_ = __builtin_amdgcn_perm(neg_hi, neg_lo, sel);
-                Bi[u][e] = (int)((rp_ & hm) | (rn_ & ~hm));
+                Bp[u][e] = (int)__builtin_amdgcn_perm(pos_hi, pos_lo, (uint32_t)Bw[u][e]);
+                Bn[u][e] = (int)__builtin_amdgcn_perm(neg_hi, neg_lo, (uint32_t)Bc[u][e]);
               }
 #pragma unroll
             for (int set = 0; set < NSET; ++set)
@@ -1119,12 +1142,15 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
                 const v4i zero = {0, 0, 0, 0};
                 v4i Dr;
                 if (NG == 2) {
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][g], Bi[g], zero, 0, 0, 0);
+                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][g], Bp[g], zero, 0, 0, 0);
+                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][g], Bn[g], Dr, 0, 0, 0);
                 } else {
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bi[0], zero, 0, 0, 0);
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bi[1], Dr, 0, 0, 0);
+                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bp[0], zero, 0, 0, 0);
+                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bp[1], Dr, 0, 0, 0);
+                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bn[0], Dr, 0, 0, 0);
+                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bn[1], Dr, 0, 0, 0);
                 }
-                const float ec = eps_sh[c][((g == 0) ? Sx[j] : (Sx[j] >> 16)) & 0x7fu];
+                const float ec = eps_sh[c][((g == 0) ? sw : (sw >> 16)) & 0x7fu];
                 acc_s[set][g] = __builtin_fmaf(ec, (float)((Dr[2] << 8) + Dr[1]), acc_s[set][g]);
               }
           }
@@ -1132,7 +1158,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           for (int set = 0; set < NSET; ++set) {
             float score = 0.f;
 #pragma unroll
-            for (int g = 0; g < NG; ++g) score = __builtin_fmaf(acc_s[set][g], sgj[j][g] * qsc[set][g], score);
+            for (int g = 0; g < NG; ++g)
+              score = __builtin_fmaf(acc_s[set][g], bf16_to_f32((uint16_t)((g == 0) ? (sw & 0xffffu) : (sw >> 16))) * qsc[set][g], score);
             const int h = set * 4 + lg;
             if ((G % 4 == 0) || h < G) {
               sc[h * L + tok] = score;
@@ -1311,7 +1338,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         uint32_t Sc[4] = {0u, 0u, 0u, 0u}, Zc[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          if (!SPREP || j == 0) Sc[j] = reg_copy(cur.s[SPREP ? 0 : j]);
+          if (!SL || j == 0) Sc[j] = reg_copy(cur.s[SL ? 0 : j]);
           Zc[j] = KA ? reg_copy(cur.z[KA ? j : 0]) : 0u;
         }
         if constexpr (it + 2 < MAXIT) cur = issue_k(min(chunk + 2 * NW, nch_cover - 1));
@@ -1396,7 +1423,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           const uint32_t x0 = Xj[j][mi][0], x1 = Xj[j][mi][1];
           Bm[mi] = (v4i){(int)((x0 >> 4) & 0x0f0f0f0fu), (int)(x0 & 0x0f0f0f0fu), (int)((x1 >> 4) & 0x0f0f0f0fu), (int)(x1 & 0x0f0f0f0fu)};
         }
-        const float ks = bf16_to_f32((uint16_t)Sx[j]);
+        const float ks = bf16_to_f32((uint16_t)scale_word(Sx, j));
         const int tok = chunk * 64 + 16 * j + t16;
 #pragma unroll
         for (int set = 0; set < NSET; ++set) {
@@ -1426,9 +1453,9 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         KBuf& cur = (it & 1) ? Kb : Ka;
         stash_k(cur);
         wave_lds_fence();
-        uint32_t Sc[4], Zc[4] = {0u, 0u, 0u, 0u};
+        uint32_t Sc[4] = {0u, 0u, 0u, 0u}, Zc[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) Sc[j] = reg_copy(cur.s[j]);
+        for (int j = 0; j < (SL ? 1 : 4); ++j) Sc[j] = reg_copy(cur.s[SL ? 0 : j]);
         if constexpr (it + 2 < MAXIT) cur = issue_k(min(chunk + 2 * NW, nch_cover - 1));
         const int n_local = n - chunk * 64;  // (uniform)
         if (n_local > 0) {
