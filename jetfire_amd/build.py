@@ -24,6 +24,11 @@ SOURCES = (     # (the long compilations first: the pool starts them together)
     "fused_full_c.hip",
     "fused_full_d.hip",
     "fused_full_e.hip",
+    "fused_short_a.hip",
+    "fused_short_b.hip",
+    "fused_short_c.hip",
+    "fused_short_d.hip",
+    "fused_short_e.hip",
     "quant_write.hip",
     "unpack.hip",
     "shadow_write.hip",

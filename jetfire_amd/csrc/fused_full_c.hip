@@ -1,8 +1,8 @@
 // One-pass scan kernels of the fused decode step, INT3 / INT4 keys with INT3 values
-// (see launch_full_scan_* in fused_scan_impl.h).
+// (see JF_SCAN_FAMILY in fused_scan_impl.h).
 #include "fused_scan_impl.h"
 
-int jf::launch_full_scan_c(int scheme, int G, int NG, const void* params, void* stream) {
+int jf::JF_SCAN_ENTRY(c)(int scheme, int G, int NG, const void* params, void* stream) {
   if (scheme == JF_SCHEME_K3V3)
     return NG == 2 ? launch_full_by_group<JF_SCHEME_K3V3, 2>(G, params, stream)
                    : launch_full_by_group<JF_SCHEME_K3V3, 1>(G, params, stream);

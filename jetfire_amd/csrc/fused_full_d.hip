@@ -1,8 +1,8 @@
 // One-pass scan kernels of the fused decode step, asymmetric INT2 keys
-// (see launch_full_scan_* in fused_scan_impl.h).
+// (see JF_SCAN_FAMILY in fused_scan_impl.h).
 #include "fused_scan_impl.h"
 
-int jf::launch_full_scan_d(int scheme, int G, int NG, const void* params, void* stream) {
+int jf::JF_SCAN_ENTRY(d)(int scheme, int G, int NG, const void* params, void* stream) {
   if (scheme == JF_SCHEME_A2V2)
     return NG == 2 ? launch_full_by_group<JF_SCHEME_A2V2, 2>(G, params, stream)
                    : launch_full_by_group<JF_SCHEME_A2V2, 1>(G, params, stream);

@@ -78,12 +78,24 @@ constexpr bool kDebugHooks = true;
 constexpr bool kDebugHooks = false;
 #endif
 // The one-pass scan kernels are instantiated in five translation units (fused_full_*.hip), one per family of
-// schemes, so that they compile side by side; `params` points to the launcher's FusedParams.
-int launch_full_scan_a(int scheme, int G, int NG, const void* params, void* stream);  // K3V2, K4V4, K3V4, K4V2
-int launch_full_scan_b(int scheme, int G, int NG, const void* params, void* stream);  // K2V2, K2V3, K2V4
-int launch_full_scan_c(int scheme, int G, int NG, const void* params, void* stream);  // K3V3, K4V3
-int launch_full_scan_d(int scheme, int G, int NG, const void* params, void* stream);  // A2V2, A2V3, A2V4
-int launch_full_scan_e(int scheme, int G, int NG, const void* params, void* stream);  // B4V2, B4V3, B4V4
+// schemes, and five more for the form for short splits (fused_short_*.hip: the same files with JF_SHORT_FORM), so that they
+// compile side by side; `params` points to the launcher's FusedParams.
+#define JF_SCAN_FAMILY(F)                                                                        \
+  int launch_full_scan_##F(int scheme, int G, int NG, const void* params, void* stream);         \
+  int launch_short_scan_##F(int scheme, int G, int NG, const void* params, void* stream);
+JF_SCAN_FAMILY(a)  // K3V2, K4V4, K3V4, K4V2
+JF_SCAN_FAMILY(b)  // K2V2, K2V3, K2V4
+JF_SCAN_FAMILY(c)  // K3V3, K4V3
+JF_SCAN_FAMILY(d)  // A2V2, A2V3, A2V4
+JF_SCAN_FAMILY(e)  // B4V2, B4V3, B4V4
+#undef JF_SCAN_FAMILY
+#ifdef JF_SHORT_FORM
+#define JF_SCAN_ENTRY(F) launch_short_scan_##F
+constexpr bool kShortForm = true;
+#else
+#define JF_SCAN_ENTRY(F) launch_full_scan_##F
+constexpr bool kShortForm = false;
+#endif
 
 namespace {
 
@@ -498,7 +510,15 @@ struct PreCorr {
 // barriers), 18 us at 1024 rows; the same steps from LDS, four wavefronts per head, cost 4 to 8 us at the end of the
 // scan.  Per layer, MI355X, graph replay: 32 sequences x 2048 positions, K3V2, 8 kv-heads, top-k 256 37.5 -> 26.7 us;
 // 32 x 464, K3V4, 4 kv-heads, top-k 64 30.1 -> 19.4; 7 x 311, K4V4, 8 kv-heads, G = 2 20.7 -> 16.5.
-template <int MODE, int SCHEME, int G, int NG, bool ONE = false>
+//
+// SHORT: at most one chunk per wavefront (splits of up to NW * 64 positions).  Its V rows are requested along with the key
+// rows; the form for longer splits requests V rows with the last two of four key chunks, which a short split never
+// reaches, so that it would wait for them from a standing start.  Wavefronts without a chunk request no keys: sixteen
+// wavefronts' loads are issued one after the other, some twelve cycles each, before the query set-up's barrier.  Per layer:
+// 4 x 8100 positions, B4V4 in 64-channel groups (splits of 1024) 28.0 -> 26.4 us; 1 x 4096, K4V4 (256) 18.3 -> 17.5.
+// (Two chunks per wavefront, all four requested at once: 2 to 4 % slower on 32 x 2048.  One form for all lengths that puts
+// V rows into the key buffers at run time: the compiler's waits, counted for the shorter path, cost long splits 2 %.)
+template <int MODE, int SCHEME, int G, int NG, bool ONE = false, bool SHORT = false>
 __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kernel(FusedParams p) {
   using Lds = ScanLds<SCHEME, G, NG>;
   constexpr bool HAS_K = (MODE == FS_FULL || MODE == FS_STAGE_A);  // key stream and phase A
@@ -517,7 +537,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   constexpr int AR = Lds::ACC_REGS;
   constexpr float LOG2E = 1.44269504088896340736f;
   constexpr int NW = Lds::NW, NT = Lds::NT;
-  constexpr int MAXIT = Lds::LMAX / 64 / NW;  // chunks per wavefront
+  static_assert(!SHORT || MODE == FS_FULL, "the stage-wise forms have no short variant");
+  constexpr int MAXIT = SHORT ? 1 : Lds::LMAX / 64 / NW;  // chunks per wavefront
 
   extern __shared__ __align__(16) uint8_t smem[];
   const int L = p.L;
@@ -688,25 +709,35 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   };
   // first two chunks of this wavefront and the V scales of the split start now, before the query set-up
   KBuf Ka = {}, Kb = {};
-  // (every wavefront requests, on a clamped chunk if it has none of its own: the number of loads in flight at each
-  // later wait is then the same on every path, and the compiler's waits leave the younger loads in flight)
-  if constexpr (HAS_K) Ka = issue_k(min(wave, nch_cover - 1));
-  constexpr int VSPT = Lds::LMAX / NT;
+  // (every wavefront requests, chunk or not: the number of loads in flight at each later wait is then the same on every
+  // path, and the compiler's waits leave the younger loads in flight)
+  if constexpr (HAS_K && !SHORT) Ka = issue_k(min(wave, nch_cover - 1));
+  constexpr int VSPT = MAXIT;  // one word per thread and step
   // (positions past the split's end read the scale of its last row again: straight-line code whose loads leave
   // together, and the only use of these values is their maximum)
-  uint32_t vsw[VSPT], vs_slot[VSPT];
+  uint32_t vsw[VSPT];
 #pragma unroll
-  for (int i = 0; i < VSPT; ++i) {
-    const int t = min(tid + i * NT, n - 1);
-    vs_slot[i] = HAS_V ? (uint32_t)(sbase[t >> 4] + (t & 15)) : 0u;
-  }
+  for (int i = 0; i < VSPT; ++i) vsw[i] = 0u;
+  auto request_vs = [&]() {
+    uint32_t vs_slot[VSPT];
 #pragma unroll
-  for (int i = 0; i < VSPT; ++i) {
-    vsw[i] = 0u;
-    if constexpr (HAS_V) {
+    for (int i = 0; i < VSPT; ++i) {
+      const int t = min(tid + i * NT, n - 1);
+      vs_slot[i] = (uint32_t)(sbase[t >> 4] + (t & 15));
+    }
+#pragma unroll
+    for (int i = 0; i < VSPT; ++i) {
       if (NG == 2) vsw[i] = *reinterpret_cast<const uint32_t*>(vsbase + (size_t)(vs_slot[i] * 4u));
       else vsw[i] = (uint32_t) * reinterpret_cast<const uint16_t*>(vsbase + (size_t)(vs_slot[i] * 2u));
     }
+  };
+  if constexpr (SHORT) {
+    if (wave < nch_cover) {  // (a wavefront without a chunk requests nothing: its loads would only be in the others' way)
+      Ka = issue_k(wave);
+      request_vs();
+    }
+  } else if constexpr (HAS_V) {
+    request_vs();
   }
   if constexpr (!HAS_K) {
     // the scores are an input: no query constants
@@ -834,7 +865,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     }
   }
   lds_barrier();
-  if constexpr (HAS_K) Kb = issue_k(min(wave + NW, nch_cover - 1));
+  if constexpr (HAS_K && !SHORT) Kb = issue_k(min(wave + NW, nch_cover - 1));
   if (clk && tid == 0) clk[7] = JF_CLK();
 
   // ---- V stream, set-up (same scheme as the key stream)
@@ -858,18 +889,21 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   };
   auto issue_v = [&](int chunk) -> VBuf {
     VBuf vbuf;
+    // (SHORT, a chunk the wavefront does not have: all lanes read one place)
+    const uint32_t lm = (!SHORT || chunk < nch) ? 0xffffffffu : 0u;
+    if constexpr (SHORT) chunk = (lm != 0u) ? chunk : 0;
 #pragma unroll
     for (int i = 0; i < VLD; ++i) {
-      const uint32_t sb = (uint32_t)sbase[chunk * 4 + vl_page[i]];
-      vbuf.r[i] = *reinterpret_cast<const v4u*>(vbase + (size_t)(sb * (uint32_t)VP + vl_off[i]));
+      const uint32_t sb = (uint32_t)sbase[chunk * 4 + (vl_page[i] & lm)];
+      vbuf.r[i] = *reinterpret_cast<const v4u*>(vbase + (size_t)(sb * (uint32_t)VP + (vl_off[i] & lm)));
     }
     return vbuf;
   };
   // the first two V chunks are requested while the last key chunks are being worked on
   VBuf Va = {}, Vb = {};
-  bool va_requested = false, vb_requested = false;  // (uniform per wavefront)
+  bool va_requested = SHORT, vb_requested = SHORT;  // (uniform per wavefront)
   auto prefetch_v = [&](int it) {
-    if constexpr (MODE == FS_FULL) {
+    if constexpr (MODE == FS_FULL && !SHORT) {
       if (it == MAXIT - 2) {
         Va = issue_v(min(wave, nch - 1));
         va_requested = true;
@@ -880,6 +914,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       }
     }
   };
+  if constexpr (SHORT) Va = issue_v(wave);
   if constexpr (MODE == FS_STAGE_B) {  // nothing to wait for: the value stream starts at once
     Va = issue_v(min(wave, nch - 1));
     Vb = issue_v(min(wave + NW, nch - 1));
@@ -3488,12 +3523,12 @@ inline WsLayout ws_layout(int B, int H_q, int ns, int kc, int parts, int top_k) 
   return w;
 }
 
-template <int MODE, int SCHEME, int G, int NG>
+template <int MODE, int SCHEME, int G, int NG, bool SHORT = false>
 int launch_scan(const FusedParams& p, hipStream_t st) {
   using Lds = ScanLds<SCHEME, G, NG>;
   const bool one = p.one_split != 0;
   const size_t smem = Lds::total(p.L) + (one ? ScanTail<G, Lds::SEG>::bytes(p.top_k, p.Kc) : 0);
-  auto kern = one ? fused_scan_kernel<MODE, SCHEME, G, NG, true> : fused_scan_kernel<MODE, SCHEME, G, NG, false>;
+  auto kern = one ? fused_scan_kernel<MODE, SCHEME, G, NG, true, SHORT> : fused_scan_kernel<MODE, SCHEME, G, NG, false, SHORT>;
   // per instantiation: raise the dynamic-LDS limit only when it grows (launches may come from several threads)
   static std::mutex attr_mu;
   static size_t attr_smem[2] = {0, 0};
@@ -3525,17 +3560,17 @@ int launch_scan(const FusedParams& p, hipStream_t st) {
   return JF_OK;
 }
 
-// One scheme of the one-pass form: the GQA group picks the instantiation.
+// One scheme of the one-pass form: the GQA group picks the instantiation (of this translation unit's form).
 template <int SCHEME, int NG>
 int launch_full_by_group(int G, const void* params, void* stream) {
   const FusedParams& p = *static_cast<const FusedParams*>(params);
   hipStream_t st = (hipStream_t)stream;
   switch (G) {
-    case 1: return launch_scan<FS_FULL, SCHEME, 1, NG>(p, st);
-    case 2: return launch_scan<FS_FULL, SCHEME, 2, NG>(p, st);
-    case 4: return launch_scan<FS_FULL, SCHEME, 4, NG>(p, st);
-    case 8: return launch_scan<FS_FULL, SCHEME, 8, NG>(p, st);
-    default: return launch_scan<FS_FULL, SCHEME, 16, NG>(p, st);
+    case 1: return launch_scan<FS_FULL, SCHEME, 1, NG, kShortForm>(p, st);
+    case 2: return launch_scan<FS_FULL, SCHEME, 2, NG, kShortForm>(p, st);
+    case 4: return launch_scan<FS_FULL, SCHEME, 4, NG, kShortForm>(p, st);
+    case 8: return launch_scan<FS_FULL, SCHEME, 8, NG, kShortForm>(p, st);
+    default: return launch_scan<FS_FULL, SCHEME, 16, NG, kShortForm>(p, st);
   }
 }
 
@@ -3681,11 +3716,15 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
     default: JF_FUSED_CASE(SCH, 16, NGG); break;       \
   }
   if constexpr (MODE == FS_FULL) {  // (instantiated elsewhere, by family)
-    if (scheme_has_zp(scheme)) rc = launch_full_scan_d(scheme, G, NGv, &p, stream);
-    else if (scheme / 10 == 5) rc = launch_full_scan_e(scheme, G, NGv, &p, stream);
-    else if (scheme / 10 == 2) rc = launch_full_scan_b(scheme, G, NGv, &p, stream);
-    else if (scheme == JF_SCHEME_K3V3 || scheme == JF_SCHEME_K4V3) rc = launch_full_scan_c(scheme, G, NGv, &p, stream);
-    else rc = launch_full_scan_a(scheme, G, NGv, &p, stream);
+    // one chunk of 64 positions per wavefront at most (see SHORT)
+    const bool is_short = (p.L < max_S ? p.L : max_S) <= 64 * (G <= 4 ? 16 : 8);
+#define JF_SCAN_OF(F) rc = is_short ? launch_short_scan_##F(scheme, G, NGv, &p, stream) : launch_full_scan_##F(scheme, G, NGv, &p, stream)
+    if (scheme_has_zp(scheme)) JF_SCAN_OF(d);
+    else if (scheme / 10 == 5) JF_SCAN_OF(e);
+    else if (scheme / 10 == 2) JF_SCAN_OF(b);
+    else if (scheme == JF_SCHEME_K3V3 || scheme == JF_SCHEME_K4V3) JF_SCAN_OF(c);
+    else JF_SCAN_OF(a);
+#undef JF_SCAN_OF
   } else if constexpr (MODE == FS_TOPK) {
     JF_FUSED_BY_G(JF_SCHEME_K4V4, 1)
   } else if (scheme == JF_SCHEME_K3V2) {
