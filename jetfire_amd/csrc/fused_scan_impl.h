@@ -634,6 +634,11 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     return;
   }
 
+  // A candidate list with room for all of the split's positions takes them all, in place: no selection buckets, no cut, no
+  // compaction.  1 x 4096 positions, K4V4, top-k 64 (splits of 256), per layer 17.4 -> 15.5 us.  (Short splits only: the
+  // test in the value stream costs the long ones, which have room for all of them in the widest corrections only, 0.8 %.)
+  const bool take_all = SHORT && !ONE && n <= p.Kc;  // (uniform)
+
   // Page table of the split: one entry per 16 positions of every 64-token chunk that is touched.  Table
   // entries past the last valid position may hold anything: those pages read slot 0 instead, so every row
   // address formed below is in bounds (those rows' scores are masked to -inf, their softmax weights are
@@ -1544,7 +1549,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   if constexpr (MODE == FS_STAGE_A)
     if (p.scores_only) return;
   if constexpr (HAS_TOPK)
-    for (int i = tid; i < Lds::HIST / 4; i += NT) hist[i] = 0;
+    if (!take_all)
+      for (int i = tid; i < Lds::HIST / 4; i += NT) hist[i] = 0;
   if (tid < G) {
     float m = red_f[0][tid], lo = red_f[0][G + tid];
 #pragma unroll
@@ -1640,7 +1646,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         lsum[h] += pw;
 #pragma unroll
         for (int g = 0; g < NG; ++g) bits[h][g] = __builtin_bit_cast(uint32_t, __builtin_fmaf(pw, vsf[g], 8388608.0f));
-        if constexpr (HAS_TOPK) {
+        if (HAS_TOPK && !take_all) {
           // (positions past the end add zero instead of branching around the add: their score is -inf or, with a
           // degenerate range, gives a NaN, and either clamps to a bucket inside the table)
           const uint32_t bin = (uint32_t)__builtin_amdgcn_fmed3f(__builtin_fmaf(s, bin_a[h], bin_bv[h]), 0.f, clamp_hi);
@@ -1908,6 +1914,29 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   for (int hs = wave; HAS_TOPK && hs < G * SEG; hs += NW) {
     const int h = hs / SEG, seg = hs % SEG;
     if (h >= GA) continue;
+    if (SHORT && !ONE && take_all) {
+      const float* srow = sc + h * L;
+      uint32_t* ck = p.cand_key + (part_base + (size_t)h * p.n_splits) * Kcap;
+      int32_t* ci = p.cand_idx + (part_base + (size_t)h * p.n_splits) * Kcap;
+      for (int t = (seg * 64 + lane) * 4; t < Kcap; t += SEG * 256) {  // (the list's length is a multiple of 4, at most L)
+        const v4f x = *reinterpret_cast<const v4f*>(srow + t);
+        v4u key;
+        v4i pos;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          key[u] = (t + u < n) ? score_key(x[u]) : 0u;  // unused slots hold key 0
+          pos[u] = s0 + t + u;
+        }
+        *reinterpret_cast<v4u*>(ck + t) = key;
+        *reinterpret_cast<v4i*>(ci + t) = pos;
+      }
+      if (seg == 0) {  // the smallest score
+        float lo = -red_f[lane & (NW - 1)][G + h];
+        JF_DPP_ROW_REDUCE(lo, op_fmax, float, -INFINITY);
+        if (lane == 15) p.cand_edge[part_base + (size_t)h * p.n_splits] = -lo;
+      }
+      continue;
+    }
     // Every wavefront of a head searches the cut itself (same histograms, same result): no exchange, no barrier
     // between the search and the emission.
     const float ba = uniform_f(bin_a_sh[h]);
