@@ -387,6 +387,23 @@ __device__ inline float uniform_f(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
 
+// |x| as an integer of the same order; zero for a NaN, which takes no part in a maximum
+__device__ inline uint32_t abs_bits(float x) { return (x == x) ? __builtin_bit_cast(uint32_t, x) & 0x7fffffffu : 0u; }
+// Reductions over each half of a wavefront (32 lanes), the result in every lane of the half: DPP row shifts and the first
+// row broadcast.  (Five shuffles through the LDS crossbar, one after the other, take some 600 cycles.)
+__device__ inline uint32_t half_max_u(uint32_t v) {
+  JF_DPP_ROW_REDUCE(v, op_umax, uint32_t, 0u);
+  v = op_umax(v, (uint32_t)dpp_mov<0x142, 0xa>(0, (int)v));
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)v, 31), hi = (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+  return (threadIdx.x & 32) ? hi : lo;
+}
+__device__ inline int half_sum_i(int v) {
+  JF_DPP_ROW_REDUCE(v, op_iadd, int, 0);
+  v += dpp_mov<0x142, 0xa>(0, v);
+  const int lo = __builtin_amdgcn_readlane(v, 31), hi = __builtin_amdgcn_readlane(v, 63);
+  return (threadIdx.x & 32) ? hi : lo;
+}
+
 // Range-checked loads through a buffer descriptor (raw, the offsets in bytes): past its end a load returns zero, and the
 // scalar base and offset take the place of 64-bit vector address arithmetic.
 __device__ inline __amdgpu_buffer_rsrc_t buffer_of(const void* base, int bytes) {
@@ -791,7 +808,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         if (c * 64 >= QN) continue;    // uniform per wavefront
         const int i = it * NT + tid, h = i >> 7, d = i & 127;
         const float x = q_elem(it);
-        const float amax = wave_max(fabsf(x));
+        const float amax = __builtin_bit_cast(float, wave_max_u(abs_bits(x)));
         int e = 0;
         if (amax > 0.f && isfinite(amax)) (void)frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
         const int qf = (int)rintf(ldexpf(x, 22 - e));
@@ -807,7 +824,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       for (int it = 0; it < QPT; ++it) {
         const int c = it * NW + wave;  // 64-channel half row of this wavefront
         if (c * 64 < QN) {             // uniform per wavefront
-          const float am = wave_max(fabsf(q_elem(it)));
+          const float am = __builtin_bit_cast(float, wave_max_u(abs_bits(q_elem(it))));
           if (lane == 0) prep->amax_w[c] = am;
         }
       }
@@ -846,15 +863,11 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       if (i < QN) {  // uniform per wavefront: QN is a multiple of 64
         const int h = i >> 7, d = i & 127, kk = d >> 5;
         const float x = q_elem(it);
-        float a = fabsf(x);
-#pragma unroll
-        for (int off = 16; off >= 1; off >>= 1) a = fmaxf(a, __shfl_xor(a, off));
+        const float a = __builtin_bit_cast(float, half_max_u(abs_bits(x)));
         const float sq = fmaxf(a / 127.0f, 1e-12f);
         const float inv = 1.0f / sq;
         const int v = max(-128, min(127, (int)rintf(x * inv)));
-        int sv = v;
-#pragma unroll
-        for (int off = 16; off >= 1; off >>= 1) sv += __shfl_xor(sv, off);
+        const int sv = half_sum_i(v);
         // channel d sits in MFMA d>>6, k-block (d>>4)&3; inside the k-block's 16 bytes the nibble spread of two
         // packed dwords yields: even channels of bytes 0-3, odd channels of bytes 0-3, then the same for bytes 4-7
         const int set = h >> 2, hh = h & 3, mi = d >> 6, kb = (d >> 4) & 3;
@@ -2098,9 +2111,40 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           sco = s_next;
         }
       };
+      if constexpr (SHORT) {
+        // Segments of at most 256 positions (512 beyond four heads): one position per lane, 64 at a time; all scores first,
+        // then the sums' atomics, which would otherwise be ahead of them in the LDS queue.  (Sixteen positions per lane,
+        // as below, leave a segment of 256 to sixteen lanes.)
+        constexpr int STEPS = Lds::NT / SEG / 64;
+        float x[STEPS];
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) x[i] = srow[min(tb + 64 * i + lane, L - 1)];
+        if (HAS_V && !acc_issued) {
+          add_acc_range(0, ACC_TOTAL * 4);
+          acc_issued = true;
+        }
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+          if (tb + 64 * i < te) {
+            const int t = tb + 64 * i + lane;
+            const bool emit = t < te && !(__builtin_fmaf(x[i], ba, bb) >= thr);
+            const unsigned long long em = __builtin_amdgcn_ballot_w64(emit);
+            const uint32_t o = (uint32_t)(count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(em >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)em, 0u)));
+            count += __popcll(em);
+            if (emit && o < (uint32_t)Kcap) {  // the bound only matters for non-finite scores
+              if constexpr (ONE) {
+                cl[o] = (uint16_t)t;
+              } else {
+                ck[o] = score_key(x[i]);
+                ci[o] = s0 + t;
+              }
+            }
+          }
+        }
+      }
       constexpr std::integral_constant<int, -1> plain{};
-      int t0 = tb;
-      if (HAS_V && !acc_issued && te > tb) {  // the first block (or the first two) of this wavefront carry the sums
+      int t0 = SHORT ? te : tb;
+      if (!SHORT && HAS_V && !acc_issued && te > tb) {  // the first block (or the first two) of this wavefront carry the sums
         if (te - tb > 1024) {
           emit_block(tb, std::integral_constant<int, 0>{});
           emit_block(tb + 1024, std::integral_constant<int, 1>{});
