@@ -419,6 +419,10 @@ __device__ inline float buffer_f32(__amdgpu_buffer_rsrc_t r, int voffset, int so
   return __builtin_bit_cast(float, buffer_i32(r, voffset, soffset));
 }
 
+// The streams' steps must be part of the kernel: as calls (the compiler's choice for some instantiations) they keep every
+// captured array in scratch memory, at three times the run time.
+#define JF_INLINE __attribute__((always_inline))
+
 // Pre-correction terms over the winners' packed V rows, shared by the merge kernel and the scan's in-kernel merge: DW
 // lanes per row, lane dwi holds dword dwi of it (INT2, INT4) or two bytes of each of the three planes (INT3) = CPD
 // codes; a wavefront instruction covers WPI rows, sixteen wavefronts (or roles) and UNR requests per lane 256 rows.
@@ -646,8 +650,11 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       p.part_l[part_base + (size_t)tid * p.n_splits] = 0.f;
       p.cand_edge[part_base + (size_t)tid * p.n_splits] = -INFINITY;
     }
-    for (int i = tid; i < GA * p.Kc; i += NT)  // unused candidate slots hold key 0 (no score maps to it)
-      p.cand_key[(part_base + (size_t)(i / p.Kc) * p.n_splits) * p.Kc + (i % p.Kc)] = 0u;
+    // unused candidate slots hold key 0 (no score maps to it); a list's length is a multiple of 4
+    for (int h = wave / (NW / 4); HAS_TOPK && h < GA; h += 4) {
+      uint32_t* ck = p.cand_key + (part_base + (size_t)h * p.n_splits) * p.Kc;
+      for (int i = (wave % (NW / 4) * 64 + lane) * 4; i < p.Kc; i += NW / 4 * 256) *reinterpret_cast<v4u*>(ck + i) = (v4u){0u, 0u, 0u, 0u};
+    }
     return;
   }
 
@@ -943,7 +950,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // scale words become copies of the last valid row, so the stream's arithmetic runs without a validity select per
   // score (a copy of a valid score changes neither extremum), and `mask_tail` afterwards stores -inf over what those
   // positions produced.  A chunk past the end (n_local <= 0) is not worked through at all.
-  auto clone_last_row = [&](int n_local, uint32_t (&Sx)[4], uint32_t (&Zx)[4]) {
+  auto clone_last_row = [&](int n_local, uint32_t (&Sx)[4], uint32_t (&Zx)[4]) JF_INLINE {
     const int last = n_local - 1, jl = last >> 4;
     if constexpr (SL) {  // one scale word per lane (= token): Sx[0]
       const uint32_t sl = (uint32_t)__builtin_amdgcn_readlane((int)Sx[0], last);
@@ -1056,7 +1063,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     for (int set = 0; set < NSET; ++set)
 #pragma unroll
       for (int g = 0; g < NG; ++g) Cin[set][g] = (v4i){-sq4[set][g], 0, 0, 0};
-    auto body = [&](int chunk, const uint32_t (&Sx)[4], const uint32_t (&Zx)[4]) {
+    auto body = [&](int chunk, const uint32_t (&Sx)[4], const uint32_t (&Zx)[4]) JF_INLINE {
       (void)Zx;
       // all LDS reads of the chunk first (plane dwords of the four pages, rounding coefficients), then arithmetic
       uint32_t Pj[4][3];
@@ -1379,7 +1386,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     // loads leaves the loads of the following chunks in flight
     // (step it + 1 sits inside step it's block, and the chunk two ahead is requested unconditionally, clamped: no
     // two paths with different numbers of loads in flight meet before a wait)
-    auto key_step = [&](auto self, auto it_tag) -> void {
+    auto key_step = [&](auto self, auto it_tag) JF_INLINE -> void {
       constexpr int it = decltype(it_tag)::value;
       const int chunk = wave + it * NW;
       prefetch_v(it);
@@ -1459,7 +1466,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       mxl[set] = -INFINITY;
       mnl[set] = INFINITY;
     }
-    auto body = [&](int chunk, const uint32_t (&Sx)[4]) {
+    auto body = [&](int chunk, const uint32_t (&Sx)[4]) JF_INLINE {
       v2u Xj[4][2];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -1497,7 +1504,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         }
       }
     };
-    auto key_step = [&](auto self, auto it_tag) -> void {  // (nested, as for the other key formats)
+    auto key_step = [&](auto self, auto it_tag) JF_INLINE -> void {  // (nested, as for the other key formats)
       constexpr int it = decltype(it_tag)::value;
       const int chunk = wave + it * NW;
       prefetch_v(it);
@@ -1640,7 +1647,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   const int tr_tok = (((r16 >> 1) & 3) << 1) | ((r16 >> 3) & 1);
   const uint8_t* wrow = wl + (kb4 * 16 + tr_tok) * 16 + (r16 & 1) * 8;
   const int seg_chunks = L / 64 / SEG;  // chunks per emission segment
-  auto body_v = [&](int chunk, uint32_t vsw) {
+  auto body_v = [&](int chunk, uint32_t vsw) JF_INLINE {
     const int t = chunk * 64 + lane;
     float vsf[NG];
     vsf[0] = ldexpf(bf16_to_f32((uint16_t)(vsw & 0xffffu)), E[0]);
@@ -1789,7 +1796,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     if (!va_requested) Va = issue_v(min(wave, nch - 1));
     if (!vb_requested) Vb = issue_v(min(wave + NW, nch - 1));
   }
-  auto value_step = [&](auto self, auto it_tag) -> void {  // (nested like the key stream's steps)
+  auto value_step = [&](auto self, auto it_tag) JF_INLINE -> void {  // (nested like the key stream's steps)
     constexpr int it = decltype(it_tag)::value;
     const int chunk = wave + it * NW;
     if (chunk < nch) {
@@ -2054,7 +2061,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       // few set bits of every lane.  The lane reads its four 16-byte quads starting at quad (lane >> 2) & 3 (the
       // four lanes that share a bank group then read different banks) and rotates its bit mask back afterwards.
       const int rot4 = ((lane >> 2) & 3) * 4;
-      auto emit_block = [&](int t0, auto acc_tag) {
+      auto emit_block = [&](int t0, auto acc_tag) JF_INLINE {
         constexpr int ACCSEL = decltype(acc_tag)::value;  // accumulator sums issued along the comparisons: -1 none, 0 / 1 a half, 2 all
         constexpr int A_LO = (ACCSEL == 1) ? ACC_HALF * 4 : 0;
         constexpr int A_HI = (ACCSEL < 0) ? 0 : ((ACCSEL == 0) ? ACC_HALF * 4 : ACC_TOTAL * 4);
