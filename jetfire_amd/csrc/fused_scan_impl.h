@@ -572,9 +572,11 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   __shared__ uint32_t vmax_sh[NW][2];
   __shared__ float m_sh[G], bin_a_sh[G], bin_b_sh[G], lsum_sh[NW][G];
   __shared__ int e_sh[2];
-  // rounding coefficients 256 * (bf16(c s) - c s) / s for s = 1 + m/128 (INT3: c = 3; INT4, bf16 model: c = 3, 5, 7).
+  // Rounding of bf16(c s) for s = 1 + m/128.  INT3: the coefficient 256 * (bf16(3 s) - 3 s) / s.  INT4 (bf16 model): what
+  // the roundings are multiples of, 256 / (128 s), and the byte tables they are looked up in (see phase A).
   // Static, so that a look-up's address is the index plus a constant the instruction carries.
-  __shared__ float eps_sh[KB4 ? 3 : 1][128];
+  __shared__ float eps_sh[128];
+  __shared__ v4u rnd_sh[KB4 ? 128 : 1];
   __shared__ unsigned long long tmax_sh;
   if (threadIdx.x == 0) tmax_sh = 0ull;
 
@@ -779,10 +781,21 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     if ((K3 || KB4) && tid >= EPS_T0 && tid < EPS_T0 + 128) {
       const int m = tid - EPS_T0;
       const float sm = 1.0f + (float)m * (1.0f / 128.0f);
-#pragma unroll
-      for (int i = 0; i < (KB4 ? 3 : 1); ++i) {
-        const float t = (float)(3 + 2 * i) * sm;  // 3 s, 5 s, 7 s: exact in fp32
-        eps_sh[i][m] = 256.0f * ((bf16_to_f32(f32_to_bf16(t)) - t) / sm);
+      if constexpr (KB4) {
+        // in units of 1/128 a rounding is a whole number of at most 4
+        auto rounding = [&](float c) -> int { return (int)(128.0f * (bf16_to_f32(f32_to_bf16(c * sm)) - c * sm)); };
+        const int r3 = rounding(3.f), r5 = rounding(5.f), r7 = rounding(7.f);
+        auto bytes = [](int b0, int b1, int b2, int b3) -> uint32_t {
+          return (uint32_t)(b0 & 255) | ((uint32_t)(b1 & 255) << 8) | ((uint32_t)(b2 & 255) << 16) | ((uint32_t)b3 << 24);
+        };
+        // first the codes 0..7, then -8..-1; each entry less what the other table's look-up yields for the same code
+        const int n1 = -r7 + (r3 < 0 ? 1 : 0), n2 = -2 * r3 + (r5 < -1 ? 1 : 0), n3 = -r5 + (r7 < -1 ? 1 : 0), n5 = 1 - r3;
+        rnd_sh[m] = (v4u){bytes(n1 < 0 ? 1 : 0, n3 < 0 ? 1 : 0, n5 < 0 ? 1 : 0, r3), bytes(0, r5 + 1, 2 * r3 + 1, r7 + 1),
+                          bytes(0, n1, n2, n3), bytes(0, n5, 1, 1)};
+        eps_sh[m] = 2.0f / sm;
+      } else {
+        const float t = 3.0f * sm;  // exact in fp32
+        eps_sh[m] = 256.0f * ((bf16_to_f32(f32_to_bf16(t)) - t) / sm);
       }
     }
     // stores the three limbs of element (h, d) in the byte order of the MFMA A operand
@@ -1098,10 +1111,10 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         } else if constexpr (!KB4) {
           const uint32_t sw = scale_word(Sx, j);
           sgj[j][0] = bf16_to_f32((uint16_t)(sw & 0xffffu));
-          egj[j][0] = K3 ? eps_sh[0][sw & 0x7fu] : 0.f;  // (INT4: three coefficients, read where they are used)
+          egj[j][0] = K3 ? eps_sh[sw & 0x7fu] : 0.f;
           if (NG == 2) {
             sgj[j][NG - 1] = bf16_to_f32((uint16_t)(sw >> 16));
-            egj[j][NG - 1] = K3 ? eps_sh[0][(sw >> 16) & 0x7fu] : 0.f;
+            egj[j][NG - 1] = K3 ? eps_sh[(sw >> 16) & 0x7fu] : 0.f;
           }
         }
       }
@@ -1148,15 +1161,16 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           }
         }
         if constexpr (KB4) {
-          // khat = bf16((u - 8) s) for the unsigned nibble u: exact for |u - 8| in {0, 1, 2, 4, 8}; for 3, 5, 7 (and 6 =
-          // 2 * 3) the rounding is eps_c(s) * s with the sign of the code, eps_c a function of the scale's mantissa
-          // alone.  So next to the code contraction there are three with the signed indicators r3 = [c = +-3] +
-          // 2 [c = +-6], r5 = [c = +-5], r7 = [c = +-7], each the sum of two byte look-ups: one that is right for the codes
-          // >= 0 (selector u ^ 8 = c) and one for the codes < 0 (selector u = c + 8).  Selectors 8..15 of v_perm_b32 are
-          // not table entries but constants (8..11 the signs of bytes 1, 3, 5, 7, 12 zero, 13..15 minus one); the tables
-          // hold what makes the two sums come out, and the matrix cores, which are idle mostly, do the adding: seven
-          // vector instructions per dword.  (Masking the selectors and choosing between the two results per byte took
-          // fourteen.)  4 x 8100 positions, B4V4 in 64-channel groups, per layer: 29.0 -> 28.0 us, and no scratch any more.
+          // khat = bf16((u - 8) s) for the unsigned nibble u and s = 2^e (1 + m/128) is (c + r_c(m) / (128 + m)) s, c = u - 8,
+          // with whole numbers r_c, |r_c| <= 4, that depend on the scale's mantissa alone: zero but for c = +-3, 5, 7 (and
+          // +-6 = 2 * +-3), and odd in c.  So next to the code contraction there is one with the bytes r_c, each the sum of two
+          // byte look-ups in tables of the lane's token: one that is right for the codes >= 0 (selector u ^ 8 = c) and one for
+          // the codes < 0 (selector u = c + 8).  Selectors 8..15 of v_perm_b32 are not table entries but constants (8..11 the
+          // signs of bytes 1, 3, 5, 7, 12 zero, 13..15 minus one); the tables hold what makes the two sums come out, and the
+          // matrix cores, which are idle mostly, do the adding: three vector instructions per dword.
+          // (Three contractions with the signed indicators of +-3, +-5 and +-7 from constant tables, each with its own
+          // coefficient per token, took seven and the scan's phase A 12.5 k cycles instead of 8.6 k: 4 x 8100 positions,
+          // B4V4 in 64-channel groups, per layer 25.8 -> 24.2 us.  Scores are off the 64-bit ones by 4.9e-8, 5.2e-8 before.)
           const uint32_t sw = scale_word(Sx, j);
           const int tok = chunk * 64 + 16 * j + t16;
           float acc_s[NSET][NG];
@@ -1164,7 +1178,6 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           for (int set = 0; set < NSET; ++set)
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
-              const v4i zero = {0, 0, 0, 0};
               v4i Dc;
               if (NG == 2) {
                 Dc = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][g], Bc[g], Cin[set][g], 0, 0, 0);
@@ -1172,48 +1185,42 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
                 Dc = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bc[0], Cin[set][0], 0, 0, 0);
                 Dc = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bc[1], Dc, 0, 0, 0);
               }
-              (void)zero;
               acc_s[set][g] = (float)join_limbs(Dc[2], Dc[1], Dc[0]);
             }
-          v4i Bw[2];  // u ^ 8
+          v4i Bp[2], Bn[2];
+          v4u rnd[NG];
+          float unit[NG];
+#pragma unroll
+          for (int g = 0; g < NG; ++g) {
+            const uint32_t m = ((g == 0) ? sw : (sw >> 16)) & 0x7fu;
+            rnd[g] = rnd_sh[m];
+            unit[g] = eps_sh[m];
+          }
 #pragma unroll
           for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) Bw[u][e] = Bc[u][e] ^ 0x08080808;
+            for (int e = 0; e < 4; ++e) {
+              const v4u r = rnd[(NG == 2) ? u : 0];
+              Bp[u][e] = (int)__builtin_amdgcn_perm(r[1], r[0], (uint32_t)(Bc[u][e] ^ 0x08080808));
+              Bn[u][e] = (int)__builtin_amdgcn_perm(r[3], r[2], (uint32_t)Bc[u][e]);
+            }
 #pragma unroll
-          for (int c = 0; c < 3; ++c) {  // c = 0, 1, 2: the indicators of +-3 (and +-6), +-5, +-7
-            const uint32_t pos_hi = (c == 0) ? 0x01030100u : ((c == 1) ? 0x01010200u : 0x02010100u);
-            const uint32_t pos_lo = (c == 0) ? 0x01000000u : ((c == 1) ? 0x00000100u : 0x00000001u);
-            const uint32_t neg_hi = (c == 0) ? 0x01010000u : ((c == 1) ? 0x01010100u : 0x01010100u);
-            const uint32_t neg_lo = (c == 0) ? 0x00fe0000u : ((c == 1) ? 0xff000000u : 0x0000ff00u);
-            __builtin_amdgcn_sched_barrier(0);
-            v4i Bp[2], Bn[2];
+          for (int set = 0; set < NSET; ++set)
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                Bp[u][e] = (int)__builtin_amdgcn_perm(pos_hi, pos_lo, (uint32_t)Bw[u][e]);
-                Bn[u][e] = (int)__builtin_amdgcn_perm(neg_hi, neg_lo, (uint32_t)Bc[u][e]);
+            for (int g = 0; g < NG; ++g) {
+              const v4i zero = {0, 0, 0, 0};
+              v4i Dr;
+              if (NG == 2) {
+                Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][g], Bp[g], zero, 0, 0, 0);
+                Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][g], Bn[g], Dr, 0, 0, 0);
+              } else {
+                Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bp[0], zero, 0, 0, 0);
+                Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bp[1], Dr, 0, 0, 0);
+                Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bn[0], Dr, 0, 0, 0);
+                Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bn[1], Dr, 0, 0, 0);
               }
-#pragma unroll
-            for (int set = 0; set < NSET; ++set)
-#pragma unroll
-              for (int g = 0; g < NG; ++g) {
-                const v4i zero = {0, 0, 0, 0};
-                v4i Dr;
-                if (NG == 2) {
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][g], Bp[g], zero, 0, 0, 0);
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][g], Bn[g], Dr, 0, 0, 0);
-                } else {
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bp[0], zero, 0, 0, 0);
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bp[1], Dr, 0, 0, 0);
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bn[0], Dr, 0, 0, 0);
-                  Dr = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bn[1], Dr, 0, 0, 0);
-                }
-                const float ec = eps_sh[c][((g == 0) ? sw : (sw >> 16)) & 0x7fu];
-                acc_s[set][g] = __builtin_fmaf(ec, (float)((Dr[2] << 8) + Dr[1]), acc_s[set][g]);
-              }
-          }
+              acc_s[set][g] = __builtin_fmaf(unit[g], (float)((Dr[2] << 8) + Dr[1]), acc_s[set][g]);
+            }
 #pragma unroll
           for (int set = 0; set < NSET; ++set) {
             float score = 0.f;
@@ -1409,10 +1416,10 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
             const uint32_t sw = Sc[0];
             uint8_t* sp = kst + Lds::KST + lane * Lds::SCT;
             const float s0f = bf16_to_f32((uint16_t)(sw & 0xffffu));
-            const float e0f = K3 ? eps_sh[0][sw & 0x7fu] : 0.f;
+            const float e0f = K3 ? eps_sh[sw & 0x7fu] : 0.f;
             if (NG == 2) {
               const float s1f = bf16_to_f32((uint16_t)(sw >> 16));
-              const float e1f = K3 ? eps_sh[0][(sw >> 16) & 0x7fu] : 0.f;
+              const float e1f = K3 ? eps_sh[(sw >> 16) & 0x7fu] : 0.f;
               *reinterpret_cast<v4f*>(sp) = (v4f){s0f, s1f, e0f, e1f};
             } else {
               *reinterpret_cast<v2f*>(sp) = (v2f){s0f, e0f};
@@ -3378,7 +3385,7 @@ template <int SCHEME, int G, int NG>
 long lds_room_for() {
   using Lds = ScanLds<SCHEME, G, NG>;
   const size_t budget = (G <= 4 && Lds::NW == 8) ? LDS_BUDGET_2WG : LDS_BUDGET_1WG;
-  const size_t fixed = Lds::AUX + Lds::stage_bytes() + 64 + 832 + (Lds::KB4 ? 1536 : (Lds::K3 ? 512 : 0));  // + static LDS of the kernel (incl. the rounding tables)
+  const size_t fixed = Lds::AUX + Lds::stage_bytes() + 64 + 832 + (Lds::KB4 ? 2560 : (Lds::K3 ? 512 : 0));  // + static LDS of the kernel (incl. the rounding tables)
   return (long)budget - (long)fixed;
 }
 
