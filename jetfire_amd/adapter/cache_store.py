@@ -124,12 +124,20 @@ class JetFireInt4CacheStore:
     # ------------------------------------------------------------------ append
     def _prepare(self, key, value, slot_mapping):
         n = min(int(slot_mapping.numel()), int(key.shape[0]), int(value.shape[0]))
-        slots = slot_mapping[:n].to(device=self.device, dtype=torch.long).contiguous()
-        key_tok, value_tok = key[:n], value[:n]
+        # (what needs no cut and no conversion is taken as it is: the views and conversions that would change nothing are
+        # half of a decode token's time on the host, 8 us)
+        dev = self.k_data.device
+        if not (slot_mapping.shape == (n,) and slot_mapping.dtype is torch.long and slot_mapping.device == dev):
+            slot_mapping = slot_mapping[:n].to(device=self.device, dtype=torch.long)
+        slots = slot_mapping.contiguous()
+        key_tok = key if key.shape[0] == n else key[:n]
+        value_tok = value if value.shape[0] == n else value[:n]
         if key_tok.shape[1:] != (self.num_kv_heads, self.head_dim) or value_tok.shape[1:] != key_tok.shape[1:]:
             raise ValueError(f"key/value must be (T, {self.num_kv_heads}, {self.head_dim}); got {tuple(key.shape)}, {tuple(value.shape)}")
-        key_tok = key_tok.to(device=self.device, dtype=torch.bfloat16)
-        value_tok = value_tok.to(device=self.device, dtype=torch.bfloat16)
+        if key_tok.dtype is not torch.bfloat16 or key_tok.device != dev:
+            key_tok = key_tok.to(device=self.device, dtype=torch.bfloat16)
+        if value_tok.dtype is not torch.bfloat16 or value_tok.device != dev:
+            value_tok = value_tok.to(device=self.device, dtype=torch.bfloat16)
         return n, slots, key_tok, value_tok
 
     def _quantise(self, key_tok, value_tok, slots) -> None:

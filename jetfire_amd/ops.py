@@ -259,7 +259,8 @@ def append_rows(key_tok, value_tok, slot_idx, k_data, k_scales, k_zp, v_data, v_
     kds, kss, vds, vss = k_data.stride(), k_scales.stride(), v_data.stride(), v_scales.stride()
     kp, vp = key_tok.data_ptr(), value_tok.data_ptr()
     if (kst[2] != 1 or vst[2] != 1 or (kp | vp) & 15 or (kst[0] | kst[1] | vst[0] | vst[1]) & 7
-            or not all(0 <= n < 1 << 32 for n in (kst[0], vst[0], kds[1], kss[1], vds[1], vss[1]))):
+            or min(kst[0], vst[0], kds[1], kss[1], vds[1], vss[1]) < 0
+            or max(kst[0], vst[0], kds[1], kss[1], vds[1], vss[1]) >= 1 << 32):
         return False
     S, ng = k_data.size(1), D // group_size
     for d, s, ds, ss, bits in ((k_data, k_scales, kds, kss, k_nbits), (v_data, v_scales, vds, vss, v_nbits)):
