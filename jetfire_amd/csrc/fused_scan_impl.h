@@ -3812,8 +3812,9 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
     default: JF_FUSED_CASE(SCH, 16, NGG); break;       \
   }
   if constexpr (MODE == FS_FULL) {  // (instantiated elsewhere, by family)
-    // one chunk of 64 positions per wavefront at most (see SHORT)
-    const bool is_short = (p.L < max_S ? p.L : max_S) <= 64 * (G <= 4 ? 16 : 8);
+    // One chunk of 64 positions per wavefront at most (see SHORT).  It is the split's length that counts, not the sequence's:
+    // the emission's segments are parts of L, and the form works through 64 positions per wavefront of each.
+    const bool is_short = p.L <= 64 * (G <= 4 ? 16 : 8);
 #define JF_SCAN_OF(F) rc = is_short ? launch_short_scan_##F(scheme, G, NGv, &p, stream) : launch_full_scan_##F(scheme, G, NGv, &p, stream)
     if (scheme_has_zp(scheme)) JF_SCAN_OF(d);
     else if (scheme / 10 == 5) JF_SCAN_OF(e);

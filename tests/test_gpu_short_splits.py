@@ -28,3 +28,22 @@ def test_short_splits_match_the_oracle(scheme, G, S, lens, split_len):
     check_against_oracle(scheme, c, S, 64, out)
     again = run_fused(scheme, c, d, S, 64)
     assert torch.equal(out[4], again[4]) and torch.equal(out[7], again[7])
+
+
+# (four emission segments of L / 4 positions each: the short form works through 256 of each)
+@pytest.mark.parametrize("G,S,lens,split_len,K", [
+    (4, 1000, [1000, 513], 1280, 64), (4, 1000, [1000, 257], 1280, 512), (4, 700, [700, 641], 2048, 64),
+    (1, 300, [300, 257], 2048, 64), (2, 1024, [1024, 770], 4096, 256)])
+@pytest.mark.parametrize("scheme", ["k3v2", "k4v4", "b4v4", "a2v2"])
+def test_a_split_longer_than_the_sequence_keeps_every_position(scheme, G, S, lens, split_len, K):
+    """Split lengths beyond one chunk per wavefront for a sequence that has no more positions than that."""
+    from jetfire_amd import _lib
+    kb, vb, gs = SCHEME_GEOMETRY[scheme]
+    c = make_case(57 + S + G, 2, G, 1, S, kb, vb, gs, lens=lens, extra_blocks=2, k_asym=scheme.startswith("a"))
+    d = to_device(c)
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
+    try:
+        out = [t.clone() for t in run_fused(scheme, c, d, S, K)]
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    check_against_oracle(scheme, c, S, K, out)
