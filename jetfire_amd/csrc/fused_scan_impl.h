@@ -227,7 +227,7 @@ inline MergeParams merge_params(const FusedParams& p, bool first) {
 template <int NSET>
 struct K3Prep {
   int8_t aop[NSET][16][4][2][16];  // A operand bytes: [set][row = 4*head + limb][k-block][MFMA][byte]
-  int sq4[NSET * 4][2];            // 4 * sum of the fixed-point query over the scale group
+  int sq4[NSET * 4][2];            // code offset * sum of the fixed-point query over the scale group (WIDE_SUM: the sum)
   float qsc[NSET * 4][2];          // 2^(e-22) * attn_scale of the (head, group)
   float amax_w[NSET * 8];          // per 64-channel half row: |q| maximum, fixed-point sum, exponent
   int sum_w[NSET * 8];
@@ -546,6 +546,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   constexpr bool HAS_V = (MODE == FS_FULL || MODE == FS_STAGE_B);  // value stream and the P.V part of phase B
   constexpr bool HAS_TOPK = (MODE != FS_STAGE_B);                  // histograms and phase C
   constexpr bool K3 = Lds::K3, KLIMB = Lds::KLIMB, KA = Lds::KA, KB4 = Lds::KB4;
+  // INT4 keys over 128 channels in one group: their sums reach 128 * 2^22 * 8 = 2^32 and are put together in two parts
+  constexpr bool WIDE_SUM = KB4 && NG == 1;
   constexpr bool V2 = Lds::V2, V3 = Lds::V3;
   constexpr int NSET = Lds::NSET;
   constexpr int SEG = Lds::SEG;
@@ -819,7 +821,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       prep->aop[set][4 * hh + 2][kb][mi][by] = (int8_t)l2;
       prep->aop[set][4 * hh + 3][kb][mi][by] = 0;
     };
-    constexpr int CODE_OFF4 = KB4 ? 8 : (K3 ? 4 : 2);  // the codes are used unsigned: offset 8 (INT4), 4 (INT3) or 2 (INT2)
+    // the codes are used unsigned: offset 8 (INT4), 4 (INT3) or 2 (INT2); WIDE_SUM keeps the query's sum itself
+    constexpr int CODE_OFF4 = KB4 ? (WIDE_SUM ? 1 : 8) : (K3 ? 4 : 2);
     if constexpr (NG == 2) {
       // a wavefront's 64 elements are one scale group of one head: its statistics never leave the wavefront
 #pragma unroll
@@ -1075,7 +1078,13 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
 #pragma unroll
     for (int set = 0; set < NSET; ++set)
 #pragma unroll
-      for (int g = 0; g < NG; ++g) Cin[set][g] = (v4i){-sq4[set][g], 0, 0, 0};
+      for (int g = 0; g < NG; ++g) {
+        if constexpr (WIDE_SUM) {  // 8 sum(q) = 256 * (sum(q) >> 5) + 8 * (sum(q) & 31), the parts to two limbs
+          Cin[set][g] = (v4i){-8 * (sq4[set][g] & 31), -(sq4[set][g] >> 5), 0, 0};
+        } else {
+          Cin[set][g] = (v4i){-sq4[set][g], 0, 0, 0};
+        }
+      }
     auto body = [&](int chunk, const uint32_t (&Sx)[4], const uint32_t (&Zx)[4]) JF_INLINE {
       (void)Zx;
       // all LDS reads of the chunk first (plane dwords of the four pages, rounding coefficients), then arithmetic
@@ -1185,7 +1194,10 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
                 Dc = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][0], Bc[0], Cin[set][0], 0, 0, 0);
                 Dc = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aop[set][1], Bc[1], Dc, 0, 0, 0);
               }
-              acc_s[set][g] = (float)join_limbs(Dc[2], Dc[1], Dc[0]);
+              // (WIDE_SUM: the upper limbs' part is at most 2^24 in size and a whole number, so the one rounding is that of
+              // the sum, as where it fits 32 bits)
+              acc_s[set][g] = WIDE_SUM ? __builtin_fmaf((float)((Dc[2] << 8) + Dc[1]), 256.0f, (float)Dc[0])
+                                       : (float)join_limbs(Dc[2], Dc[1], Dc[0]);
             }
           v4i Bp[2], Bn[2];
           v4u rnd[NG];

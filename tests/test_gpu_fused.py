@@ -204,6 +204,32 @@ def test_fused_scan_on_degenerate_queries(scheme, G, Hkv, S, K, split_len, mode)
     check_against_oracle(scheme, c, S, K, out, atol_out=6e-6)
 
 
+@pytest.mark.parametrize("G,split_len", [(4, 256), (4, 2048), (8, 1024)])
+@pytest.mark.parametrize("scheme", ["b4v4_g128", "b4v2_g128", "b4v4", "b4v3", "k3v2_g128", "k2v2_g128", "a2v2_g128", "k3v2", "k4v4"])
+def test_fused_scan_on_flat_queries_and_extreme_codes(scheme, G, split_len):
+    """Queries whose channels all have one magnitude, with the largest mantissa among them, against rows that hold the
+    largest or the smallest code throughout: the largest sums the integer arithmetic of the scores can meet (128 channels
+    of 22 bits times codes of up to -8 go to 2^32)."""
+    from jetfire_amd import _lib
+    kb, vb, gs = SCHEME_GEOMETRY[scheme]
+    S, K = 1300, 64
+    c = make_case(616, 2, G, 1, S, kb, vb, gs, lens=[S, S - 37], extra_blocks=1, k_asym=scheme.startswith("a"))
+    # (bf16 values; the shared exponent makes the integers the same whatever the size, and at this one no few positions hold
+    # all of the softmax: N fixed-point weights of 2^-23 of the largest value scale are off by sqrt(N / 12) units in sum, which
+    # against a sum of weights of one would be 6e-6 for these sequences)
+    flat = np.resize(np.float32([1.9921875, -1.8984375, 1.0, -1.9921875, 1.25]), (2, G, 1)) / 1024
+    c["q"][...] = flat
+    rows = np.random.default_rng(5).permutation(c["kd"].shape[1])
+    c["kd"][:, rows[:100]], c["kd"][:, rows[100:200]] = 0xff, 0
+    d = to_device(c)
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
+    try:
+        out = [t.clone() for t in run_fused(scheme, c, d, S, K)]
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    check_against_oracle(scheme, c, S, K, out, atol_out=6e-6)
+
+
 @pytest.mark.parametrize("gs", (128, 64))
 def test_int2_single_call_names_of_the_reference(gs):
     """int2_fused_attn_topk and int2_fused_attn_topk_v1 (jetfire_vllm/csrc/int2_fused_attn_topk.cu:403-417,
