@@ -246,7 +246,9 @@ struct QInt8F {
 // LDS carve-up shared by the kernel and its launcher.
 //   sc     [G][L] fp32 scores of the split
 //   sbase  [L/16] first slot of every 16-position page
-//   aux    phase A: query constants (K3Prep / QInt8F); afterwards: selection histograms [G][SEG][256]
+//   aux    phase A: query constants (K3Prep / QInt8F) and the rounding tables of the bf16-model INT4 keys; afterwards:
+//          selection histograms [G][SEG][256].  With those keys it lies in front of sc instead of behind sbase, so that a
+//          look-up's address is the index plus a constant the instruction carries
 //   stage  one private staging area per wavefront: key rows in phase A, V rows + weight rows in phase B
 // After phase B the staging area holds the sum of the wavefronts' P.V accumulators.
 template <int SCHEME, int G, int NG>
@@ -296,7 +298,13 @@ struct ScanLds {
   // tighter) two 16-bit counters per word: a (head, segment) histogram counts at most LMAX / SEG <= 4096 positions
   static constexpr bool H16 = !(KLIMB && V2);
   static constexpr int HIST = G * SEG * 256 * (H16 ? 2 : 4);
-  static constexpr int AUX = ((PREP > HIST ? PREP : HIST) + 15) & ~15;
+  // Rounding tables: 128 entries of 16 bytes, then 128 of four.  In LDS of their own they cost the format the splits of 4096
+  // positions: 4 x 32768 positions, 8 kv-heads, G = 4, top-k 256, B4V4 in one group took 16 splits of 2048 instead of 8 and
+  // two rounds of workgroups, per layer 52.5 us, now 40.1 (B4V3 in 64-channel groups 55.5 / 42.4; 1 x 131072, top-k 512, B4V4
+  // in one group 62.5 / 48.0).
+  static constexpr int RND_AT = (PREP + 15) & ~15, RND = KB4 ? 128 * (16 + 4) : 0;
+  static constexpr int AUX = ((RND_AT + RND > HIST ? RND_AT + RND : HIST) + 15) & ~15;
+  static constexpr int SC_AT = KB4 ? AUX : 0;
   __host__ __device__ static constexpr int stage_bytes() { return NW * WAVE_STAGE; }
   static_assert(NW * WAVE_STAGE >= XACC + NW * 1024, "the staging area must hold the accumulator sums and the selection scratch");
   __host__ __device__ static constexpr size_t per_position() { return (size_t)G * 4; }
@@ -565,20 +573,21 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
 
   extern __shared__ __align__(16) uint8_t smem[];
   const int L = p.L;
-  float* sc = reinterpret_cast<float*>(smem);                     // [G][L]
-  int* sbase = reinterpret_cast<int*>(smem + (size_t)G * L * 4);  // [L/16] first slot of each page
-  uint8_t* aux = smem + Lds::aux_offset(L);
-  uint8_t* stage = aux + Lds::AUX;
+  float* sc = reinterpret_cast<float*>(smem + Lds::SC_AT);                     // [G][L]
+  int* sbase = reinterpret_cast<int*>(smem + Lds::SC_AT + (size_t)G * L * 4);  // [L/16] first slot of each page
+  uint8_t* aux = (Lds::SC_AT != 0) ? smem : smem + Lds::aux_offset(L);
+  uint8_t* stage = smem + Lds::aux_offset(L) + Lds::AUX;
   int* hist = reinterpret_cast<int*>(aux);  // [G][SEG][256], valid after phase A
   __shared__ float red_f[NW][2 * G];
   __shared__ uint32_t vmax_sh[NW][2];
   __shared__ float m_sh[G], bin_a_sh[G], bin_b_sh[G], lsum_sh[NW][G];
   __shared__ int e_sh[2];
-  // Rounding of bf16(c s) for s = 1 + m/128.  INT3: the coefficient 256 * (bf16(3 s) - 3 s) / s.  INT4 (bf16 model): what
-  // the roundings are multiples of, 256 / (128 s), and the byte tables they are looked up in (see phase A).
-  // Static, so that a look-up's address is the index plus a constant the instruction carries.
-  __shared__ float eps_sh[128];
-  __shared__ v4u rnd_sh[KB4 ? 128 : 1];
+  // Rounding of bf16(c s) for s = 1 + m/128.  INT3: the coefficient 256 * (bf16(3 s) - 3 s) / s.  INT4 (bf16 model): the
+  // byte tables the roundings are looked up in and what they are multiples of, 256 / (128 s) (see phase A).
+  // At a place known when this is compiled, so that a look-up's address is the index plus a constant the instruction carries.
+  __shared__ float eps_k3[K3 ? 128 : 1];
+  v4u* const rnd_sh = reinterpret_cast<v4u*>(smem + Lds::RND_AT);
+  float* const eps_sh = KB4 ? reinterpret_cast<float*>(smem + Lds::RND_AT + 128 * 16) : eps_k3;
   __shared__ unsigned long long tmax_sh;
   if (threadIdx.x == 0) tmax_sh = 0ull;
 
@@ -3397,7 +3406,7 @@ template <int SCHEME, int G, int NG>
 long lds_room_for() {
   using Lds = ScanLds<SCHEME, G, NG>;
   const size_t budget = (G <= 4 && Lds::NW == 8) ? LDS_BUDGET_2WG : LDS_BUDGET_1WG;
-  const size_t fixed = Lds::AUX + Lds::stage_bytes() + 64 + 832 + (Lds::KB4 ? 2560 : (Lds::K3 ? 512 : 0));  // + static LDS of the kernel (incl. the rounding tables)
+  const size_t fixed = Lds::AUX + Lds::stage_bytes() + 64 + 832 + (Lds::K3 ? 512 : 0);  // + static LDS of the kernel (INT3: incl. the rounding table)
   return (long)budget - (long)fixed;
 }
 
@@ -3570,6 +3579,12 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
   // positions, A2V2, G = 2, top-k 1024 in one split 28.9 us, in splits of 256 25.5; 4 x 1, 1262 positions, A2V4 24.4 / 22.6.
   // (With one group, or at 0.8, as many shapes lost as gained.)
   const double lone_split = scheme / 10 == 5 ? 0.8 : (scheme / 10 == 1 && NG == 2) ? 0.65 : 0.5;
+  // These keys, more than 256 winners, a sequence that two splits in the short form hold: one split for all of it takes that
+  // much longer against those than the figures say.  28 sequences x 4 kv-heads, 1361 positions, G = 4, B4V4 in 64-channel
+  // groups, top-k 512 in one split 32.2 us, in two of 768 30.0 (256 winners 26.9 / 26.5, 64 22.8 / 24.9).  Of 1600 random
+  // shapes 21 are cut otherwise, 20 of them for the better, by up to 20 %, one 1.3 % slower; charged whatever the number of
+  // winners a dozen lose 8 to 22 %.
+  const double lone_wide = (scheme / 10 == 5 && top_k > 256 && max_S <= 2 * 64 * nw) ? 3.5 : 0.0;
   int L = 256;
   double best = -1.0;
   for (int cand = 256; cand <= lmax; cand += 256) {
@@ -3583,7 +3598,7 @@ inline void fused_plan(int scheme, int NG, int B, int H_q, int H_kv, int max_S, 
     if (rem > 0) cost += kScanFixed + stream * (lone + (1.0 - lone) * (double)rem / kCUs);
     const int kc = (top_k + FS_CAND_SLACK) < cand ? (top_k + FS_CAND_SLACK) : cand;
     if (nsp == 1 && one_split_merges(FS_FULL, scheme, G, NG, B, H_q, H_kv, max_S, cand, top_k, kc))
-      cost += one_split_us(G, units, max_S, top_k);
+      cost += one_split_us(G, units, max_S, top_k) + (cand > 64 * nw ? lone_wide : 0.0);
     else
       cost += merge_us(rows, max_S, (int)nsp, kc, top_k);
     if (best < 0.0 || cost <= best) {

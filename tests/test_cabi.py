@@ -405,6 +405,22 @@ def test_fused_plan_geometry_is_consistent(scheme, gs, B, Hq, Hkv, S, K):
     assert out[0].value == L
 
 
+@pytest.mark.parametrize("scheme,gs,B,Hq,Hkv,S,K,split_len,n_splits", [
+    (54, 128, 4, 32, 8, 32768, 256, 4096, 8),     # one round of workgroups
+    (53, 64, 4, 32, 8, 32768, 256, 4096, 8), (53, 128, 4, 32, 8, 32768, 256, 4096, 8),
+    (54, 128, 1, 32, 8, 131072, 512, 4096, 32),
+    (54, 64, 28, 16, 4, 1361, 512, 768, 2), (54, 64, 24, 32, 8, 1361, 512, 1536, 1),
+])
+def test_plan_of_the_bf16_model_int4_keys(scheme, gs, B, Hq, Hkv, S, K, split_len, n_splits):
+    """Their rounding tables take no LDS from the longest splits; measured shapes on both sides of the line between one
+    split and two short ones."""
+    import ctypes as C
+    from jetfire_amd import _lib
+    out = [C.c_int() for _ in range(2)]
+    _lib.check(_lib.load().jf_fused_plan(scheme, gs, B, Hq, Hkv, S, K, *[C.byref(o) for o in out], None, None))
+    assert [o.value for o in out] == [split_len, n_splits]
+
+
 @pytest.mark.parametrize("stage,scheme,gs,B,Hq,Hkv,S,K,merges", [
     (0, 44, 128, 1, 32, 8, 777, 64, True),       # a chat turn
     (0, 32, 64, 32, 32, 8, 2048, 256, True),     # a full batch: a merge launch of 1024 rows
