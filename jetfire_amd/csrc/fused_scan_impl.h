@@ -2698,6 +2698,12 @@ constexpr int MG_LIGHT_THREADS = 256, MG_LIGHT_REGK = 16, MG_LIGHT_TOPK = 512;  
 // ranked all pairs at once, in every wavefront.  Six barriers instead of twelve.  Per layer, graph replay, before / now:
 // 1 x 4096 positions, K4V4, top-k 64 20.5 / 18.3 us; 4 x 8100, B4V4 30.3 / 28.9; 4 x 32768, K3V2 36.1 / 35.0;
 // the same with G = 8 33.4 / 32.3; 1 x 131072, K4V4, top-k 512 (two stages) 49.3 / 48.0.
+// Lane masks are short-lived: no comparison of the candidates is made twice in a form the compiler could recognise (an unused
+// slot's bucket lies behind all others instead of a second test of its key; the bounds of the second pass are opaque; counts
+// are taken at once).  Kept from one pass to the next the masks took 93 scalar registers in the first stage, which with the
+// trap handler's 16 leaves one workgroup per CU instead of two, and 190 spilled words in the shape of 32 candidates.  First
+// stage, 1024 / 1664 workgroups of 7000 candidates, top-k 1024 35.9 -> 22.5, 55.0 -> 33.7 us; 32-candidate shape, 16 / 512 /
+// 1376 rows 22.2 -> 15.6, 80.9 -> 67.6, 257 -> 223 us.
 // PARTIAL = true is the first stage of the two-stage merge: blockIdx.z selects a run of mg_spp candidate
 // lists, steps 2 and 3 run on those alone and the winners (still in position order) are written out as one
 // new candidate list; the final merge (PARTIAL = false, mg_parts > 1) reads these lists instead of the
@@ -2907,18 +2913,18 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) 
   };
   int bin[MG_REGK];
 #pragma unroll
-  for (int r = 0; r < MG_REGK; ++r) bin[r] = MG_BINS - 1;
+  for (int r = 0; r < MG_REGK; ++r) bin[r] = MG_BINS;  // (unused slots, behind all buckets: a winner's or a member's bin says it all)
   if constexpr (HAS_LISTS) {
     if (take_all) {
 #pragma unroll
-      for (int r = 0; r < MG_REGK; ++r) bin[r] = (kreg[r] != 0u) ? 0 : MG_BINS - 1;
+      for (int r = 0; r < MG_REGK; ++r) bin[r] = (kreg[r] != 0u) ? 0 : MG_BINS;
     } else if (!exact) {
 #pragma unroll
       for (int g = 0; g < NGRP; ++g)
         if (g == 0 || 4 * g < per) {
 #pragma unroll
           for (int r = 4 * g; r < 4 * g + 4; ++r) {
-            bin[r] = bin_of(kreg[r]);
+            bin[r] = (kreg[r] != 0u) ? bin_of(kreg[r]) : MG_BINS;
             if (bin[r] < MG_BINS - 1) atomicAdd(&hist[bin[r]], 1);
           }
         }
@@ -3021,7 +3027,7 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) 
 #pragma unroll
           for (int r = 4 * g; r < 4 * g + 4; ++r) {
             n_above += __popcll(__builtin_amdgcn_ballot_w64(bin[r] < cut));
-            const bool member = bin[r] == cut && kreg[r] != 0u;
+            const bool member = bin[r] == cut;
             if (__builtin_amdgcn_ballot_w64(member) != 0ull) {
               has_members = true;
               if (member) list_member(kreg[r], f_of(r));
@@ -3085,7 +3091,7 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) 
             const int r = 4 * g + j;
             win[j] = bin[r] < cut;
             if (has_members)  // (uniform)
-              win[j] = win[j] || (bin[r] == cut && kreg[r] != 0u && (kreg[r] > tk || (kreg[r] == tk && f_of(r) <= tf)));
+              win[j] = win[j] || (bin[r] == cut && (kreg[r] > tk || (kreg[r] == tk && f_of(r) <= tf)));
             mine += win[j] ? 1 : 0;
           }
           const int incl = wave_incl_scan_i(mine);
@@ -3168,14 +3174,20 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) 
         quota = K - ((tau == 0xffffffffu) ? 0 : count_ge(tau + 1u));
       }
       // ordered compaction: winners (key above tau) and ties of every wavefront, then its own, register by register
-      auto is_above = [&](uint32_t key) { return key != 0u && (take_all || key > tau); };
-      auto is_tie = [&](uint32_t key) { return key != 0u && !take_all && key == tau; };
+      // (unused slots have key 0: never above, and equal to tau only where every candidate wins, with a quota of none)
+      if (!take_all) tau = max(tau, 1u);
+      auto is_above = [&](uint32_t key) { return key > tau; };
+      auto is_tie = [&](uint32_t key) { return key == tau; };
       int na = 0, nt = 0;
 #pragma unroll
       for (int r = 0; r < MG_REGK; ++r) {
         na += __popcll(__builtin_amdgcn_ballot_w64(is_above(kreg[r])));
         nt += __popcll(__builtin_amdgcn_ballot_w64(is_tie(kreg[r])));
+        asm volatile("" : "+s"(na), "+s"(nt));  // (counted at once: all masks together do not fit the scalar registers)
       }
+      // (a bound the compiler takes for a new one: it would otherwise carry the lane masks of all these comparisons across the
+      // barrier, four scalar registers per candidate register)
+      asm volatile("" : "+v"(tau));
       lds_barrier();  // (wred_i has been read)
       if (lane == 0) {
         wred_i[wave] = na;
