@@ -3330,7 +3330,7 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) 
   const int g_of_lane = (NG == 1) ? 0 : ((dwi * CPD) / (D / NG));
   constexpr int UNR = Pre::UNR;  // 256 winners per pass
   // A workgroup of fewer than sixteen wavefronts takes several roles per wavefront, ROLES at a time: the rows of those are
-  // requested together.  All four at once: one gather latency instead of four, 105 - 126 registers and so four workgroups
+  // requested together.  All four at once: one gather latency instead of four, 101 - 125 registers and so four workgroups
   // of the light shape per CU; one at a time: 73, five workgroups, and no rows fetched for roles without winners.  Per
   // layer, one / four at a time: 16 sequences x 32 heads, 700 positions, K4V4, top-k 256 37.1 / 36.3 us; 32 x 64 heads of
   // 512, top-k 128 53.6 / 55.6; 22 x 128 heads of 39, INT4 with 64-channel groups, top-k 128 54.8 / 60.8.
@@ -3371,8 +3371,11 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) 
         }
     };
     for (int kb = (wave + r0 * MG_WAVES) * WPI; kb < n_out; kb += UNR * VWAVES * WPI) {
-      // (narrow corrections: no rows are fetched for winners there are none of)
-      if (UNR > 1 && n_out - (kb - (wave + r0 * MG_WAVES) * WPI) <= VWAVES * WPI) gather(kb, std::integral_constant<int, 1>{});
+      // (narrow corrections: no rows are fetched for winners there are none of.  Not with several roles at a time, where the
+      // second body costs INT2 and INT3 values 158 registers instead of 111 to 125, three workgroups per CU instead of four.
+      // Per layer, K3V2, top-k 256, three / four: 32 sequences x 32 heads, 8192 positions 73.0 / 68.0 us, 16 x 64 of 6000 62.3 /
+      // 55.4; K3V3 32 x 32 of 8192 80.4 / 75.3.)
+      if (ROLES == 1 && UNR > 1 && n_out - (kb - (wave + r0 * MG_WAVES) * WPI) <= VWAVES * WPI) gather(kb, std::integral_constant<int, 1>{});
       else gather(kb, std::integral_constant<int, UNR>{});
     }
 #pragma unroll

@@ -55,3 +55,9 @@ def test_merge_kernels_keep_their_lane_masks_out_of_vector_registers():
     went to vector lanes, 81 to 190 words of them."""
     ks = [k for n, k in _kernels().items() if "fused_merge_kernelI" in n]
     assert ks and max(k[".sgpr_spill_count"] for k in ks) < 16
+
+
+def test_light_merge_that_gathers_at_once_runs_four_workgroups_per_compute_unit():
+    """256 threads x 16 candidates, all four roles of a wavefront together: launched for up to four rows per unit."""
+    ks = [k for n, k in _kernels().items() if "fused_merge_kernelI" in n and "ELi256ELi16ELb0ELb0ELi4E" in n]
+    assert len(ks) == 6 and min(_workgroups_per_cu(k) for k in ks) == 4
