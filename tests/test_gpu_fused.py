@@ -149,8 +149,9 @@ def test_fused_scan_matches_oracle(scheme, B, Hq, Hkv, S, lens, K):
     ("k3v2", 3000, [3000], 64, 1024),      # longer than the planner would pick for this size
     ("k3v4", 10000, [9989], 256, 512), ("k4v2", 10000, [9000], 512, 768),      # two-stage merges of the mixed pairs
     ("k3v2", 20000, [19989], 2048, 512),   # every position a candidate, 40 lists: two-stage merge at the widest correction
-    ("k4v4", 40000, [39000], 2048, 0),     # the planner's own split: lists of 2304 entries, first stage beyond the registers
-    ("k3v2", 40000, [39990], 4096, 0),     # every position a candidate; two-stage merge whose parts exceed the registers
+    ("k4v4", 40000, [39000], 2048, 0),     # the planner's own split: 79 lists of 512, the first stage's parts beyond 8192 candidates
+    ("k4v4", 56000, [55000], 2048, 4096),  # lists of 2304 entries, four of them to a part, likewise
+    ("k3v2", 40000, [39990], 4096, 0),     # every position a candidate; two-stage merge in the wide shapes
     ("k4v4", 20000, [19000], 8192, 1024),  # single stage over every position, most candidates re-read from global memory
 ])
 def test_fused_scan_with_forced_split_length(scheme, S, lens, K, split_len):

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from tests.helpers import make_case, to_device
-from tests.test_gpu_fused import run_fused
+from tests.test_gpu_fused import check_against_oracle, run_fused
 
 pytestmark = pytest.mark.gpu
 
@@ -86,6 +86,71 @@ def test_winners_crowd_into_few_lists(B, split_len, order, K):
             n = min(K, S)
             want[:n] = np.sort(np.lexsort((np.arange(S), -scores[b, h, :S]))[:n])
             assert np.array_equal(idx[b, h], want), (b, h)
+
+
+@pytest.mark.parametrize("order", ["falling", "rising", "infinite", "nan"])
+@pytest.mark.parametrize("S,K,split_len,first,final", [
+    (20000, 64, 256, 1280, 1024),         # two stages, lists longer than the correction: each part bounded by its largest cut
+    (40000, 2048, 256, 10240, 8192),      # lists shorter than it (the smallest cut); parts of the 32-candidate shape
+    (40000, 2048, 2048, 10240, 8192),     # ... lists as long as it
+    (65536, 4096, 256, 16384, 16384),     # 256 lists; winners in dynamic LDS in both stages
+    (33100, 8192, 256, 0, 33280),         # one stage, 130 lists, candidates beyond the registers
+])
+def test_winners_crowd_into_few_lists_of_two_stages(S, K, split_len, first, final, order):
+    """The first stage hands the second a lower bound with every part's list, and the shapes of 32 candidates per thread look
+    up a winner's position when it is known: the same orders of scores as above, and scores that are NaN."""
+    import ctypes as C
+    from jetfire_amd import _lib
+    Hq, Hkv = 8, 1
+    c = make_case(97, 1, Hq, Hkv, S, 4, 4, 128, lens=[S])
+    d = to_device(c)
+    base = run_fused("k4v4", c, d, S, 32)
+    pos = torch.arange(S, device="cuda")
+    slot = d["bt"][0][pos // 16] * 16 + pos % 16
+    by_score = torch.argsort(base[7][0, 0], descending=order != "rising", stable=True)
+    d["kd"], d["ks"] = d["kd"].clone(), d["ks"].clone()
+    if order in ("infinite", "nan"):
+        d["ks"][:, slot[by_score[[700, S // 2]]]] = float("inf" if order == "infinite" else "nan")
+    else:
+        d["kd"][:, slot], d["ks"][:, slot] = d["kd"][:, slot[by_score]], d["ks"][:, slot[by_score]]
+    L, ns, cap, parts = [C.c_int() for _ in range(4)]
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
+    try:
+        _lib.check(_lib.load().jf_fused_plan(44, 128, 1, Hq, Hkv, S, K, *[C.byref(x) for x in (L, ns, cap, parts)]))
+        out = run_fused("k4v4", c, d, S, K)
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    if parts.value > 1:
+        assert (-(-ns.value // parts.value) * cap.value, parts.value * K) == (first, final)
+    else:
+        assert (0, ns.value * cap.value) == (first, final)
+    scores, idx, slots = out[7].cpu().numpy(), out[4].cpu().numpy(), out[1].cpu().numpy()
+    for h in range(Hq):
+        # the order of the kernels' keys: NaNs with the sign bit below everything, the others above
+        u = scores[0, h].view(np.uint32)
+        key = np.where(u >> 31, ~u, u | np.uint32(1 << 31)).astype(np.int64)
+        want = np.sort(np.lexsort((np.arange(S), -key))[:K])
+        assert np.array_equal(idx[0, h], want), h
+        assert np.array_equal(slots[0, h], slot.cpu().numpy()[want]), h
+
+
+@pytest.mark.parametrize("scheme,kb,vb,gs,S,K", [
+    ("k4v4", 4, 4, 128, 33100, 64),       # 130 splits, the third group of 64; two stages
+    ("k3v2", 3, 2, 64, 50000, 8192),      # 196 splits, the fourth; one stage
+    ("k3v2", 3, 2, 64, 65536, 256),       # 256 splits, the most there are
+])
+def test_up_to_256_splits_match_the_oracle(scheme, kb, vb, gs, S, K):
+    """The merge keeps the splits' statistics in the lanes, 64 splits at a time: all four groups of them, and sequences that
+    end in the third, the second and the first, behind which the splits are empty."""
+    from jetfire_amd import _lib
+    c = make_case(98, 4, 2, 1, S, kb, vb, gs, lens=[S, 129 * 256, 100 * 256 + 7, 300])
+    d = to_device(c)
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(256))
+    try:
+        out = [t.clone() for t in run_fused(scheme, c, d, S, K)]
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    check_against_oracle(scheme, c, S, K, out)
 
 
 def test_five_rows_of_the_light_shape_share_a_compute_unit():
