@@ -28,8 +28,9 @@
 //            scores per lane and block.  Heavily tied scores fall back to a radix select.
 //   sum of the wavefronts' integer accumulators with LDS integer atomics (issued along the emission's
 //   comparisons), exact int64 recombination -> partial o.
-// Launch 2, fused_merge_kernel, grid (B, H_q): selects the global top-k among the candidates (ties to
-// the lower position, ascending output), merges the split partials
+// Launch 2, fused_merge_kernel, grid (G, H_kv, B) (ahead of it, with many candidates per row, a first stage of it on grid
+// (B, H_q, parts)): selects the global top-k among the candidates (ties to the lower position, ascending output), merges
+// the split partials
 //   M = max m_i, l = sum l_i e^{m_i-M}, o_hat = sum o_i e^{m_i-M} / l
 // (the split-KV combine of jetfire_vllm/csrc/fused_decode_wmma.cu:1226-1253), and computes the
 // pre-correction terms o_old_unnorm, W over the winners (jetfire_vllm/csrc/int2_softmax_v.cu:738-788).
@@ -441,17 +442,25 @@ struct PreCorr {
   static constexpr int CPD = (VBITS == 3) ? 16 : 32 / VBITS;
   static constexpr int WPI = 64 / DW;
   static constexpr int UNR = (256 / (16 * WPI) > 0) ? 256 / (16 * WPI) : 1;
-  static __device__ inline void fetch(const uint8_t* vbase, uint32_t slot, int dwi, uint32_t& word, uint32_t& word_b) {
-    if constexpr (VBITS == 3) {  // bytes 2*dwi, 2*dwi+1 of every plane -> the 24-bit words of two 8-code groups
+  // INT3: all rows of a batch are requested before the first is used.  Left to itself the compiler requests a row or two and
+  // waits: 19 sequences x 16 heads over 4 kv-heads, 4955 positions, K4V3, top-k 512 38.4 us, 35.6 with this.  (The others' one
+  // load per row goes ahead anyway, and holding all of them costs registers: 28 x 32 heads over 4 kv-heads, 887 positions,
+  // INT4 in 64-channel groups, top-k 512 33.2 us, 37.0 with this.)
+  static constexpr bool ALL_AHEAD = VBITS == 3;
+  // what a lane requests of a row: its dword, or (INT3) bytes 2*dwi, 2*dwi+1 of every plane
+  struct Row {
+    uint32_t w[VBITS == 3 ? 3 : 1];
+  };
+  static __device__ inline Row fetch(const uint8_t* vbase, uint32_t slot, int dwi) {
+    Row x;
+    if constexpr (VBITS == 3) {
       const uint8_t* row = vbase + (size_t)(slot * (uint32_t)VP) + dwi * 2;
-      const uint32_t h0 = *reinterpret_cast<const uint16_t*>(row), h1 = *reinterpret_cast<const uint16_t*>(row + 16),
-                     h2 = *reinterpret_cast<const uint16_t*>(row + 32);
-      word = ((h0 & 0xffu) << 16) | ((h1 & 0xffu) << 8) | (h2 & 0xffu);
-      word_b = ((h0 >> 8) << 16) | ((h1 >> 8) << 8) | (h2 >> 8);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) x.w[i] = *reinterpret_cast<const uint16_t*>(row + 16 * i);
     } else {
-      word = *reinterpret_cast<const uint32_t*>(vbase + (size_t)(slot * (uint32_t)VP) + dwi * 4);
-      word_b = 0;
+      x.w[0] = *reinterpret_cast<const uint32_t*>(vbase + (size_t)(slot * (uint32_t)VP) + dwi * 4);
     }
+    return x;
   }
   // acc[c] += ws * (code c - offset).  Byte `byte` of the dword holds its codes MSB first; channel of code c in the
   // dword = dwi*CPD + c.  code - offset is the code with its top bit flipped, read as a two's complement field.  INT4
@@ -459,9 +468,13 @@ struct PreCorr {
   // sixteenth (INT2: a quarter) of its value; the factor, a power of two, sits in the weight, so every product is the
   // same number.  Two instructions per code; the bit-field extract, conversion and multiply-add of the INT3 words
   // take three, and with 256 winners for each of a workgroup's four heads the multiply-adds fill the vector ALU.
-  static __device__ inline void add(uint32_t word, uint32_t word_b, float ws, float (&acc)[CPD]) {
-    if constexpr (VBITS == 3) {
-      const uint32_t xa = word ^ 0x00924924u, xb = word_b ^ 0x00924924u;
+  static __device__ inline void add(const Row& row, float ws, float (&acc)[CPD]) {
+    const uint32_t word = row.w[0];
+    if constexpr (VBITS == 3) {  // the 24-bit words of two 8-code groups
+      const uint32_t h0 = row.w[0], h1 = row.w[1], h2 = row.w[2];
+      const uint32_t wa = ((h0 & 0xffu) << 16) | ((h1 & 0xffu) << 8) | (h2 & 0xffu);
+      const uint32_t wb = ((h0 >> 8) << 16) | ((h1 >> 8) << 8) | (h2 >> 8);
+      const uint32_t xa = wa ^ 0x00924924u, xb = wb ^ 0x00924924u;
 #pragma unroll
       for (int c = 0; c < CPD; ++c) {
         const int sh = 21 - 3 * (c & 7);
@@ -2573,34 +2586,45 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         float acc[Pre::CPD], accw = 0.f;
 #pragma unroll
         for (int c = 0; c < Pre::CPD; ++c) acc[c] = 0.f;
-        auto gather = [&](int first, auto count) {  // `count` rows per lane from winner `first` + part * WPI on
+        auto gather = [&](int first, auto count, auto all) JF_INLINE {  // `count` rows per lane (`all`: every one a winner) from winner `first` + part * WPI on
           constexpr int NU = decltype(count)::value;
-          uint32_t word[NU], word_b[NU];
+          typename Pre::Row row[NU];
           uint16_t sb[NU];
+          int slot[NU];
           float wv[NU];
+          // (all look-ups ahead of all rows: one round trip to LDS instead of one for each row's request)
 #pragma unroll
           for (int u = 0; u < NU; ++u) {
-            const int k = first + (u * WPH + part) * Pre::WPI + w_in, kc = h * K + min(k, n_out - 1);
-            const int slot = (k < n_out) ? tl_wslot[kc] : -1;
-            wv[u] = (slot >= 0) ? tl_ww[kc] : 0.f;
-            const uint32_t sl = (uint32_t)max(slot, 0);
-            Pre::fetch(vbase, sl, dwi, word[u], word_b[u]);
+            const int k = first + (u * WPH + part) * Pre::WPI + w_in, kc = h * K + (decltype(all)::value ? k : min(k, n_out - 1));
+            slot[u] = tl_wslot[kc];
+            wv[u] = tl_ww[kc];
+            if (!decltype(all)::value) slot[u] = (k < n_out) ? slot[u] : -1;
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int u = 0; u < NU; ++u) {
+            wv[u] = (slot[u] >= 0) ? wv[u] : 0.f;
+            const uint32_t sl = (uint32_t)max(slot[u], 0);
+            row[u] = Pre::fetch(vbase, sl, dwi);
             sb[u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
           }
+          if constexpr (Pre::ALL_AHEAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int u = 0; u < NU; ++u) {
-            Pre::add(word[u], word_b[u], wv[u] * bf16_to_f32(sb[u]), acc);
+            Pre::add(row[u], wv[u] * bf16_to_f32(sb[u]), acc);
             if (dwi == 0) accw += wv[u];
           }
         };
         // (as many rows as are left: a correction of 64 with four wavefronts per head is four INT4 rows per lane; sixteen,
         // twelve of them absent, took 9 k cycles at the end of a scan of 777 positions, four 3 k)
         constexpr int ROWS = WPH * Pre::WPI;  // winners per row of every lane
-        for (int first = 0; first < n_out; first += PB * ROWS) {
-          if (n_out - first <= PB / 4 * ROWS) gather(first, std::integral_constant<int, PB / 4>{});
-          else if (n_out - first <= PB / 2 * ROWS) gather(first, std::integral_constant<int, PB / 2>{});
-          else gather(first, std::integral_constant<int, PB>{});
+        int first = 0;
+        for (; n_out - first >= PB * ROWS; first += PB * ROWS) gather(first, std::integral_constant<int, PB>{}, std::true_type{});
+        while (n_out - first > PB / 4 * ROWS) {
+          gather(first, std::integral_constant<int, PB / 2>{}, std::false_type{});
+          first += PB / 2 * ROWS;
         }
+        if (n_out - first > 0) gather(first, std::integral_constant<int, PB / 4>{}, std::false_type{});
         const int chan = Pre::reduce(acc, lane);
         old_sh[hw * D + chan] = acc[0];
         old_sh[hw * D + chan + 1] = acc[1];
@@ -2710,7 +2734,7 @@ constexpr int MG_LIGHT_THREADS = 256, MG_LIGHT_REGK = 16, MG_LIGHT_TOPK = 512;  
 // scan's.  The top K of a union is the top K of the parts' top K's, ties included: a candidate that a part
 // drops is beaten by K candidates of that part.
 template <int MODE, int VBITS, int NG, int MG_THREADS, int MG_REGK, bool PARTIAL, bool WIDE = false, int ROLES = 1>
-__global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) {
+__global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void fused_merge_kernel(MergeParams p) {  // (wavefronts per SIMD: four workgroups of the gather for all roles)
   static_assert(!(PARTIAL && MODE == FS_STAGE_B), "Stage B alone selects nothing");
   constexpr int MG_WAVES = MG_THREADS / 64;
   using Pre = PreCorr<VBITS>;
@@ -3345,38 +3369,54 @@ __global__ __launch_bounds__(MG_THREADS) void fused_merge_kernel(MergeParams p) 
 #pragma unroll
       for (int c = 0; c < CPD; ++c) acc[r][c] = 0.f;
     }
-    auto gather = [&](int kb, auto count) {  // `count` rows per lane and role from winner kb on
+    auto gather = [&](int kb, auto count) JF_INLINE {  // `count` rows per lane and role from winner kb on
       constexpr int NU = decltype(count)::value;
-      uint32_t word[RP][NU], word_b[RP][NU];  // (word_b: INT3 only)
+      typename Pre::Row row[RP][NU];
       uint16_t sbits[RP][NU];
+      int slot[RP][NU];
       float wv[RP][NU];
+      // (all look-ups ahead of all rows: one round trip to LDS instead of one for each row's request)
 #pragma unroll
       for (int r = 0; r < RP; ++r)
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-          const int k = kb + (r * MG_WAVES + u * VWAVES) * WPI + w_in;
-          const int slot = (k < n_out) ? win_idx[k] : -1;
-          wv[r][u] = (slot >= 0) ? __builtin_bit_cast(float, win_key[k]) : 0.f;
-          const uint32_t sl = (uint32_t)max(slot, 0);
-          Pre::fetch(vbase, sl, dwi, word[r][u], word_b[r][u]);
+          const int k = kb + (r * MG_WAVES + u * VWAVES) * WPI + w_in, kc = min(k, n_out - 1);
+          const int named = win_idx[kc];
+          wv[r][u] = __builtin_bit_cast(float, win_key[kc]);
+          slot[r][u] = (k < n_out) ? named : -1;
+        }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < RP; ++r)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          wv[r][u] = (slot[r][u] >= 0) ? wv[r][u] : 0.f;
+          const uint32_t sl = (uint32_t)max(slot[r][u], 0);
+          row[r][u] = Pre::fetch(vbase, sl, dwi);
           sbits[r][u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
         }
+      if constexpr (Pre::ALL_AHEAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int r = 0; r < RP; ++r)
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
           const float ws = wv[r][u] * bf16_to_f32(sbits[r][u]);  // zero for padding rows
-          Pre::add(word[r][u], word_b[r][u], ws, acc[r]);
+          Pre::add(row[r][u], ws, acc[r]);
           if (dwi == 0) accw[r] += wv[r][u];
         }
     };
-    for (int kb = (wave + r0 * MG_WAVES) * WPI; kb < n_out; kb += UNR * VWAVES * WPI) {
-      // (narrow corrections: no rows are fetched for winners there are none of.  Not with several roles at a time, where the
-      // second body costs INT2 and INT3 values 158 registers instead of 111 to 125, three workgroups per CU instead of four.
-      // Per layer, K3V2, top-k 256, three / four: 32 sequences x 32 heads, 8192 positions 73.0 / 68.0 us, 16 x 64 of 6000 62.3 /
-      // 55.4; K3V3 32 x 32 of 8192 80.4 / 75.3.)
-      if (ROLES == 1 && UNR > 1 && n_out - (kb - (wave + r0 * MG_WAVES) * WPI) <= VWAVES * WPI) gather(kb, std::integral_constant<int, 1>{});
-      else gather(kb, std::integral_constant<int, UNR>{});
+    const int kb0 = (wave + r0 * MG_WAVES) * WPI;
+    if constexpr (ROLES == 1 && UNR > 1) {
+      // (narrow corrections, and the end of wide ones: no rows are fetched for winners there are none of.  Behind the loop: a
+      // choice between the two bodies inside it made 2048 winners' sums 25 to 35 % longer, 17.8 -> 24.5 k cycles.  Not with
+      // several roles at a time, where the second body costs INT2 and INT3 values 158 registers instead of 111 to 125, three
+      // workgroups per CU instead of four.  Per layer, K3V2, top-k 256, three / four: 32 sequences x 32 heads, 8192 positions
+      // 73.0 / 68.0 us, 16 x 64 of 6000 62.3 / 55.4; K3V3 32 x 32 of 8192 80.4 / 75.3.)
+      int done = 0;
+      for (; n_out - done > VWAVES * WPI; done += UNR * VWAVES * WPI) gather(kb0 + done, std::integral_constant<int, UNR>{});
+      if (kb0 + done < n_out) gather(kb0 + done, std::integral_constant<int, 1>{});
+    } else {
+      for (int kb = kb0; kb < n_out; kb += UNR * VWAVES * WPI) gather(kb, std::integral_constant<int, UNR>{});
     }
 #pragma unroll
     for (int r = 0; r < RP; ++r) {  // over the WPI winners of a wavefront instruction; then over the roles through LDS
