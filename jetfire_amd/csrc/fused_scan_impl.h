@@ -443,7 +443,7 @@ struct PreCorr {
   static constexpr int WPI = 64 / DW;
   static constexpr int UNR = (256 / (16 * WPI) > 0) ? 256 / (16 * WPI) : 1;
   // INT3: all rows of a batch are requested before the first is used.  Left to itself the compiler requests a row or two and
-  // waits: 19 sequences x 16 heads over 4 kv-heads, 4955 positions, K4V3, top-k 512 38.4 us, 35.6 with this.  (The others' one
+  // waits: 19 sequences x 16 heads over 4 kv-heads, 4955 positions, K4V3, top-k 512 38.4 us, 36.3 with this.  (The others' one
   // load per row goes ahead anyway, and holding all of them costs registers: 28 x 32 heads over 4 kv-heads, 887 positions,
   // INT4 in 64-channel groups, top-k 512 33.2 us, 37.0 with this.)
   static constexpr bool ALL_AHEAD = VBITS == 3;
@@ -2694,7 +2694,7 @@ __device__ inline void waves_prefix_i(const int* arr, int lane, int wave, int* b
 
 // ---------------------------------------------------------------------------------------------------
 constexpr int MG_MAX_SPLITS = 256;
-constexpr int MG_BINS = 512;       // linear score buckets of the threshold search; the last one holds all that lies below
+constexpr int MG_BINS = 512;       // linear score buckets of the threshold search (32 candidates per thread: twice as many); the last one holds all that lies below
 constexpr int MG_LIST = 1024;      // members of the cut bucket resolved by rank counting
 constexpr int MG_RANK = 16;        // up to here all pairs at once in every wavefront, beyond over the list in LDS
 constexpr int MG_BT_LDS = 4096;    // block-table entries cached in LDS (65536 positions)
@@ -2749,7 +2749,9 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
   // the light shape (many rows per launch, few candidates per row) trades table sizes for workgroups per CU
   constexpr int MG_BT = (MG_THREADS >= 1024) ? MG_BT_LDS : 1024;  // block-table entries cached in LDS
   constexpr int MG_WIN = (MG_THREADS >= 1024) ? FS_LDS_TOPK : 512;  // widest correction of this shape (WIDE: any)
-  __shared__ __align__(16) int hist[MG_BINS];
+  // (the shape of 32 candidates per thread meets wide corrections, whose cut lies where the scores are densest: twice the buckets)
+  constexpr int BINS = (MG_REGK > 16) ? 2 * MG_BINS : MG_BINS;
+  __shared__ __align__(16) int hist[BINS];
   __shared__ uint32_t lkey[MG_LIST];
   __shared__ int lpos[MG_RANK];  // candidate number of the first members
   __shared__ int bt_sh[MG_BT];
@@ -2873,7 +2875,7 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
   uint16_t blend_raw = 0;
   if constexpr (MODE == FS_FULL && !PARTIAL)  // (no blend: any readable address)
     blend_raw = *(p.blend_o_new ? p.blend_o_new + bh * D + (tid & (D - 1)) : reinterpret_cast<const uint16_t*>(ck));
-  for (int i = tid; i < MG_BINS; i += MG_THREADS) hist[i] = 0;
+  for (int i = tid; i < BINS; i += MG_THREADS) hist[i] = 0;
   if (tid == 0) lcount_sh = 0;
   lds_barrier();
 
@@ -2920,14 +2922,14 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
   }
   // (bucket 0 = largest scores; the last one, for what lies below `lo`, is not counted)
   const float range = hi - lo;
-  const float iw = ((float)MG_BINS - 1.5f) * __builtin_amdgcn_rcpf(range);
+  const float iw = ((float)BINS - 1.5f) * __builtin_amdgcn_rcpf(range);
   const float bb = hi * iw;
   // No usable range (all cuts at the largest score, infinite scores), or a NaN among the scores, whose place in the order
   // of the keys the buckets do not know (its split's sum of weights is a NaN too): bisection over the keys.
   const bool exact = !take_all && !(range > 0.f && isfinite(range) && isfinite(iw) && isfinite(bb) && lsum == lsum);  // (uniform)
   // (an unused slot's key 0 stands for a NaN, which the minimum turns into the last bucket)
   auto bin_of = [&](uint32_t k) -> int {
-    return (int)__builtin_fmaxf(__builtin_fminf(__builtin_fmaf(key_to_score(k), -iw, bb), (float)(MG_BINS - 1)), 0.f);
+    return (int)__builtin_fmaxf(__builtin_fminf(__builtin_fmaf(key_to_score(k), -iw, bb), (float)(BINS - 1)), 0.f);
   };
   // key of candidate f in pass-over-all-candidates loops: registers first, global memory beyond
   const int rounds = (flat + MG_THREADS - 1) / MG_THREADS;
@@ -2937,26 +2939,26 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
   };
   int bin[MG_REGK];
 #pragma unroll
-  for (int r = 0; r < MG_REGK; ++r) bin[r] = MG_BINS;  // (unused slots, behind all buckets: a winner's or a member's bin says it all)
+  for (int r = 0; r < MG_REGK; ++r) bin[r] = BINS;  // (unused slots, behind all buckets: a winner's or a member's bin says it all)
   if constexpr (HAS_LISTS) {
     if (take_all) {
 #pragma unroll
-      for (int r = 0; r < MG_REGK; ++r) bin[r] = (kreg[r] != 0u) ? 0 : MG_BINS;
+      for (int r = 0; r < MG_REGK; ++r) bin[r] = (kreg[r] != 0u) ? 0 : BINS;
     } else if (!exact) {
 #pragma unroll
       for (int g = 0; g < NGRP; ++g)
         if (g == 0 || 4 * g < per) {
 #pragma unroll
           for (int r = 4 * g; r < 4 * g + 4; ++r) {
-            bin[r] = (kreg[r] != 0u) ? bin_of(kreg[r]) : MG_BINS;
-            if (bin[r] < MG_BINS - 1) atomicAdd(&hist[bin[r]], 1);
+            bin[r] = (kreg[r] != 0u) ? bin_of(kreg[r]) : BINS;
+            if (bin[r] < BINS - 1) atomicAdd(&hist[bin[r]], 1);
           }
         }
       for (int r = MG_REGK; r < rounds; ++r) {
         const uint32_t k = key_of(r);
         if (k != 0u) {
           const int c = bin_of(k);
-          if (c < MG_BINS - 1) atomicAdd(&hist[c], 1);
+          if (c < BINS - 1) atomicAdd(&hist[c], 1);
         }
       }
     }
@@ -3011,7 +3013,7 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
     // list of that bucket's members
     int cut = 1, need = 0;  // (every candidate wins: they are in bucket 0)
     if (!take_all && !exact) {
-      constexpr int BPL = MG_BINS / 64;  // lane l owns buckets BPL * l .. (ascending bucket = descending score)
+      constexpr int BPL = BINS / 64;  // lane l owns buckets BPL * l .. (ascending bucket = descending score)
       static_assert(BPL % 4 == 0, "16-byte reads");
       int mine = 0;
 #pragma unroll
@@ -3021,7 +3023,7 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
       }
       const int incl = wave_incl_scan_i(mine);
       const unsigned long long who = __builtin_amdgcn_ballot_w64(incl >= K);
-      cut = MG_BINS - 1;
+      cut = BINS - 1;
       int above = __builtin_amdgcn_readlane(incl, 63);
       if (who != 0ull) {
         const int src = __ffsll((long long)who) - 1;
@@ -3283,11 +3285,26 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
   if (mclk && tid == 0) mclk[2] = JF_CLK();
   lds_barrier();
   if (mclk && tid == 0) mclk[3] = JF_CLK();
+  constexpr bool BATCHED = LAZY && HAS_LISTS && WIDE, LOOK_UP = LAZY && HAS_LISTS && !WIDE;
+  if constexpr (BATCHED) {
+    // the winners' positions, every thread those of the winners it goes on with, four requests in flight (one after the
+    // other, in the loops below, 8192 winners' slots and weights took 11.4 k cycles instead of 6.5 k; up to 2048 winners, two
+    // per thread, are quicker looked up there)
+    constexpr int PB = 4;
+    for (int r = tid; r < n_out; r += PB * MG_THREADS) {
+      int pos[PB];
+#pragma unroll
+      for (int u = 0; u < PB; ++u) pos[u] = buffer_i32(ri, win_idx[(r + u * MG_THREADS < n_out) ? r + u * MG_THREADS : r] * 4, 0);
+#pragma unroll
+      for (int u = 0; u < PB; ++u)
+        if (r + u * MG_THREADS < n_out) win_idx[r + u * MG_THREADS] = pos[u];
+    }
+  }
   if (PARTIAL) {  // the winners become one candidate list of the final merge
     const size_t at = (bh * p.mg_parts + part) * (size_t)K;
     for (int r = tid; r < K; r += MG_THREADS) {
       p.out_key[at + r] = (r < n_out) ? win_key[r] : 0u;  // unused slots: key 0
-      if (r < n_out) p.out_idx[at + r] = LAZY ? ci[win_idx[r]] : win_idx[r];
+      if (r < n_out) p.out_idx[at + r] = LOOK_UP ? ci[win_idx[r]] : win_idx[r];
     }
     if (tid == 0) p.out_edge[bh * p.mg_parts + part] = edge;
     return;
@@ -3312,7 +3329,7 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
     int wslot = -1;
     float ww = 0.f;
     if (r < n_out && win_idx[r] >= 0) {
-      position = (LAZY && HAS_LISTS) ? ci[win_idx[r]] : win_idx[r];
+      position = LOOK_UP ? ci[win_idx[r]] : win_idx[r];
       const int blk = (int)(position / BS);
       if (blk < p.max_blocks) slot = (int64_t)((blk < nblk_lds) ? (int64_t)bt_sh[blk] : bt[blk]) * BS + (position % BS);
       wslot = (slot >= 0 && slot < p.num_slots) ? (int)slot : -1;
