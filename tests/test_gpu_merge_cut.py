@@ -153,6 +153,27 @@ def test_up_to_256_splits_match_the_oracle(scheme, kb, vb, gs, S, K):
     check_against_oracle(scheme, c, S, K, out)
 
 
+@pytest.mark.parametrize("G,copies,split_len", [
+    (4, 1, 256), (8, 1, 256),     # a merge launch, 1024 threads
+    (8, 3, 256), (4, 12, 256),    # ... 256 threads, all roles at once and one at a time
+    (1, 1, 768), (4, 1, 768), (8, 1, 768),     # the scan that merges by itself: sixteen wavefronts per head to one
+])
+@pytest.mark.parametrize("scheme,kb,vb,gs", [("k3v2", 3, 2, 64), ("k3v3", 3, 3, 64), ("k4v4", 4, 4, 128), ("b4v4", 4, 4, 64)])
+def test_sums_over_the_winners_at_the_edges_of_their_batches(scheme, kb, vb, gs, G, copies, split_len):
+    """Value rows are gathered in full batches and a short one behind them: as many winners as positions, around every
+    multiple a batch can have."""
+    from jetfire_amd import _lib
+    lens = [1, 7, 9, 31, 33, 64, 65, 127, 129, 192, 255, 256, 257, 320, 383, 385, 449, 511, 512, 600] * copies
+    c = make_case(99, len(lens), G, 1, 600, kb, vb, gs, lens=lens)
+    d = to_device(c)
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
+    try:
+        out = [t.clone() for t in run_fused(scheme, c, d, 600, 512)]
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    check_against_oracle(scheme, c, 600, 512, out)
+
+
 def test_five_rows_of_the_light_shape_share_a_compute_unit():
     """What the light shape is for (many rows, few candidates each): its registers and LDS leave room for five
     workgroups per compute unit."""
