@@ -124,8 +124,8 @@ class JetFireInt4CacheStore:
     # ------------------------------------------------------------------ append
     def _prepare(self, key, value, slot_mapping):
         n = min(int(slot_mapping.numel()), int(key.shape[0]), int(value.shape[0]))
-        # (what needs no cut and no conversion is taken as it is: the views and conversions that would change nothing are
-        # half of a decode token's time on the host, 8 us)
+        # (what needs no cut and no conversion is taken as it is: the views and conversions that would change nothing took 3.5 us
+        # of a decode token's 17)
         dev = self.k_data.device
         if not (slot_mapping.shape == (n,) and slot_mapping.dtype is torch.long and slot_mapping.device == dev):
             slot_mapping = slot_mapping[:n].to(device=self.device, dtype=torch.long)
