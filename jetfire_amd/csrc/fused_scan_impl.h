@@ -3562,13 +3562,24 @@ inline double merge_pass_us(double fixed, long cands) {
   return cands <= MG_REG_CANDS ? fixed + kPerCand * (double)cands : fixed + 1.5 + kPerCandBig * (double)cands;
 }
 
+// One stage of the shape that keeps 32 candidates per thread, against two stages at the same split length, 36 shapes of 9472 to
+// 30720 candidates, 16 to 256 rows, per layer: up to 16384 candidates 1.5 - 9 us shorter, around 22000 as long, 2.4 us longer at
+// 30720 (rows 16; with 64 rows and more it is the shorter way throughout).  3 x 28076 positions, 8 kv-heads, G = 4, K3V2, top-k
+// 1024 (12800 candidates, 96 rows) 47.9 -> 42.4 us; 2 x 61876, K4V4, top-k 512 (12288, 64) 45.1 -> 42.6; 1 x 131072, K4V4, top-k
+// 512 (24576, 32) stays at two, 46.1 against 47.2.
+constexpr double kOneStageFixed = 11.6, kOneStagePerCand = 0.00032;
+inline double merge_one_stage_us(long cands) {
+  return cands > MG_REG_CANDS && cands <= 4 * MG_REG_CANDS ? kOneStageFixed + kOneStagePerCand * (double)cands
+                                                           : merge_pass_us(kMergeFixed, cands);
+}
+
 // Two-stage merge when one workgroup per row would face more than MG_REG_CANDS candidates: the number of
 // parts (at most MG_REG_CANDS / top_k, so that the final merge keeps its candidates in registers, and at least
 // two lists per part) with the smallest estimated time, which is returned.  parts == 1: single stage.
 inline double merge_plan(int rows, int ns, int kc, int top_k, int* parts_out, int* spp_out) {
   *parts_out = 1;
   *spp_out = ns;
-  double best = merge_pass_us(kMergeFixed, (long)ns * kc);
+  double best = merge_one_stage_us((long)ns * kc);
   if ((long long)ns * kc <= MG_REG_CANDS || ns < 4) return best;
   // (wide corrections run the 32-register shape throughout: its 32768 candidates bound the final merge)
   int cap = (top_k > FS_LDS_TOPK ? 4 * MG_REG_CANDS : MG_REG_CANDS) / top_k;
