@@ -316,12 +316,12 @@ struct ScanLds {
 };
 
 // LDS behind the staging area of a scan workgroup that holds the whole sequence and merges by itself (ONE): per head
-// the candidate positions, the members of the cut bucket, the winners' slots and weights, o_hat and a few words.
+// the members of the cut bucket, the winners' positions, slots and weights, o_hat and a few words.
 template <int G, int SEG>
 struct ScanTail {
   static constexpr int MEM = 64;  // members of the cut bucket that are selected from a list, one per lane
   static constexpr int RANK = 24;  // up to here against each other, beyond by bits
-  static constexpr int INTS = ((5 + SEG + 3) * G * 4 + 15) & ~15;
+  static constexpr int INTS = ((3 + SEG + 3) * G * 4 + 15) & ~15;
   __host__ __device__ static constexpr size_t bytes(int top_k, int kc) {
     return INTS + (size_t)G * (D * 4 + 8 * (size_t)top_k + 8 * MEM + 2 * (size_t)kc);
   }
@@ -1612,8 +1612,27 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   if constexpr (HAS_TOPK)
     if (!take_all)
       for (int i = tid; i < Lds::HIST / 4; i += NT) hist[i] = 0;
+  // ONE: what the in-kernel merge keeps behind the staging area (see ScanTail)
+  using Tail = ScanTail<G, SEG>;
+  const int Kcap = p.Kc;
+  [[maybe_unused]] const int K = p.top_k;
+  uint8_t* tail = stage + Lds::stage_bytes() + 64;
+  [[maybe_unused]] int* tl_put = reinterpret_cast<int*>(tail);              // [G] members put into the head's list
+  [[maybe_unused]] int* tl_mem = tl_put + G;                                // [G] members of the cut bucket
+  [[maybe_unused]] int* tl_nout = tl_mem + G;                               // [G] winners (Stage B); the selection's words
+  [[maybe_unused]] int* tl_segc = tl_nout + G;                              // [G][SEG] winners per wavefront
+  [[maybe_unused]] float* tl_m = reinterpret_cast<float*>(tl_segc + G * SEG);  // [G] softmax maximum, 1 / sum, e^{m - M}
+  [[maybe_unused]] float* tl_iz = tl_m + G;
+  [[maybe_unused]] float* tl_coef = tl_iz + G;
+  [[maybe_unused]] float* tl_ohat = reinterpret_cast<float*>(tail + Tail::INTS);          // [G][D]
+  [[maybe_unused]] int* tl_wslot = reinterpret_cast<int*>(tl_ohat + G * D);               // [G][top_k] paged slot of a winner
+  [[maybe_unused]] float* tl_ww = reinterpret_cast<float*>(tl_wslot + (size_t)G * K);     // [G][top_k] its softmax weight
+  // [G][MEM] members of the cut bucket, as rank words
+  [[maybe_unused]] unsigned long long* tl_mlist = reinterpret_cast<unsigned long long*>(tl_ww + (size_t)G * K);
+  [[maybe_unused]] uint16_t* tl_list = reinterpret_cast<uint16_t*>(tl_mlist + G * Tail::MEM);  // [G][Kcap] the winners' positions, ascending
   if (tid < G) {
     float m = red_f[0][tid], lo = red_f[0][G + tid];
+    if constexpr (ONE) tl_put[tid] = 0;
 #pragma unroll
     for (int w = 1; w < NW; ++w) {
       m = fmaxf(m, red_f[w][tid]);
@@ -1880,26 +1899,6 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // the constant row (75 * sum of codes) for l = 3.  Item j = (register i = j >> 2 of set i / AR, component j & 3)
   // lives at xacc[j * 64 + lane].
   int* xacc = reinterpret_cast<int*>(stage);
-  // ONE: what the in-kernel merge keeps behind the staging area (see ScanTail)
-  using Tail = ScanTail<G, SEG>;
-  const int Kcap = p.Kc;
-  [[maybe_unused]] const int K = p.top_k;
-  uint8_t* tail = stage + Lds::stage_bytes() + 64;
-  [[maybe_unused]] int* tl_cnt = reinterpret_cast<int*>(tail);              // [G] candidates of the head
-  [[maybe_unused]] int* tl_cut = tl_cnt + G;                                // [G] the cut bucket
-  [[maybe_unused]] int* tl_need = tl_cut + G;                               // [G] winners among the cut bucket's members; -1: every candidate wins
-  [[maybe_unused]] int* tl_mem = tl_need + G;                               // [G] members of the cut bucket
-  [[maybe_unused]] int* tl_nout = tl_mem + G;                               // [G] winners
-  [[maybe_unused]] int* tl_segc = tl_nout + G;                              // [G][SEG] winners per wavefront
-  [[maybe_unused]] float* tl_m = reinterpret_cast<float*>(tl_segc + G * SEG);  // [G] softmax maximum, 1 / sum, e^{m - M}
-  [[maybe_unused]] float* tl_iz = tl_m + G;
-  [[maybe_unused]] float* tl_coef = tl_iz + G;
-  [[maybe_unused]] float* tl_ohat = reinterpret_cast<float*>(tail + Tail::INTS);          // [G][D]
-  [[maybe_unused]] int* tl_wslot = reinterpret_cast<int*>(tl_ohat + G * D);               // [G][top_k] paged slot of a winner
-  [[maybe_unused]] float* tl_ww = reinterpret_cast<float*>(tl_wslot + (size_t)G * K);     // [G][top_k] its softmax weight
-  // [G][MEM] members of the cut bucket, as rank words
-  [[maybe_unused]] unsigned long long* tl_mlist = reinterpret_cast<unsigned long long*>(tl_ww + (size_t)G * K);
-  [[maybe_unused]] uint16_t* tl_list = reinterpret_cast<uint16_t*>(tl_mlist + G * Tail::MEM);  // [G][Kcap] candidate positions, ascending
   if constexpr (ONE) {
     if (tid < G) {
       float l = 0.f;
@@ -1911,7 +1910,6 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       tl_m[tid] = M;
       tl_coef[tid] = coef;
       tl_iz[tid] = (l > 0.f) ? 1.0f / l : 0.f;
-      tl_mem[tid] = 0;
     }
   }
   constexpr int ACC_TOTAL = NSET * AR, ACC_HALF = (ACC_TOTAL + 1) / 2;
@@ -1972,37 +1970,58 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // emitted, one wavefront per (head, segment of the split), each segment starting where the counts of the segments
   // before it end.  Otherwise (heavily tied scores) one wavefront falls back to an exact radix select over the keys.
   const int Kt = min(p.top_k, n);
-  for (int hs = wave; HAS_TOPK && hs < G * SEG; hs += NW) {
-    const int h = hs / SEG, seg = hs % SEG;
-    if (h >= GA) continue;
-    if (SHORT && !ONE && take_all) {
-      const float* srow = sc + h * L;
-      uint32_t* ck = p.cand_key + (part_base + (size_t)h * p.n_splits) * Kcap;
-      int32_t* ci = p.cand_idx + (part_base + (size_t)h * p.n_splits) * Kcap;
-      for (int t = (seg * 64 + lane) * 4; t < Kcap; t += SEG * 256) {  // (the list's length is a multiple of 4, at most L)
-        const v4f x = *reinterpret_cast<const v4f*>(srow + t);
-        v4u key;
-        v4i pos;
+  // Blocks of 1024 positions, 16 consecutive ones per lane: the lane's candidates are consecutive in the output,
+  // so a block costs one comparison per position, one wavefront scan of the lanes' counts, and a loop over the
+  // few set bits of every lane.  The lane reads its four 16-byte quads starting at quad (lane >> 2) & 3 (the
+  // four lanes that share a bank group then read different banks) and rotates its bit mask back afterwards.
+  const int rot4 = ((lane >> 2) & 3) * 4;
+  // -> bit i: position t0 + 16 * lane + i lies before `thr` in the buckets; ONE: `sure`, likewise before `thr_lo`
+  auto block_mask = [&](const float* lp, float ba, float bb, float thr, float thr_lo, int nvalid, auto acc_tag, uint32_t& sure) JF_INLINE -> uint32_t {
+    constexpr int ACCSEL = decltype(acc_tag)::value;  // accumulator sums issued along the comparisons: -1 none, 0 / 1 a half, 2 all
+    constexpr int A_LO = (ACCSEL == 1) ? ACC_HALF * 4 : 0;
+    constexpr int A_HI = (ACCSEL < 0) ? 0 : ((ACCSEL == 0) ? ACC_HALF * 4 : ACC_TOTAL * 4);
+    constexpr int PER = (A_HI - A_LO + 15) / 16;      // a few behind every comparison: the LDS queue never fills
+    v4f x[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          key[u] = (t + u < n) ? score_key(x[u]) : 0u;  // unused slots hold key 0
-          pos[u] = s0 + t + u;
+    for (int q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const v4f*>(lp + ((4 * q + rot4) & 15));
+    uint32_t ge = 0u, ge_lo = 0u;  // bit 4q + e set: element e of quad register q falls behind the cut (not emitted)
+#pragma unroll
+    for (int bi = 15; bi >= 0; --bi) {
+      // ge = 2 * ge + [value >= thr]: the comparison's lane mask is the carry of one add
+      const float v = __builtin_fmaf(x[bi >> 2][bi & 3], ba, bb);
+      const unsigned long long c = __builtin_amdgcn_ballot_w64(v >= thr);
+      // (the two wait states between a vector instruction's scalar result and a vector instruction that reads it
+      // are the compiler's job everywhere else; it does not look inside an asm statement)
+      asm("s_nop 1\n\tv_addc_co_u32_e64 %0, vcc, %1, %1, %2" : "=v"(ge) : "v"(ge), "s"(c) : "vcc");
+      if constexpr (ONE) {
+        const unsigned long long c_lo = __builtin_amdgcn_ballot_w64(v >= thr_lo);
+        asm("s_nop 1\n\tv_addc_co_u32_e64 %0, vcc, %1, %1, %2" : "=v"(ge_lo) : "v"(ge_lo), "s"(c_lo) : "vcc");
+      }
+      if constexpr (HAS_V && PER > 0) {
+        const int lo = A_LO + (15 - bi) * PER;
+        if (lo < A_HI) {
+          add_acc_range(lo, (lo + PER < A_HI) ? lo + PER : A_HI);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        *reinterpret_cast<v4u*>(ck + t) = key;
-        *reinterpret_cast<v4i*>(ci + t) = pos;
       }
-      if (seg == 0) {  // the smallest score
-        float lo = -red_f[lane & (NW - 1)][G + h];
-        JF_DPP_ROW_REDUCE(lo, op_fmax, float, -INFINITY);
-        if (lane == 15) p.cand_edge[part_base + (size_t)h * p.n_splits] = -lo;
-      }
-      continue;
     }
-    // Every wavefront of a head searches the cut itself (same histograms, same result): no exchange, no barrier
-    // between the search and the emission.
-    const float ba = uniform_f(bin_a_sh[h]);
-    float bb = uniform_f(bin_b_sh[h]);
-    asm volatile("" : "+v"(bb));  // (kept in a vector register: the multiply-add takes one scalar operand only)
+    // register bit b is position (b + rot4) mod 16 of the lane's run
+    auto in_order = [&](uint32_t m) -> uint32_t {
+      m = ~m & 0xffffu;
+      m |= m << 16;
+      return (m >> (16 - rot4)) & ((1u << nvalid) - 1u);
+    };
+    if constexpr (ONE) sure = in_order(ge_lo);
+    return in_order(ge);
+  };
+  // The cut of a head's histograms: the bucket, the positions up to and with it, those before it, and in the segments before
+  // `seg` those up to and with it and those before it.  Every wavefront of a head searches it for itself (same histograms, same
+  // result): no exchange, no barrier between the search and the emission.
+  struct Cut {
+    bool found;
+    int cut, tot, above_cut, before_me, before_above;
+  };
+  auto find_cut = [&](int h, int seg) JF_INLINE -> Cut {
     const int* h0 = hist + h * (SEG * 256) / (Lds::H16 ? 2 : 1);
     // lane l owns buckets 4l .. 4l+3 (ascending bucket = descending score) of every segment's histogram
     int cs[SEG][4], c[4], mine;
@@ -2041,14 +2060,13 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     // the first lane whose inclusive total reaches Kt holds the cut bucket; the rest is scalar arithmetic on that
     // lane's four counts
     const unsigned long long who = __ballot((incl & 0xffff) >= Kt);
-    bool ok = false;
-    int cut = 255, tot = 0, before_me = 0, above_cut = 0;
+    bool found = false;
+    int cut = 255, tot = 0, before_me = 0, above_cut = 0, before_above = 0;
     if (who != 0ull) {
       const int src = __ffsll((long long)who) - 1;
       const int ex = __builtin_amdgcn_readlane(incl - packed, src);  // exclusive sums at that lane
       int run = ex & 0xffff;
       before_me = ex >> 16;
-      bool found = false;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int cu = __builtin_amdgcn_readlane(c[u], src), mu = __builtin_amdgcn_readlane(cum[u], src);
@@ -2058,25 +2076,51 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           if (run >= Kt) {
             found = true;
             above_cut = run - cu;
+            before_above = before_me - mu;
             cut = 4 * src + u;
             tot = run;
           }
         }
       }
-      ok = tot <= Kcap;
     }
-    // A NaN falls into bucket 0, which says nothing about its place in the order of the keys, the order a merge launch
-    // goes by.  Nobody looks at the keys of the buckets before the cut here, so such a head takes the exact selection;
-    // its sum of weights is a NaN too (and where a score is +infinity or all are -infinity).
-    if constexpr (ONE) {
-      const float lw = lsum_sh[min(lane, NW - 1)][h];
-      ok = ok && __builtin_amdgcn_ballot_w64(lw != lw) == 0ull;
+    return {found, cut, tot, above_cut, before_me, before_above};
+  };
+  for (int hs = wave; HAS_TOPK && !ONE && hs < G * SEG; hs += NW) {
+    const int h = hs / SEG, seg = hs % SEG;
+    if (h >= GA) continue;
+    if (SHORT && take_all) {
+      const float* srow = sc + h * L;
+      uint32_t* ck = p.cand_key + (part_base + (size_t)h * p.n_splits) * Kcap;
+      int32_t* ci = p.cand_idx + (part_base + (size_t)h * p.n_splits) * Kcap;
+      for (int t = (seg * 64 + lane) * 4; t < Kcap; t += SEG * 256) {  // (the list's length is a multiple of 4, at most L)
+        const v4f x = *reinterpret_cast<const v4f*>(srow + t);
+        v4u key;
+        v4i pos;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          key[u] = (t + u < n) ? score_key(x[u]) : 0u;  // unused slots hold key 0
+          pos[u] = s0 + t + u;
+        }
+        *reinterpret_cast<v4u*>(ck + t) = key;
+        *reinterpret_cast<v4i*>(ci + t) = pos;
+      }
+      if (seg == 0) {  // the smallest score
+        float lo = -red_f[lane & (NW - 1)][G + h];
+        JF_DPP_ROW_REDUCE(lo, op_fmax, float, -INFINITY);
+        if (lane == 15) p.cand_edge[part_base + (size_t)h * p.n_splits] = -lo;
+      }
+      continue;
     }
+    const float ba = uniform_f(bin_a_sh[h]);
+    float bb = uniform_f(bin_b_sh[h]);
+    asm volatile("" : "+v"(bb));  // (kept in a vector register: the multiply-add takes one scalar operand only)
+    const Cut c = find_cut(h, seg);
+    const bool ok = c.found && c.tot <= Kcap;
+    const int cut = c.cut, tot = c.tot, before_me = c.before_me;
     if (clk && tid == 0) clk[6] = JF_CLK();
     const float* srow = sc + h * L;
     uint32_t* ck = p.cand_key + (part_base + (size_t)h * p.n_splits) * Kcap;
     int32_t* ci = p.cand_idx + (part_base + (size_t)h * p.n_splits) * Kcap;
-    uint16_t* cl = tl_list + h * Kcap;
     if (ok) {
       // bucket(s) <= cut  <=>  not (s * ba + bb >= cut + 1): the bucket is the floor of that value clamped to
       // [0, 255]; with cut = 255 every position qualifies
@@ -2088,52 +2132,12 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       // unused slots hold key 0 (no score maps to it); the planned total is known, so the head's wavefronts
       // share the padding and its stores leave before the emission's
       const int etot = min(Kcap, tot);
-      if constexpr (ONE) {
-        if (seg == 0 && lane == 0) {
-          tl_cnt[h] = etot;
-          tl_cut[h] = cut;
-          tl_need[h] = (etot == Kt) ? -1 : Kt - above_cut;
-        }
-      } else {
-        for (int i = etot + seg * 64 + lane; i < Kcap; i += SEG * 64) ck[i] = 0u;
-      }
-      // Blocks of 1024 positions, 16 consecutive ones per lane: the lane's candidates are consecutive in the output,
-      // so a block costs one comparison per position, one wavefront scan of the lanes' counts, and a loop over the
-      // few set bits of every lane.  The lane reads its four 16-byte quads starting at quad (lane >> 2) & 3 (the
-      // four lanes that share a bank group then read different banks) and rotates its bit mask back afterwards.
-      const int rot4 = ((lane >> 2) & 3) * 4;
+      for (int i = etot + seg * 64 + lane; i < Kcap; i += SEG * 64) ck[i] = 0u;
       auto emit_block = [&](int t0, auto acc_tag) JF_INLINE {
-        constexpr int ACCSEL = decltype(acc_tag)::value;  // accumulator sums issued along the comparisons: -1 none, 0 / 1 a half, 2 all
-        constexpr int A_LO = (ACCSEL == 1) ? ACC_HALF * 4 : 0;
-        constexpr int A_HI = (ACCSEL < 0) ? 0 : ((ACCSEL == 0) ? ACC_HALF * 4 : ACC_TOTAL * 4);
-        constexpr int PER = (A_HI - A_LO + 15) / 16;      // a few behind every comparison: the LDS queue never fills
         const int lt = t0 + 16 * lane;                    // first position of this lane
         const float* lp = srow + lt;
-        v4f x[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const v4f*>(lp + ((4 * q + rot4) & 15));
-        uint32_t ge = 0u;  // bit 4q + e set: element e of quad register q falls behind the cut (not emitted)
-#pragma unroll
-        for (int bi = 15; bi >= 0; --bi) {
-          // ge = 2 * ge + [value >= thr]: the comparison's lane mask is the carry of one add
-          const unsigned long long c = __builtin_amdgcn_ballot_w64(__builtin_fmaf(x[bi >> 2][bi & 3], ba, bb) >= thr);
-          // (the two wait states between a vector instruction's scalar result and a vector instruction that reads it
-          // are the compiler's job everywhere else; it does not look inside an asm statement)
-          asm("s_nop 1\n\tv_addc_co_u32_e64 %0, vcc, %1, %1, %2" : "=v"(ge) : "v"(ge), "s"(c) : "vcc");
-          if constexpr (HAS_V && PER > 0) {
-            const int lo = A_LO + (15 - bi) * PER;
-            if (lo < A_HI) {
-              add_acc_range(lo, (lo + PER < A_HI) ? lo + PER : A_HI);
-              __builtin_amdgcn_sched_barrier(0);
-            }
-          }
-        }
-        // register bit b is position (b + rot4) mod 16 of the lane's run
-        uint32_t m2 = ~ge & 0xffffu;
-        m2 |= m2 << 16;
-        uint32_t mask = (m2 >> (16 - rot4)) & 0xffffu;
-        const int nvalid = max(0, min(16, te - lt));
-        mask &= (1u << nvalid) - 1u;
+        uint32_t none;
+        uint32_t mask = block_mask(lp, ba, bb, thr, 0.f, max(0, min(16, te - lt)), acc_tag, none);
         const int mine = __popc(mask);
         const int incl = wave_incl_scan_i(mine);
         uint32_t o = (uint32_t)(count + incl - mine);
@@ -2147,12 +2151,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           const int i_next = (mask != 0u) ? __ffs((int)mask) - 1 : 0;
           const float s_next = lp[i_next];
           if (o < (uint32_t)Kcap) {  // the bound only matters for non-finite scores
-            if constexpr (ONE) {
-              cl[o] = (uint16_t)(lt + i);
-            } else {
-              ck[o] = score_key(sco);
-              ci[o] = s0 + lt + i;
-            }
+            ck[o] = score_key(sco);
+            ci[o] = s0 + lt + i;
           }
           ++o;
           i = i_next;
@@ -2180,12 +2180,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
             const uint32_t o = (uint32_t)(count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(em >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)em, 0u)));
             count += __popcll(em);
             if (emit && o < (uint32_t)Kcap) {  // the bound only matters for non-finite scores
-              if constexpr (ONE) {
-                cl[o] = (uint16_t)t;
-              } else {
-                ck[o] = score_key(x[i]);
-                ci[o] = s0 + t;
-              }
+              ck[o] = score_key(x[i]);
+              ci[o] = s0 + t;
             }
           }
         }
@@ -2204,7 +2200,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         acc_issued = true;
       }
       for (; t0 < te; t0 += 1024) emit_block(t0, plain);
-      if (!ONE && seg == SEG - 1) {
+      if (seg == SEG - 1) {
         // the lower edge of the cut bucket (a degenerate range: one bucket, the largest score)
         if (lane == 0) p.cand_edge[part_base + (size_t)h * p.n_splits] = (ba < 0.f) ? (bb - (float)(cut + 1)) * __builtin_amdgcn_rcpf(-ba) : m_sh[h];
         for (int i = count + lane; i < etot; i += 64) ck[i] = 0u;  // (only if a segment emitted less than planned)
@@ -2276,26 +2272,109 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         if (above || (tie && pt < quota)) {
           const int pos = pa + min(pt, quota);
           if (pos < Kcap) {
-            if constexpr (ONE) {
-              cl[pos] = (uint16_t)t;
-            } else {
-              ck[pos] = k;
-              ci[pos] = s0 + t;
-            }
+            ck[pos] = k;
+            ci[pos] = s0 + t;
           }
         }
         count += __popcll(ma);
         base_tie += __popcll(mt);
       }
       count += min(base_tie, quota);
-      if constexpr (ONE) {
-        if (lane == 0) {
-          tl_cnt[h] = min(Kcap, count);
-          tl_need[h] = -1;
+      if (lane == 0) p.cand_edge[part_base + (size_t)h * p.n_splits] = key_to_score(T);
+      for (int i = count + lane; i < Kcap; i += 64) ck[i] = 0u;
+    }
+  }
+  // ONE: the workgroup holds all scores, so the winners are marked where they stand.  The positions whose bucket lies before the
+  // cut bucket win; of the cut bucket's members the `need` largest (ties: the lowest positions).  A wavefront has the positions
+  // of its (head, segment) in two masks per lane and puts its members, a dozen per head, into the head's list; where the
+  // segments' winners go follows from the histograms and that list, so behind one barrier every wavefront finds the last
+  // winner and writes its own.  A list of candidates as the merge kernel takes it, gone over once for the members, once for the
+  // winners and once for their outputs with a barrier each, took longer, per layer: 1 x 777 positions, K4V4, top-k 64 15.1 us, now
+  // 14.1; 20 x 1000, K3V2, 128 17.9 / 17.2; 32 x 1900, K3V2, 512 29.5 / 28.8; 32 x 2048, K4V4, 256 26.8 / 26.6.
+  // (rank word: key over inverted position, 32 + 12 bits, so that the larger word is the earlier winner)
+  constexpr int NHS = (G * SEG + NW - 1) / NW;  // (head, segment) pairs per wavefront
+  static_assert(Lds::LMAX <= 4096 && Lds::LMAX / SEG <= 2048, "a position takes twelve bits, a lane's share of a segment 32");
+  constexpr int STEPS = SHORT ? NT / SEG / 64 : 1;
+  static_assert(!SHORT || STEPS <= 32, "one bit a step");
+  [[maybe_unused]] uint32_t sure[NHS], memb[NHS];  // SHORT: bit i is position 64 i + lane of the segment; else 1024 (i / 16) + 16 lane + i % 16
+  [[maybe_unused]] int need[NHS], members[NHS], before[NHS];  // winners among the head's members, members, sure winners in the segments before
+  [[maybe_unused]] auto rank_word = [](uint32_t key, int pos) { return ((unsigned long long)key << 12) | (uint32_t)(4095 - pos); };
+  [[maybe_unused]] auto place_of = [&](int i) -> int { return SHORT ? 64 * i + lane : (i >> 4) * 1024 + 16 * lane + (i & 15); };
+  if constexpr (ONE && HAS_TOPK) {
+#pragma unroll
+    for (int it = 0; it < NHS; ++it) {
+      const int hs = wave + it * NW, h = hs / SEG, seg = hs % SEG;
+      sure[it] = memb[it] = 0u;
+      need[it] = members[it] = before[it] = 0;
+      if (hs >= G * SEG || h >= GA) continue;
+      const float ba = uniform_f(bin_a_sh[h]);
+      float bb = uniform_f(bin_b_sh[h]);
+      asm volatile("" : "+v"(bb));
+      const Cut c = find_cut(h, seg);
+      const float lw = lsum_sh[min(lane, NW - 1)][h];
+      if (clk && tid == 0) clk[6] = JF_CLK();
+      const bool all = Kt == n;  // every position wins
+      // No range to cut into buckets, or a NaN among the scores (its sum of weights is one too), whose place in the order of the
+      // keys the buckets do not know: all positions are members.
+      const bool exact = !all && (!c.found || !(ba < 0.f) || __builtin_amdgcn_ballot_w64(lw != lw) != 0ull);
+      const int tb = seg * (L / SEG), te = min(n, tb + L / SEG);
+      need[it] = all ? 0 : (exact ? Kt : Kt - c.above_cut);
+      members[it] = all ? 0 : (exact ? n : c.tot - c.above_cut);
+      before[it] = all ? tb : (exact ? 0 : c.before_above);
+      // bucket(s) <= cut  <=>  not (s * ba + bb >= cut + 1): the bucket is the floor of that value clamped to [0, 255]
+      const float thr = uniform_f((all || exact || c.cut >= 255) ? INFINITY : (float)(c.cut + 1));
+      const float thr_lo = uniform_f((c.cut == 0) ? -INFINITY : (float)c.cut);
+      const float* srow = sc + h * L;
+      uint32_t upto = 0u, lower = 0u;
+      if constexpr (SHORT) {
+        float x[STEPS];
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) x[i] = srow[min(tb + 64 * i + lane, L - 1)];
+        if (HAS_V && !acc_issued) {
+          add_acc_range(0, ACC_TOTAL * 4);
+          acc_issued = true;
+        }
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+          const float v = __builtin_fmaf(x[i], ba, bb);
+          const bool in = tb + 64 * i + lane < te;
+          upto |= (in && !(v >= thr) ? 1u : 0u) << i;
+          lower |= (in && !(v >= thr_lo) ? 1u : 0u) << i;
         }
       } else {
-        if (lane == 0) p.cand_edge[part_base + (size_t)h * p.n_splits] = key_to_score(T);
-        for (int i = count + lane; i < Kcap; i += 64) ck[i] = 0u;
+        auto block = [&](int t0, auto acc_tag) JF_INLINE {
+          const int lt = t0 + 16 * lane;
+          uint32_t lo;
+          const uint32_t m = block_mask(srow + lt, ba, bb, thr, thr_lo, max(0, min(16, te - lt)), acc_tag, lo);
+          const int at = (t0 > tb) ? 16 : 0;
+          upto |= m << at;
+          lower |= lo << at;
+        };
+        constexpr std::integral_constant<int, -1> plain{};
+        if (HAS_V && !acc_issued && te > tb) {
+          if (te - tb > 1024) {
+            block(tb, std::integral_constant<int, 0>{});
+            block(tb + 1024, std::integral_constant<int, 1>{});
+          } else {
+            block(tb, std::integral_constant<int, 2>{});
+          }
+          acc_issued = true;
+        } else {
+          if (te > tb) block(tb, plain);
+          if (te > tb + 1024) block(tb + 1024, plain);
+        }
+      }
+      sure[it] = all ? upto : (exact ? 0u : upto & lower);
+      memb[it] = all ? 0u : upto & ~sure[it];
+      if (seg == 0 && lane == 0) tl_mem[h] = members[it];
+      if (members[it] <= Tail::MEM) {  // (uniform)
+        uint32_t m = memb[it];
+        while (m != 0u) {
+          const int pos = tb + place_of(__ffs((int)m) - 1);
+          m &= m - 1u;
+          const int k = atomicAdd(&tl_put[h], 1);
+          if (k < Tail::MEM) tl_mlist[h * Tail::MEM + k] = rank_word(score_key(srow[pos]), pos);
+        }
       }
     }
   }
@@ -2314,88 +2393,67 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
 #pragma unroll
       for (int set = 0; set < NSET; ++set) combine(set);
     }
-    constexpr int NHS = (G * SEG + NW - 1) / NW;  // (head, segment) pairs per wavefront
-    if constexpr (HAS_TOPK) {
-      // The candidates whose bucket lies before the cut bucket win; of the cut bucket's members the `need` largest
-      // (ties: the lowest positions).  A wavefront takes a contiguous run of its head's list.
-      // (rank word: key over inverted position, 32 + 12 bits, so that the larger word is the earlier winner)
-      static_assert(Lds::LMAX <= 4096, "a position takes twelve bits");
-      auto rank_word = [](uint32_t key, int pos) { return ((unsigned long long)key << 12) | (uint32_t)(4095 - pos); };
-      auto pair_of = [&](int it, int& h, int& lo, int& hi) -> int {  // -> segment, -1: nothing for this wavefront
-        const int hs = wave + it * NW;
-        h = hs / SEG;
-        if (hs >= G * SEG || h >= GA) return -1;
-        const int cnt = __builtin_amdgcn_readfirstlane(tl_cnt[h]);
-        const int run = (cnt + SEG * 64 - 1) / (SEG * 64) * 64;
-        lo = (hs % SEG) * run;
-        hi = min(cnt, lo + run);
-        return hs % SEG;
-      };
+    // what the blend takes is requested here; behind the last barrier its first touch was waited for (20 x 1000 positions, K3V2,
+    // top-k 128 18.2 us per layer, 17.9 with this; 32 x 2048, K4V4, 256 27.0 / 26.75)
+    constexpr int OPT = (G * D + NT - 1) / NT;  // outputs per thread
+    [[maybe_unused]] uint16_t o_new[OPT];
+    if constexpr (MODE == FS_FULL) {
 #pragma unroll
-      for (int it = 0; it < NHS; ++it) {
-        int h, lo, hi;
-        if (pair_of(it, h, lo, hi) < 0 || tl_need[h] < 0) continue;
-        const int cut = tl_cut[h];
-        const float ba = bin_a_sh[h], bb = bin_b_sh[h], thr = (float)cut;
-        for (int i = lo + lane; i < hi; i += 64) {
-          const int pos = min((int)tl_list[h * Kcap + i], n - 1);
-          const float s = sc[h * L + pos];
-          // (bucket 0: also the degenerate ranges, whose buckets say nothing about the order)
-          if (cut == 0 || __builtin_fmaf(s, ba, bb) >= thr) {
-            const int k = atomicAdd(&tl_mem[h], 1);
-            if (k < Tail::MEM) tl_mlist[h * Tail::MEM + k] = rank_word(score_key(s), pos);
-            tl_list[h * Kcap + i] = (uint16_t)(pos | 0x8000);  // (positions are below 4096)
-          }
-        }
-      }
-      lds_barrier();
+      for (int it = 0; it < OPT; ++it)  // (no blend: any readable address)
+        o_new[it] = *(p.blend_o_new ? p.blend_o_new + head0 * D + min(it * NT + tid, GA * D - 1) : p.q + head0 * D);
+    }
+    if constexpr (HAS_TOPK) {
       // More members than a rank list holds: the buckets are linear between the smallest and the largest score, so one
       // outlying score (an attention sink) makes them wide, a correction of thousands puts hundreds of positions in
       // one, and equal scores share one.  Radix select over the rank words, eight bits a pass from the highest bit in
-      // which a head's members differ: the head's wavefronts count the digits of their runs, each finds the digit of
+      // which a head's members differ: the head's wavefronts count the digits of their members, each finds the digit of
       // the last winner, and the head is done when the members left are as many as the winners left.  At most six
       // passes (the words are distinct), two or three where scores differ.  Ranking each such member against the whole
       // list, as this did at first, took 67 us per layer for 32 sequences x 2048 positions, K3V2, 8 kv-heads, top-k 256
       // and one score at 40 sigma (this: 29.5, no outlier: 24.9, splits of 256 with a merge launch: 103), and 1055 us
       // for 16 x 3900, K2V2, one head per kv-head, top-k 2048 and no outlier at all (31.6; 81).
       unsigned long long last[NHS] = {};  // the last winner among the head's members
-      // (the same in every wavefront; this wavefront's heads are read along)
-      const int any_need = tl_need[min(lane, G - 1)], any_mem = tl_mem[min(lane, G - 1)];
-      int need_of[NHS], mem_of[NHS];
-#pragma unroll
-      for (int it = 0; it < NHS; ++it) {
-        const int h = min((wave + it * NW) / SEG, G - 1);
-        need_of[it] = tl_need[h];
-        mem_of[it] = tl_mem[h];
-      }
-      const unsigned long long crowded = __builtin_amdgcn_ballot_w64(lane < GA && any_need >= 0 && any_mem > Tail::MEM);
+      int ahead[NHS] = {};                // members that win in the segments before
+      auto pair_of = [&](int it, int& h, int& seg) -> bool {  // (false: nothing for this wavefront)
+        const int hs = wave + it * NW;
+        h = hs / SEG;
+        seg = hs % SEG;
+        return hs < G * SEG && h < GA;
+      };
+      const int any_mem = tl_mem[min(lane, G - 1)];  // (the same in every wavefront)
+      const unsigned long long crowded = __builtin_amdgcn_ballot_w64(lane < GA && any_mem > Tail::MEM);
       if (__builtin_expect(crowded != 0ull, 0)) {
-        // (the staging area is dead since `combine`) per head the digit counts, the smallest and the largest member's key
+        if constexpr (HAS_V) lds_barrier();  // (the sums in the staging area have been read)
+        // per head the digit counts, the smallest and the largest member's key
         int* rh = reinterpret_cast<int*>(stage);
         uint32_t* ends = reinterpret_cast<uint32_t*>(rh + G * 256);
         static_assert(NW * Lds::WAVE_STAGE >= G * (256 * 4 + 8), "the digit counts lie in the staging area");
-        auto for_members = [&](int h, int lo, int hi, auto&& f) {  // four list entries per lane in flight
-          for (int i0 = lo + lane; i0 - lane < hi; i0 += 256) {
-            uint32_t e[4];
-            float sv[4];
+        auto for_members = [&](int it, int h, int seg, auto&& f) {  // four scores per lane in flight
+          const int tb = seg * (L / SEG);
+          const float* srow = sc + h * L;
+          for (int i0 = 0; i0 < (SHORT ? STEPS : 32); i0 += 4) {
+            float x[4];
+            int pos[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) e[u] = (i0 + 64 * u < hi) ? tl_list[h * Kcap + i0 + 64 * u] : 0u;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) sv[u] = sc[h * L + min((int)(e[u] & 0x7fffu), n - 1)];
+            for (int u = 0; u < 4; ++u) {
+              pos[u] = min(tb + place_of(i0 + u), n - 1);
+              x[u] = srow[pos[u]];
+            }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-              if (e[u] & 0x8000u) f(rank_word(score_key(sv[u]), min((int)(e[u] & 0x7fffu), n - 1)));
+              if ((memb[it] >> (i0 + u)) & 1u) f(i0 + u, rank_word(score_key(x[u]), pos[u]));
           }
         };
         for (int i = tid; i < G * 256; i += NT) rh[i] = 0;
         if (tid < 2 * G) ends[tid] = (tid & 1) ? 0u : 0xffffffffu;
+        if (tid < G) tl_nout[tid] = 0;
         lds_barrier();
 #pragma unroll
         for (int it = 0; it < NHS; ++it) {
-          int h, lo, hi;
-          if (pair_of(it, h, lo, hi) < 0 || !((crowded >> h) & 1ull)) continue;
+          int h, seg;
+          if (!pair_of(it, h, seg) || !((crowded >> h) & 1ull)) continue;
           uint32_t kmin = 0xffffffffu, kmax = 0u;
-          for_members(h, lo, hi, [&](unsigned long long w) { kmin = min(kmin, (uint32_t)(w >> 12)); kmax = max(kmax, (uint32_t)(w >> 12)); });
+          for_members(it, h, seg, [&](int, unsigned long long w) { kmin = min(kmin, (uint32_t)(w >> 12)); kmax = max(kmax, (uint32_t)(w >> 12)); });
           kmin = wave_min_u(kmin);
           kmax = wave_max_u(kmax);
           if (lane == 0) {
@@ -2404,47 +2462,46 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           }
         }
         lds_barrier();
-        int bits[NHS], need[NHS], left[NHS];
+        int bits[NHS], want[NHS], left[NHS];
         unsigned long long top[NHS];  // members in the running have these bits above the lowest `bits` ones
 #pragma unroll
         for (int it = 0; it < NHS; ++it) {
-          int h, lo, hi;
-          bits[it] = need[it] = left[it] = 0;
+          int h, seg;
+          bits[it] = want[it] = left[it] = 0;
           top[it] = 0ull;
-          if (pair_of(it, h, lo, hi) < 0 || !((crowded >> h) & 1ull)) continue;
+          if (!pair_of(it, h, seg) || !((crowded >> h) & 1ull)) continue;
           const uint32_t kmin = __builtin_amdgcn_readfirstlane(ends[2 * h]), kmax = __builtin_amdgcn_readfirstlane(ends[2 * h + 1]);
           bits[it] = 12 + ((kmin == kmax) ? 0 : 32 - __clz((int)(kmin ^ kmax)));
           top[it] = rank_word(kmax, 0) >> bits[it];
-          need[it] = __builtin_amdgcn_readfirstlane(need_of[it]);
-          left[it] = __builtin_amdgcn_readfirstlane(mem_of[it]);
+          want[it] = need[it];
+          left[it] = members[it];
         }
         for (int pass = 0; pass < 6; ++pass) {
 #pragma unroll
           for (int it = 0; it < NHS; ++it) {
-            int h, lo, hi;
-            if (pair_of(it, h, lo, hi) < 0 || left[it] == need[it]) continue;
+            int h, seg;
+            if (!pair_of(it, h, seg) || left[it] == want[it]) continue;
             const int shift = max(0, bits[it] - 8);
-            for_members(h, lo, hi, [&](unsigned long long w) {
+            for_members(it, h, seg, [&](int, unsigned long long w) {
               if ((w >> bits[it]) == top[it]) atomicAdd(&rh[h * 256 + (int)((w >> shift) & ((1u << (bits[it] - shift)) - 1u))], 1);
             });
           }
           lds_barrier();
 #pragma unroll
           for (int it = 0; it < NHS; ++it) {
-            int h, lo, hi;
-            const int seg = pair_of(it, h, lo, hi);
-            if (seg < 0) continue;
-            if (left[it] != need[it]) {
+            int h, seg;
+            if (!pair_of(it, h, seg)) continue;
+            if (left[it] != want[it]) {
               // lane l owns the digits 255 - 4l .. 252 - 4l: a scan over the lanes counts from the largest digit down
               const v4i c = *reinterpret_cast<const v4i*>(rh + h * 256 + 252 - 4 * lane);
               const int mine = (c[0] + c[1]) + (c[2] + c[3]);
-              int above = wave_incl_scan_i(mine) - mine, digit = -1, count = 0, before = 0;
+              int above = wave_incl_scan_i(mine) - mine, digit = -1, count = 0, less = 0;
 #pragma unroll
               for (int u = 3; u >= 0; --u) {
-                if (above < need[it] && need[it] <= above + c[u]) {
+                if (above < want[it] && want[it] <= above + c[u]) {
                   digit = 252 - 4 * lane + u;
                   count = c[u];
-                  before = above;
+                  less = above;
                 }
                 above += c[u];
               }
@@ -2452,32 +2509,46 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
               const int src = (who != 0ull) ? __ffsll((long long)who) - 1 : 0;
               const int shift = max(0, bits[it] - 8);
               top[it] = (top[it] << (bits[it] - shift)) | (uint32_t)__builtin_amdgcn_readlane(digit, src);
-              need[it] -= __builtin_amdgcn_readlane(before, src);
+              want[it] -= __builtin_amdgcn_readlane(less, src);
               left[it] = __builtin_amdgcn_readlane(count, src);
               bits[it] = shift;
             }
-            if (seg == 0 && lane == 0) tl_nout[h] = left[it] - need[it];  // (free until the winners are counted)
+            if (seg == 0 && lane == 0) tl_nout[h] = left[it] - want[it];
           }
           lds_barrier();
           if (__builtin_amdgcn_ballot_w64(lane < GA && tl_nout[min(lane, G - 1)] != 0) == 0ull) break;
           for (int i = tid; i < G * 256; i += NT) rh[i] = 0;
           lds_barrier();
         }
+        // the members that win join the sure winners; how many every segment has goes through LDS
 #pragma unroll
-        for (int it = 0; it < NHS; ++it) last[it] = top[it] << bits[it];
+        for (int it = 0; it < NHS; ++it) {
+          int h, seg;
+          if (!pair_of(it, h, seg) || !((crowded >> h) & 1ull)) continue;
+          last[it] = top[it] << bits[it];
+          const uint32_t alone = sure[it];
+          for_members(it, h, seg, [&](int i, unsigned long long w) { sure[it] |= (w >= last[it] ? 1u : 0u) << i; });
+          const int won = wave_sum_i(__popc(sure[it]) - __popc(alone));
+          if (lane == 0) tl_segc[h * SEG + seg] = won;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int it = 0; it < NHS; ++it) {
+          int h, seg;
+          if (!pair_of(it, h, seg) || !((crowded >> h) & 1ull)) continue;
+#pragma unroll
+          for (int sg = 0; sg < SEG; ++sg) ahead[it] += (sg < seg) ? tl_segc[h * SEG + sg] : 0;
+        }
       }
-      uint32_t wmask[NHS];  // bit j: this lane's candidate of step j wins (at most 32 steps: one_split_fits)
 #pragma unroll
       for (int it = 0; it < NHS; ++it) {
-        wmask[it] = 0u;
-        int h, lo, hi;
-        const int seg = pair_of(it, h, lo, hi);
-        if (seg < 0) continue;
-        const int need = __builtin_amdgcn_readfirstlane(need_of[it]), m = __builtin_amdgcn_readfirstlane(mem_of[it]);
-        const uint16_t* cl = tl_list + h * Kcap;
+        int h, seg;
+        if (!pair_of(it, h, seg)) continue;
+        const int tb = seg * (L / SEG), m = members[it];
+        const float* srow = sc + h * L;
         // a short list: every wavefront of the head finds the last winner itself, one member per lane (no exchange): few
         // members are ranked against each other as scalars (40 ns per member), more by bits (1 us)
-        if (need >= 0 && m <= Tail::MEM) {
+        if (m > 0 && m <= Tail::MEM) {
           const unsigned long long own = (lane < m) ? tl_mlist[h * Tail::MEM + lane] : 0ull;
           unsigned long long held;
           if (m <= Tail::RANK) {
@@ -2487,67 +2558,67 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
                                            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, k);
               rank += (o > own) ? 1 : 0;
             }
-            held = __builtin_amdgcn_ballot_w64(lane < m && rank == need - 1);
+            held = __builtin_amdgcn_ballot_w64(lane < m && rank == need[it] - 1);
           } else {
             held = (m < 64) ? (1ull << m) - 1ull : ~0ull;
-            int place = need;
+            int place = need[it];
             nth_largest((uint32_t)(own >> 12), held, place);   // the key,
             nth_largest((uint32_t)own & 4095u, held, place);   // and among equal ones the position
           }
           const int src = (held != 0ull) ? __ffsll((long long)held) - 1 : 0;
           last[it] = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), src) << 32) |
                      (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)own, src);
-        }
-        int total = 0;
-        for (int i0 = lo, j = 0; i0 < hi; i0 += 64, ++j) {
-          const int i = i0 + lane;
-          const uint32_t e = (i < hi) ? cl[i] : 0u;
-          bool win = i < hi;
-          if (e & 0x8000u) {
-            const int pos = min((int)(e & 0x7fffu), n - 1);
-            win = rank_word(score_key(sc[h * L + pos]), pos) >= last[it];
+          ahead[it] = __popcll(__builtin_amdgcn_ballot_w64(lane < m && own >= last[it] && 4095 - (int)((uint32_t)own & 4095u) < tb));
+          uint32_t mm = memb[it];
+          while (mm != 0u) {
+            const int i = __ffs((int)mm) - 1, pos = tb + place_of(i);
+            mm &= mm - 1u;
+            sure[it] |= (rank_word(score_key(srow[pos]), pos) >= last[it] ? 1u : 0u) << i;
           }
-          wmask[it] |= (win ? 1u : 0u) << j;
-          total += __popcll(__builtin_amdgcn_ballot_w64(win));
         }
-        if (lane == 0) tl_segc[h * SEG + seg] = total;
-      }
-      lds_barrier();
-      // the winners in position order: outputs, and slot and weight for the pre-correction
+        // this wavefront's winners in position order
+        uint16_t* cl = tl_list + h * Kcap;
+        const int base = before[it] + ahead[it];
+        int count = base;
+        if constexpr (SHORT) {
 #pragma unroll
-      for (int it = 0; it < NHS; ++it) {
-        int h, lo, hi;
-        const int seg = pair_of(it, h, lo, hi);
-        if (seg < 0) continue;
-        int base = 0, all = 0;
+          for (int i = 0; i < STEPS; ++i) {
+            const bool win = ((sure[it] >> i) & 1u) != 0u;
+            const unsigned long long mw = __builtin_amdgcn_ballot_w64(win);
+            const int r = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mw >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mw, 0u));
+            count += __popcll(mw);
+            if (win && r < Kt) cl[r] = (uint16_t)(tb + 64 * i + lane);
+          }
+        } else {
 #pragma unroll
-        for (int sg = 0; sg < SEG; ++sg) {
-          const int c = tl_segc[h * SEG + sg];
-          base += (sg < seg) ? c : 0;
-          all += c;
-        }
-        const int n_out = min(K, all);
-        if (seg == 0 && lane == 0) tl_nout[h] = n_out;
-        int64_t* out_idx = p.topk_idx + (head0 + h) * (size_t)K;
-        int64_t* out_slot = p.topk_slots + (head0 + h) * (size_t)K;
-        const float M = tl_m[h], iz = tl_iz[h];
-        for (int i0 = lo, j = 0; i0 < hi; i0 += 64, ++j) {
-          const bool win = ((wmask[it] >> j) & 1u) != 0u;
-          const unsigned long long mw = __builtin_amdgcn_ballot_w64(win);
-          const int r = base + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mw >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mw, 0u));
-          base += __popcll(mw);
-          if (win && r < K) {
-            const int pos = min((int)(tl_list[h * Kcap + i0 + lane] & 0x7fffu), n - 1);
-            const int slot = sbase[pos >> 4] + (pos & 15);
-            out_idx[r] = pos;
-            out_slot[r] = slot;
-            if constexpr (HAS_V) {
-              tl_wslot[h * K + r] = (slot >= 0 && slot < p.num_slots) ? slot : -1;
-              tl_ww[h * K + r] = __expf(sc[h * L + pos] - M) * iz;
+          for (int blk = 0; blk < Lds::LMAX / SEG / 1024; ++blk) {
+            uint32_t w = (sure[it] >> (16 * blk)) & 0xffffu;
+            const int mine = __popc(w), incl = wave_incl_scan_i(mine);
+            int r = count + incl - mine;
+            count += __builtin_amdgcn_readlane(incl, 63);
+            while (w != 0u) {
+              if (r < Kt) cl[r] = (uint16_t)(tb + 1024 * blk + 16 * lane + __ffs((int)w) - 1);
+              ++r;
+              w &= w - 1u;
             }
           }
         }
-        for (int r = n_out + seg * 64 + lane; r < K; r += SEG * 64) {
+        wave_lds_fence();
+        // outputs, and slot and weight for the pre-correction, one winner per lane
+        int64_t* out_idx = p.topk_idx + (head0 + h) * (size_t)K;
+        int64_t* out_slot = p.topk_slots + (head0 + h) * (size_t)K;
+        const float M = tl_m[h], iz = tl_iz[h];
+        for (int r = base + lane; r < min(count, Kt); r += 64) {
+          const int pos = min((int)cl[r], n - 1);
+          const int slot = sbase[pos >> 4] + (pos & 15);
+          out_idx[r] = pos;
+          out_slot[r] = slot;
+          if constexpr (HAS_V) {
+            tl_wslot[h * K + r] = (slot >= 0 && slot < p.num_slots) ? slot : -1;
+            tl_ww[h * K + r] = __expf(srow[pos] - M) * iz;
+          }
+        }
+        for (int r = Kt + seg * 64 + lane; r < K; r += SEG * 64) {
           out_idx[r] = -1;
           out_slot[r] = -1;
         }
@@ -2582,7 +2653,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       float* old_sh = reinterpret_cast<float*>(stage);  // [G][WPH][D] (the accumulator sums are dead)
       float* w_sh = old_sh + G * WPH * D;               // [G][WPH]
       for (int hw = wave; hw < GA * WPH; hw += NW) {
-        const int h = hw / WPH, part = hw % WPH, n_out = __builtin_amdgcn_readfirstlane(tl_nout[h]);
+        const int h = hw / WPH, part = hw % WPH, n_out = HAS_TOPK ? Kt : __builtin_amdgcn_readfirstlane(tl_nout[h]);
         float acc[Pre::CPD], accw = 0.f;
 #pragma unroll
         for (int c = 0; c < Pre::CPD; ++c) acc[c] = 0.f;
@@ -2632,8 +2703,10 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         if (lane == 0) w_sh[hw] = wsum;
       }
       lds_barrier();
-      for (int i = tid; i < GA * D; i += NT) {
-        const int h = i >> 7, d = i & 127;
+#pragma unroll
+      for (int it = 0; it < OPT; ++it) {
+        const int i = it * NT + tid, h = i >> 7, d = i & 127;
+        if (i >= GA * D) break;
         float o = 0.f, wt = 0.f;
 #pragma unroll
         for (int w = 0; w < WPH; ++w) {
@@ -2644,7 +2717,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         if (d == 0) p.W[head0 + h] = wt;
         if (MODE == FS_FULL && p.blend_out) {
           const size_t at = (head0 + h) * D + d;
-          p.blend_out[at] = f32_to_bf16(__builtin_fmaf(wt, bf16_to_f32(p.blend_o_new[at]), tl_ohat[h * D + d]) - o);
+          p.blend_out[at] = f32_to_bf16(__builtin_fmaf(wt, bf16_to_f32(o_new[it]), tl_ohat[h * D + d]) - o);
         }
       }
     }
@@ -3531,27 +3604,10 @@ inline size_t scan_tail_bytes(int G, int top_k, int kc) {
                   ScanTail<16, 1>::bytes(top_k, kc);
 }
 
-// Entries a head's candidate list can have where the scan merges by itself: a wavefront's share fits the 32 bits of its
-// win mask.
-inline int one_split_list_max(int G) { return (G <= 4 ? 4 : 1) * 64 * 32; }
-
 // Whether a scan whose single split of L positions covers the sequence can merge by itself: its tables fit the LDS
-// that is left, and so does a list of kc candidates.
+// that is left, and so does the list of winners (kc counts their most and more).
 inline bool one_split_fits(int scheme, int G, int NG, int L, int top_k, int kc) {
-  return kc <= one_split_list_max(G) &&
-         (long)((4 * G + 1) * (long)L + (long)scan_tail_bytes(G, top_k, kc)) <= lds_room(scheme, G, NG);
-}
-
-// The candidate list such a scan gets: as much of the LDS that is left (one workgroup per CU either way) as the split can
-// fill.  A bucket at the cut with more positions than the list has room for (one outlying score makes the buckets wide)
-// takes the exact selection, one wavefront per head; a list that holds them goes on with all of the head's wavefronts:
-// 16 sequences x 8 kv-heads, 3900 positions, K2V2, one head each, top-k 1024, per layer with no outlier / one score at 20
-// / at 40 sigma: top_k + 256 entries 26.8 / 52.8 / 61.1 us, this 26.7 / 28.8 / 29.5 (splits of 2048 and a merge launch:
-// 28.5 / 29.2 / 35.3).
-inline int one_split_list(int scheme, int G, int NG, int L, int top_k, int kc) {
-  const long room = lds_room(scheme, G, NG) - (4 * G + 1) * (long)L - (long)scan_tail_bytes(G, top_k, kc);
-  const long most = L < one_split_list_max(G) ? L : one_split_list_max(G), more = kc + room / (2 * G);
-  return (int)(more < most ? more : most);
+  return (long)((4 * G + 1) * (long)L + (long)scan_tail_bytes(G, top_k, kc)) <= lds_room(scheme, G, NG);
 }
 
 // Estimated microseconds of the merge (fitted on MI355X): a fixed part per launch plus a part proportional to
@@ -3561,7 +3617,6 @@ constexpr int MG_REG_CANDS = 8192;  // candidates the common merge shape keeps i
 inline double merge_pass_us(double fixed, long cands) {
   return cands <= MG_REG_CANDS ? fixed + kPerCand * (double)cands : fixed + 1.5 + kPerCandBig * (double)cands;
 }
-
 // One stage of the shape that keeps 32 candidates per thread, against two stages at the same split length, 36 shapes of 9472 to
 // 30720 candidates, 16 to 256 rows, per layer: up to 16384 candidates 1.5 - 9 us shorter, around 22000 as long, 2.4 us longer at
 // 30720 (rows 16; with 64 rows and more it is the shorter way throughout).  3 x 28076 positions, 8 kv-heads, G = 4, K3V2, top-k
@@ -3887,7 +3942,6 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
     JF_CHECK_ARG(workspace && workspace_bytes >= wl.total, "fused_scan: workspace too small (%zu < %zu)", workspace_bytes, wl.total);
     JF_CHECK_ARG(((uintptr_t)workspace & 255) == 0, "fused_scan: workspace must be 256-byte aligned");
   }
-  if (p.one_split) p.Kc = one_split_list(scheme, G, NGv, p.L, top_k, p.Kc);  // (in LDS, not in the workspace)
   uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
   p.scores = HAS_K ? scores : nullptr;
   p.scores_in = scores_in;
