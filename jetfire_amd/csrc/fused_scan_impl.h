@@ -47,6 +47,7 @@
 #include <atomic>
 #include <type_traits>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 namespace jf {
@@ -432,6 +433,210 @@ __device__ inline float buffer_f32(__amdgpu_buffer_rsrc_t r, int voffset, int so
 // captured array in scratch memory, at three times the run time.
 #define JF_INLINE __attribute__((always_inline))
 
+// Value codes as MFMA B operands.  64 packed V rows lie in LDS (`stash_row`, or the value stream's own stores to the same
+// places), and transposed reads hand every lane 16 tokens of a channel or two, which are spread to one code per byte.  Tile t,
+// column c of the products is channel `channel(t, c)`.
+template <int VBITS, int NG>
+struct VTiles {
+  static constexpr bool V2 = VBITS == 2, V3 = VBITS == 3;
+  static constexpr int VP = D * VBITS / 8;
+  // LDS pitch of a staged V row.  INT2 rows (32 bytes) are padded so that 16 consecutive rows hit 16 distinct
+  // bank pairs; INT4 rows (64 bytes) keep their pitch and swap their 16-byte quarters instead (quarter q of row r
+  // sits at q ^ ((r >> 2) & 3)), which has the same effect without the padding bytes.  INT3 rows (48 bytes: 16
+  // consecutive rows already hit distinct bank pairs) swap the 8-byte halves of every plane in rows 16..31 and
+  // 48..63, so that the two 16-row groups one 8-byte read serves in a cycle do not meet either.
+  static constexpr bool VSWZ = !(V2 || V3);
+  static constexpr int VROW = (VSWZ || V3) ? VP : VP + 8;
+  static constexpr int VST = 64 * VROW;
+  static constexpr int OFFSET = V2 ? 2 : (V3 ? 4 : 8);  // of the codes
+  // even INT2 tiles hold four times their codes
+  static constexpr int times(int tile) { return V2 && !(tile & 1) ? 4 : 1; }
+  static __device__ inline int channel(int tile, int col) {
+    if (V2) return (tile >> 1) * 32 + (col >> 1) * 4 + ((col & 1) ? 0 : 2) + (tile & 1);
+    // tile = 4 * (64-channel half) + code within the lane's four; odd columns hold codes 0..3
+    if (V3) return (tile >> 2) * 64 + (col >> 1) * 8 + ((col & 1) ? 0 : 4) + (tile & 3);
+    return tile * 16 + 2 * (col >> 1) + (1 - (col & 1));
+  }
+  // piece i (16 bytes) of row `row` to its place
+  static __device__ inline void stash_piece(uint8_t* vst, int row, int i, const v4u& x) {
+    uint8_t* dst = vst + row * VROW;
+    if constexpr (VSWZ) {
+      *reinterpret_cast<v4u*>(dst + ((i ^ ((row >> 2) & 3)) * 16)) = x;
+    } else {
+      const int first = V3 ? 8 * ((row >> 4) & 1) : 0;  // (INT3: first half's place)
+      *reinterpret_cast<v2u*>(dst + 16 * i + first) = (v2u){x[0], x[1]};
+      *reinterpret_cast<v2u*>(dst + 16 * i + (8 - first)) = (v2u){x[2], x[3]};
+    }
+  }
+  // calls f(tile, scale group, operand) for the eight tiles of 16 channels
+  template <class F>
+  static __device__ JF_INLINE void spread(const uint8_t* vst, int lane, F&& f) {
+    // the nibble spread of a transposed V dword yields tokens 0,2,4,6 | 1,3,5,7 | 8,10,12,14 | 9,11,13,15 of the
+    // lane group's 16 tokens: token r sits in byte (r&8) | ((r&1)<<2) | ((r>>1)&3)
+    const uint8_t* vrow = vst + lane * VROW;
+    spread_from(vrow, lane, f, std::make_integer_sequence<int, V2 ? 4 : (V3 ? 2 : 8)>{});
+  }
+  template <class F, int... Q>
+  static __device__ JF_INLINE void spread_from(const uint8_t* vrow, int lane, F&& f, std::integer_sequence<int, Q...>) {
+    (step<Q>(vrow, lane, f), ...);
+  }
+  template <int Q, class F>
+  static __device__ JF_INLINE void step(const uint8_t* vrow, int lane, F&& f) {
+    if constexpr (V2) {
+      const v2i x = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(vrow + 8 * Q));
+      const uint32_t x0 = (uint32_t)x[0], x1 = (uint32_t)x[1], y0 = x0 >> 4, y1 = x1 >> 4;
+      // the upper code of every nibble stays where it is: tile 2 * Q accumulates 4 * code (undone where the sums are read)
+      const v4i Ba = {(int)(x0 & 0x0c0c0c0cu), (int)(y0 & 0x0c0c0c0cu), (int)(x1 & 0x0c0c0c0cu), (int)(y1 & 0x0c0c0c0cu)};
+      const v4i Bb = {(int)(x0 & 0x03030303u), (int)(y0 & 0x03030303u), (int)(x1 & 0x03030303u), (int)(y1 & 0x03030303u)};
+      const int g = (NG == 1) ? 0 : (Q >> 1);
+      f(std::integral_constant<int, 2 * Q>{}, g, Ba);
+      f(std::integral_constant<int, 2 * Q + 1>{}, g, Bb);
+    } else if constexpr (V3) {
+      // Planar INT3: bytes j of the three 16-byte planes form the 24-bit word of channels 8j .. 8j+7, code i at
+      // bits 23-3i .. 21-3i.  A transposed read of one plane's 8-byte half hands lane c the nibble c of 16 tokens:
+      // odd lanes the high nibbles of byte c >> 1, even lanes the low ones.  With one exchange inside the lane
+      // pair (the odd lane needs its partner's plane-0 nibble, the even lane its partner's plane-2 nibble) the odd
+      // lane holds what codes 0..3 of the word are made of and the even lane what codes 4..7 are made of, in the
+      // same three positions: a = [c0 c0 c0 c1], b = [c1 c1 c2 c2], c = [c2 c3 c3 c3] (msb first).
+      const bool odd = (lane & 1) != 0;
+      const int hsw = 8 * ((lane >> 4) & 1);  // rows 16..31, 48..63 keep their plane halves swapped
+      const uint8_t* src = vrow + (Q ? 8 - hsw : hsw);
+      const v2i x0 = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(src));
+      const v2i x1 = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(src + 16));
+      const v2i x2 = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(src + 32));
+      v4i Bc[4];
+#pragma unroll
+      for (int hw = 0; hw < 2; ++hw) {  // tokens 0..7 and 8..15 of the lane group, one nibble each
+        const int send = odd ? x2[hw] : x0[hw];
+        const uint32_t b = (uint32_t)dpp_mov<0xb1, 0xf>(0, send);  // quad_perm [1,0,3,2]: the pair partner's value
+        const uint32_t a = (uint32_t)(odd ? x0[hw] : x1[hw]), c = (uint32_t)(odd ? x1[hw] : x2[hw]);
+        // per nibble (bit 3 of the two middle codes is cleared by the byte masks below)
+        const uint32_t n1 = ((b >> 2) & 0x33333333u) | ((a << 2) & ~0x33333333u);
+        const uint32_t n2 = ((c >> 3) & 0x11111111u) | ((b << 1) & ~0x11111111u);
+        Bc[0][2 * hw] = (int)((a >> 1) & 0x07070707u);
+        Bc[0][2 * hw + 1] = (int)((a >> 5) & 0x07070707u);
+        Bc[1][2 * hw] = (int)(n1 & 0x07070707u);
+        Bc[1][2 * hw + 1] = (int)((n1 >> 4) & 0x07070707u);
+        Bc[2][2 * hw] = (int)(n2 & 0x07070707u);
+        Bc[2][2 * hw + 1] = (int)((n2 >> 4) & 0x07070707u);
+        Bc[3][2 * hw] = (int)(c & 0x07070707u);
+        Bc[3][2 * hw + 1] = (int)((c >> 4) & 0x07070707u);
+      }
+      const int g = (NG == 1) ? 0 : Q;
+      f(std::integral_constant<int, 4 * Q>{}, g, Bc[0]);
+      f(std::integral_constant<int, 4 * Q + 1>{}, g, Bc[1]);
+      f(std::integral_constant<int, 4 * Q + 2>{}, g, Bc[2]);
+      f(std::integral_constant<int, 4 * Q + 3>{}, g, Bc[3]);
+    } else {
+      const int vx = 16 * ((lane >> 2) & 3);  // quarter swap of this lane's row
+      const v2i x = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(vrow + ((8 * Q) ^ vx)));
+      const uint32_t x0 = (uint32_t)x[0], x1 = (uint32_t)x[1];
+      const v4i Bv = {(int)(x0 & 0x0f0f0f0fu), (int)((x0 >> 4) & 0x0f0f0f0fu),
+                      (int)(x1 & 0x0f0f0f0fu), (int)((x1 >> 4) & 0x0f0f0f0fu)};
+      f(std::integral_constant<int, Q>{}, (NG == 1) ? 0 : (Q >> 2), Bv);
+    }
+  }
+};
+
+// Byte j of an A operand is token tr8_token of the lane group's 16: what pairs a transposed read of 16-byte rows with the
+// byte order of VTiles' operands (the lane pair (2j, 2j+1) supplies the two halves of the row that must land in byte j).
+__device__ inline int tr8_token(int lane) { return (((lane >> 1) & 3) << 1) | ((lane >> 3) & 1); }
+
+// Pre-correction terms over the winners' packed V rows where a wavefront has 64 winners of a head at a time (one per lane): the
+// contraction of phase B on v_mfma_i32_16x16x64_i8, with one head's weights in four rows of the operand.  The weights are held
+// to 24 bits of the largest among the 64 (exact integers in float), in limbs of 7, 7, 7 and 3 bits, so that no limb needs a
+// sign; the products are exact, and each of the 64-winner sums is rounded once.
+// What a conversion and a multiply-add per code take instead, per
+// layer: 32 sequences x 2048 positions, K3V2, top-k 256 25.2 us, this 24.1; K4V4 26.6 / 25.5; 32 x 1900, K3V2, 512 28.9 / 26.8;
+// 16 x 1024, K4V4, 512 21.7 / 19.3; 32 x 500, eight heads, K3V2, 256 22.1 / 20.5.
+template <int VBITS, int NG>
+struct WinnerSums {
+  using Tiles = VTiles<VBITS, NG>;
+  static constexpr int PIECES = Tiles::VP / 16;
+  static constexpr int STAGE = Tiles::VST + NG * 1024;  // LDS per wavefront: the rows, and a 16-byte weight row per winner and group
+  struct Rows {
+    v4u r[PIECES];
+    uint32_t s;  // scale word
+    float w;     // weight, zero for no winner
+  };
+  // winners first .. first + 63 of n; slots (-1: none) and weights of the head's winners in LDS.  The lanes of a row lie side by
+  // side: a lane per row touched sixty-four
+  // lines with every load (32 sequences x 2048 positions, K4V4, top-k 256 27.3 us per layer, 25.8 with this).
+  static __device__ JF_INLINE Rows fetch(const uint8_t* vbase, const uint8_t* vsbase, const int* slots, const float* weights, int first, int n, int lane) {
+    Rows x;
+    int slot[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) slot[i] = slots[min(first + (1024 * i + 16 * lane) / Tiles::VP, n - 1)];
+    const int own = min(first + lane, n - 1);
+    const int mine = slots[own];
+    const float w = weights[own];
+    const bool valid = first + lane < n && mine >= 0;
+    x.w = valid ? w : 0.f;
+    const uint32_t sl = (uint32_t)max(mine, 0);
+    if (NG == 2) x.s = *reinterpret_cast<const uint32_t*>(vsbase + (size_t)(sl * 4u));
+    else x.s = (uint32_t) * reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * 2u));
+    if (!valid) x.s = 0u;  // (whatever scale that slot has)
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      x.r[i] = *reinterpret_cast<const v4u*>(vbase + (size_t)((uint32_t)max(slot[i], 0) * (uint32_t)Tiles::VP + (uint32_t)(1024 * i + 16 * lane) % Tiles::VP));
+    return x;
+  }
+  // o[t] += the sums of tile t, column lane (lanes 0 .. 15; the other lanes' are of no use)
+  static __device__ JF_INLINE void add(const Rows& x, uint8_t* st, int lane, float (&o)[8]) {
+    uint8_t* wl = st + Tiles::VST;
+    float top[NG];
+    int E[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const float v = x.w * bf16_to_f32((uint16_t)(g ? x.s >> 16 : x.s & 0xffffu));
+      const uint32_t most = wave_max_u(__builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
+      top[g] = uniform_f(__builtin_bit_cast(float, most));
+      int e = 0;
+      float f;
+      if (isfinite(top[g])) {  // (uniform)
+        if (top[g] > 0.f) (void)frexpf(top[g], &e);  // top = f * 2^e, f in [0.5, 1)
+        f = ldexpf(v, 24 - e);
+      } else {  // an infinite weight or a NaN: it alone counts, and `top` becomes the sums' factor
+        f = (__builtin_bit_cast(uint32_t, v) & 0x7fffffffu) == most ? 1.f : 0.f;
+      }
+      E[g] = 24 - e;
+      const uint32_t w = (uint32_t)rintf(f);
+      *reinterpret_cast<uint32_t*>(wl + (g * 64 + lane) * 16) = (w & 0x7fu) | ((w << 1) & 0x7f00u) | ((w << 2) & 0x7f0000u) | ((w << 3) & 0x7f000000u);
+    }
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) Tiles::stash_piece(st, (1024 * i + 16 * lane) / Tiles::VP, (1024 * i + 16 * lane) % Tiles::VP / 16, x.r[i]);
+    wave_lds_fence();
+    const uint8_t* wrow = wl + ((lane >> 4) * 16 + tr8_token(lane)) * 16 + (lane & 1) * 8;
+    v4i A[NG], sw[NG], acc[8];
+    const v4i zero = {0, 0, 0, 0}, ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const v2i x0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(wrow + g * 1024));
+      const v2i x1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(wrow + g * 1024 + 128));
+      A[g] = (v4i){x0[0], x0[1], x1[0], x1[1]};
+      sw[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g], ones, zero, 0, 0, 0);
+    }
+    Tiles::spread(st, lane, [&](auto tile, int g, const v4i& B) JF_INLINE {
+      acc[decltype(tile)::value] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g], B, zero, 0, 0, 0);
+    });
+    int lo[NG], hi[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      lo[g] = Tiles::OFFSET * (sw[g][0] + (sw[g][1] << 7));
+      hi[g] = Tiles::OFFSET * (sw[g][2] + (sw[g][3] << 7));
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const int g = (NG == 1) ? 0 : t / 4, m = Tiles::times(t);
+      // (both below 2^24: floats hold them)
+      const float a = (float)(acc[t][0] + (acc[t][1] << 7) - m * lo[g]), b = (float)(acc[t][2] + (acc[t][3] << 7) - m * hi[g]);
+      const float sum = __builtin_fmaf(b, 16384.f, a) * (m == 4 ? 0.25f : 1.f);
+      o[t] += isfinite(top[g]) ? ldexpf(sum, -E[g]) : sum * top[g];
+    }
+    wave_lds_fence();
+  }
+};
+
 // Pre-correction terms over the winners' packed V rows, shared by the merge kernel and the scan's in-kernel merge: DW
 // lanes per row, lane dwi holds dword dwi of it (INT2, INT4) or two bytes of each of the three planes (INT3) = CPD
 // codes; a wavefront instruction covers WPI rows, sixteen wavefronts (or roles) and UNR requests per lane 256 rows.
@@ -576,7 +781,9 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   constexpr int KROW = Lds::KROW;
   constexpr int VP = Lds::VP;
   constexpr int VROW = Lds::VROW;
-  constexpr int VOFF = V2 ? 2 : (V3 ? 4 : 8);  // code offset of the V format
+  using Tiles = VTiles<SCHEME % 10, NG>;
+  constexpr int VOFF = Tiles::OFFSET;  // code offset of the V format
+  static_assert(VROW == Tiles::VROW, "one layout of the staged V rows");
   constexpr int NTILE = 8;          // 8 MFMA column tiles of 16 channels
   constexpr int AR = Lds::ACC_REGS;
   constexpr float LOG2E = 1.44269504088896340736f;
@@ -1612,27 +1819,9 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   if constexpr (HAS_TOPK)
     if (!take_all)
       for (int i = tid; i < Lds::HIST / 4; i += NT) hist[i] = 0;
-  // ONE: what the in-kernel merge keeps behind the staging area (see ScanTail)
-  using Tail = ScanTail<G, SEG>;
-  const int Kcap = p.Kc;
-  [[maybe_unused]] const int K = p.top_k;
-  uint8_t* tail = stage + Lds::stage_bytes() + 64;
-  [[maybe_unused]] int* tl_put = reinterpret_cast<int*>(tail);              // [G] members put into the head's list
-  [[maybe_unused]] int* tl_mem = tl_put + G;                                // [G] members of the cut bucket
-  [[maybe_unused]] int* tl_nout = tl_mem + G;                               // [G] winners (Stage B); the selection's words
-  [[maybe_unused]] int* tl_segc = tl_nout + G;                              // [G][SEG] winners per wavefront
-  [[maybe_unused]] float* tl_m = reinterpret_cast<float*>(tl_segc + G * SEG);  // [G] softmax maximum, 1 / sum, e^{m - M}
-  [[maybe_unused]] float* tl_iz = tl_m + G;
-  [[maybe_unused]] float* tl_coef = tl_iz + G;
-  [[maybe_unused]] float* tl_ohat = reinterpret_cast<float*>(tail + Tail::INTS);          // [G][D]
-  [[maybe_unused]] int* tl_wslot = reinterpret_cast<int*>(tl_ohat + G * D);               // [G][top_k] paged slot of a winner
-  [[maybe_unused]] float* tl_ww = reinterpret_cast<float*>(tl_wslot + (size_t)G * K);     // [G][top_k] its softmax weight
-  // [G][MEM] members of the cut bucket, as rank words
-  [[maybe_unused]] unsigned long long* tl_mlist = reinterpret_cast<unsigned long long*>(tl_ww + (size_t)G * K);
-  [[maybe_unused]] uint16_t* tl_list = reinterpret_cast<uint16_t*>(tl_mlist + G * Tail::MEM);  // [G][Kcap] the winners' positions, ascending
   if (tid < G) {
     float m = red_f[0][tid], lo = red_f[0][G + tid];
-    if constexpr (ONE) tl_put[tid] = 0;
+    if constexpr (ONE) reinterpret_cast<int*>(stage + Lds::stage_bytes() + 64)[tid] = 0;  // (tl_put, see below)
 #pragma unroll
     for (int w = 1; w < NW; ++w) {
       m = fmaxf(m, red_f[w][tid]);
@@ -1704,7 +1893,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // transposed weight read: 16-lane group kb4 fetches the rows of tokens 16*kb4 .. +15; the lane pair (2j, 2j+1)
   // supplies the two halves of the row that must land in byte j, i.e. of the token whose byte position in the
   // V operand (see below) is j
-  const int tr_tok = (((r16 >> 1) & 3) << 1) | ((r16 >> 3) & 1);
+  const int tr_tok = tr8_token(lane);
   const uint8_t* wrow = wl + (kb4 * 16 + tr_tok) * 16 + (r16 & 1) * 8;
   const int seg_chunks = L / 64 / SEG;  // chunks per emission segment
   auto body_v = [&](int chunk, uint32_t vsw) JF_INLINE {
@@ -1767,78 +1956,11 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
 #pragma unroll
       for (int set = 0; set < NSET; ++set)
         accw[set][g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g][set], ones, accw[set][g], 0, 0, 0);
-    // the nibble spread of a transposed V dword yields tokens 0,2,4,6 | 1,3,5,7 | 8,10,12,14 | 9,11,13,15 of the
-    // lane group's 16 tokens: token r sits in byte (r&8) | ((r&1)<<2) | ((r>>1)&3)
-    const uint8_t* vrow = vst + lane * VROW;
-    if (V2) {
+    Tiles::spread(vst, lane, [&](auto tile, int g, const v4i& Bv) JF_INLINE {
 #pragma unroll
-      for (int qc = 0; qc < 4; ++qc) {
-        const v2i x = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(vrow + 8 * qc));
-        const uint32_t x0 = (uint32_t)x[0], x1 = (uint32_t)x[1], y0 = x0 >> 4, y1 = x1 >> 4;
-        // the upper code of every nibble stays where it is: tile 2*qc accumulates 4 * code (undone in `combine`)
-        const v4i Ba = {(int)(x0 & 0x0c0c0c0cu), (int)(y0 & 0x0c0c0c0cu), (int)(x1 & 0x0c0c0c0cu), (int)(y1 & 0x0c0c0c0cu)};
-        const v4i Bb = {(int)(x0 & 0x03030303u), (int)(y0 & 0x03030303u), (int)(x1 & 0x03030303u), (int)(y1 & 0x03030303u)};
-        const int g = (NG == 1) ? 0 : (qc >> 1);
-#pragma unroll
-        for (int set = 0; set < NSET; ++set) {
-          acc[set][2 * qc] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g][set], Ba, acc[set][2 * qc], 0, 0, 0);
-          acc[set][2 * qc + 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g][set], Bb, acc[set][2 * qc + 1], 0, 0, 0);
-        }
-      }
-    } else if (V3) {
-      // Planar INT3: bytes j of the three 16-byte planes form the 24-bit word of channels 8j .. 8j+7, code i at
-      // bits 23-3i .. 21-3i.  A transposed read of one plane's 8-byte half hands lane c the nibble c of 16 tokens:
-      // odd lanes the high nibbles of byte c >> 1, even lanes the low ones.  With one exchange inside the lane
-      // pair (the odd lane needs its partner's plane-0 nibble, the even lane its partner's plane-2 nibble) the odd
-      // lane holds what codes 0..3 of the word are made of and the even lane what codes 4..7 are made of, in the
-      // same three positions: a = [c0 c0 c0 c1], b = [c1 c1 c2 c2], c = [c2 c3 c3 c3] (msb first).
-      const bool odd = (lane & 1) != 0;
-      const int hsw = 8 * ((lane >> 4) & 1);  // rows 16..31, 48..63 keep their plane halves swapped
-#pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        const uint8_t* src = vrow + (w ? 8 - hsw : hsw);
-        const v2i x0 = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(src));
-        const v2i x1 = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(src + 16));
-        const v2i x2 = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(src + 32));
-        v4i Bc[4];
-#pragma unroll
-        for (int hw = 0; hw < 2; ++hw) {  // tokens 0..7 and 8..15 of the lane group, one nibble each
-          const int send = odd ? x2[hw] : x0[hw];
-          const uint32_t b = (uint32_t)dpp_mov<0xb1, 0xf>(0, send);  // quad_perm [1,0,3,2]: the pair partner's value
-          const uint32_t a = (uint32_t)(odd ? x0[hw] : x1[hw]), c = (uint32_t)(odd ? x1[hw] : x2[hw]);
-          // per nibble (bit 3 of the two middle codes is cleared by the byte masks below)
-          const uint32_t n1 = ((b >> 2) & 0x33333333u) | ((a << 2) & ~0x33333333u);
-          const uint32_t n2 = ((c >> 3) & 0x11111111u) | ((b << 1) & ~0x11111111u);
-          Bc[0][2 * hw] = (int)((a >> 1) & 0x07070707u);
-          Bc[0][2 * hw + 1] = (int)((a >> 5) & 0x07070707u);
-          Bc[1][2 * hw] = (int)(n1 & 0x07070707u);
-          Bc[1][2 * hw + 1] = (int)((n1 >> 4) & 0x07070707u);
-          Bc[2][2 * hw] = (int)(n2 & 0x07070707u);
-          Bc[2][2 * hw + 1] = (int)((n2 >> 4) & 0x07070707u);
-          Bc[3][2 * hw] = (int)(c & 0x07070707u);
-          Bc[3][2 * hw + 1] = (int)((c >> 4) & 0x07070707u);
-        }
-        const int g = (NG == 1) ? 0 : w;
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-#pragma unroll
-          for (int set = 0; set < NSET; ++set)
-            acc[set][4 * w + m] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g][set], Bc[m], acc[set][4 * w + m], 0, 0, 0);
-      }
-    } else {
-      const int vx = 16 * ((lane >> 2) & 3);  // quarter swap of this lane's row
-#pragma unroll
-      for (int qc = 0; qc < 8; ++qc) {
-        const v2i x = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)(vrow + (Lds::VSWZ ? ((8 * qc) ^ vx) : 8 * qc)));
-        const uint32_t x0 = (uint32_t)x[0], x1 = (uint32_t)x[1];
-        const v4i Bv = {(int)(x0 & 0x0f0f0f0fu), (int)((x0 >> 4) & 0x0f0f0f0fu),
-                        (int)(x1 & 0x0f0f0f0fu), (int)((x1 >> 4) & 0x0f0f0f0fu)};
-        const int g = (NG == 1) ? 0 : (qc >> 2);
-#pragma unroll
-        for (int set = 0; set < NSET; ++set)
-          acc[set][qc] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g][set], Bv, acc[set][qc], 0, 0, 0);
-      }
-    }
+      for (int set = 0; set < NSET; ++set)
+        acc[set][decltype(tile)::value] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g][set], Bv, acc[set][decltype(tile)::value], 0, 0, 0);
+    });
     wave_lds_fence();
   };
   auto stash_v = [&](const VBuf& vbuf) {
@@ -1899,6 +2021,24 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // the constant row (75 * sum of codes) for l = 3.  Item j = (register i = j >> 2 of set i / AR, component j & 3)
   // lives at xacc[j * 64 + lane].
   int* xacc = reinterpret_cast<int*>(stage);
+  // ONE: what the in-kernel merge keeps behind the staging area (see ScanTail)
+  using Tail = ScanTail<G, SEG>;
+  const int Kcap = p.Kc;
+  [[maybe_unused]] const int K = p.top_k;
+  uint8_t* tail = stage + Lds::stage_bytes() + 64;
+  [[maybe_unused]] int* tl_put = reinterpret_cast<int*>(tail);              // [G] members put into the head's list
+  [[maybe_unused]] int* tl_mem = tl_put + G;                                // [G] members of the cut bucket
+  [[maybe_unused]] int* tl_nout = tl_mem + G;                               // [G] winners (Stage B); the selection's words
+  [[maybe_unused]] int* tl_segc = tl_nout + G;                              // [G][SEG] winners per wavefront
+  [[maybe_unused]] float* tl_m = reinterpret_cast<float*>(tl_segc + G * SEG);  // [G] softmax maximum, 1 / sum, e^{m - M}
+  [[maybe_unused]] float* tl_iz = tl_m + G;
+  [[maybe_unused]] float* tl_coef = tl_iz + G;
+  [[maybe_unused]] float* tl_ohat = reinterpret_cast<float*>(tail + Tail::INTS);          // [G][D]
+  [[maybe_unused]] int* tl_wslot = reinterpret_cast<int*>(tl_ohat + G * D);               // [G][top_k] paged slot of a winner
+  [[maybe_unused]] float* tl_ww = reinterpret_cast<float*>(tl_wslot + (size_t)G * K);     // [G][top_k] its softmax weight
+  // [G][MEM] members of the cut bucket, as rank words
+  [[maybe_unused]] unsigned long long* tl_mlist = reinterpret_cast<unsigned long long*>(tl_ww + (size_t)G * K);
+  [[maybe_unused]] uint16_t* tl_list = reinterpret_cast<uint16_t*>(tl_mlist + G * Tail::MEM);  // [G][Kcap] the winners' positions, ascending
   if constexpr (ONE) {
     if (tid < G) {
       float l = 0.f;
@@ -1924,21 +2064,14 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       atomicAdd(xacc + j * 64 + lane, v[c]);
     }
   };
+  [[maybe_unused]] float* late_o_hat = nullptr;  // ONE: see below
   auto combine = [&](int set) {
     // thread -> (tile, head, column)
     for (int i = tid; i < 4 * D; i += NT) {
       const int col = i & 15, hh = (i >> 4) & 3, tile = i >> 6;
       const int h = set * 4 + hh;
       if (h >= GA) continue;
-      int d;
-      if (V2) {
-        const int e = ((col & 1) ? 0 : 2) + (tile & 1);
-        d = (tile >> 1) * 32 + (col >> 1) * 4 + e;
-      } else if (V3) {  // tile = 4 * (64-channel half) + code within the lane's four; odd columns hold codes 0..3
-        d = (tile >> 2) * 64 + (col >> 1) * 8 + ((col & 1) ? 0 : 4) + (tile & 3);
-      } else {
-        d = tile * 16 + 2 * (col >> 1) + (1 - (col & 1));
-      }
+      const int d = Tiles::channel(tile, col);
       const int g = (NG == 1) ? 0 : (d / (D / NG));
       const int* ta = xacc + ((set * AR + tile) * 4) * 64 + 16 * hh + col;   // row 4*hh + l of the tile: component l, lane 16*hh + col
       const int* wa = xacc + ((set * AR + NTILE + g) * 4) * 64 + 16 * hh;    // weight sums: any column of the all-ones tile
@@ -1955,7 +2088,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       const float o = (float)ldexp((double)tot, -E[g]);
       if constexpr (ONE) {
         const float o_hat = __builtin_fmaf(o, tl_coef[h], 0.f) * tl_iz[h];
-        p.o_hat[(head0 + h) * D + d] = o_hat;
+        late_o_hat[(head0 + h) * D + d] = o_hat;
         tl_ohat[h * D + d] = o_hat;
       } else {
         p.part_o[(part_base + (size_t)h * p.n_splits) * D + d] = o;
@@ -1996,6 +2129,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       if constexpr (ONE) {
         const unsigned long long c_lo = __builtin_amdgcn_ballot_w64(v >= thr_lo);
         asm("s_nop 1\n\tv_addc_co_u32_e64 %0, vcc, %1, %1, %2" : "=v"(ge_lo) : "v"(ge_lo), "s"(c_lo) : "vcc");
+        __builtin_amdgcn_sched_barrier(0);  // (all lane masks together do not fit the scalar registers)
       }
       if constexpr (HAS_V && PER > 0) {
         const int lo = A_LO + (15 - bi) * PER;
@@ -2024,7 +2158,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   auto find_cut = [&](int h, int seg) JF_INLINE -> Cut {
     const int* h0 = hist + h * (SEG * 256) / (Lds::H16 ? 2 : 1);
     // lane l owns buckets 4l .. 4l+3 (ascending bucket = descending score) of every segment's histogram
-    int cs[SEG][4], c[4], mine;
+    int cs[SEG][4];
 #pragma unroll
     for (int sg = 0; sg < SEG; ++sg) {
       if (Lds::H16) {
@@ -2039,10 +2173,9 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         for (int u = 0; u < 4; ++u) cs[sg][u] = x[u];
       }
     }
-    // c[u]: the bucket's count over all segments; cum[u]: over the segments before this wavefront's
-    int cum[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int u = 0; u < 4; ++u) c[u] = 0;
+    // pk[u]: the bucket's count over all segments in the low half, over the segments before this wavefront's in the high half (each
+    // sum <= 4096)
+    int c[4] = {0, 0, 0, 0}, cum[4] = {0, 0, 0, 0}, pk[4];
 #pragma unroll
     for (int sg = 0; sg < SEG; ++sg) {
       if (sg == seg) {  // (uniform)
@@ -2052,38 +2185,21 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
 #pragma unroll
       for (int u = 0; u < 4; ++u) c[u] += cs[sg][u];
     }
-    mine = (c[0] + c[1]) + (c[2] + c[3]);
-    const int cumt = (cum[0] + cum[1]) + (cum[2] + cum[3]);
-    // one scan for both: the totals in the low half, the earlier segments' in the high half (each sum <= 4096)
-    const int packed = mine | (cumt << 16);
-    const int incl = wave_incl_scan_i(packed);
-    // the first lane whose inclusive total reaches Kt holds the cut bucket; the rest is scalar arithmetic on that
-    // lane's four counts
-    const unsigned long long who = __ballot((incl & 0xffff) >= Kt);
-    bool found = false;
-    int cut = 255, tot = 0, before_me = 0, above_cut = 0, before_above = 0;
-    if (who != 0ull) {
-      const int src = __ffsll((long long)who) - 1;
-      const int ex = __builtin_amdgcn_readlane(incl - packed, src);  // exclusive sums at that lane
-      int run = ex & 0xffff;
-      before_me = ex >> 16;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int cu = __builtin_amdgcn_readlane(c[u], src), mu = __builtin_amdgcn_readlane(cum[u], src);
-        if (!found) {
-          run += cu;
-          before_me += mu;
-          if (run >= Kt) {
-            found = true;
-            above_cut = run - cu;
-            before_above = before_me - mu;
-            cut = 4 * src + u;
-            tot = run;
-          }
-        }
-      }
-    }
-    return {found, cut, tot, above_cut, before_me, before_above};
+    for (int u = 0; u < 4; ++u) pk[u] = c[u] | (cum[u] << 16);
+    const int packed = (pk[0] + pk[1]) + (pk[2] + pk[3]);
+    const int incl = wave_incl_scan_i(packed);
+    // the first lane whose inclusive total reaches Kt holds the cut bucket; every lane finds the bucket that would be the cut were
+    // it that lane
+    const unsigned long long who = __builtin_amdgcn_ballot_w64((incl & 0xffff) >= Kt);
+    const int r_1 = incl - packed, r0 = r_1 + pk[0], r1 = r0 + pk[1], r2 = r1 + pk[2];  // sums up to the bucket
+    const bool t0 = (r0 & 0xffff) < Kt, t1 = (r1 & 0xffff) < Kt, t2 = (r2 & 0xffff) < Kt;
+    const int with = t2 ? incl : (t1 ? r2 : (t0 ? r1 : r0)), without = t2 ? r2 : (t1 ? r1 : (t0 ? r0 : r_1));
+    const int bucket = 4 * lane + (t0 ? 1 : 0) + (t1 ? 1 : 0) + (t2 ? 1 : 0);
+    const bool found = who != 0ull;
+    const int src = found ? __ffsll((long long)who) - 1 : 63;
+    const uint32_t upto = (uint32_t)__builtin_amdgcn_readlane(with, src), before = (uint32_t)__builtin_amdgcn_readlane(without, src);
+    return {found, __builtin_amdgcn_readlane(bucket, src), (int)(upto & 0xffffu), (int)(before & 0xffffu), (int)(upto >> 16), (int)(before >> 16)};
   };
   for (int hs = wave; HAS_TOPK && !ONE && hs < G * SEG; hs += NW) {
     const int h = hs / SEG, seg = hs % SEG;
@@ -2383,11 +2499,31 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   if constexpr (HAS_V) {  // whatever the emission did not carry (no batch of this wavefront, a short split, the exact selection)
     if (!acc_issued) add_acc_range(0, ACC_TOTAL * 4);
   }
+  // ONE: the outputs' addresses are read from the argument block again here (the compiler keeps what it has read, and with the
+  // streams' own values the scalar registers do not hold it: some twenty of them went to vector lanes), all together ahead of
+  // the barrier: read where each is used they were waited for one after the other (20 x 1000 positions, K3V2, top-k 128
+  // 17.4 us per layer, all together 17.35).
+  struct {
+    int64_t *topk_idx, *topk_slots;
+    float *o_hat, *o_old, *W, *softmax_m, *softmax_inv_z;
+    const uint16_t* blend_o_new;
+    uint16_t* blend_out;
+    int64_t num_slots;
+  } late = {};
+  if constexpr (ONE) {
+    auto args = (const __attribute__((address_space(4))) FusedParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    late = {args->topk_idx, args->topk_slots, args->o_hat, args->o_old, args->W, args->softmax_m, args->softmax_inv_z,
+            args->blend_o_new, args->blend_out, args->num_slots};
+    asm volatile("" : "+s"(late.topk_idx), "+s"(late.topk_slots), "+s"(late.o_hat), "+s"(late.o_old), "+s"(late.W),
+                      "+s"(late.softmax_m), "+s"(late.softmax_inv_z), "+s"(late.blend_o_new), "+s"(late.blend_out), "+s"(late.num_slots));
+    late_o_hat = late.o_hat;
+  }
   if constexpr (HAS_V || ONE) lds_barrier();
   if constexpr (ONE) {
-    if (p.softmax_m && tid < GA) {
-      p.softmax_m[head0 + tid] = tl_m[tid];
-      p.softmax_inv_z[head0 + tid] = tl_iz[tid];
+    if (late.softmax_m && tid < GA) {
+      late.softmax_m[head0 + tid] = tl_m[tid];
+      late.softmax_inv_z[head0 + tid] = tl_iz[tid];
     }
     if constexpr (HAS_V) {
 #pragma unroll
@@ -2400,7 +2536,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     if constexpr (MODE == FS_FULL) {
 #pragma unroll
       for (int it = 0; it < OPT; ++it)  // (no blend: any readable address)
-        o_new[it] = *(p.blend_o_new ? p.blend_o_new + head0 * D + min(it * NT + tid, GA * D - 1) : p.q + head0 * D);
+        o_new[it] = *(late.blend_o_new ? late.blend_o_new + head0 * D + min(it * NT + tid, GA * D - 1) : p.q + head0 * D);
     }
     if constexpr (HAS_TOPK) {
       // More members than a rank list holds: the buckets are linear between the smallest and the largest score, so one
@@ -2431,6 +2567,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         auto for_members = [&](int it, int h, int seg, auto&& f) {  // four scores per lane in flight
           const int tb = seg * (L / SEG);
           const float* srow = sc + h * L;
+#pragma unroll 1  // (unrolled, its lane masks spill)
           for (int i0 = 0; i0 < (SHORT ? STEPS : 32); i0 += 4) {
             float x[4];
             int pos[4];
@@ -2605,8 +2742,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         }
         wave_lds_fence();
         // outputs, and slot and weight for the pre-correction, one winner per lane
-        int64_t* out_idx = p.topk_idx + (head0 + h) * (size_t)K;
-        int64_t* out_slot = p.topk_slots + (head0 + h) * (size_t)K;
+        int64_t* out_idx = late.topk_idx + (head0 + h) * (size_t)K;
+        int64_t* out_slot = late.topk_slots + (head0 + h) * (size_t)K;
         const float M = tl_m[h], iz = tl_iz[h];
         for (int r = base + lane; r < min(count, Kt); r += 64) {
           const int pos = min((int)cl[r], n - 1);
@@ -2614,7 +2751,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           out_idx[r] = pos;
           out_slot[r] = slot;
           if constexpr (HAS_V) {
-            tl_wslot[h * K + r] = (slot >= 0 && slot < p.num_slots) ? slot : -1;
+            tl_wslot[h * K + r] = (slot >= 0 && slot < late.num_slots) ? slot : -1;
             tl_ww[h * K + r] = __expf(srow[pos] - M) * iz;
           }
         }
@@ -2624,15 +2761,15 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         }
       }
     } else {  // Stage B alone: the winners are given (or none)
-      const int n_out = p.topk_idx ? K : 0;
+      const int n_out = late.topk_idx ? K : 0;
       if (tid < G) tl_nout[tid] = 0;
       lds_barrier();
       for (int i = tid; i < GA * n_out; i += NT) {
         const int h = i / K;
-        const int64_t pos = p.topk_idx[head0 * K + i];
+        const int64_t pos = late.topk_idx[head0 * K + i];
         const bool valid = pos >= 0 && pos < n;
         const int slot = valid ? sbase[(int)pos >> 4] + ((int)pos & 15) : -1;
-        tl_wslot[i] = (slot >= 0 && slot < p.num_slots) ? slot : -1;
+        tl_wslot[i] = (slot >= 0 && slot < late.num_slots) ? slot : -1;
         tl_ww[i] = valid ? __expf(sc[h * L + (int)pos] - tl_m[h]) * tl_iz[h] : 0.f;
         // A head's list ends with its last entry that names a position (the padding of a short sequence is not gone
         // over: 1024 entries for eight heads over 16 positions took 50 us).  K >= 32: 32 lanes hold entries of one head.
@@ -2643,64 +2780,89 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     if constexpr (HAS_V) {
       lds_barrier();
       // ---- pre-correction over the winners
-      using Pre = PreCorr<SCHEME % 10>;
-      const int dwi = lane % Pre::DW, w_in = lane / Pre::DW;
-      const int g_of_lane = (NG == 1) ? 0 : ((dwi * Pre::CPD) / (D / NG));
-      // WPH wavefronts per head (more heads than wavefronts: one after the other), each a contiguous-stride share of the
-      // winners, PB requests per lane in flight; one reduction over the lanes per wavefront and head
-      constexpr int WPH = (NW >= G) ? NW / G : 1, PB = (Pre::CPD == 16) ? 8 : 16;
-      static_assert(NW * Lds::WAVE_STAGE >= G * WPH * (D + 1) * 4, "the wavefronts' sums lie in the staging area");
-      float* old_sh = reinterpret_cast<float*>(stage);  // [G][WPH][D] (the accumulator sums are dead)
-      float* w_sh = old_sh + G * WPH * D;               // [G][WPH]
+      // WPH wavefronts per head (more heads than wavefronts: one after the other), which take its winners 64 at a time in turn
+      using Sums = WinnerSums<SCHEME % 10, NG>;
+      constexpr int WPH = (NW >= G) ? NW / G : 1;
+      // a wavefront's staging area: the rows of 64 winners; then (more heads than wavefronts: behind them) the head's sums
+      constexpr int RES_AT = (G > NW) ? Sums::STAGE : 0, RES = (D + 4) * 4;
+      static_assert(Lds::WAVE_STAGE >= Sums::STAGE && Lds::WAVE_STAGE >= RES_AT + (G + NW - 1) / NW * RES, "the sums lie in the staging area");
+      static_assert(Lds::WAVE_STAGE % 16 == 0, "16-byte rows");
+      uint8_t* st = stage + wave * Lds::WAVE_STAGE;
       for (int hw = wave; hw < GA * WPH; hw += NW) {
         const int h = hw / WPH, part = hw % WPH, n_out = HAS_TOPK ? Kt : __builtin_amdgcn_readfirstlane(tl_nout[h]);
-        float acc[Pre::CPD], accw = 0.f;
+        const int* slots = tl_wslot + h * K;
+        const float* weights = tl_ww + h * K;
+        float* res = reinterpret_cast<float*>(st + RES_AT + hw / NW * RES);
+        float wsum = 0.f;
+        if (K <= 32 * WPH) {  // (the correction's width, not the winners': Stage B is given a list of that length)
+          // Few winners: code by code, WPI rows per wavefront instruction, four requests per lane at a time; a shorter chain than
+          // the staged rows'.  1 x 777 positions, K4V4, top-k 64 14.35 us per layer, 14.8 the other way; 16 x 2048, K3V2, 64 20.6 /
+          // 21.7.  (With up to half as many 20 x 1000, K3V2, 128 17.4 us, 17.6 the other way; 24 x 500, G = 8, 32 15.6 / 15.8.)
+          using Pre = PreCorr<SCHEME % 10>;
+          const int dwi = lane % Pre::DW, w_in = lane / Pre::DW;
+          const int g_of_lane = (NG == 1) ? 0 : ((dwi * Pre::CPD) / (D / NG));
+          float acc[Pre::CPD];
 #pragma unroll
-        for (int c = 0; c < Pre::CPD; ++c) acc[c] = 0.f;
-        auto gather = [&](int first, auto count, auto all) JF_INLINE {  // `count` rows per lane (`all`: every one a winner) from winner `first` + part * WPI on
-          constexpr int NU = decltype(count)::value;
-          typename Pre::Row row[NU];
-          uint16_t sb[NU];
-          int slot[NU];
-          float wv[NU];
-          // (all look-ups ahead of all rows: one round trip to LDS instead of one for each row's request)
+          for (int c = 0; c < Pre::CPD; ++c) acc[c] = 0.f;
+          auto gather = [&](int first, auto count) JF_INLINE {  // `count` rows per lane from winner `first` on
+            constexpr int NU = decltype(count)::value;
+            typename Pre::Row row[NU];
+            uint16_t sb[NU];
+            int slot[NU];
+            float wv[NU];
+            // (all look-ups ahead of all rows: one round trip to LDS instead of one for each row's request)
 #pragma unroll
-          for (int u = 0; u < NU; ++u) {
-            const int k = first + (u * WPH + part) * Pre::WPI + w_in, kc = h * K + (decltype(all)::value ? k : min(k, n_out - 1));
-            slot[u] = tl_wslot[kc];
-            wv[u] = tl_ww[kc];
-            if (!decltype(all)::value) slot[u] = (k < n_out) ? slot[u] : -1;
+            for (int u = 0; u < NU; ++u) {
+              const int k = first + (u * WPH + part) * Pre::WPI + w_in, kc = min(k, n_out - 1);
+              const int named = slots[kc];
+              wv[u] = weights[kc];
+              slot[u] = (k < n_out) ? named : -1;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < NU; ++u) {
+              wv[u] = (slot[u] >= 0) ? wv[u] : 0.f;
+              const uint32_t sl = (uint32_t)max(slot[u], 0);
+              row[u] = Pre::fetch(vbase, sl, dwi);
+              sb[u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
+            }
+            if constexpr (Pre::ALL_AHEAD) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < NU; ++u) {
+              Pre::add(row[u], wv[u] * bf16_to_f32(sb[u]), acc);
+              if (dwi == 0) wsum += wv[u];
+            }
+          };
+          constexpr int ROWS = WPH * Pre::WPI;  // winners per row of every lane
+          int first = 0;
+          for (; n_out - first > 2 * ROWS; first += 4 * ROWS) gather(first, std::integral_constant<int, 4>{});
+          if (first < n_out) gather(first, std::integral_constant<int, 2>{});
+          const int chan = Pre::reduce(acc, lane);
+          res[chan] = acc[0];
+          res[chan + 1] = acc[1];
+        } else {
+          float o[8] = {};
+          int first = part * 64;
+          if (first < n_out) {
+            typename Sums::Rows x = Sums::fetch(vbase, vsbase, slots, weights, first, n_out, lane);
+            for (;;) {
+              const bool more = first + WPH * 64 < n_out;  // (uniform)
+              typename Sums::Rows next = x;
+              if (more) next = Sums::fetch(vbase, vsbase, slots, weights, first + WPH * 64, n_out, lane);
+              wsum += x.w;
+              Sums::add(x, st, lane, o);
+              if (!more) break;
+              x = next;
+              first += WPH * 64;
+            }
           }
-          __builtin_amdgcn_sched_barrier(0);
+          if (lane < 16) {
 #pragma unroll
-          for (int u = 0; u < NU; ++u) {
-            wv[u] = (slot[u] >= 0) ? wv[u] : 0.f;
-            const uint32_t sl = (uint32_t)max(slot[u], 0);
-            row[u] = Pre::fetch(vbase, sl, dwi);
-            sb[u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
+            for (int t = 0; t < 8; ++t) res[Tiles::channel(t, lane)] = o[t];
           }
-          if constexpr (Pre::ALL_AHEAD) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int u = 0; u < NU; ++u) {
-            Pre::add(row[u], wv[u] * bf16_to_f32(sb[u]), acc);
-            if (dwi == 0) accw += wv[u];
-          }
-        };
-        // (as many rows as are left: a correction of 64 with four wavefronts per head is four INT4 rows per lane; sixteen,
-        // twelve of them absent, took 9 k cycles at the end of a scan of 777 positions, four 3 k)
-        constexpr int ROWS = WPH * Pre::WPI;  // winners per row of every lane
-        int first = 0;
-        for (; n_out - first >= PB * ROWS; first += PB * ROWS) gather(first, std::integral_constant<int, PB>{}, std::true_type{});
-        while (n_out - first > PB / 4 * ROWS) {
-          gather(first, std::integral_constant<int, PB / 2>{}, std::false_type{});
-          first += PB / 2 * ROWS;
         }
-        if (n_out - first > 0) gather(first, std::integral_constant<int, PB / 4>{}, std::false_type{});
-        const int chan = Pre::reduce(acc, lane);
-        old_sh[hw * D + chan] = acc[0];
-        old_sh[hw * D + chan + 1] = acc[1];
-        const float wsum = wave_sum(accw);
-        if (lane == 0) w_sh[hw] = wsum;
+        wsum = wave_sum(wsum);
+        if (lane == 0) res[D] = wsum;
       }
       lds_barrier();
 #pragma unroll
@@ -2710,14 +2872,16 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         float o = 0.f, wt = 0.f;
 #pragma unroll
         for (int w = 0; w < WPH; ++w) {
-          o += old_sh[(h * WPH + w) * D + d];
-          wt += w_sh[h * WPH + w];
+          const int hw = h * WPH + w;
+          const float* res = reinterpret_cast<const float*>(stage + hw % NW * Lds::WAVE_STAGE + RES_AT + hw / NW * RES);
+          o += res[d];
+          wt += res[D];
         }
-        p.o_old[(head0 + h) * D + d] = o;
-        if (d == 0) p.W[head0 + h] = wt;
-        if (MODE == FS_FULL && p.blend_out) {
+        late.o_old[(head0 + h) * D + d] = o;
+        if (d == 0) late.W[head0 + h] = wt;
+        if (MODE == FS_FULL && late.blend_out) {
           const size_t at = (head0 + h) * D + d;
-          p.blend_out[at] = f32_to_bf16(__builtin_fmaf(wt, bf16_to_f32(o_new[it]), tl_ohat[h * D + d]) - o);
+          late.blend_out[at] = f32_to_bf16(__builtin_fmaf(wt, bf16_to_f32(o_new[it]), tl_ohat[h * D + d]) - o);
         }
       }
     }
