@@ -553,7 +553,7 @@ template <int VBITS, int NG>
 struct WinnerSums {
   using Tiles = VTiles<VBITS, NG>;
   static constexpr int PIECES = Tiles::VP / 16;
-  static constexpr int STAGE = Tiles::VST + NG * 1024;  // LDS per wavefront: the rows, and a 16-byte weight row per winner and group
+  static constexpr int STAGE = Tiles::VST + 1024;  // LDS per wavefront: the rows, and a 16-byte weight row per winner
   struct Rows {
     v4u r[PIECES];
     uint32_t s;  // scale word
@@ -581,11 +581,16 @@ struct WinnerSums {
       x.r[i] = *reinterpret_cast<const v4u*>(vbase + (size_t)((uint32_t)max(slot[i], 0) * (uint32_t)Tiles::VP + (uint32_t)(1024 * i + 16 * lane) % Tiles::VP));
     return x;
   }
-  // o[t] += the sums of tile t, column lane (lanes 0 .. 15; the other lanes' are of no use)
-  static __device__ JF_INLINE void add(const Rows& x, uint8_t* st, int lane, float (&o)[8]) {
+  // channel of o[i] in `add`
+  static __device__ inline int channel(int lane, int i) { return Tiles::channel(2 * (lane >> 4) + i, lane & 15); }
+  // o[0], o[1] += the sums of two channels per lane.  A weight row holds the limbs four times, once for each lane group of the
+  // products (the first two take the first scale group's, the others the second's).  Tiles 2q and 2q + 1 are multiplied with the
+  // rows of lane group q alone, so two accumulators hold all eight and every lane has two channels.
+  static __device__ JF_INLINE void add(const Rows& x, uint8_t* st, int lane, float (&o)[2]) {
     uint8_t* wl = st + Tiles::VST;
     float top[NG];
     int E[NG];
+    uint32_t limbs[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       const float v = x.w * bf16_to_f32((uint16_t)(g ? x.s >> 16 : x.s & 0xffffu));
@@ -601,52 +606,51 @@ struct WinnerSums {
       }
       E[g] = 24 - e;
       const uint32_t w = (uint32_t)rintf(f);
-      *reinterpret_cast<uint32_t*>(wl + (g * 64 + lane) * 16) = (w & 0x7fu) | ((w << 1) & 0x7f00u) | ((w << 2) & 0x7f0000u) | ((w << 3) & 0x7f000000u);
+      limbs[g] = (w & 0x7fu) | ((w << 1) & 0x7f00u) | ((w << 2) & 0x7f0000u) | ((w << 3) & 0x7f000000u);
     }
+    *reinterpret_cast<v4u*>(wl + lane * 16) = (v4u){limbs[0], limbs[0], limbs[NG - 1], limbs[NG - 1]};
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) Tiles::stash_piece(st, (1024 * i + 16 * lane) / Tiles::VP, (1024 * i + 16 * lane) % Tiles::VP / 16, x.r[i]);
     wave_lds_fence();
     const uint8_t* wrow = wl + ((lane >> 4) * 16 + tr8_token(lane)) * 16 + (lane & 1) * 8;
-    v4i A[NG], sw[NG], acc[8];
-    const v4i zero = {0, 0, 0, 0}, ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    const v2i x0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(wrow));
+    const v2i x1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(wrow + 128));
+    const v4i A = {x0[0], x0[1], x1[0], x1[1]}, zero = {0, 0, 0, 0}, ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    const v4i sw = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, ones, zero, 0, 0, 0);
+    v4i acc[2] = {zero, zero};
+    Tiles::spread(st, lane, [&](auto tile, int, const v4i& B) JF_INLINE {
+      constexpr int t = decltype(tile)::value;
+      const bool own = ((lane & 15) >> 2) == t / 2;  // (lane: a row of the operand)
+      v4i Aq;
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      const v2i x0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(wrow + g * 1024));
-      const v2i x1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)(wrow + g * 1024 + 128));
-      A[g] = (v4i){x0[0], x0[1], x1[0], x1[1]};
-      sw[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g], ones, zero, 0, 0, 0);
-    }
-    Tiles::spread(st, lane, [&](auto tile, int g, const v4i& B) JF_INLINE {
-      acc[decltype(tile)::value] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[g], B, zero, 0, 0, 0);
+      for (int c = 0; c < 4; ++c) Aq[c] = own ? A[c] : 0;
+      acc[t & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aq, B, acc[t & 1], 0, 0, 0);
     });
-    int lo[NG], hi[NG];
+    const int lo = Tiles::OFFSET * (sw[0] + (sw[1] << 7)), hi = Tiles::OFFSET * (sw[2] + (sw[3] << 7));
+    const bool upper = (lane & 32) != 0;
+    const float factor = upper ? top[NG - 1] : top[0];
+    const int e = upper ? E[NG - 1] : E[0];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      lo[g] = Tiles::OFFSET * (sw[g][0] + (sw[g][1] << 7));
-      hi[g] = Tiles::OFFSET * (sw[g][2] + (sw[g][3] << 7));
-    }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int g = (NG == 1) ? 0 : t / 4, m = Tiles::times(t);
+    for (int i = 0; i < 2; ++i) {
+      constexpr int m[2] = {Tiles::times(0), Tiles::times(1)};
+      const v4i a = acc[i];
       // (both below 2^24: floats hold them)
-      const float a = (float)(acc[t][0] + (acc[t][1] << 7) - m * lo[g]), b = (float)(acc[t][2] + (acc[t][3] << 7) - m * hi[g]);
-      const float sum = __builtin_fmaf(b, 16384.f, a) * (m == 4 ? 0.25f : 1.f);
-      o[t] += isfinite(top[g]) ? ldexpf(sum, -E[g]) : sum * top[g];
+      const float low = (float)(a[0] + (a[1] << 7) - m[i] * lo), high = (float)(a[2] + (a[3] << 7) - m[i] * hi);
+      const float sum = __builtin_fmaf(high, 16384.f, low) * (m[i] == 4 ? 0.25f : 1.f);
+      o[i] += isfinite(factor) ? ldexpf(sum, -e) : sum * factor;
     }
     wave_lds_fence();
   }
 };
 
-// Pre-correction terms over the winners' packed V rows, shared by the merge kernel and the scan's in-kernel merge: DW
-// lanes per row, lane dwi holds dword dwi of it (INT2, INT4) or two bytes of each of the three planes (INT3) = CPD
-// codes; a wavefront instruction covers WPI rows, sixteen wavefronts (or roles) and UNR requests per lane 256 rows.
+// The same terms code by code, for few winners of a scan that merges by itself: DW lanes per row, lane dwi holds dword dwi of it
+// (INT2, INT4) or two bytes of each of the three planes (INT3) = CPD codes; a wavefront instruction covers WPI rows.
 template <int VBITS>
 struct PreCorr {
   static constexpr int VP = D * VBITS / 8;
   static constexpr int DW = (VBITS == 3) ? 8 : VP / 4;
   static constexpr int CPD = (VBITS == 3) ? 16 : 32 / VBITS;
   static constexpr int WPI = 64 / DW;
-  static constexpr int UNR = (256 / (16 * WPI) > 0) ? 256 / (16 * WPI) : 1;
   // INT3: all rows of a batch are requested before the first is used.  Left to itself the compiler requests a row or two and
   // waits: 19 sequences x 16 heads over 4 kv-heads, 4955 positions, K4V3, top-k 512 38.4 us, 36.3 with this.  (The others' one
   // load per row goes ahead anyway, and holding all of them costs registers: 28 x 32 heads over 4 kv-heads, 887 positions,
@@ -2794,7 +2798,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         const float* weights = tl_ww + h * K;
         float* res = reinterpret_cast<float*>(st + RES_AT + hw / NW * RES);
         float wsum = 0.f;
-        if (K <= 32 * WPH) {  // (the correction's width, not the winners': Stage B is given a list of that length)
+        if (K <= 16 * WPH) {  // (the correction's width, not the winners': Stage B is given a list of that length)
           // Few winners: code by code, WPI rows per wavefront instruction, four requests per lane at a time; a shorter chain than
           // the staged rows'.  1 x 777 positions, K4V4, top-k 64 14.35 us per layer, 14.8 the other way; 16 x 2048, K3V2, 64 20.6 /
           // 21.7.  (With up to half as many 20 x 1000, K3V2, 128 17.4 us, 17.6 the other way; 24 x 500, G = 8, 32 15.6 / 15.8.)
@@ -2841,7 +2845,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
           res[chan] = acc[0];
           res[chan + 1] = acc[1];
         } else {
-          float o[8] = {};
+          float o[2] = {};
           int first = part * 64;
           if (first < n_out) {
             typename Sums::Rows x = Sums::fetch(vbase, vsbase, slots, weights, first, n_out, lane);
@@ -2856,10 +2860,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
               first += WPH * 64;
             }
           }
-          if (lane < 16) {
 #pragma unroll
-            for (int t = 0; t < 8; ++t) res[Tiles::channel(t, lane)] = o[t];
-          }
+          for (int i = 0; i < 2; ++i) res[Sums::channel(lane, i)] = o[i];
         }
         wsum = wave_sum(wsum);
         if (lane == 0) res[D] = wsum;
@@ -2970,28 +2972,41 @@ constexpr int MG_LIGHT_THREADS = 256, MG_LIGHT_REGK = 16, MG_LIGHT_TOPK = 512;  
 // new candidate list; the final merge (PARTIAL = false, mg_parts > 1) reads these lists instead of the
 // scan's.  The top K of a union is the top K of the parts' top K's, ties included: a candidate that a part
 // drops is beaten by K candidates of that part.
-template <int MODE, int VBITS, int NG, int MG_THREADS, int MG_REGK, bool PARTIAL, bool WIDE = false, int ROLES = 1>
-__global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void fused_merge_kernel(MergeParams p) {  // (wavefronts per SIMD: four workgroups of the gather for all roles)
+template <int MODE, int VBITS, int NG, int MG_THREADS, int MG_REGK, bool PARTIAL, bool WIDE = false, int PER_CU = 1>
+__global__ __launch_bounds__(MG_THREADS, PER_CU == 4 ? 4 : MG_THREADS / 256) void fused_merge_kernel(MergeParams p) {
   static_assert(!(PARTIAL && MODE == FS_STAGE_B), "Stage B alone selects nothing");
   constexpr int MG_WAVES = MG_THREADS / 64;
-  using Pre = PreCorr<VBITS>;
-  constexpr int DW = Pre::DW, CPD = Pre::CPD;  // lanes per winner row, codes per lane
-  constexpr int WPI = Pre::WPI;         // winners per wavefront instruction
+  // PER_CU = 4, light shape: four workgroups per CU are all there are, and a wavefront has registers for the rows of both its turns
+  constexpr bool AHEAD = PER_CU == 4;
   // The floating-point sums (o_hat over the splits, the pre-correction terms over the winners) are organised
-  // as if eight thread groups of 128 and sixteen wavefronts were at work, whatever MG_THREADS is: a smaller
+  // as if eight thread groups of 128 and eight wavefronts were at work, whatever MG_THREADS is: a smaller
   // workgroup takes several of those roles one after the other, so every shape of this kernel adds the same
   // numbers in the same order and the results do not depend on which shape the launcher picks.
-  constexpr int VGRP = 8, VWAVES = 16;
-  static_assert(MG_THREADS % D == 0 && VGRP % (MG_THREADS / D) == 0 && VWAVES % MG_WAVES == 0, "whole roles per thread group / wavefront");
+  constexpr int VGRP = 8;
+  static_assert(MG_THREADS % D == 0 && VGRP % (MG_THREADS / D) == 0 && (MG_WAVES >= VGRP || VGRP % MG_WAVES == 0), "whole roles per thread group / wavefront");
   // the light shape (many rows per launch, few candidates per row) trades table sizes for workgroups per CU
   constexpr int MG_BT = (MG_THREADS >= 1024) ? MG_BT_LDS : 1024;  // block-table entries cached in LDS
   constexpr int MG_WIN = (MG_THREADS >= 1024) ? FS_LDS_TOPK : 512;  // widest correction of this shape (WIDE: any)
   // (the shape of 32 candidates per thread meets wide corrections, whose cut lies where the scores are densest: twice the buckets)
   constexpr int BINS = (MG_REGK > 16) ? 2 * MG_BINS : MG_BINS;
-  __shared__ __align__(16) int hist[BINS];
-  __shared__ uint32_t lkey[MG_LIST];
+  // The sums over the winners need a staging area; what the selection needs lies in the same place (a barrier lies between).  Side by
+  // side the two took the 1024-thread shape longer to start than they saved: 16 sequences x 4096 positions, K3V2, top-k 1024 46.6 us
+  // per layer, this 46.0; 1 x 131072, K4V4, 512 46.4 / 46.05.
+  using Sums = WinnerSums<VBITS, NG>;
+  constexpr bool HAS_SUMS = !PARTIAL && MODE != FS_STAGE_A;
+  constexpr int SUM_WAVES = MG_WAVES < VGRP ? MG_WAVES : VGRP;
+  constexpr int EARLY = (BINS + MG_LIST + MG_BT + VGRP * D) * 4, AREAS = (AHEAD && VBITS < 4) ? 2 : 1,  // one for each turn (INT4 rows: that would be three workgroups per CU)
+                STAGED = HAS_SUMS ? AREAS * SUM_WAVES * Sums::STAGE : 0;
+  __shared__ __align__(16) uint8_t pool[!HAS_SUMS ? 16 : (EARLY > STAGED ? EARLY : STAGED)];
+  __shared__ __align__(16) int hist_s[HAS_SUMS ? 1 : BINS];
+  __shared__ uint32_t lkey_s[HAS_SUMS ? 1 : MG_LIST];
+  __shared__ int bt_s[HAS_SUMS ? 1 : MG_BT];
+  __shared__ float red_s[HAS_SUMS ? 1 : VGRP][D];
+  int* const hist = HAS_SUMS ? reinterpret_cast<int*>(pool) : hist_s;
+  uint32_t* const lkey = HAS_SUMS ? reinterpret_cast<uint32_t*>(pool) + BINS : lkey_s;
+  int* const bt_sh = HAS_SUMS ? reinterpret_cast<int*>(pool) + BINS + MG_LIST : bt_s;
+  float (*const red_sh)[D] = HAS_SUMS ? reinterpret_cast<float (*)[D]>(pool + (BINS + MG_LIST + MG_BT) * 4) : red_s;
   __shared__ int lpos[MG_RANK];  // candidate number of the first members
-  __shared__ int bt_sh[MG_BT];
   // winners: key and position while they are selected; the thread that turns winner r into its softmax weight and
   // paged slot overwrites the two entries in place (weight bits over the key, slot over the position)
   // (WIDE, corrections beyond FS_LDS_TOPK: the two arrays are the launch's dynamic LDS, top_k entries each)
@@ -3000,10 +3015,9 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
   extern __shared__ __align__(16) uint32_t win_dyn[];
   uint32_t* const win_key = WIDE ? win_dyn : win_key_s;
   int* const win_idx = WIDE ? reinterpret_cast<int*>(win_dyn + p.top_k) : win_idx_s;
-  __shared__ float red_sh[VGRP][D];
-  __shared__ float old_sh[VWAVES][D];
+  __shared__ float sum_sh[HAS_SUMS ? SUM_WAVES : 1][D];
   __shared__ float ohat_sh[D];
-  __shared__ float w_sh[VWAVES];
+  __shared__ float w_sh[VGRP];
   __shared__ uint32_t wred_u[MG_WAVES], wred_k[MG_WAVES];
   __shared__ int wred_i[MG_WAVES], wred_j[MG_WAVES];
   __shared__ int lcount_sh, quota_sh;
@@ -3599,110 +3613,75 @@ __global__ __launch_bounds__(MG_THREADS, ROLES == 4 ? 4 : MG_THREADS / 256) void
   lds_barrier();
   if (mclk && tid == 0) mclk[4] = JF_CLK();
 
-  // ---- pre-correction over the winners.  One winner row per DW lanes: lane (w_in, dwi) holds dword dwi of
-  // the winner's packed V row (CPD codes) and accumulates its CPD channels; winners are visited in a fixed
-  // order, so the sums are run-to-run deterministic.  UNR rows per lane are requested before any is used.
-  const uint8_t* vbase = p.v_data + (size_t)hkv * p.num_slots * Pre::VP;
-  const uint8_t* vsbase = reinterpret_cast<const uint8_t*>(p.v_scales + (size_t)hkv * p.num_slots * NG);
-  const int dwi = lane % DW, w_in = lane / DW;
-  const int g_of_lane = (NG == 1) ? 0 : ((dwi * CPD) / (D / NG));
-  constexpr int UNR = Pre::UNR;  // 256 winners per pass
-  // A workgroup of fewer than sixteen wavefronts takes several roles per wavefront, ROLES at a time: the rows of those are
-  // requested together.  All four at once: one gather latency instead of four, 101 - 125 registers and so four workgroups
-  // of the light shape per CU; one at a time: 73, five workgroups, and no rows fetched for roles without winners.  Per
-  // layer, one / four at a time: 16 sequences x 32 heads, 700 positions, K4V4, top-k 256 37.1 / 36.3 us; 32 x 64 heads of
-  // 512, top-k 128 53.6 / 55.6; 22 x 128 heads of 39, INT4 with 64-channel groups, top-k 128 54.8 / 60.8.
-  constexpr int RPW = VWAVES / MG_WAVES, RP = ROLES;
-  static_assert(RPW % RP == 0, "whole turns");
-#pragma unroll
-  for (int r0 = 0; r0 < RPW; r0 += RP) {
-    float acc[RP][CPD], accw[RP];
-#pragma unroll
-    for (int r = 0; r < RP; ++r) {
-      accw[r] = 0.f;
-#pragma unroll
-      for (int c = 0; c < CPD; ++c) acc[r][c] = 0.f;
-    }
-    auto gather = [&](int kb, auto count) JF_INLINE {  // `count` rows per lane and role from winner kb on
-      constexpr int NU = decltype(count)::value;
-      typename Pre::Row row[RP][NU];
-      uint16_t sbits[RP][NU];
-      int slot[RP][NU];
-      float wv[RP][NU];
-      // (all look-ups ahead of all rows: one round trip to LDS instead of one for each row's request)
-#pragma unroll
-      for (int r = 0; r < RP; ++r)
-#pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          const int k = kb + (r * MG_WAVES + u * VWAVES) * WPI + w_in, kc = min(k, n_out - 1);
-          const int named = win_idx[kc];
-          wv[r][u] = __builtin_bit_cast(float, win_key[kc]);
-          slot[r][u] = (k < n_out) ? named : -1;
+  // ---- pre-correction over the winners, 64 at a time on the matrix cores, in eight groups whatever MG_THREADS is (four
+  // wavefronts: two groups each, added as the first step of the sum over eight would).  What a conversion and a multiply-add per
+  // code in all wavefronts took instead, per layer: 32 sequences x 3000 positions, K4V4, top-k 2048 100.5 us, this 95.0; 32 x 3000,
+  // K3V2, 1024 66.4 / 64.1; 24 x 2500, eight heads, K3V2, 512 72.7 / 69.7; 32 x 6000, K3V2, 256 58.8 / 56.8; 12 x 8192, K4V4, 64
+  // 33.4 / 31.6; 16 of 983 .. 16384, K4V4, 256 60.2 / 59.1; 4 x 32768, K3V2, 256 34.4 / 34.2.
+  if constexpr (HAS_SUMS) {
+    const uint8_t* vbase = p.v_data + (size_t)hkv * p.num_slots * Sums::Tiles::VP;
+    const uint8_t* vsbase = reinterpret_cast<const uint8_t*>(p.v_scales + (size_t)hkv * p.num_slots * NG);
+    if (wave < SUM_WAVES) {
+      uint8_t* st = pool + wave * Sums::STAGE;
+      auto fetch = [&](int first) JF_INLINE { return Sums::fetch(vbase, vsbase, win_idx, reinterpret_cast<const float*>(win_key), first, n_out, lane); };
+      float sum[2] = {}, wsum = 0.f;
+      if constexpr (AHEAD) {  // (at most 512 winners: two turns of 64)
+        static_assert(VGRP == 2 * SUM_WAVES && MG_WIN <= VGRP * 64, "a turn for each of two groups");
+        const int second = (wave + SUM_WAVES) * 64;
+        if (wave * 64 < n_out) {
+          const typename Sums::Rows x = fetch(wave * 64), y = fetch(min(second, n_out - 1));
+          __builtin_amdgcn_sched_barrier(0);
+          Sums::add(x, st, lane, sum);
+          wsum = wave_sum(x.w);
+          if (second < n_out) {  // (uniform)
+            float o[2] = {};
+            Sums::add(y, st + (AREAS - 1) * SUM_WAVES * Sums::STAGE, lane, o);
+            sum[0] += o[0];
+            sum[1] += o[1];
+            wsum += wave_sum(y.w);
+          }
         }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < RP; ++r)
-#pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          wv[r][u] = (slot[r][u] >= 0) ? wv[r][u] : 0.f;
-          const uint32_t sl = (uint32_t)max(slot[r][u], 0);
-          row[r][u] = Pre::fetch(vbase, sl, dwi);
-          sbits[r][u] = *reinterpret_cast<const uint16_t*>(vsbase + (size_t)(sl * (uint32_t)(NG * 2)) + g_of_lane * 2);
+      } else {
+#pragma unroll 1
+        for (int vg = wave; vg < VGRP; vg += SUM_WAVES) {
+          float o[2] = {}, ws = 0.f;
+#pragma unroll 1
+          for (int first = vg * 64; first < n_out; first += VGRP * 64) {
+            const typename Sums::Rows x = fetch(first);
+            ws += x.w;
+            Sums::add(x, st, lane, o);
+          }
+          sum[0] += o[0];
+          sum[1] += o[1];
+          wsum += wave_sum(ws);
         }
-      if constexpr (Pre::ALL_AHEAD) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < RP; ++r)
-#pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          const float ws = wv[r][u] * bf16_to_f32(sbits[r][u]);  // zero for padding rows
-          Pre::add(row[r][u], ws, acc[r]);
-          if (dwi == 0) accw[r] += wv[r][u];
-        }
-    };
-    const int kb0 = (wave + r0 * MG_WAVES) * WPI;
-    if constexpr (ROLES == 1 && UNR > 1) {
-      // (narrow corrections, and the end of wide ones: no rows are fetched for winners there are none of.  Behind the loop: a
-      // choice between the two bodies inside it made 2048 winners' sums 25 to 35 % longer, 17.8 -> 24.5 k cycles.  Not with
-      // several roles at a time, where the second body costs INT2 and INT3 values 158 registers instead of 111 to 125, three
-      // workgroups per CU instead of four.  Per layer, K3V2, top-k 256, three / four: 32 sequences x 32 heads, 8192 positions
-      // 73.0 / 68.0 us, 16 x 64 of 6000 62.3 / 55.4; K3V3 32 x 32 of 8192 80.4 / 75.3.)
-      int done = 0;
-      for (; n_out - done > VWAVES * WPI; done += UNR * VWAVES * WPI) gather(kb0 + done, std::integral_constant<int, UNR>{});
-      if (kb0 + done < n_out) gather(kb0 + done, std::integral_constant<int, 1>{});
-    } else {
-      for (int kb = kb0; kb < n_out; kb += UNR * VWAVES * WPI) gather(kb, std::integral_constant<int, UNR>{});
-    }
-#pragma unroll
-    for (int r = 0; r < RP; ++r) {  // over the WPI winners of a wavefront instruction; then over the roles through LDS
-      const int vw = wave + (r0 + r) * MG_WAVES;
-      const int chan = Pre::reduce(acc[r], lane);
-      old_sh[vw][chan] = acc[r][0];
-      old_sh[vw][chan + 1] = acc[r][1];
-      const float wsum = wave_sum(accw[r]);  // only the dwi == 0 lanes hold weights
-      if (lane == 0) w_sh[vw] = wsum;
-    }
-  }
-  lds_barrier();
-  if (tid < D) {
-    float o16[VWAVES], w16[VWAVES];
-#pragma unroll
-    for (int w = 0; w < VWAVES; ++w) {
-      o16[w] = old_sh[w][tid];
-      w16[w] = w_sh[w];
-    }
-#pragma unroll
-    for (int n = VWAVES / 2; n >= 1; n /= 2) {  // fixed order
-#pragma unroll
-      for (int w = 0; w < n; ++w) {
-        o16[w] += o16[w + n];
-        w16[w] += w16[w + n];
       }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) sum_sh[wave][Sums::channel(lane, i)] = sum[i];
+      if (lane == 0) w_sh[wave] = wsum;
     }
-    const float o = o16[0], wt = w16[0];  // (the same wt in every thread)
-    p.o_old[bh * D + tid] = o;
-    if (tid == 0) p.W[bh] = wt;
-    // the blend of jetfire_vllm/csrc/blend.cu:202-226 for callers that hold o_new already
-    if (MODE == FS_FULL && p.blend_out) p.blend_out[bh * D + tid] = f32_to_bf16(__builtin_fmaf(wt, bf16_to_f32(blend_raw), ohat_sh[tid]) - o);
+    lds_barrier();
+    if (tid < D) {
+      float o8[SUM_WAVES], w8[SUM_WAVES];
+#pragma unroll
+      for (int q = 0; q < SUM_WAVES; ++q) {
+        o8[q] = sum_sh[q][tid];
+        w8[q] = w_sh[q];
+      }
+#pragma unroll
+      for (int n = SUM_WAVES / 2; n >= 1; n /= 2) {  // fixed order
+#pragma unroll
+        for (int q = 0; q < n; ++q) {
+          o8[q] += o8[q + n];
+          w8[q] += w8[q + n];
+        }
+      }
+      const float o = o8[0], wt = w8[0];  // (the same wt in every thread)
+      p.o_old[bh * D + tid] = o;
+      if (tid == 0) p.W[bh] = wt;
+      // the blend of jetfire_vllm/csrc/blend.cu:202-226 for callers that hold o_new already
+      if (MODE == FS_FULL && p.blend_out) p.blend_out[bh * D + tid] = f32_to_bf16(__builtin_fmaf(wt, bf16_to_f32(blend_raw), ohat_sh[tid]) - o);
+    }
   }
   if (mclk && tid == 0) mclk[5] = JF_CLK();
 }
@@ -4186,12 +4165,12 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
                    (p.mg_parts > 1 ? (long long)p.mg_parts * top_k : (long long)p.n_splits * p.Kc) > MG_REG_CANDS;
   // Many rows with few candidates each (large batches of short or medium sequences): four wavefronts per row and
   // small tables, so that five rows share a CU instead of one (measured from 257 rows up: 42.5 against 47.5 us per
-  // layer at 384 rows of 2048 candidates, 38 against 57 at 1024 rows of 512).  Same results (see VGRP / VWAVES in
+  // layer at 384 rows of 2048 candidates, 38 against 57 at 1024 rows of 512).  Same results (see VGRP in
   // the kernel).
   const bool light = (MODE == FS_FULL) && !big && p.mg_parts == 1 && top_k <= MG_LIGHT_TOPK &&
                      (long long)B * H_q > (long long)device_cus() && (long long)p.n_splits * p.Kc <= MG_LIGHT_THREADS * MG_LIGHT_REGK;
-  // its gathers all at once where four workgroups per CU hold every row and most roles have winners (see ROLES)
-  const bool gather = light && (long long)B * H_q <= 4ll * device_cus() && top_k >= 256 && max_S >= 256;
+  // the rows of both of a wavefront's turns at once where there are two and four workgroups per CU hold every row (see PER_CU)
+  const bool gather = light && top_k > 256 && (long long)B * H_q <= 4ll * device_cus();
   (void)gather;
 #define JF_MERGE(VB, NGG)                                                                                            \
   do {                                                                                                               \

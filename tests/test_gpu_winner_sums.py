@@ -1,0 +1,62 @@
+"""Sums over the winners' value rows, 64 at a time with 24-bit weights: rows whose scales lie far apart, an infinite scale or a
+NaN among them, and one in a slot that only padding names; in the scan that merges by itself and both shapes of the merge."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import jetfire_oracle as O
+from tests.helpers import bits_to_bf16, make_case, to_device
+from tests.test_gpu_fused import run_fused
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(x):
+    return O.f32_to_bf16_bits(np.asarray(x, np.float32))
+
+
+@pytest.mark.parametrize("kind", ["range", "infinite", "nan", "unused"])
+@pytest.mark.parametrize("copies,split_len,K", [(1, 768, 64), (1, 768, 256), (1, 256, 64), (1, 256, 512), (20, 256, 256), (20, 256, 512)])
+@pytest.mark.parametrize("scheme,kb,vb,gs", [("k3v2", 3, 2, 64), ("k3v2", 3, 2, 128), ("k3v3", 3, 3, 64), ("k4v4", 4, 4, 128), ("b4v4", 4, 4, 64)])
+def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
+    from jetfire_amd import _lib
+    S, G, Hkv = 700, 8, 2
+    lens = [S, 70] * copies
+    c = make_case(101, len(lens), G * Hkv, Hkv, S, kb, vb, gs, lens=lens, extra_blocks=1)
+    c["bt"] = (np.random.default_rng(5).permutation(c["bt"].size) + 1).reshape(c["bt"].shape).astype(np.int64)  # (block 0: nobody's)
+    d = to_device(c)
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
+    try:
+        if kind != "range":
+            out = [t.cpu().numpy() for t in run_fused(scheme, c, d, S, K)]
+            bad = np.float32(np.nan if kind == "nan" else np.inf)
+            slot = 0 if kind == "unused" else int(out[1][0, 0, 5])
+            c["vs"][0, slot, -1] = _bits([bad])[0]
+        else:
+            vs = O.bf16_bits_to_f32(c["vs"])
+            c["vs"] = _bits(vs * np.exp2(np.random.default_rng(6).integers(-20, 21, vs.shape)).astype(np.float32))
+        d["vs"] = bits_to_bf16(c["vs"]).cuda()
+        out = [t.cpu().numpy() for t in run_fused(scheme, c, d, S, K)]
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    _, slots, o_old, W, idx, m, iz, scores = out
+    codes = O.decode_codes(c["vd"], vb).astype(np.float64) - O.offset(vb)
+    vs = O.bf16_bits_to_f32(c["vs"]).astype(np.float64)
+    for b in range(2):      # (the others are further copies)
+        for hq in range(G * Hkv):
+            won = idx[b, hq] >= 0
+            p = np.exp(scores[b, hq, idx[b, hq][won]].astype(np.float64) - m[b, hq]) * iz[b, hq]
+            sl = slots[b, hq][won]
+            for g in range(128 // gs):
+                w = p * vs[hq // G, sl, g]
+                got = o_old[b, hq, g * gs:(g + 1) * gs]
+                if not np.isfinite(w).all():
+                    assert not np.isfinite(got).any(), (b, hq, g)
+                    continue
+                v = codes[hq // G, sl, g * gs:(g + 1) * gs]
+                # the weights' own fp32 error (scores, exponential, products): 4e-6 of the sum of magnitudes; half a unit of 24
+                # bits of the largest for each of 64 weights and codes of up to 8
+                top = sum(w[i:i + 64].max(initial=0.0) for i in range(0, len(w), 64))
+                tol = 4e-6 * (w[:, None] * np.abs(v)).sum(0) + 64 * 8 * 2.0 ** -25 * top
+                assert (np.abs(got - (w[:, None] * v).sum(0)) <= tol).all(), (b, hq, g)
+            assert abs(W[b, hq] - p.sum()) <= 4e-6 * max(1.0, p.sum())
