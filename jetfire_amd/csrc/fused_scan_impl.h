@@ -292,9 +292,9 @@ struct ScanLds {
   static constexpr int SCT = 8 * NG;
   static constexpr bool SPREP = (K3 || (K2 && !KA)) && (WAVE_STAGE >= KST + 64 * SCT);
   static constexpr int ACC_REGS = 8 + NG;                   // v4i accumulators per set: 8 channel tiles + NG weight sums
-  // sum of the wavefronts' accumulators: one int per (set, accumulator register, component, lane), in the staging
+  // sum of the wavefronts' accumulators: two ints per (set, accumulator register, lane) and one per (set, tile, column), in the staging
   // area (dead after phase B), followed by one kilobyte per wavefront for the exact selection's histogram
-  static constexpr int XACC = NSET * ACC_REGS * 4 * 64 * 4;
+  static constexpr int XACC = NSET * (ACC_REGS * 2 * 64 + 8 * 16) * 4;
   static constexpr int PREP = KLIMB ? (int)sizeof(K3Prep<NSET>) : (int)sizeof(QInt8F<NSET>);
   // selection histograms: 32-bit counters, or (any INT4 side, where the staging areas are larger and LDS is
   // tighter) two 16-bit counters per word: a (head, segment) histogram counts at most LMAX / SEG <= 4096 positions
@@ -2022,8 +2022,10 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // at a time along the comparisons of its first emission blocks: they drain in the LDS pipe while the vector ALU
   // works.
   // D layout: row r of a tile sits in lane 16*(r>>2) + column, register r&3; row 4*head + l is limb l for l < 3 and
-  // the constant row (75 * sum of codes) for l = 3.  Item j = (register i = j >> 2 of set i / AR, component j & 3)
-  // lives at xacc[j * 64 + lane].
+  // the constant row (75 * sum of codes) for l = 3.  The two lower limbs go in as one number, 256 * limb 1 + limb 0 (at most
+  // 4096 * 128 * 257 * 15 in size: 31 bits), and the constant rows, which are the same for every head, from the first lane group
+  // alone.  Item j = 2 * (register i of set i / AR) + {0: lower limbs, 1: limb 2} lies at xacc[j * 64 + lane], the constant row of
+  // tile t of set s behind all items, at [(s * 8 + t) * 16 + column].
   int* xacc = reinterpret_cast<int*>(stage);
   // ONE: what the in-kernel merge keeps behind the staging area (see ScanTail)
   using Tail = ScanTail<G, SEG>;
@@ -2056,16 +2058,22 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       tl_iz[tid] = (l > 0.f) ? 1.0f / l : 0.f;
     }
   }
-  constexpr int ACC_TOTAL = NSET * AR, ACC_HALF = (ACC_TOTAL + 1) / 2;
+  constexpr int ACC_ITEMS = NSET * AR * 2, ACC_HALF = NSET * AR;
   // (uniform) this wavefront's sums are on their way (or it had no chunk: a short split occupies a few wavefronts only)
   bool acc_issued = wave >= nch;
   auto add_acc_range = [&](const int first, const int last) {  // (constants once the caller's loop is unrolled)
 #pragma unroll
-    for (int j = 0; j < ACC_TOTAL * 4; ++j) {
+    for (int j = 0; j < ACC_ITEMS; ++j) {
       if (j < first || j >= last) continue;
-      const int i = j >> 2, c = j & 3, set = i / AR, r = i % AR;
+      const int i = j >> 1, set = i / AR, r = i % AR;
       const v4i v = (r < NTILE) ? acc[set][r < NTILE ? r : 0] : accw[set][r >= NTILE ? r - NTILE : 0];
-      atomicAdd(xacc + j * 64 + lane, v[c]);
+      atomicAdd(xacc + j * 64 + lane, (j & 1) ? v[2] : v[0] + (v[1] << 8));
+    }
+    if (last == ACC_ITEMS && lane < 16) {
+#pragma unroll
+      for (int set = 0; set < NSET; ++set)
+#pragma unroll
+        for (int t = 0; t < NTILE; ++t) atomicAdd(xacc + ACC_ITEMS * 64 + (set * NTILE + t) * 16 + lane, acc[set][t][3]);
     }
   };
   [[maybe_unused]] float* late_o_hat = nullptr;  // ONE: see below
@@ -2077,18 +2085,16 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       if (h >= GA) continue;
       const int d = Tiles::channel(tile, col);
       const int g = (NG == 1) ? 0 : (d / (D / NG));
-      const int* ta = xacc + ((set * AR + tile) * 4) * 64 + 16 * hh + col;   // row 4*hh + l of the tile: component l, lane 16*hh + col
-      const int* wa = xacc + ((set * AR + NTILE + g) * 4) * 64 + 16 * hh;    // weight sums: any column of the all-ones tile
-      int i0 = ta[0], i1 = ta[64], i2 = ta[128], cs = ta[192] / 75;          // (row 4*hh + 3 holds 75 * sum of the codes)
+      const int* ta = xacc + ((set * AR + tile) * 2) * 64 + 16 * hh + col;
+      const int* wa = xacc + ((set * AR + NTILE + g) * 2) * 64 + 16 * hh;    // weight sums: any column of the all-ones tile
+      int lo = ta[0], i2 = ta[64], cs = xacc[ACC_ITEMS * 64 + (set * NTILE + tile) * 16 + col] / 75;
       if (V2 && !(tile & 1)) {  // even INT2 tiles hold four times their sums (exact multiples)
-        i0 >>= 2;
-        i1 >>= 2;
+        lo >>= 2;
         i2 >>= 2;
         cs >>= 2;
       }
-      const int w0 = wa[0], w1 = wa[64], w2 = wa[128];   // |sum| < 2^24: no overflow
-      const long long wsum = (long long)w2 * 65536ll + (long long)w1 * 256ll + (long long)w0 + 32896ll * 64ll * (long long)nch;
-      const long long tot = (long long)i2 * 65536ll + (long long)i1 * 256ll + (long long)i0 + 32896ll * (long long)cs - (long long)VOFF * wsum;
+      const long long wsum = (long long)wa[64] * 65536ll + (long long)wa[0] + 32896ll * 64ll * (long long)nch;
+      const long long tot = (long long)i2 * 65536ll + (long long)lo + 32896ll * (long long)cs - (long long)VOFF * wsum;
       const float o = (float)ldexp((double)tot, -E[g]);
       if constexpr (ONE) {
         const float o_hat = __builtin_fmaf(o, tl_coef[h], 0.f) * tl_iz[h];
@@ -2115,8 +2121,8 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // -> bit i: position t0 + 16 * lane + i lies before `thr` in the buckets; ONE: `sure`, likewise before `thr_lo`
   auto block_mask = [&](const float* lp, float ba, float bb, float thr, float thr_lo, int nvalid, auto acc_tag, uint32_t& sure) JF_INLINE -> uint32_t {
     constexpr int ACCSEL = decltype(acc_tag)::value;  // accumulator sums issued along the comparisons: -1 none, 0 / 1 a half, 2 all
-    constexpr int A_LO = (ACCSEL == 1) ? ACC_HALF * 4 : 0;
-    constexpr int A_HI = (ACCSEL < 0) ? 0 : ((ACCSEL == 0) ? ACC_HALF * 4 : ACC_TOTAL * 4);
+    constexpr int A_LO = (ACCSEL == 1) ? ACC_HALF : 0;
+    constexpr int A_HI = (ACCSEL < 0) ? 0 : ((ACCSEL == 0) ? ACC_HALF : ACC_ITEMS);
     constexpr int PER = (A_HI - A_LO + 15) / 16;      // a few behind every comparison: the LDS queue never fills
     v4f x[4];
 #pragma unroll
@@ -2288,7 +2294,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
 #pragma unroll
         for (int i = 0; i < STEPS; ++i) x[i] = srow[min(tb + 64 * i + lane, L - 1)];
         if (HAS_V && !acc_issued) {
-          add_acc_range(0, ACC_TOTAL * 4);
+          add_acc_range(0, ACC_ITEMS);
           acc_issued = true;
         }
 #pragma unroll
@@ -2451,7 +2457,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
 #pragma unroll
         for (int i = 0; i < STEPS; ++i) x[i] = srow[min(tb + 64 * i + lane, L - 1)];
         if (HAS_V && !acc_issued) {
-          add_acc_range(0, ACC_TOTAL * 4);
+          add_acc_range(0, ACC_ITEMS);
           acc_issued = true;
         }
 #pragma unroll
@@ -2501,7 +2507,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   if (clk && tid == 0) clk[3] = JF_CLK();
 
   if constexpr (HAS_V) {  // whatever the emission did not carry (no batch of this wavefront, a short split, the exact selection)
-    if (!acc_issued) add_acc_range(0, ACC_TOTAL * 4);
+    if (!acc_issued) add_acc_range(0, ACC_ITEMS);
   }
   // ONE: the outputs' addresses are read from the argument block again here (the compiler keeps what it has read, and with the
   // streams' own values the scalar registers do not hold it: some twenty of them went to vector lanes), all together ahead of

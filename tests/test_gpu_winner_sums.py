@@ -60,3 +60,28 @@ def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
                 tol = 4e-6 * (w[:, None] * np.abs(v)).sum(0) + 64 * 8 * 2.0 ** -25 * top
                 assert (np.abs(got - (w[:, None] * v).sum(0)) <= tol).all(), (b, hq, g)
             assert abs(W[b, hq] - p.sum()) <= 4e-6 * max(1.0, p.sum())
+
+
+@pytest.mark.parametrize("code", ["lowest", "highest"])
+@pytest.mark.parametrize("G", [1, 4, 8])
+@pytest.mark.parametrize("scheme,kb,vb,gs", [("k3v2", 3, 2, 64), ("k3v3", 3, 3, 64), ("k4v4", 4, 4, 128), ("b4v4", 4, 4, 64)])
+def test_longest_splits_of_equal_weights_and_codes(scheme, kb, vb, gs, G, code):
+    """Equal scores and scales that are powers of two: every weight is the largest and its two lower limbs are -128 each, every
+    code the largest there is, so the accumulator sums of the longest split reach the end of their range."""
+    from jetfire_amd import _lib
+    S, Hkv, K = 8192, 2, 64
+    c = make_case(102, 1, G * Hkv, Hkv, S, kb, vb, gs, lens=[S])
+    top = (1 << vb) - 1 if code == "highest" else 0
+    c["q"] = np.zeros_like(c["q"])
+    c["vd"] = np.broadcast_to(O.pack_codes(np.full(128, top), vb), c["vd"].shape).copy()
+    c["vs"] = np.full_like(c["vs"], _bits([0.25])[0])
+    d = to_device(c)
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(4096 if G <= 4 else 2048))
+    try:
+        out = [t.cpu().numpy() for t in run_fused(scheme, c, d, S, K)]
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    value = 0.25 * (top - O.offset(vb))
+    assert np.abs(out[0] - value).max() <= 3e-6 * abs(value)
+    assert np.abs(out[2] - value * K / S).max() <= 3e-6 * abs(value) * K / S
+    assert np.array_equal(out[4][0], np.broadcast_to(np.arange(K), out[4][0].shape))
