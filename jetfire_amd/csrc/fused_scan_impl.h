@@ -293,7 +293,7 @@ struct ScanLds {
   static constexpr bool SPREP = (K3 || (K2 && !KA)) && (WAVE_STAGE >= KST + 64 * SCT);
   static constexpr int ACC_REGS = 8 + NG;                   // v4i accumulators per set: 8 channel tiles + NG weight sums
   // sum of the wavefronts' accumulators: two ints per (set, accumulator register, lane) and one per (set, tile, column), in the staging
-  // area (dead after phase B), followed by one kilobyte per wavefront for the exact selection's histogram
+  // area (dead after phase B), followed by what the emission needs per wavefront
   static constexpr int XACC = NSET * (ACC_REGS * 2 * 64 + 8 * 16) * 4;
   static constexpr int PREP = KLIMB ? (int)sizeof(K3Prep<NSET>) : (int)sizeof(QInt8F<NSET>);
   // selection histograms: 32-bit counters, or (any INT4 side, where the staging areas are larger and LDS is
@@ -308,7 +308,9 @@ struct ScanLds {
   static constexpr int AUX = ((RND_AT + RND > HIST ? RND_AT + RND : HIST) + 15) & ~15;
   static constexpr int SC_AT = KB4 ? AUX : 0;
   __host__ __device__ static constexpr int stage_bytes() { return NW * WAVE_STAGE; }
-  static_assert(NW * WAVE_STAGE >= XACC + NW * 1024, "the staging area must hold the accumulator sums and the selection scratch");
+  // per wavefront behind it: the candidates of a block of 1024 positions, or the exact selection's histogram
+  static constexpr int EMIT = 2048;
+  static_assert(NW * WAVE_STAGE >= XACC + NW * EMIT, "the staging area must hold the accumulator sums and the selection scratch");
   __host__ __device__ static constexpr size_t per_position() { return (size_t)G * 4; }
   __host__ __device__ static size_t aux_offset(int L) { return (per_position() * L + (size_t)(L / 16) * 4 + 15) & ~(size_t)15; }
   __host__ __device__ static size_t total(int L) {
@@ -2259,6 +2261,11 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       // share the padding and its stores leave before the emission's
       const int etot = min(Kcap, tot);
       for (int i = etot + seg * 64 + lane; i < Kcap; i += SEG * 64) ck[i] = 0u;
+      // A block's candidates go to a list in the wavefront's own LDS first, then out one per lane: stored from the loop over a
+      // lane's set bits, keys and positions took a dozen partly filled stores each instead of two or three.  Per layer: 32 sequences x 3000
+      // positions, K4V4, top-k 2048 94.8 us, this 84.4; 1 x 65536, eight heads, K3V2, 512 40.9 / 37.1; 16 x 4096, K3V2, 1024 45.4 / 42.1;
+      // 4 x 32768, eight heads, 256 31.8 / 31.6.
+      uint16_t* cl = reinterpret_cast<uint16_t*>(stage + Lds::XACC + wave * Lds::EMIT);
       auto emit_block = [&](int t0, auto acc_tag) JF_INLINE {
         const int lt = t0 + 16 * lane;                    // first position of this lane
         const float* lp = srow + lt;
@@ -2266,24 +2273,20 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         uint32_t mask = block_mask(lp, ba, bb, thr, 0.f, max(0, min(16, te - lt)), acc_tag, none);
         const int mine = __popc(mask);
         const int incl = wave_incl_scan_i(mine);
-        uint32_t o = (uint32_t)(count + incl - mine);
+        const int start = count;
+        int at = incl - mine;
         count += __builtin_amdgcn_readlane(incl, 63);
-        // (the score of the next set bit is requested before the current one is stored: one LDS latency per lane run,
-        // not one per candidate)
-        int i = (mask != 0u) ? __ffs((int)mask) - 1 : 0;
-        float sco = lp[i];
         while (mask != 0u) {
+          cl[at++] = (uint16_t)(lt + __ffs((int)mask) - 1);
           mask &= mask - 1u;
-          const int i_next = (mask != 0u) ? __ffs((int)mask) - 1 : 0;
-          const float s_next = lp[i_next];
-          if (o < (uint32_t)Kcap) {  // the bound only matters for non-finite scores
-            ck[o] = score_key(sco);
-            ci[o] = s0 + lt + i;
-          }
-          ++o;
-          i = i_next;
-          sco = s_next;
         }
+        wave_lds_fence();
+        for (int r = start + lane; r < min(count, Kcap); r += 64) {  // (the bound only matters for non-finite scores)
+          const int t = cl[r - start];
+          ck[r] = score_key(srow[t]);
+          ci[r] = s0 + t;
+        }
+        wave_lds_fence();
       };
       if constexpr (SHORT) {
         // Segments of at most 256 positions (512 beyond four heads): one position per lane, 64 at a time; all scores first,
@@ -2334,7 +2337,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
     } else if (seg == 0) {
       // exact fallback: 8-bit radix select over the order-preserving keys (bits shared by every key skipped),
       // then the keys above the K-th and the lowest-position ties that fill the quota
-      int* rh = reinterpret_cast<int*>(stage + Lds::XACC + wave * 1024);
+      int* rh = reinterpret_cast<int*>(stage + Lds::XACC + wave * Lds::EMIT);
       uint32_t T = 0;
       int quota = 0;
       uint32_t kmin = 0xffffffffu, kmax = 0u;
