@@ -2947,6 +2947,7 @@ constexpr int MG_LIST = 1024;      // members of the cut bucket resolved by rank
 constexpr int MG_RANK = 16;        // up to here all pairs at once in every wavefront, beyond over the list in LDS
 constexpr int MG_BT_LDS = 4096;    // block-table entries cached in LDS (65536 positions)
 constexpr int MG_LIGHT_THREADS = 256, MG_LIGHT_REGK = 16, MG_LIGHT_TOPK = 512;  // the light shape of the merge
+constexpr int MG_MEDIUM_THREADS = 512, MG_MEDIUM_REGK = 16;                     // the medium one
 
 // Launch 2: one workgroup per (sequence, query head).
 //   1. split statistics -> M, l, o_hat; a lower bound of the K-th largest score from the splits' own cuts
@@ -2958,8 +2959,8 @@ constexpr int MG_LIGHT_THREADS = 256, MG_LIGHT_REGK = 16, MG_LIGHT_TOPK = 512;  
 //   4. slots, softmax weights, and the pre-correction terms over the winners' V rows.
 // The first MG_REGK * MG_THREADS candidates stay in registers from a single load; anything beyond that is
 // re-read from global memory in every pass.
-// Two shapes: 1024 threads x 8 register-resident candidates each (up to 8192 candidates, the common case)
-// and 1024 x 32 for first-stage parts that exceed it.
+// Shapes: 1024 threads x 8 register-resident candidates each (up to 8192 candidates, the common case), 1024 x 32 beyond, and
+// 512 x 16 and 256 x 16 where there are more rows than CUs.
 //
 // What bounds it is neither memory nor launch: run a second time over warm caches the same workgroup takes as long.  It
 // is the length of the chain every wavefront goes through, some 900 instructions and a dozen round trips to LDS, which
@@ -2994,8 +2995,8 @@ __global__ __launch_bounds__(MG_THREADS, PER_CU == 4 ? 4 : MG_THREADS / 256) voi
   constexpr int VGRP = 8;
   static_assert(MG_THREADS % D == 0 && VGRP % (MG_THREADS / D) == 0 && (MG_WAVES >= VGRP || VGRP % MG_WAVES == 0), "whole roles per thread group / wavefront");
   // the light shape (many rows per launch, few candidates per row) trades table sizes for workgroups per CU
-  constexpr int MG_BT = (MG_THREADS >= 1024) ? MG_BT_LDS : 1024;  // block-table entries cached in LDS
-  constexpr int MG_WIN = (MG_THREADS >= 1024) ? FS_LDS_TOPK : 512;  // widest correction of this shape (WIDE: any)
+  constexpr int MG_BT = (MG_THREADS > MG_LIGHT_THREADS) ? MG_BT_LDS : 1024;  // block-table entries cached in LDS
+  constexpr int MG_WIN = (MG_THREADS > MG_LIGHT_THREADS) ? FS_LDS_TOPK : 512;  // widest correction of this shape (WIDE: any)
   // (the shape of 32 candidates per thread meets wide corrections, whose cut lies where the scores are densest: twice the buckets)
   constexpr int BINS = (MG_REGK > 16) ? 2 * MG_BINS : MG_BINS;
   // The sums over the winners need a staging area; what the selection needs lies in the same place (a barrier lies between).  Side by
@@ -4178,6 +4179,13 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   // the kernel).
   const bool light = (MODE == FS_FULL) && !big && p.mg_parts == 1 && top_k <= MG_LIGHT_TOPK &&
                      (long long)B * H_q > (long long)device_cus() && (long long)p.n_splits * p.Kc <= MG_LIGHT_THREADS * MG_LIGHT_REGK;
+  // More rows than CUs that the light shape does not take: half the wavefronts with twice the candidates each.  What every wavefront
+  // does for itself is done half as often, and up to three rows share a CU: per layer, 1024 threads / this, 288 rows of 8 lists
+  // (9 x 4096 positions, K3V2, top-k 1024) 36.9 / 31.7 us, 384 (12 x 2500) 35.6 / 30.4, 512 (16 x 4096) 42.1 / 37.2, 1024 (32 x
+  // 3000) 61.4 / 49.3, K4V4, 2048 84.0 / 73.5.  With a row per CU the sixteen wavefronts are the shorter way: 256 rows 25.2 / 25.8,
+  // 128 (4 x 32768, 256) 33.7 / 34.45.
+  const bool medium = (MODE == FS_FULL) && !wide && !big && !light && (long long)B * H_q > (long long)device_cus();
+  (void)medium;
   // the rows of both of a wavefront's turns at once where there are two and four workgroups per CU hold every row (see PER_CU)
   const bool gather = light && top_k > 256 && (long long)B * H_q <= 4ll * device_cus();
   (void)gather;
@@ -4192,6 +4200,8 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
         if (gather) hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false, false, 4>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, mp); \
         else hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_LIGHT_THREADS, MG_LIGHT_REGK, false>), mgrid, dim3(MG_LIGHT_THREADS), 0, st, mp); \
       }                                                                                                              \
+    } else if (medium) {                                                                                               \
+      if constexpr (MODE == FS_FULL) hipLaunchKernelGGL((fused_merge_kernel<FS_FULL, VB, NGG, MG_MEDIUM_THREADS, MG_MEDIUM_REGK, false>), mgrid, dim3(MG_MEDIUM_THREADS), 0, st, mp); \
     } else hipLaunchKernelGGL((fused_merge_kernel<MODE, VB, NGG, 1024, 8, false>), mgrid, dim3(1024), 0, st, mp);       \
   } while (0)
   if constexpr (MODE == FS_STAGE_A || MODE == FS_TOPK) {  // no value rows are read: one instantiation serves every format

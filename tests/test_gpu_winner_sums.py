@@ -85,3 +85,30 @@ def test_longest_splits_of_equal_weights_and_codes(scheme, kb, vb, gs, G, code):
     assert np.abs(out[0] - value).max() <= 3e-6 * abs(value)
     assert np.abs(out[2] - value * K / S).max() <= 3e-6 * abs(value) * K / S
     assert np.array_equal(out[4][0], np.broadcast_to(np.arange(K), out[4][0].shape))
+
+
+@pytest.mark.parametrize("scheme,kb,vb,gs,S,K,split_len", [
+    ("k3v2", 3, 2, 64, 700, 64, 256), ("k4v4", 4, 4, 128, 700, 256, 256), ("b4v4", 4, 4, 64, 1500, 512, 768),    # 256 threads a row
+    ("k3v3", 3, 3, 64, 1200, 512, 512),                                                # ... with two turns of winners at once
+    ("k3v2", 3, 2, 64, 2040, 1024, 256), ("k4v4", 4, 4, 128, 1111, 1024, 512),         # 512 threads
+    ("k3v2", 3, 2, 64, 8192, 2048, 2048), ("k3v3", 3, 3, 128, 6000, 64, 256),          # ... as many candidates as they hold; few winners
+    ("k4v4", 4, 4, 128, 9000, 2048, 2048),                                             # beyond: 32 candidates per thread
+])
+def test_shapes_of_the_merge_give_the_same_bits(scheme, kb, vb, gs, S, K, split_len):
+    """More rows than compute units, whose merge has fewer wavefronts per row, and the same rows a few at a time."""
+    from jetfire_amd import _lib, ops
+    G, Hkv, B = 8, 4, 10            # 320 rows, and 96 or fewer
+    c = make_case(103, B, G * Hkv, Hkv, S, kb, vb, gs, lens=[max(1, S - 97 * b * b) for b in range(B)])
+    d = to_device(c)
+    _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
+    try:
+        whole = [t.clone() for t in run_fused(scheme, c, d, S, K)]
+        for lo in range(0, B, 3):
+            at = slice(lo, min(B, lo + 3))
+            part = ops.fused_attn_topk(scheme, d["q"][at].contiguous(), d["kd"], d["ks"], d["vd"], d["vs"], d["bt"][at].contiguous(),
+                                       d["lens"][at].contiguous(), S, G * Hkv, Hkv, 16, K, 128 ** -0.5, return_scores=True,
+                                       return_stats=True)
+            for a, b in zip(whole, part):
+                assert torch.equal(a[at], b)
+    finally:
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
