@@ -761,8 +761,9 @@ struct PreCorr {
 // fetch: it selects the winners, forms the pre-correction terms and writes the step's outputs itself, and no merge is
 // launched.  A merge launch costs 9 - 10 us whatever it merges (its loads are first touches, its intervals a chain of
 // barriers), 18 us at 1024 rows; the same steps from LDS, four wavefronts per head, cost 4 to 8 us at the end of the
-// scan.  Per layer, MI355X, graph replay: 32 sequences x 2048 positions, K3V2, 8 kv-heads, top-k 256 37.5 -> 26.7 us;
-// 32 x 464, K3V4, 4 kv-heads, top-k 64 30.1 -> 19.4; 7 x 311, K4V4, 8 kv-heads, G = 2 20.7 -> 16.5.
+// scan.  Per layer, MI355X, graph replay, when it was made: 32 sequences x 2048 positions, K3V2, 8 kv-heads, top-k 256 37.5 -> 26.7
+// us (22.8 since its winners are marked in place and summed on the matrix cores); 32 x 464, K3V4, 4 kv-heads, top-k 64 30.1 -> 19.4;
+// 7 x 311, K4V4, 8 kv-heads, G = 2 20.7 -> 16.5.
 //
 // SHORT: at most one chunk per wavefront (splits of up to NW * 64 positions).  Its V rows are requested along with the key
 // rows; the form for longer splits requests V rows with the last two of four key chunks, which a short split never
@@ -3825,7 +3826,8 @@ inline double merge_us(int rows, int max_S, int ns, int kc, int top_k) {
 // wavefronts (more heads than wavefronts: one after the other), and all wavefronts of a SIMD share its vector ALU.
 // Measured against the merge launch at the same split length, up to 256 rows: 64-row batches per wavefront 1 / 2 / 4 with
 // sixteen wavefronts 3 us faster / equal / 4 us slower, 1 / 2 / 4 / 8 with eight wavefronts 4 and 2 us faster, 2 and up to 10
-// slower; with more rows the launch takes longer and the workgroups here do not.
+// slower; with more rows the launch takes longer and the workgroups here do not.  (Both ways' sums have moved to the matrix cores
+// since; over 450 random shapes, each timed in every split length, the planner's choice is 1.2 % off the best one's time in the mean.)
 inline double one_split_us(int G, int units, int max_S, int top_k) {
   constexpr double kFixed = 1.4, kPerBatch = 0.25;
   const int nw = G <= 4 ? 16 : 8, per_head = nw >= G ? nw / G : 1, winners = top_k < max_S ? top_k : max_S;
