@@ -1835,9 +1835,10 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       lo = fminf(lo, red_f[w][G + tid]);
     }
     m_sh[tid] = m;
-    // bucket of a score: min(255, (m - s) * 255 / (m - lo)), bucket 0 = largest; monotone in s
-    const float range = m - lo;
-    const float iw = (range > 0.f && isfinite(range)) ? 254.99f / range : 0.f;
+    // bucket of a score: min(255, (m - s) * 255 / (m - lo)), bucket 0 = largest; monotone in s.  No slope where the range has no
+    // width or no end, or is so narrow (below 7.5e-37) that its slope has none: all scores in bucket 0.
+    const float range = m - lo, slope = 254.99f / range;
+    const float iw = (range > 0.f && isfinite(range) && isfinite(slope)) ? slope : 0.f;
     bin_a_sh[tid] = -iw;
     bin_b_sh[tid] = isfinite(m) ? m * iw : 0.f;
   }

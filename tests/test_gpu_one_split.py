@@ -151,6 +151,68 @@ def test_one_split_selects_from_a_crowded_bucket(scheme, kb, vb, gs, G, S, K, ki
             assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -1).all()
 
 
+def _winners_by_key(scores, n, K):
+    """Positions of the K largest of scores[:n] in the order of the kernels' keys, ties to the lowest position."""
+    u = scores[:n].view(np.uint32)
+    key = np.where(u >> 31, ~u, u | np.uint32(1 << 31)).astype(np.int64)
+    return np.sort(np.lexsort((np.arange(n), -key))[:K])
+
+
+# a head's finite scores this close together have no finite number of buckets per unit: 254.99 / range overflows
+NARROW = 254.99 / float(np.finfo(np.float32).max)
+
+
+@pytest.mark.parametrize("scheme,kb,vb,gs,G,S,K", [
+    ("k3v2", 3, 2, 64, 4, 1024, 512),      # more winners than one of the head's four segments has positions
+    ("k3v2", 3, 2, 64, 8, 1000, 128),
+    ("k2v2", 2, 2, 64, 1, 3900, 2048),
+    ("b4v4", 4, 4, 64, 4, 900, 64),
+])
+def test_one_split_scores_within_a_range_too_narrow_for_buckets(scheme, kb, vb, gs, G, S, K):
+    Hkv, lens = 2, [S, S - S // 5]
+    c = make_case(97, 2, G * Hkv, Hkv, S, kb, vb, gs, lens=lens)
+    d = to_device(c)
+    d["ks"] = (d["ks"].float() * 2.0 ** -122).to(torch.bfloat16)
+    one, cut = _both(scheme, c, d, S, K)
+    scores = one[7].cpu().numpy()
+    narrow = 0
+    for b, n in enumerate(lens):
+        for h in range(G * Hkv):
+            s = scores[b, h, :n]
+            narrow += 0 < float(s.max()) - float(s.min()) < NARROW
+            want, got = _winners_by_key(s, n, K), one[4][b, h].cpu().numpy()
+            assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -1).all(), (b, h)
+    assert narrow > 0
+    assert torch.equal(one[4], cut[4]) and torch.equal(one[1], cut[1])
+    for a, b in ((one[0], cut[0]), (one[2], cut[2]), (one[3], cut[3])):
+        assert float((a - b).abs().max()) <= 6e-6
+
+
+@pytest.mark.parametrize("width", [1e-40, 1e-37, 4e-37, 7e-37, 8e-37])
+@pytest.mark.parametrize("Hq,S,K", [(4, 2048, 1024), (4, 777, 64), (2, 1000, 512), (1, 3900, 2048)])
+def test_selection_from_given_scores_within_a_range_too_narrow_for_buckets(Hq, S, K, width):
+    from jetfire_amd import _lib, ops
+    rng = np.random.default_rng(98)
+    lens = np.array([S, S - 100], np.int32)
+    scores = (rng.random((2, Hq, S)) - rng.choice([0.0, 0.5, 1.0], (2, Hq, 1))).astype(np.float32) * np.float32(width)
+    table = torch.randperm(2 * ((S + 15) // 16)).reshape(2, -1).cuda()
+    got = []
+    for split in (-(-S // 256) * 256, 256):
+        _lib.check(_lib.debug_hook("jf_debug_split_len")(split))
+        try:
+            got.append(ops._topk(torch.from_numpy(scores).cuda(), table, torch.from_numpy(lens).cuda(), S, Hq, 16, K, True, "topk"))
+        finally:
+            _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    for b, n in enumerate(lens):
+        for h in range(Hq):
+            want = _winners_by_key(scores[b, h], n, K)
+            for idx, slots, _, _ in got:
+                i = idx[b, h].cpu().numpy()
+                assert np.array_equal(i[:len(want)], want) and (i[len(want):] == -1).all(), (b, h)
+                pos = idx[b, h, :len(want)]
+                assert torch.equal(slots[b, h, :len(want)], table[b, pos // 16] * 16 + pos % 16)
+
+
 @pytest.mark.parametrize("kind", ["outlier", "levels", "plain"])
 @pytest.mark.parametrize("scheme,kb,vb,gs,B,Hkv,G,S,K,other", [
     ("k2v2", 2, 2, 64, 16, 8, 1, 3900, 2048, 256),
