@@ -1921,8 +1921,11 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
         // masked positions hold -inf: their weight is exactly zero
         const float pw = __builtin_amdgcn_exp2f(__builtin_fmaf(s, LOG2E, nml[h]));
         lsum[h] += pw;
+        // A weight that is a NaN (an infinite or NaN score) is the sum's affair, which makes the head's outputs what they are.  Here
+        // it counts zero: converted, it would change the word's top byte, which the other heads of the set take their code sums from.
+        const float pv = fmaxf(pw, 0.f);
 #pragma unroll
-        for (int g = 0; g < NG; ++g) bits[h][g] = __builtin_bit_cast(uint32_t, __builtin_fmaf(pw, vsf[g], 8388608.0f));
+        for (int g = 0; g < NG; ++g) bits[h][g] = __builtin_bit_cast(uint32_t, __builtin_fmaf(pv, vsf[g], 8388608.0f));
         if (HAS_TOPK && !take_all) {
           // (positions past the end add zero instead of branching around the add: their score is -inf or, with a
           // degenerate range, gives a NaN, and either clamps to a bucket inside the table)
