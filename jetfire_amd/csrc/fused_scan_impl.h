@@ -546,8 +546,8 @@ __device__ inline int tr8_token(int lane) { return (((lane >> 1) & 3) << 1) | ((
 
 // Pre-correction terms over the winners' packed V rows where a wavefront has 64 winners of a head at a time (one per lane): the
 // contraction of phase B on v_mfma_i32_16x16x64_i8, with one head's weights in four rows of the operand.  The weights are held
-// to 24 bits of the largest among the 64 (exact integers in float), in limbs of 7, 7, 7 and 3 bits, so that no limb needs a
-// sign; the products are exact, and each of the 64-winner sums is rounded once.
+// to 24 bits of the largest among the 64 (exact integers in float), in limbs of 7, 7, 7 and 3 bits with the weight's
+// sign in each; the products are exact, and each of the 64-winner sums is rounded once.
 // What a conversion and a multiply-add per code take instead, per
 // layer: 32 sequences x 2048 positions, K3V2, top-k 256 25.2 us, this 24.1; K4V4 26.6 / 25.5; 32 x 1900, K3V2, 512 28.9 / 26.8;
 // 16 x 1024, K4V4, 512 21.7 / 19.3; 32 x 500, eight heads, K3V2, 256 22.1 / 20.5.
@@ -602,13 +602,14 @@ struct WinnerSums {
       float f;
       if (isfinite(top[g])) {  // (uniform)
         if (top[g] > 0.f) (void)frexpf(top[g], &e);  // top = f * 2^e, f in [0.5, 1)
-        f = ldexpf(v, 24 - e);
+        f = ldexpf(fabsf(v), 24 - e);
       } else {  // an infinite weight or a NaN: it alone counts, and `top` becomes the sums' factor
         f = (__builtin_bit_cast(uint32_t, v) & 0x7fffffffu) == most ? 1.f : 0.f;
       }
       E[g] = 24 - e;
       const uint32_t w = (uint32_t)rintf(f);
       limbs[g] = (w & 0x7fu) | ((w << 1) & 0x7f00u) | ((w << 2) & 0x7f0000u) | ((w << 3) & 0x7f000000u);
+      if (v < 0.f) limbs[g] = (0x80808080u - limbs[g]) ^ 0x80808080u;  // (a negative scale: every limb negated; none borrows)
     }
     *reinterpret_cast<v4u*>(wl + lane * 16) = (v4u){limbs[0], limbs[0], limbs[NG - 1], limbs[NG - 1]};
 #pragma unroll

@@ -1,5 +1,6 @@
-"""Sums over the winners' value rows, 64 at a time with 24-bit weights: rows whose scales lie far apart, an infinite scale or a
-NaN among them, and one in a slot that only padding names; in the scan that merges by itself and both shapes of the merge."""
+"""Sums over the winners' value rows, 64 at a time with 24-bit weights: rows whose scales lie far apart or are negative, an infinite
+scale or a NaN among them, and one in a slot that only padding names; in the scan that merges by itself and both shapes of the
+merge."""
 import numpy as np
 import pytest
 import torch
@@ -15,7 +16,7 @@ def _bits(x):
     return O.f32_to_bf16_bits(np.asarray(x, np.float32))
 
 
-@pytest.mark.parametrize("kind", ["range", "infinite", "nan", "unused"])
+@pytest.mark.parametrize("kind", ["range", "signed", "infinite", "nan", "unused"])
 @pytest.mark.parametrize("copies,split_len,K", [(1, 768, 64), (1, 768, 256), (1, 256, 64), (1, 256, 512), (20, 256, 256), (20, 256, 512)])
 @pytest.mark.parametrize("scheme,kb,vb,gs", [("k3v2", 3, 2, 64), ("k3v2", 3, 2, 128), ("k3v3", 3, 3, 64), ("k4v4", 4, 4, 128), ("b4v4", 4, 4, 64)])
 def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
@@ -27,7 +28,10 @@ def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
     d = to_device(c)
     _lib.check(_lib.debug_hook("jf_debug_split_len")(split_len))
     try:
-        if kind != "range":
+        if kind == "signed":
+            vs = O.bf16_bits_to_f32(c["vs"])
+            c["vs"] = _bits(np.where(np.random.default_rng(7).random(vs.shape) < 0.4, -vs, vs))
+        elif kind != "range":
             out = [t.cpu().numpy() for t in run_fused(scheme, c, d, S, K)]
             bad = np.float32(np.nan if kind == "nan" else np.inf)
             slot = 0 if kind == "unused" else int(out[1][0, 0, 5])
@@ -56,10 +60,31 @@ def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
                 v = codes[hq // G, sl, g * gs:(g + 1) * gs]
                 # the weights' own fp32 error (scores, exponential, products): 4e-6 of the sum of magnitudes; half a unit of 24
                 # bits of the largest for each of 64 weights and codes of up to 8
-                top = sum(w[i:i + 64].max(initial=0.0) for i in range(0, len(w), 64))
-                tol = 4e-6 * (w[:, None] * np.abs(v)).sum(0) + 64 * 8 * 2.0 ** -25 * top
+                top = sum(np.abs(w[i:i + 64]).max(initial=0.0) for i in range(0, len(w), 64))
+                tol = 4e-6 * (np.abs(w[:, None] * v)).sum(0) + 64 * 8 * 2.0 ** -25 * top
                 assert (np.abs(got - (w[:, None] * v).sum(0)) <= tol).all(), (b, hq, g)
             assert abs(W[b, hq] - p.sum()) <= 4e-6 * max(1.0, p.sum())
+
+
+@pytest.mark.parametrize("Hq,Hkv,S,lens,K", [(8, 2, 700, [700, 70], 64), (8, 1, 2000, [2000, 1999], 512), (32, 8, 300, [300] * 10, 256)])
+def test_negative_scales_in_the_int8_tiles_form(Hq, Hkv, S, lens, K):
+    """The form whose o_hat takes scales of either sign: o_old_unnorm does too."""
+    from jetfire_amd import ops
+    c = make_case(104, len(lens), Hq, Hkv, S, 4, 4, 128, lens=lens)
+    vs = O.bf16_bits_to_f32(c["vs"])
+    c["vs"] = _bits(np.where(np.random.default_rng(8).random(vs.shape) < 0.4, -vs, vs))
+    d = to_device(c)
+    sc = O.scores_int8_model(c["q"], c["kd"], c["ks"], c["bt"], c["lens"], S, Hq, Hkv, 16, 128 ** -0.5)
+    idx, _ = O.topk_select(sc, c["lens"], c["bt"], S, K)
+    m, iz = O.softmax_stats(sc, c["lens"], S)
+    got = ops.int8tc_softmax_v_with_pre_corr_reg_stats(
+        torch.from_numpy(sc).cuda(), torch.from_numpy(m).cuda(), torch.from_numpy(iz).cuda(), d["vd"], d["vs"], d["bt"], d["lens"],
+        torch.from_numpy(idx).cuda(), S, Hq, Hkv, 16, K)
+    want = O.softmax_v_int8_tiles(sc, m, iz, c["vd"], c["vs"], c["bt"], c["lens"], idx, S, Hq, Hkv, 16)
+    # o_hat: a weight at half a quantum may round either way (a quantum is the tile's largest weight over 127); the others as there
+    quantum = float((np.exp(sc - m[..., None]) * iz[..., None]).max()) * float(np.abs(vs).max()) / 127 * 8
+    for g, w, tol in zip(got, want, (3e-6 + 2 * quantum, 3e-6, 3e-6)):
+        np.testing.assert_allclose(g.cpu().numpy(), w, atol=tol, rtol=2e-5)
 
 
 @pytest.mark.parametrize("code", ["lowest", "highest"])
