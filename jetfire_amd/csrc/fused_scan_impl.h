@@ -2848,7 +2848,7 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
             if constexpr (Pre::ALL_AHEAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
-              Pre::add(row[u], wv[u] * bf16_to_f32(sb[u]), acc);
+              Pre::add(row[u], slot[u] >= 0 ? wv[u] * bf16_to_f32(sb[u]) : 0.f, acc);  // (whatever scale slot 0 has)
               if (dwi == 0) wsum += wv[u];
             }
           };

@@ -66,6 +66,36 @@ def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
             assert abs(W[b, hq] - p.sum()) <= 4e-6 * max(1.0, p.sum())
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("G,K", [(4, 32), (4, 64), (1, 256), (8, 32), (4, 256)])     # code by code, and 64 at a time
+@pytest.mark.parametrize("scheme,kb,vb,gs", [("k3v2", 3, 2, 64), ("k3v3", 3, 3, 64), ("k4v4", 4, 4, 128), ("b4v4", 4, 4, 64)])
+def test_scale_of_the_slot_that_stands_in_for_no_winner(scheme, kb, vb, gs, G, K, bad):
+    """Fewer winners than the correction is wide, and Stage B with lists that have holes: entries without a position read slot 0,
+    which is nobody's, and whose scale makes no difference."""
+    from jetfire_amd import _lib, ops
+    S, Hkv = 700, 2
+    c = make_case(105, 3, G * Hkv, Hkv, S, kb, vb, gs, lens=[S, 9, 33], extra_blocks=1)
+    c["bt"] = (np.random.default_rng(5).permutation(c["bt"].size) + 1).reshape(c["bt"].shape).astype(np.int64)
+    d = to_device(c)
+    idx = torch.arange(K, device="cuda").expand(3, G * Hkv, K).clone()
+    idx[..., 1::3] = -1
+    stage_b = {2: ops.int2_softmax_v_with_pre_corr_wvs2, 3: ops.int3_softmax_v_with_pre_corr_wvs2,
+               4: ops.int4_softmax_v_with_pre_corr_wvs2_scores}[vb]
+    res = []
+    for scale in (1.0, bad):
+        d["vs"][:, 0] = scale
+        for split in (768, 256):
+            _lib.check(_lib.debug_hook("jf_debug_split_len")(split))
+            try:
+                full = run_fused(scheme, c, d, S, K)
+                res.append([t.clone() for t in list(full) + list(stage_b(full[7], d["vd"], d["vs"], d["bt"], d["lens"], idx, S, G * Hkv, Hkv, 16, K))])
+            finally:
+                _lib.check(_lib.debug_hook("jf_debug_split_len")(0))
+    for plain, odd in ((res[0], res[2]), (res[1], res[3])):
+        for a, b in zip(plain, odd):
+            assert torch.equal(a, b), a.shape
+
+
 @pytest.mark.parametrize("Hq,Hkv,S,lens,K", [(8, 2, 700, [700, 70], 64), (8, 1, 2000, [2000, 1999], 512), (32, 8, 300, [300] * 10, 256)])
 def test_negative_scales_in_the_int8_tiles_form(Hq, Hkv, S, lens, K):
     """The form whose o_hat takes scales of either sign: o_old_unnorm does too."""
