@@ -546,8 +546,10 @@ __device__ inline int tr8_token(int lane) { return (((lane >> 1) & 3) << 1) | ((
 
 // Pre-correction terms over the winners' packed V rows where a wavefront has 64 winners of a head at a time (one per lane): the
 // contraction of phase B on v_mfma_i32_16x16x64_i8, with one head's weights in four rows of the operand.  The weights are held
-// to 24 bits of the largest among the 64 (exact integers in float), in limbs of 7, 7, 7 and 3 bits with the weight's
-// sign in each; the products are exact, and each of the 64-winner sums is rounded once.
+// to 30 bits of the largest among the 64 (a float times a power of two is exact, 30 bits are what four signed digits of eight
+// take without an overflow), so a weight 2^-6 of the largest keeps all its bits; the products are exact, and each of the
+// 64-winner sums is rounded once.  (24 bits were off by up to three times what sums code by code in fp32 are where one score
+// stands out.)
 // What a conversion and a multiply-add per code take instead, per
 // layer: 32 sequences x 2048 positions, K3V2, top-k 256 25.2 us, this 24.1; K4V4 26.6 / 25.5; 32 x 1900, K3V2, 512 28.9 / 26.8;
 // 16 x 1024, K4V4, 512 21.7 / 19.3; 32 x 500, eight heads, K3V2, 256 22.1 / 20.5.
@@ -602,14 +604,12 @@ struct WinnerSums {
       float f;
       if (isfinite(top[g])) {  // (uniform)
         if (top[g] > 0.f) (void)frexpf(top[g], &e);  // top = f * 2^e, f in [0.5, 1)
-        f = ldexpf(fabsf(v), 24 - e);
+        f = ldexpf(v, 30 - e);
       } else {  // an infinite weight or a NaN: it alone counts, and `top` becomes the sums' factor
-        f = (__builtin_bit_cast(uint32_t, v) & 0x7fffffffu) == most ? 1.f : 0.f;
+        f = (__builtin_bit_cast(uint32_t, v) & 0x7fffffffu) == most ? copysignf(1.f, v) : 0.f;
       }
-      E[g] = 24 - e;
-      const uint32_t w = (uint32_t)rintf(f);
-      limbs[g] = (w & 0x7fu) | ((w << 1) & 0x7f00u) | ((w << 2) & 0x7f0000u) | ((w << 3) & 0x7f000000u);
-      if (v < 0.f) limbs[g] = (0x80808080u - limbs[g]) ^ 0x80808080u;  // (a negative scale: every limb negated; none borrows)
+      E[g] = 30 - e;
+      limbs[g] = ((uint32_t)(int)rintf(f) + 0x808080u) ^ 0x808080u;
     }
     *reinterpret_cast<v4u*>(wl + lane * 16) = (v4u){limbs[0], limbs[0], limbs[NG - 1], limbs[NG - 1]};
 #pragma unroll
@@ -629,7 +629,7 @@ struct WinnerSums {
       for (int c = 0; c < 4; ++c) Aq[c] = own ? A[c] : 0;
       acc[t & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Aq, B, acc[t & 1], 0, 0, 0);
     });
-    const int lo = Tiles::OFFSET * (sw[0] + (sw[1] << 7)), hi = Tiles::OFFSET * (sw[2] + (sw[3] << 7));
+    const int lo = Tiles::OFFSET * (sw[0] + (sw[1] << 8)), hi = Tiles::OFFSET * (sw[2] + (sw[3] << 8));
     const bool upper = (lane & 32) != 0;
     const float factor = upper ? top[NG - 1] : top[0];
     const int e = upper ? E[NG - 1] : E[0];
@@ -637,9 +637,9 @@ struct WinnerSums {
     for (int i = 0; i < 2; ++i) {
       constexpr int m[2] = {Tiles::times(0), Tiles::times(1)};
       const v4i a = acc[i];
-      // (both below 2^24: floats hold them)
-      const float low = (float)(a[0] + (a[1] << 7) - m[i] * lo), high = (float)(a[2] + (a[3] << 7) - m[i] * hi);
-      const float sum = __builtin_fmaf(high, 16384.f, low) * (m[i] == 4 ? 0.25f : 1.f);
+      // (floats hold both: `high` is below 2^24, `low` below 1.004 * 2^24, where it may be rounded to an even number)
+      const float low = (float)(a[0] + (a[1] << 8) - m[i] * lo), high = (float)(a[2] + (a[3] << 8) - m[i] * hi);
+      const float sum = __builtin_fmaf(high, 65536.f, low) * (m[i] == 4 ? 0.25f : 1.f);
       o[i] += isfinite(factor) ? ldexpf(sum, -e) : sum * factor;
     }
     wave_lds_fence();

@@ -1,6 +1,6 @@
-"""Sums over the winners' value rows, 64 at a time with 24-bit weights: rows whose scales lie far apart or are negative, an infinite
-scale or a NaN among them, and one in a slot that only padding names; in the scan that merges by itself and both shapes of the
-merge."""
+"""Sums over the winners' value rows, 64 at a time with 30-bit weights: rows whose scales lie far apart or are negative, a large
+weight whose codes are zero, an infinite scale or a NaN among them, and one in a slot that only padding names; in the scan that
+merges by itself and the shapes of the merge."""
 import numpy as np
 import pytest
 import torch
@@ -16,7 +16,7 @@ def _bits(x):
     return O.f32_to_bf16_bits(np.asarray(x, np.float32))
 
 
-@pytest.mark.parametrize("kind", ["range", "signed", "infinite", "nan", "unused"])
+@pytest.mark.parametrize("kind", ["range", "signed", "zero", "infinite", "nan", "unused"])
 @pytest.mark.parametrize("copies,split_len,K", [(1, 768, 64), (1, 768, 256), (1, 256, 64), (1, 256, 512), (20, 256, 256), (20, 256, 512)])
 @pytest.mark.parametrize("scheme,kb,vb,gs", [("k3v2", 3, 2, 64), ("k3v2", 3, 2, 128), ("k3v3", 3, 3, 64), ("k4v4", 4, 4, 128), ("b4v4", 4, 4, 64)])
 def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
@@ -31,6 +31,15 @@ def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
         if kind == "signed":
             vs = O.bf16_bits_to_f32(c["vs"])
             c["vs"] = _bits(np.where(np.random.default_rng(7).random(vs.shape) < 0.4, -vs, vs))
+        elif kind == "zero":        # one weight 2^16 times the others', in channels to which it adds nothing
+            out = [t.cpu().numpy() for t in run_fused(scheme, c, d, S, K)]
+            vs = O.bf16_bits_to_f32(c["vs"])
+            for hkv in range(Hkv):
+                slot = int(out[1][0, hkv * G, 5])
+                vs[hkv, slot] *= 2.0 ** 16
+                c["vd"][hkv, slot] = O.pack_codes(np.full(128, O.offset(vb)), vb)
+            c["vs"] = _bits(vs)
+            d["vd"] = torch.from_numpy(c["vd"]).cuda()
         elif kind != "range":
             out = [t.cpu().numpy() for t in run_fused(scheme, c, d, S, K)]
             bad = np.float32(np.nan if kind == "nan" else np.inf)
@@ -58,10 +67,11 @@ def test_scales_of_any_size(scheme, kb, vb, gs, copies, split_len, K, kind):
                     assert not np.isfinite(got).any(), (b, hq, g)
                     continue
                 v = codes[hq // G, sl, g * gs:(g + 1) * gs]
-                # the weights' own fp32 error (scores, exponential, products): 4e-6 of the sum of magnitudes; half a unit of 24
-                # bits of the largest for each of 64 weights and codes of up to 8
-                top = sum(np.abs(w[i:i + 64]).max(initial=0.0) for i in range(0, len(w), 64))
-                tol = 4e-6 * (np.abs(w[:, None] * v)).sum(0) + 64 * 8 * 2.0 ** -25 * top
+                # the weights' own fp32 error (scores, exponential, products): 4e-6 of the sum of magnitudes; half a unit of 30
+                # bits of the largest of 64 for each code, and a unit where the sums of the limbs are joined
+                tol = 4e-6 * (np.abs(w[:, None] * v)).sum(0)
+                for i in range(0, len(w), 64):
+                    tol += 2.0 ** (np.frexp(np.abs(w[i:i + 64]).max())[1] - 31) * (np.abs(v[i:i + 64]).sum(0) + 2)
                 assert (np.abs(got - (w[:, None] * v).sum(0)) <= tol).all(), (b, hq, g)
             assert abs(W[b, hq] - p.sum()) <= 4e-6 * max(1.0, p.sum())
 
