@@ -2988,8 +2988,10 @@ constexpr int MG_MEDIUM_THREADS = 512, MG_MEDIUM_REGK = 16;                     
 // new candidate list; the final merge (PARTIAL = false, mg_parts > 1) reads these lists instead of the
 // scan's.  The top K of a union is the top K of the parts' top K's, ties included: a candidate that a part
 // drops is beaten by K candidates of that part.
+// (Stage B alone keeps no candidates: registers for two workgroups per CU.  One more than the 64 that allows, INT3 values, and 512 rows (16
+// sequences x 4096 positions, top-k 256) took 27.6 us per layer, 24.5 with the bound.)
 template <int MODE, int VBITS, int NG, int MG_THREADS, int MG_REGK, bool PARTIAL, bool WIDE = false, int PER_CU = 1>
-__global__ __launch_bounds__(MG_THREADS, PER_CU == 4 ? 4 : MG_THREADS / 256) void fused_merge_kernel(MergeParams p) {
+__global__ __launch_bounds__(MG_THREADS, PER_CU == 4 ? 4 : (MODE == FS_STAGE_B ? 2 : 1) * MG_THREADS / 256) void fused_merge_kernel(MergeParams p) {
   static_assert(!(PARTIAL && MODE == FS_STAGE_B), "Stage B alone selects nothing");
   constexpr int MG_WAVES = MG_THREADS / 64;
   // PER_CU = 4, light shape: four workgroups per CU are all there are, and a wavefront has registers for the rows of both its turns

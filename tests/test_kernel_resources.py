@@ -61,3 +61,10 @@ def test_light_merge_that_gathers_at_once_runs_four_workgroups_per_compute_unit(
     """256 threads x 16 candidates, all four roles of a wavefront together: launched for up to four rows per unit."""
     ks = [k for n, k in _kernels().items() if "fused_merge_kernelI" in n and "ELi256ELi16ELb0ELb0ELi4E" in n]
     assert len(ks) == 6 and min(_workgroups_per_cu(k) for k in ks) == 4
+
+
+def test_merge_of_stage_b_runs_two_workgroups_per_compute_unit():
+    """1024 threads, which hold no candidates; beyond FS_LDS_TOPK winners the launch adds LDS for them, eight bytes each."""
+    ks = [(n, k) for n, k in _kernels().items() if "fused_merge_kernelILi2E" in n]
+    assert len(ks) >= 12 and all(_workgroups_per_cu(k) == 2 for _, k in ks)
+    assert all(k[".vgpr_spill_count"] == 0 for _, k in ks)
