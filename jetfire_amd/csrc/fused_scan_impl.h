@@ -783,6 +783,15 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   // INT4 keys over 128 channels in one group: their sums reach 128 * 2^22 * 8 = 2^32 and are put together in two parts
   constexpr bool WIDE_SUM = KB4 && NG == 1;
   constexpr bool V2 = Lds::V2, V3 = Lds::V3;
+  // What the outputs and the winners' rows are addressed by follows from the thread's number; the compiler forms it ahead of phase B,
+  // and where the value rows in flight leave no registers for it (16 wavefronts, 128 registers) it waits for a chunk of them to put
+  // that into scratch memory.  Behind phase B those kernels take the number as a value of its own, for the winners' rows (TIGHT) and
+  // for all outputs (TIGHTER): the ones that spilled.  Forming it anew costs the others, which have the registers, 1 to 4 %.
+  // Per layer, 32 sequences x 8 kv-heads: K3V3 in two groups, 3900 positions, top-k 256, one head each 29.7 us, with this 28.2; 1900
+  // positions, four heads 28.4 / 25.1; A2V2 in two groups, 3900, 128, one head 35.6 / 34.3.
+  constexpr bool TIGHT = ONE && !SHORT && Lds::NW == 16 &&
+                         (V3 ? !(G == 1 && NG == 1 && (K3 || KA)) : NG == 2 && (KA || (!V2 && G == 4)));
+  constexpr bool TIGHTER = (TIGHT && (KA ? NG == 2 : (G > 1 && (G == 4 || NG == 2)))) || (!ONE && !SHORT && V3 && G == 4);
   constexpr int NSET = Lds::NSET;
   constexpr int SEG = Lds::SEG;
   constexpr int KP = Lds::KP;
@@ -2087,7 +2096,9 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   [[maybe_unused]] float* late_o_hat = nullptr;  // ONE: see below
   auto combine = [&](int set) {
     // thread -> (tile, head, column)
-    for (int i = tid; i < 4 * D; i += NT) {
+    int first = tid;
+    if constexpr (TIGHTER) asm volatile("" : "+v"(first));
+    for (int i = first; i < 4 * D; i += NT) {
       const int col = i & 15, hh = (i >> 4) & 3, tile = i >> 6;
       const int h = set * 4 + hh;
       if (h >= GA) continue;
@@ -2540,6 +2551,12 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
   }
   if constexpr (HAS_V || ONE) lds_barrier();
   if constexpr (ONE) {
+    int late_tid = tid, late_lane = lane;
+    if constexpr (TIGHTER) {
+      asm volatile("" : "+v"(late_tid));
+      late_lane = late_tid & 63;
+    }
+    const int tid = late_tid, lane = late_lane;
     if (late.softmax_m && tid < GA) {
       late.softmax_m[head0 + tid] = tl_m[tid];
       late.softmax_inv_z[head0 + tid] = tl_iz[tid];
@@ -2807,7 +2824,9 @@ __global__ __launch_bounds__((ScanLds<SCHEME, G, NG>::NT)) void fused_scan_kerne
       static_assert(Lds::WAVE_STAGE >= Sums::STAGE && Lds::WAVE_STAGE >= RES_AT + (G + NW - 1) / NW * RES, "the sums lie in the staging area");
       static_assert(Lds::WAVE_STAGE % 16 == 0, "16-byte rows");
       uint8_t* st = stage + wave * Lds::WAVE_STAGE;
+      if constexpr (TIGHT) asm volatile("" : "+v"(late_lane));
       for (int hw = wave; hw < GA * WPH; hw += NW) {
+        const int lane = late_lane;
         const int h = hw / WPH, part = hw % WPH, n_out = HAS_TOPK ? Kt : __builtin_amdgcn_readfirstlane(tl_nout[h]);
         const int* slots = tl_wslot + h * K;
         const float* weights = tl_ww + h * K;

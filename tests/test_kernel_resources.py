@@ -68,3 +68,12 @@ def test_merge_of_stage_b_runs_two_workgroups_per_compute_unit():
     ks = [(n, k) for n, k in _kernels().items() if "fused_merge_kernelILi2E" in n]
     assert len(ks) >= 12 and all(_workgroups_per_cu(k) == 2 for _, k in ks)
     assert all(k[".vgpr_spill_count"] == 0 for _, k in ks)
+
+
+def test_scans_of_up_to_eight_heads_keep_the_value_rows_in_registers():
+    """A spill there is a chunk of value rows waited for and put into scratch memory.  Asymmetric keys and INT3 values in two
+    groups, one or two heads, keep a word or two of the rows there."""
+    ks = {n: k[".vgpr_spill_count"] for n, k in _kernels().items() if "fused_scan_kernelI" in n and "ELi16ELi" not in n}
+    few = {n for n in ks if re.search(r"fused_scan_kernelILi0ELi13ELi[12]ELi2ELb[01]ELb0E", n)}
+    assert len(ks) > 400 and len(few) == 4
+    assert max(ks[n] for n in few) <= 8 and not any(ks[n] for n in ks if n not in few)
