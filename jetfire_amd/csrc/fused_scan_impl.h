@@ -3799,7 +3799,8 @@ inline double merge_pass_us(double fixed, long cands) {
 }
 // One stage of the shape that keeps 32 candidates per thread, against two stages at the same split length, 36 shapes of 9472 to
 // 30720 candidates, 16 to 256 rows, per layer: up to 16384 candidates 1.5 - 9 us shorter, around 22000 as long, 2.4 us longer at
-// 30720 (rows 16; with 64 rows and more it is the shorter way throughout).  3 x 28076 positions, 8 kv-heads, G = 4, K3V2, top-k
+// 30720 (rows 16; with 64 rows and more it is the shorter way throughout, which the estimate, by the candidates alone, leaves
+// out).  3 x 28076 positions, 8 kv-heads, G = 4, K3V2, top-k
 // 1024 (12800 candidates, 96 rows) 47.9 -> 42.4 us; 2 x 61876, K4V4, top-k 512 (12288, 64) 45.1 -> 42.6; 1 x 131072, K4V4, top-k
 // 512 (24576, 32) stays at two, 46.1 against 47.2.
 constexpr double kOneStageFixed = 11.6, kOneStagePerCand = 0.00032;
@@ -3853,7 +3854,8 @@ inline double merge_us(int rows, int max_S, int ns, int kc, int top_k) {
 // Measured against the merge launch at the same split length, up to 256 rows: 64-row batches per wavefront 1 / 2 / 4 with
 // sixteen wavefronts 3 us faster / equal / 4 us slower, 1 / 2 / 4 / 8 with eight wavefronts 4 and 2 us faster, 2 and up to 10
 // slower; with more rows the launch takes longer and the workgroups here do not.  (Both ways' sums have moved to the matrix cores
-// since; over 450 random shapes, each timed in every split length, the planner's choice is 1.2 % off the best one's time in the mean.)
+// since; over 450 random shapes, each timed in every split length from a graph, the planner's choice is 2.0 % off the best one's time
+// in the mean.)
 inline double one_split_us(int G, int units, int max_S, int top_k) {
   constexpr double kFixed = 1.4, kPerBatch = 0.25;
   const int nw = G <= 4 ? 16 : 8, per_head = nw >= G ? nw / G : 1, winners = top_k < max_S ? top_k : max_S;
@@ -4208,7 +4210,7 @@ static int fused_run(int scheme, int group_size, const uint16_t* q, const uint8_
   const bool light = (MODE == FS_FULL) && !big && p.mg_parts == 1 && top_k <= MG_LIGHT_TOPK &&
                      (long long)B * H_q > (long long)device_cus() && (long long)p.n_splits * p.Kc <= MG_LIGHT_THREADS * MG_LIGHT_REGK;
   // More rows than CUs that the light shape does not take: half the wavefronts with twice the candidates each.  What every wavefront
-  // does for itself is done half as often, and up to three rows share a CU: per layer, 1024 threads / this, 288 rows of 8 lists
+  // does for itself is done half as often, and two rows share a CU (82 vector registers): per layer, 1024 threads / this, 288 rows of 8 lists
   // (9 x 4096 positions, K3V2, top-k 1024) 36.9 / 31.7 us, 384 (12 x 2500) 35.6 / 30.4, 512 (16 x 4096) 42.1 / 37.2, 1024 (32 x
   // 3000) 61.4 / 49.3, K4V4, 2048 84.0 / 73.5.  With a row per CU the sixteen wavefronts are the shorter way: 256 rows 25.2 / 25.8,
   // 128 (4 x 32768, 256) 33.7 / 34.45.

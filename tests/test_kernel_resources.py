@@ -58,7 +58,7 @@ def test_merge_kernels_keep_their_lane_masks_out_of_vector_registers():
 
 
 def test_light_merge_that_gathers_at_once_runs_four_workgroups_per_compute_unit():
-    """256 threads x 16 candidates, all four roles of a wavefront together: launched for up to four rows per unit."""
+    """256 threads x 16 candidates, the rows of a wavefront's two turns requested together: launched for up to four rows per unit."""
     ks = [k for n, k in _kernels().items() if "fused_merge_kernelI" in n and "ELi256ELi16ELb0ELb0ELi4E" in n]
     assert len(ks) == 6 and min(_workgroups_per_cu(k) for k in ks) == 4
 
@@ -77,3 +77,9 @@ def test_scans_of_up_to_eight_heads_keep_the_value_rows_in_registers():
     few = {n for n in ks if re.search(r"fused_scan_kernelILi0ELi13ELi[12]ELi2ELb[01]ELb0E", n)}
     assert len(ks) > 400 and len(few) == 4
     assert max(ks[n] for n in few) <= 8 and not any(ks[n] for n in ks if n not in few)
+
+
+def test_medium_merge_runs_two_workgroups_per_compute_unit():
+    """512 threads x 16 candidates, for more rows than compute units."""
+    ks = [k for n, k in _kernels().items() if "fused_merge_kernelI" in n and "ELi512ELi16ELb0E" in n]
+    assert len(ks) == 6 and all(_workgroups_per_cu(k) == 2 for k in ks)
